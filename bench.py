@@ -401,9 +401,8 @@ def leg_single(args, wl):
 
     stamps_s = len(wl.stamps) / (ms_per_step * 1e-3)
     waves = one_call and os.environ.get("PAINTY_FUSED_SCHED", "waves") != "streams"
-    tile = 32 if os.environ.get("PAINTY_FUSED_TILE", "16") == "32" else 16
     kernel = {"plain": "k_stamp_main+k_ring_refresh", "persistent": "k_persistent",
-              "fused": ("k_stamp_wave<%d>" if waves else "k_stamp_fused<%d>") % tile,
+              "fused": "k_stamp_wave",
               "chained": "k_stamp_chain<16>"}[args.mode]
     if kern_n:
         avg_us = kern_ms * 1e3 / kern_n

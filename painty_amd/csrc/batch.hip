@@ -114,7 +114,7 @@ __device__ __forceinline__ bool wait_done(unsigned* flag, unsigned* host_err, un
 template <int kWT>
 __global__ __launch_bounds__(kWT* kWT) void k_batch(BArgs A) {
   constexpr int kBT = kWT * kWT;
-  __shared__ int sm[kWT + 2][kWT + 2];
+  __shared__ StampLds<kBT> lds;
   __shared__ int s_item;
   __shared__ int s_ok;
   const int t = threadIdx.x;
@@ -141,9 +141,6 @@ __global__ __launch_bounds__(kWT* kWT) void k_batch(BArgs A) {
       pk[c] = J.paintK[c];
       ps[c] = J.paintS[c];
     }
-    const int side = 2 * J.hr + 1;
-    const int tiles_x = (side + kWT - 1) / kWT;
-    const int ntiles = tiles_x * tiles_x;
     const int64_t m = (int64_t)J.size_map * J.size_map;
     const int gtid = rank * kBT + t;
     const int gthreads = (int)nb * kBT;
@@ -170,15 +167,18 @@ __global__ __launch_bounds__(kWT* kWT) void k_batch(BArgs A) {
         }
       }
       if (J.use_snap) {
-        ring_scan<1>(J.canvas, J.snap, J.dirty, J.fp, g, st.box, pull, gtid, gthreads);
+        ring_scan<kBT>(J.canvas, J.snap, J.dirty, J.fp, g, st.box, pull, rank, (int)nb, lds.ring);
         if (dup && !group_sync(bar, nb, rank, A.host_err)) {
           alive = false;
           break;
         }
       }
-      // ---- visits: 32x32 window tiles, round-robin over the group's blocks
+      // ---- visits: window tiles, round-robin over the group's blocks
+      const TileWin win = tile_window(g, J.fb);
+      const int ntiles = tile_count<kWT>(win);
       for (int tile = rank; tile < ntiles; tile += (int)nb)
-        window_tile<kWT>(T, J.pick.p, J.fp, J.fb, g, st, dup, pull, tile, tiles_x, sm, pk, ps);
+        window_tile<kWT, StampKind<false, true, 2>>(T, J.pick.p, J.fp, J.fb, g, st, dup, pull, tile,
+                                                    win, lds.hand, pk, ps);
       // ---- visits sharing canvas column/row 0, level by level
       for (int L = 0; L < st.dl_nlev; ++L) {
         if (!group_sync(bar, nb, rank, A.host_err)) {
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(kWT* kWT) void k_batch(BArgs A) {
           int64_t ic;
           const int mm2 = stamp_visit(g, v.x, v.y, &ic);
           if (mm2 >= 0 && J.fp[mm2] > 0.0f)
-            cached_visit(T, GlobalPick{J.pick.p, mm2}, J.fp[mm2], ic, false, pk, ps);
+            cached_visit(T, J.pick.p, mm2, J.fp[mm2], ic, false, pk, ps);
         }
       }
       if (!alive) break;

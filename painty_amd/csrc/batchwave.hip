@@ -45,7 +45,7 @@ struct BWJob {
   float* pick[kMaxChunk];
   const float* fp;
   int64_t o_st, o_dl, o_off, o_paint;  // offsets into the plan image
-  int cstride, mstride, dirty_bytes, rows, cols, hr, size_map, tiles_x, ntiles, use_snap;
+  int cstride, mstride, dirty_bytes, rows, cols, hr, size_map, use_snap;
   int fb[4];
   double pickup_rate, dep_rate, cap;
   int pad;
@@ -62,7 +62,7 @@ struct BWJobG {
   gptr<float> pick[kMaxChunk];
   gptr<const float> fp;
   int64_t o_st, o_dl, o_off, o_paint;
-  int cstride, mstride, dirty_bytes, rows, cols, hr, size_map, tiles_x, ntiles, use_snap;
+  int cstride, mstride, dirty_bytes, rows, cols, hr, size_map, use_snap;
   int fb[4];
   double pickup_rate, dep_rate, cap;
   int pad;
@@ -74,13 +74,6 @@ static_assert(sizeof(BWJobG) == sizeof(BWJob) && offsetof(BWJobG, fp) == offseto
                   offsetof(BWJobG, tmap) == offsetof(BWJob, tmap),
               "BWJobG mirrors BWJob");
 
-// 4-pixel groups per ring-scan thread in the batch's waves: twice the
-// single-canvas count, so half the ring blocks.  The batch is bound by how
-// many workgroups it runs, not by its chain of launches, and measured 2%
-// faster with 4 (1 and 2 were slower); the single canvas, bound by its
-// chain, is faster with 2.
-constexpr int kBatchRingGroups = 4;
-
 struct BWSlot {
   int job, k, kind, start, nblk, rb, chain, pad;
   // image offsets of the phase's stamp descriptor and paint: with them the
@@ -89,21 +82,28 @@ struct BWSlot {
   int64_t o_stamp, o_paint;
 };
 
+// The stamps of most waves: no clock, no stamp on canvas column/row 0, the
+// snapshot on, and no phase but stamps and map clears.  Waves with anything
+// else run the general kernel.
+using PlainStamps = StampKind<false, false, 1>;
+using AnyStamps = StampKind<true, true, 2>;
+
 // One wave: the group table gives the slot of every 8 blocks (slots start on
 // multiples of 8 blocks).
+template <class F, bool kStream>
 __global__ __launch_bounds__(kWT2, kWaveOccupancy) void k_batch_wave(const char* base, const BWJobG* jobs,
                                                      const BWSlot* slots, const int* grp) {
-  __shared__ int sm[kWT + 2][kWT + 2];
-  const BWSlot d = slots[grp[blockIdx.x >> 3]];
+  __shared__ StampLds<kWT2> lds;
+  const BWSlot d = load_const<BWSlot>(slots + load_const<int>(grp + (blockIdx.x >> 3)));
   const int b = (int)blockIdx.x - d.start;
   if (b >= d.nblk) return;
-  const BWJobG& J = jobs[d.job];
+  const BWJobG J = load_const<BWJobG>(jobs + d.job);
   SSlot S;
   S.st = reinterpret_cast<const PStamp*>(base + d.o_stamp);
   S.canvas = (float*)J.canvas;
   S.snap = (float*)J.snap;
   S.dirty = (uint8_t*)J.dirty;
-  S.pick = (float*)J.pick[d.chain];
+  S.pick = (float*)load_const<gptr<float>>(&jobs[d.job].pick[d.chain]);
   S.pick_dst = (float*)J.pick[0];  // kSCopyPick: this chain's map -> the brush's own
   S.fp = (const float*)J.fp;
   S.dl = reinterpret_cast<const int2*>(base + J.o_dl);
@@ -118,19 +118,20 @@ __global__ __launch_bounds__(kWT2, kWaveOccupancy) void k_batch_wave(const char*
   S.kind = d.kind;
   S.start = d.start;
   S.nblk = d.nblk;
-  S.ntiles = J.ntiles;
   S.rb = d.rb;
   S.hr = J.hr;
   S.size_map = J.size_map;
-  S.tiles_x = J.tiles_x;
 #pragma unroll
   for (int c = 0; c < 4; ++c) S.fb[c] = J.fb[c];
-  const float* paint = reinterpret_cast<const float*>(base + d.o_paint);
+  struct Paint {
+    float v[6];
+  };
+  const Paint paint = load_const<Paint>(base + d.o_paint);
   const bool stamp_kind = d.kind == kSStamp;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    S.pk[c] = stamp_kind ? paint[c] : 0.0f;
-    S.ps[c] = stamp_kind ? paint[3 + c] : 0.0f;
+    S.pk[c] = stamp_kind ? paint.v[c] : 0.0f;
+    S.ps[c] = stamp_kind ? paint.v[3 + c] : 0.0f;
   }
   S.pickup_rate = J.pickup_rate;
   S.dep_rate = J.dep_rate;
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(kWT2, kWaveOccupancy) void k_batch_wave(const char*
   S.dry_ms = J.dry_ms;
   S.part = 0;  // streaming phases run whole
   S.nparts = 1;
-  run_wave_slot<kBatchRingGroups>(S, b, sm);
+  run_wave_slot<F, kStream>(S, b, lds);
 }
 
 struct Phase {
@@ -160,7 +161,7 @@ struct JobPlan {
   std::vector<std::vector<Phase>> ph;
   std::vector<int> prev_on_chain;
   std::vector<float> paint;
-  std::vector<int> rb;
+  std::vector<int> rb, ntiles;  // per stamp: ring-scan blocks, window tiles
   int chains = 1;       // chains used
   int perm[kMaxChunk];  // chain -> map slot in BWJob.pick (0: the brush's own map)
   bool copy_back = false;
@@ -172,6 +173,13 @@ struct JobPlan {
   StampNeeds needs;
 };
 
+// The map cells a job's stamps run over.
+FpBox job_cells(const pnt_batch_job& job) {
+  const int* f = job.brush->fbox;
+  return cell_domain(FpBox{f[0], f[1], f[2], f[3]}, job.brush->size_map,
+                     job.canvas->clock != PNT_CLOCK_OFF && job.canvas->tmap);
+}
+
 void plan_job(const pnt_batch_job& job, int chunk, JobPlan& P) {
   pnt_brush b = job.brush;
   pnt_canvas cv = job.canvas;
@@ -181,11 +189,15 @@ void plan_job(const pnt_batch_job& job, int chunk, JobPlan& P) {
   P.U = n ? plan_units(job.stamps, P.st.data(), clear.data(), n, chunk) : std::vector<Unit>{};
   P.ph.assign(P.U.size(), {});
   P.rb.assign((size_t)n, 0);
+  P.ntiles.assign((size_t)n, 1);
+  const FpBox dom = job_cells(job);
   for (size_t i = 0; i < P.U.size(); ++i)
     for (int64_t k = P.U[i].s0; k < P.U[i].s1; ++k) {
       if (job.stamps[k].flags & PNT_STAMP_DIP) P.ph[i].push_back(Phase{k, kSClear});
       const PStamp& p = P.st[(size_t)k];
-      P.rb[(size_t)k] = b->use_snap ? ring_blocks_for(p.box, kWT2, kBatchRingGroups) : 0;
+      P.rb[(size_t)k] = b->use_snap ? ring_blocks_for(p.box, kWT2) : 0;
+      P.ntiles[(size_t)k] = tile_count<kWT>(
+          tile_window(stamp_geom(p, b->size_map, cv->rows, cv->cols), dom));
       P.ph[i].push_back(Phase{k, kSStamp});
     }
   P.prev_on_chain.assign(P.U.size(), -1);
@@ -292,11 +304,13 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
   std::vector<int> grp;
   std::vector<int64_t> ws, wg;
   std::vector<int> wb;
+  std::vector<char> wp;  // the wave's phases are plain stamps and map clears
   std::vector<std::pair<int, int>> took;  // (job, unit or -1 dry / -2 copy / -3 compose)
   std::vector<int> jfirst((size_t)n, -1), jlast((size_t)n, -1);
   for (;;) {
     const int64_t s0 = (int64_t)slots.size(), g0 = (int64_t)grp.size();
     int start = 0;
+    bool plain = true;
     took.clear();
     auto add = [&](int j, int64_t k, int kind, int nblk, int rb, int chain, int tag) {
       BWSlot d{j, (int)std::max<int64_t>(k, 0), kind, start, std::max(nblk, 1), rb, chain, 0, 0, 0};
@@ -305,6 +319,7 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
       slots.push_back(d);
       start += span;
       took.push_back({j, tag});
+      plain &= kind == kSStamp || kind == kSClear;
     };
     for (int j = 0; j < n; ++j) {
       JobPlan& J = P[(size_t)j];
@@ -344,14 +359,15 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
               }
             if (!ok) continue;
             const int rb = J.rb[(size_t)f.k];
-            const int ntl = ((2 * ((b->size_map - 1) / 2) + 1 + kWT - 1) / kWT);
-            const int ntiles = ntl * ntl;
+            const int ntiles = J.ntiles[(size_t)f.k];
             int nblk = 1;
             switch (f.kind) {
               case kSClear:
                 nblk = (int)std::min<int64_t>(64, (7 * b->mstride + 4 * kWT2 - 1) / (4 * kWT2));
                 break;
               case kSStamp:  // + the shared-pixel levels' block of a dup stamp
+                plain &= b->use_snap && !(J.st[(size_t)f.k].flags & (kStDupX | kStDupY)) &&
+                         job.canvas->clock == PNT_CLOCK_OFF;
                 nblk = ntiles + rb + (dup_levels(J.st[(size_t)f.k]) ? 1 : 0);
                 break;
               default: nblk = 1; break;
@@ -376,6 +392,7 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
     ws.push_back(s0);
     wg.push_back(g0);
     wb.push_back(start);
+    wp.push_back(plain ? 1 : 0);
     for (const auto& t : took) {
       JobPlan& J = P[(size_t)t.first];
       if (jfirst[(size_t)t.first] < 0) jfirst[(size_t)t.first] = (int)ws.size() - 1;
@@ -457,10 +474,12 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
     d.cols = cv->cols;
     d.hr = (b->size_map - 1) / 2;
     d.size_map = b->size_map;
-    d.tiles_x = (2 * d.hr + 1 + kWT - 1) / kWT;
-    d.ntiles = d.tiles_x * d.tiles_x;
+    const FpBox dom = job_cells(job);
     d.use_snap = b->use_snap ? 1 : 0;
-    for (int c = 0; c < 4; ++c) d.fb[c] = b->fbox[c];
+    d.fb[0] = dom.x0;
+    d.fb[1] = dom.y0;
+    d.fb[2] = dom.x1;
+    d.fb[3] = dom.y1;
     d.pickup_rate = b->pickup_rate;
     d.dep_rate = b->dep_rate;
     d.cap = b->cap;
@@ -485,6 +504,7 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
     W.wave_grp.push_back(o_grp + wg[w] * (int64_t)sizeof(int));
   }
   W.wave_blocks = wb;
+  W.wave_plain = std::move(wp);
   W.job_first = std::move(jfirst);
   W.job_last = std::move(jlast);
   return W;
@@ -497,7 +517,8 @@ void enqueue_waves(const BWPlan& W, const char* stage, char* dev, hipStream_t s,
   if (ev) PNT_HIP_CHECK(hipEventRecord(ev[0], s));
   const BWJobG* jobs = reinterpret_cast<const BWJobG*>(dev + W.o_jobs);
   for (size_t w = 0; w < W.wave_blocks.size(); ++w) {
-    k_batch_wave<<<(unsigned)W.wave_blocks[w], kWT2, 0, s>>>(
+    const auto kernel = W.wave_plain[w] ? k_batch_wave<PlainStamps, false> : k_batch_wave<AnyStamps, true>;
+    kernel<<<(unsigned)W.wave_blocks[w], kWT2, 0, s>>>(
         dev, jobs, reinterpret_cast<const BWSlot*>(dev + W.wave_slots[w]),
         reinterpret_cast<const int*>(dev + W.wave_grp[w]));
     PNT_HIP_CHECK(hipGetLastError());

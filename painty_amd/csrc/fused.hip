@@ -2,20 +2,30 @@
 // launch per imprint (FootprintBrush::imprint, renderer/FootprintBrush.hxx:
 // 73-143) in which the snapshot refresh and the visits run side by side.
 //
-// Blocks [0, ntiles) take one kT x kT tile of the window each (window_tile,
+// Blocks [0, ntiles) take one 16 x 16 tile of the window each (window_tile,
 // stampcore.hpp); the blocks after them scan the dirty bytes of the
 // snapshot ring (ring_scan).  The two sets touch disjoint pixels: the scan
 // skips the window interior and the border pixels that a visit refreshes
 // itself (a border visit reads the canvas value the refresh would have
 // copied and writes the snapshot back), so they need no ordering.  A stamp
 // that straddles canvas column/row 0 with a fractional centre visits some
-// pixels twice; it runs as ring | window | shared-pixel levels, three
-// launches in stream order.
+// pixels twice; one more block runs those by level (level_visits).
 //
 // Between launches the stream orders everything: no grid barrier, no
 // cooperative launch.  Consecutive stamps of a stroke overlap almost
 // entirely, and tile t of every launch runs on the same XCD
 // (tile_of_block), so a tile's pixels and map cells stay in that XCD's L2.
+//
+// Bound: a launch lasts as long as its slowest block, and a block is a chain
+// of latencies -- kernel arguments, its map cells, one round trip of visit
+// loads, the visit arithmetic, the stores -- of which the bytes moved are a
+// quarter.  What shortens the chain is therefore what was done: arguments in
+// one round of scalar loads (a slot per grid row), kernels without the code
+// a launch does not need, map cells without a halo or a division, the second
+// visit of a shared cell on its own thread, no tiles outside the rotated
+// footprint.  Per wave on 200 stamps of radius 32 on 1024^2: 13,500 cycles
+// before, 8,900 after; 4096^2, 2000 stamps: 743 launches of 13.9 us before,
+// 11.5 after.
 #include <algorithm>
 #include <atomic>
 #include <climits>
@@ -36,79 +46,164 @@ namespace pnt {
 
 namespace {
 
-struct FArgs {
-  const PStamp* st;
-  Layer7 canvas, snap;  // snap == canvas planes when the snapshot is off
-  Plane7 pick;
-  const float* fp;
-  FpBox fb;  // nonzero footprint cells
+constexpr int kT = 16;       // window tile side
+constexpr int kT2 = kT * kT;  // threads per block
+
+// What every stamp of a launch shares.
+struct StampShared {
+  float* canvas;  // canvas block and snapshot (canvas when it is off), plane strides
+  float* snap;
+  int64_t cs, ss;
   uint8_t* dirty;
   const int2* dl;
   const int* dl_off;
-  int use_snap, rows, cols, hr, size_map, tiles_x, ntiles;
   double pickup_rate, dep_rate, cap;
-  float pk[3], ps[3];  // brush paint (the last dip)
-  DryClock clk;        // the canvas' drying clock; clk.tmap == nullptr: none
+  int rows, cols, use_snap, pad;
+  int64_t* tmap;    // the canvas' drying clock (nullptr: none)
+  int64_t dry_ms;
 };
 
-// The clock of stamp `st` (its own time point); tmap == nullptr without one.
-__device__ __forceinline__ DryClock stamp_clock(const DryClock& base, const PStamp& st) {
-  DryClock c = base;
-  c.now_us = st.now_us;
-  return c;
+StampShared stamp_shared(pnt_brush_s* b, pnt_canvas_s* cv, const int2* dl, const int* dl_off) {
+  StampShared A{};
+  A.canvas = cv->base;
+  A.cs = cv->stride;
+  A.snap = b->use_snap ? b->snap : cv->base;
+  A.ss = b->use_snap ? b->snap_stride : cv->stride;
+  A.dirty = b->dirty;
+  A.dl = dl;
+  A.dl_off = dl_off;
+  A.pickup_rate = b->pickup_rate;
+  A.dep_rate = b->dep_rate;
+  A.cap = b->cap;
+  A.rows = cv->rows;
+  A.cols = cv->cols;
+  A.use_snap = b->use_snap ? 1 : 0;
+  // checkDry on every visited pixel when the canvas has a drying clock; each
+  // stamp carries its own time point (PStamp::now_us)
+  A.tmap = cv->clock != PNT_CLOCK_OFF ? cv->tmap : nullptr;
+  A.dry_ms = cv->drying_ms;
+  return A;
 }
 
-__device__ __forceinline__ StampGeom geom_of(const FArgs& A, const PStamp& st) {
-  StampGeom g;
-  g.cx = st.cx;
-  g.cy = st.cy;
-  g.c = st.c;
-  g.s = st.s;
-  g.hr = A.hr;
-  g.size_map = A.size_map;
-  g.rows = A.rows;
-  g.cols = A.cols;
-  return g;
-}
+// One phase of a launch: a stamp, or the pickup-map clear of a dip or a
+// geometry change.
+enum : int { kPhClear = 0, kPhStamp = 1 };
+struct WSlot {
+  int nblk;    // blocks with work (the grid is as wide as the largest slot)
+  int kind;    // kPh*
+  int ntiles, rb;
+  int size_map, pad;
+  int64_t mstride;
+  const float* fp;
+  float* pick;         // the unit's pickup map (7 planes of mstride)
+  FpBox dom;           // the cells its visits run over (cell_domain)
+  TileWin win;
+  float pk[3], ps[3];  // the brush paint of this stamp
+  PStamp stamp;        // its plan, passed with the launch: blocks start without a
+                       // dependent load of it
+};
 
-// Stamp j: window tiles on blocks [0, ntiles), ring scan on the next
-// ring_blocks blocks, and for a stamp on a duplicated canvas column/row 0
-// its shared-pixel visits by level on one more block.  Visits on the window
-// border refresh their own snapshot pixels (the ring scan leaves them).
-template <int kT>
-__global__ __launch_bounds__(kT* kT) void k_stamp_fused(FArgs A, int j, int ring_blocks) {
-  __shared__ int sm[kT + 2][kT + 2];
-  const PStamp& st = A.st[j];
-  const StampGeom g = geom_of(A, st);
-  const bool dup = (st.flags & (kStDupX | kStDupY)) != 0;
-  const bool pull = A.use_snap != 0;
-  const DryClock clk = stamp_clock(A.clk, st);
-  const VisitTarget T{&A.canvas, &A.snap, A.dirty, A.use_snap, A.pickup_rate, A.dep_rate, A.cap};
+template <int kSlots>
+struct WArgs {
+  StampShared sh;
+  WSlot slot[kSlots];
+};
+constexpr int kWaveSlots = 8;
+static_assert(sizeof(WArgs<kWaveSlots>) <= 4000, "wave arguments must fit the kernel argument segment");
+
+// Slot y of the grid's rows, blocks along x: a block knows its slot without
+// looking through the others' starts, so its arguments arrive in one round of
+// scalar loads.  The rows are as wide as the largest slot, rounded up to 8
+// (tiles keep their XCD); blocks past a slot's own leave at once.
+template <class F, int kSlots>
+__global__ __launch_bounds__(kT2, F::clock || F::dup ? 4 : 5) void k_stamp_wave(WArgs<kSlots> A) {
+  __shared__ StampLds<kT2> lds;
+  const WSlot& S = A.slot[kSlots > 1 ? blockIdx.y : 0];
   const int b = (int)blockIdx.x;
-  if (b < A.ntiles) {
-    window_tile<kT>(T, A.pick.p, A.fp, A.fb, g, st, dup, pull, tile_of_block(b, A.ntiles),
-                    A.tiles_x, sm, A.pk, A.ps, clk);
-  } else if (b < A.ntiles + ring_blocks) {
-    ring_scan<kRingGroups>(A.canvas, A.snap, A.dirty, A.fp, g, st.box, pull,
-                 (b - A.ntiles) * kT * kT + (int)threadIdx.x, ring_blocks * kT * kT,
-                 clk.tmap != nullptr);
-  } else if (dup) {
-    level_visits<kT * kT>(T, A.pick.p, A.fp, g, st, A.dl, A.dl_off, A.pk, A.ps, clk, pull);
+  if (b >= S.nblk) return;
+  if (S.kind == kPhClear) {  // dip() / setRadius: a clean pickup map
+    const int64_t total = 7 * S.mstride;
+    for (int64_t i = (int64_t)b * kT2 + threadIdx.x; i < total; i += (int64_t)S.nblk * kT2)
+      S.pick[i] = 0.0f;
+    return;
   }
+  const StampShared& H = A.sh;
+  const PStamp& st = S.stamp;
+  const StampGeom g = stamp_geom(st, S.size_map, H.rows, H.cols);
+  const Layer7 canvas = layer_at(H.canvas, H.cs), snap = layer_at(H.snap, H.ss);
+  const VisitTarget T{&canvas, &snap, H.dirty, H.use_snap, H.pickup_rate, H.dep_rate, H.cap};
+  float* pick[7];
+#pragma unroll
+  for (int c = 0; c < 7; ++c) pick[c] = S.pick + c * S.mstride;
+  float* R0 = H.canvas + 8 * H.cs;
+  const DryClock clk{F::clock ? H.tmap : nullptr, st.now_us, H.dry_ms,
+                     Rgb3{{R0, R0 + H.cs, R0 + 2 * H.cs}}, H.canvas + 11 * H.cs};
+  stamp_block<F>(T, pick, S.fp, S.dom, g, st, S.win, S.ntiles, S.rb, b, lds, H.dl,
+                              H.dl_off, S.pk, S.ps, clk);
+}
+
+// Launches A's first `n` slots on q with the kernel for what they need.
+template <int kSlots>
+void launch_slots(const WArgs<kSlots>& A, int n, hipStream_t q) {
+  int widest = 1;
+  bool dup = false;
+  for (int i = 0; i < n; ++i) {
+    widest = std::max(widest, A.slot[i].nblk);
+    dup |= A.slot[i].kind == kPhStamp && (A.slot[i].stamp.flags & (kStDupX | kStDupY));
+  }
+  const bool snap = A.sh.use_snap != 0;
+  void (*kernel)(WArgs<kSlots>) =
+      A.sh.tmap ? (snap ? k_stamp_wave<StampKind<true, true, 1>, kSlots>
+                        : k_stamp_wave<StampKind<true, true, 0>, kSlots>)
+      : dup     ? (snap ? k_stamp_wave<StampKind<false, true, 1>, kSlots>
+                        : k_stamp_wave<StampKind<false, true, 0>, kSlots>)
+                : (snap ? k_stamp_wave<StampKind<false, false, 1>, kSlots>
+                        : k_stamp_wave<StampKind<false, false, 0>, kSlots>);
+  kernel<<<dim3((unsigned)round_up(widest, 8), (unsigned)n), kT2, 0, q>>>(A);
+  PNT_HIP_CHECK(hipGetLastError());
+}
+
+// The launch of stamp st as one slot.
+WSlot stamp_slot(const StampShared& H, const PStamp& st, const float* fp, const FpBox& dom,
+                 int size_map, float* pick, int64_t mstride, const float* pk, const float* ps) {
+  WSlot S{};
+  S.kind = kPhStamp;
+  S.stamp = st;
+  S.size_map = size_map;
+  S.mstride = mstride;
+  S.fp = fp;
+  S.pick = pick;
+  S.dom = dom;
+  S.win = tile_window(stamp_geom(st, size_map, H.rows, H.cols), dom);
+  S.ntiles = tile_count<kT>(S.win);
+  S.rb = H.use_snap ? ring_blocks_for(st.box, kT2) : 0;
+  S.nblk = S.ntiles + S.rb + (dup_levels(st) ? 1 : 0);  // + its shared-pixel levels
+  for (int c = 0; c < 3; ++c) {
+    S.pk[c] = pk[c];
+    S.ps[c] = ps[c];
+  }
+  return S;
+}
+
+WSlot clear_slot(float* pick, int64_t mstride) {
+  WSlot S{};
+  S.kind = kPhClear;
+  S.pick = pick;
+  S.mstride = mstride;
+  S.nblk = (int)std::min<int64_t>(64, (7 * mstride + 4 * kT2 - 1) / (4 * kT2));
+  return S;
 }
 
 }  // namespace
 
-// 4-pixel groups of box b, and the blocks that scan them (each thread
-// takes kRingGroups groups per pass).
-int ring_blocks_for(const RingBox& b, int threads, int groups) {
+// Blocks that scan the ring of box b: a thread takes one unit of pixels.
+int ring_blocks_for(const RingBox& b, int threads) {
   if (b.a_x1 < b.a_x0 || b.a_y1 < b.a_y0) return 0;
   const int64_t span = b.a_x1 - b.a_x0 + 1;
-  const int64_t ngroups = ((span + 3) / 4 + 1) * (int64_t)(b.a_y1 - b.a_y0 + 1);
-  const int64_t blocks = (ngroups + groups * threads - 1) / (groups * threads);
-  return (int)std::min<int64_t>(std::max<int64_t>(blocks, 1), 1024);
+  const int64_t units =
+      ((span + kRingUnit - 1) / kRingUnit + 1) * (int64_t)(b.a_y1 - b.a_y0 + 1);
+  return (int)std::min<int64_t>((units + threads - 1) / threads, 1024);
 }
-
 
 // ---------------------------------------------------- concurrent strokes --
 // A dip cleans the pickup map (FootprintBrush.hxx:150-160), so the stamps
@@ -295,84 +390,6 @@ int fused_chains(int want) {
 // one wave touch disjoint pixels and their own pickup maps, exactly as on
 // concurrent streams, and the stream orders the waves: no events, and no
 // limit from the hardware queues.
-constexpr int kWaveSlots = 8;
-enum : int { kPhClear = 0, kPhStamp = 1 };
-
-struct WSlot {
-  int j;       // stamp index (not used by kPhClear)
-  int kind;    // kPh*
-  int start;   // first block of the slot (a multiple of 8: tiles keep their XCD)
-  int nblk;    // blocks with work (the slot's range may be padded past them)
-  int ntiles, rb;
-  int hr, size_map, tiles_x;
-  const float* fp;
-  FpBox fb;
-  float* pick;         // the unit's pickup map (7 planes of mstride)
-  int64_t mstride;
-  float pk[3], ps[3];  // the brush paint of this stamp
-  PStamp stamp;        // the stamp's plan, passed with the launch: its blocks start
-                       // without a dependent load of it
-};
-
-struct WArgs {
-  const PStamp* st;  // (the slots carry their stamps' plans; this is the whole list)
-  Layer7 canvas, snap;
-  uint8_t* dirty;
-  const int2* dl;
-  const int* dl_off;
-  int use_snap, rows, cols;
-  double pickup_rate, dep_rate, cap;
-  DryClock clk;  // the canvas' drying clock; clk.tmap == nullptr: none
-  int nslots;
-  WSlot slot[kWaveSlots];
-};
-static_assert(sizeof(WArgs) <= 4000, "wave arguments must fit the kernel argument segment");
-
-
-// 16x16 tiles: five workgroups per CU (at most 102 VGPRs; it needs 102
-// without the bound and spills nothing under it).
-template <int kT>
-__global__ __launch_bounds__(kT* kT, kT == 16 ? 5 : 1) void k_stamp_wave(WArgs A) {
-  __shared__ int sm[kT + 2][kT + 2];
-  int si = 0;
-  while (si + 1 < A.nslots && (int)blockIdx.x >= A.slot[si + 1].start) ++si;
-  const WSlot& S = A.slot[si];
-  const int b = (int)blockIdx.x - S.start;
-  if (b >= S.nblk) return;
-  if (S.kind == kPhClear) {  // dip() / setRadius: a clean pickup map
-    const int64_t total = 7 * S.mstride;
-    for (int64_t i = (int64_t)b * kT * kT + threadIdx.x; i < total; i += (int64_t)S.nblk * kT * kT)
-      S.pick[i] = 0.0f;
-    return;
-  }
-  const PStamp& st = S.stamp;
-  StampGeom g;
-  g.cx = st.cx;
-  g.cy = st.cy;
-  g.c = st.c;
-  g.s = st.s;
-  g.hr = S.hr;
-  g.size_map = S.size_map;
-  g.rows = A.rows;
-  g.cols = A.cols;
-  const bool dup = (st.flags & (kStDupX | kStDupY)) != 0;
-  const bool pull = A.use_snap != 0;  // border visits refresh their own snapshot pixels
-  const VisitTarget T{&A.canvas, &A.snap, A.dirty, A.use_snap, A.pickup_rate, A.dep_rate, A.cap};
-  float* pick[7];
-#pragma unroll
-  for (int c = 0; c < 7; ++c) pick[c] = S.pick + c * S.mstride;
-  const DryClock clk = stamp_clock(A.clk, st);
-  if (b < S.ntiles) {
-    window_tile<kT>(T, pick, S.fp, S.fb, g, st, dup, pull, tile_of_block(b, S.ntiles), S.tiles_x,
-                    sm, S.pk, S.ps, clk);
-  } else if (b < S.ntiles + S.rb) {
-    ring_scan<kRingGroups>(A.canvas, A.snap, A.dirty, S.fp, g, st.box, pull, (b - S.ntiles) * kT * kT +
-                 (int)threadIdx.x, S.rb * kT * kT, clk.tmap != nullptr);
-  } else if (dup) {  // the shared-pixel visits, beside the tiles
-    level_visits<kT * kT>(T, pick, S.fp, g, st, A.dl, A.dl_off, S.pk, S.ps, clk, pull);
-  }
-}
-
 // One brush geometry of a list: its padded footprint on the device, its side
 // and radius, and (for the brush's state after the list) the unpadded
 // footprint it came from; core == nullptr: the brush's current geometry.
@@ -387,78 +404,48 @@ struct ListGeo {
 
 // Stamps [0, n) of a list on the fused path.  Stamp k uses geometry
 // geo[k]; clear[k] cleans the pickup map before it (a geometry change).
-template <int kT>
 void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n,
                     const PlanDev& D, const std::vector<ListGeo>& geos, const std::vector<int>& geo,
                     const std::vector<uint8_t>& clear, int want_chains) {
   hipStream_t s = b->ctx->stream;
   b->last_launches = 0;
   if (b->ktimer) b->ktimer->used = 0;
-  FArgs A0;
-  A0.st = D.st;
-  A0.canvas = cv->layer();
-  A0.snap = b->use_snap ? b->snap_planes() : cv->layer();
-  A0.dirty = b->dirty;
-  A0.dl = D.dl;
-  A0.dl_off = D.dl_off;
-  A0.use_snap = b->use_snap ? 1 : 0;
-  A0.rows = cv->rows;
-  A0.cols = cv->cols;
-  A0.pickup_rate = b->pickup_rate;
-  A0.dep_rate = b->dep_rate;
-  A0.cap = b->cap;
-  // Canvas::checkDry on every visited pixel when the canvas has a drying
-  // clock; each stamp carries its own time point (PStamp::now_us)
-  A0.clk = cv->clock != PNT_CLOCK_OFF && cv->tmap
-               ? DryClock{cv->tmap, 0, cv->drying_ms, cv->R0(), cv->h()}
-               : DryClock{};
-  std::vector<FArgs> GA(geos.size(), A0);
+  const StampShared H = stamp_shared(b, cv, D.dl, D.dl_off);
+  std::vector<FpBox> gdom(geos.size());
   std::vector<int64_t> gstride(geos.size());
   int64_t max_stride = 0;
   for (size_t i = 0; i < geos.size(); ++i) {
-    FArgs& a = GA[i];
-    a.fp = geos[i].fp;
-    a.fb = geos[i].fb;
-    a.size_map = geos[i].size_map;
-    a.hr = (a.size_map - 1) / 2;
-    const int side = 2 * a.hr + 1;
-    a.tiles_x = (side + kT - 1) / kT;
-    a.ntiles = a.tiles_x * a.tiles_x;
-    gstride[i] = round_up((int64_t)a.size_map * a.size_map, 64);
+    const int sm = geos[i].size_map;
+    gdom[i] = cell_domain(geos[i].fb, sm, H.tmap != nullptr);
+    gstride[i] = round_up((int64_t)sm * sm, 64);
     max_stride = std::max(max_stride, gstride[i]);
   }
+  const auto slot_of = [&](int64_t k, float* pick, const float* pk, const float* ps) {
+    const size_t i = (size_t)geo[(size_t)k];
+    return stamp_slot(H, D.host[k], geos[i].fp, gdom[i], geos[i].size_map, pick, gstride[i], pk, ps);
+  };
 
   // one stamp on stream `q` with pickup map `pick` (7 planes of its stride)
   auto launch_stamp = [&](int64_t k, hipStream_t q, float* pick) {
-    FArgs a = GA[(size_t)geo[k]];
-    const int64_t ms = gstride[(size_t)geo[k]];
-    for (int c = 0; c < 7; ++c) a.pick.p[c] = pick + c * ms;
     if (clear[k] || (st[k].flags & PNT_STAMP_DIP))  // setRadius / dip(): a clean pickup map
-      launch_fill(pick, 7 * ms, 0.0f, q);
+      launch_fill(pick, 7 * gstride[(size_t)geo[(size_t)k]], 0.0f, q);
     if (st[k].flags & PNT_STAMP_DIP)
       for (int c = 0; c < 3; ++c) {
         b->paintK[c] = st[k].K[c];
         b->paintS[c] = st[k].S[c];
       }
-    for (int c = 0; c < 3; ++c) {
-      a.pk[c] = b->paintK[c];
-      a.ps[c] = b->paintS[c];
-    }
-    const PStamp& p = D.host[k];
-    const int rb = a.use_snap ? ring_blocks_for(p.box, kT * kT) : 0;
-    const int jk = (int)k;
+    const WArgs<1> A{H, {slot_of(k, pick, b->paintK, b->paintS)}};
     if (q == s) ktimer_mark(b, q);
-    k_stamp_fused<kT><<<a.ntiles + rb + (dup_levels(p) ? 1 : 0), kT * kT, 0, q>>>(a, jk, rb);
+    launch_slots(A, 1, q);
     if (q == s) ktimer_mark(b, q);
     b->last_launches += 1;
-    PNT_HIP_CHECK(hipGetLastError());
   };
   auto dry = [&](hipStream_t q) {
     if (b->use_snap)
       launch_dry_dirty(cv->n, cv->layer(), cv->R0(), cv->h(), b->dirty, q);
     else
       launch_dry(cv->n, cv->layer(), cv->R0(), cv->h(), q);
-    if (A0.clk.tmap)  // dryCanvas stamps every pixel's time (Canvas.hxx:105-119)
+    if (H.tmap)  // dryCanvas stamps every pixel's time (Canvas.hxx:105-119)
       launch_fill_i64(cv->tmap, cv->n, canvas_now_us(cv), q);
   };
   // the brush ends with the geometry of the list's last stamp
@@ -469,7 +456,6 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
 
   // ---- waves: the units' phases, scheduled on s ----------------------------
   auto run_waves = [&](const std::vector<Unit>& U, int used, float* const* pick) {
-    const int T2 = kT * kT;
     struct Ph {
       int64_t k;
       int kind;
@@ -492,20 +478,8 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
         }
       std::memcpy(&paint[6 * (size_t)k], cur, sizeof cur);
     }
-    WArgs W{};
-    W.st = A0.st;
-    W.canvas = A0.canvas;
-    W.snap = A0.snap;
-    W.dirty = A0.dirty;
-    W.dl = A0.dl;
-    W.dl_off = A0.dl_off;
-    W.use_snap = A0.use_snap;
-    W.rows = A0.rows;
-    W.cols = A0.cols;
-    W.pickup_rate = A0.pickup_rate;
-    W.dep_rate = A0.dep_rate;
-    W.cap = A0.cap;
-    W.clk = A0.clk;
+    WArgs<kWaveSlots> W{};
+    W.sh = H;
     std::vector<size_t> next(U.size(), 0);
     std::vector<char> done(U.size(), 0);
     std::vector<int64_t> sdone(U.size(), 0);  // stamps of each unit issued
@@ -537,39 +511,17 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
           if (ok) ready.push_back((int)i);
         }
         if (ready.empty()) break;  // the phase is done
-        W.nslots = (int)ready.size();
-        int start = 0;
-        for (int q = 0; q < W.nslots; ++q) {
+        const int nslots = (int)ready.size();
+        for (int q = 0; q < nslots; ++q) {
           const int i = ready[(size_t)q];
           const Ph& f = ph[(size_t)i][next[(size_t)i]];
-          WSlot& S = W.slot[q];
-          const FArgs& a = GA[(size_t)geo[(size_t)f.k]];
-          S.j = (int)f.k;
-          S.stamp = D.host[f.k];
-          S.kind = f.kind;
-          S.start = start;
-          S.ntiles = a.ntiles;
-          S.rb = a.use_snap ? ring_blocks_for(D.host[f.k].box, T2) : 0;
-          S.hr = a.hr;
-          S.size_map = a.size_map;
-          S.tiles_x = a.tiles_x;
-          S.fp = a.fp;
-          S.fb = a.fb;
-          S.mstride = gstride[(size_t)geo[(size_t)f.k]];
-          S.pick = pick[U[(size_t)i].chain];
-          for (int c = 0; c < 3; ++c) {
-            S.pk[c] = paint[6 * (size_t)f.k + c];
-            S.ps[c] = paint[6 * (size_t)f.k + 3 + c];
-          }
-          if (f.kind == kPhClear)
-            S.nblk = (int)std::min<int64_t>(64, (7 * S.mstride + 4 * T2 - 1) / (4 * T2));
-          else  // + the shared-pixel levels' block of a dup stamp
-            S.nblk = S.ntiles + S.rb + (dup_levels(D.host[f.k]) ? 1 : 0);
-          start += (std::max(S.nblk, 1) + 7) / 8 * 8;
+          float* map = pick[U[(size_t)i].chain];
+          const float* p = &paint[6 * (size_t)f.k];
+          W.slot[q] = f.kind == kPhClear ? clear_slot(map, gstride[(size_t)geo[(size_t)f.k]])
+                                         : slot_of(f.k, map, p, p + 3);
         }
         ktimer_mark(b, s);
-        k_stamp_wave<kT><<<(unsigned)start, T2, 0, s>>>(W);
-        PNT_HIP_CHECK(hipGetLastError());
+        launch_slots(W, nslots, s);
         ktimer_mark(b, s);
         b->last_launches += 1;
         for (int i : ready) {
@@ -686,19 +638,17 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
   }
 }
 
-template <int kT>
 void run_fused_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains) {
   const PlanDev D = upload_plan(b, cv, st, n);
   const std::vector<ListGeo> geos{ListGeo{b->fp, b->size_map, b->radius, nullptr, b->width,
                                           FpBox{b->fbox[0], b->fbox[1], b->fbox[2], b->fbox[3]}}};
-  run_fused_list<kT>(b, cv, st, n, D, geos, std::vector<int>((size_t)n, 0),
+  run_fused_list(b, cv, st, n, D, geos, std::vector<int>((size_t)n, 0),
                      std::vector<uint8_t>((size_t)n, 0), chains);
 }
 
 // A stroke list: each stroke is FootprintBrush::setRadius(radius) with its
 // footprint (a no-op within 0.5 of the current radius, FootprintBrush.hxx:
 // 46-50), then its stamps.
-template <int kT>
 void run_fused_strokes_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* S, int64_t ns) {
   std::vector<ListGeo> geos{ListGeo{b->fp, b->size_map, b->radius, nullptr, b->width,
                                     FpBox{b->fbox[0], b->fbox[1], b->fbox[2], b->fbox[3]}}};
@@ -768,7 +718,7 @@ void run_fused_strokes_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* S, 
     const PlanDev D =
         upload_plan_parts(b, cv, parts.data(), (int)parts.size(), fp_floats, fill, &d_fp);
     for (size_t g = 1; g < geos.size(); ++g) geos[g].fp = d_fp + fp_off[g];
-    run_fused_list<kT>(b, cv, all.data(), n, D, geos, geo, clear, 0);
+    run_fused_list(b, cv, all.data(), n, D, geos, geo, clear, 0);
   }
   // a geometry change after the last stamp (strokes without stamps)
   if (cur != (n > 0 ? geo.back() : 0))
@@ -791,6 +741,19 @@ void run_fused_strokes_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* S, 
 // deadlock, without a cooperative launch.  Consecutive stamps follow each
 // other at the latency of one counter, not of a kernel launch, and the host
 // issues one launch per run.
+struct FArgs {
+  const PStamp* st;
+  Layer7 canvas, snap;  // snap == canvas planes when the snapshot is off
+  Plane7 pick;
+  const float* fp;
+  FpBox fb;  // nonzero footprint cells
+  uint8_t* dirty;
+  const int2* dl;
+  const int* dl_off;
+  int use_snap, rows, cols, hr, size_map;
+  double pickup_rate, dep_rate, cap;
+};
+
 struct CArgs {
   FArgs f;              // f.st = this run's first stamp
   int n;                // stamps in the run
@@ -826,9 +789,9 @@ __device__ __forceinline__ bool chain_wait(const CArgs& A, unsigned* c, unsigned
   return true;
 }
 
-template <int kT>
-__global__ __launch_bounds__(kT* kT) void k_stamp_chain(CArgs A) {
-  __shared__ int sm[kT + 2][kT + 2];
+template <int kCT>
+__global__ __launch_bounds__(kCT* kCT) void k_stamp_chain(CArgs A) {
+  __shared__ StampLds<kCT * kCT> lds;
   __shared__ int s_v, s_ok;
   const int t = threadIdx.x;
   if (t == 0)
@@ -859,34 +822,34 @@ __global__ __launch_bounds__(kT* kT) void k_stamp_chain(CArgs A) {
   }
   __syncthreads();
   if (!s_ok) return;
-  const StampGeom g = geom_of(A.f, st);
+  const StampGeom g = stamp_geom(st, A.f.size_map, A.f.rows, A.f.cols);
   const bool pull = A.f.use_snap && !dup;
   const float* pk = A.paint + 6 * k;
   const float* ps = pk + 3;
   if (role == 0) {  // dip(): clean() the pickup map
-    for (int64_t i = (int64_t)off * kT * kT + t; i < A.pick_floats; i += (int64_t)r.x * kT * kT)
+    for (int64_t i = (int64_t)off * kCT * kCT + t; i < A.pick_floats; i += (int64_t)r.x * kCT * kCT)
       A.pick[i] = 0.0f;
   } else if (role == 1) {
-    ring_scan<kRingGroups>(A.f.canvas, A.f.snap, A.f.dirty, A.f.fp, g, st.box, pull,
-                 (off - r.x) * kT * kT + t, r.y * kT * kT);
+    ring_scan<kCT * kCT>(A.f.canvas, A.f.snap, A.f.dirty, A.f.fp, g, st.box, pull, off - r.x, r.y,
+                         lds.ring);
   } else if (role == 2) {
     const VisitTarget T{&A.f.canvas, &A.f.snap, A.f.dirty, A.f.use_snap, A.f.pickup_rate,
                         A.f.dep_rate, A.f.cap};
     float pkr[3] = {pk[0], pk[1], pk[2]}, psr[3] = {ps[0], ps[1], ps[2]};
-    window_tile<kT>(T, A.f.pick.p, A.f.fp, A.f.fb, g, st, dup, pull, off - r.x - r.y, A.f.tiles_x, sm,
-                    pkr, psr);
+    window_tile<kCT, StampKind<false, true, 2>>(T, A.f.pick.p, A.f.fp, A.f.fb, g, st, dup, pull, off - r.x - r.y,
+                    tile_window(g, A.f.fb), lds.hand, pkr, psr);
   } else {  // visits sharing canvas column/row 0, by dependency level
     const VisitTarget T{&A.f.canvas, &A.f.snap, A.f.dirty, A.f.use_snap, A.f.pickup_rate,
                         A.f.dep_rate, A.f.cap};
     float pkr[3] = {pk[0], pk[1], pk[2]}, psr[3] = {ps[0], ps[1], ps[2]};
     for (int L = 0; L < st.dl_nlev; ++L) {
       const int e0 = A.f.dl_off[st.dl_lev + L], e1 = A.f.dl_off[st.dl_lev + L + 1];
-      for (int e = e0 + t; e < e1; e += kT * kT) {
+      for (int e = e0 + t; e < e1; e += kCT * kCT) {
         const int2 vv = A.f.dl[e];
         int64_t ic;
         const int m = stamp_visit(g, vv.x, vv.y, &ic);
         if (m >= 0 && A.f.fp[m] > 0.0f)
-          cached_visit(T, GlobalPick{A.f.pick.p, m}, A.f.fp[m], ic, false, pkr, psr);
+          cached_visit(T, A.f.pick.p, m, A.f.fp[m], ic, false, pkr, psr);
       }
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
@@ -933,7 +896,7 @@ void chain_release(ChainState*& c) {
   c = nullptr;
 }
 
-template <int kT>
+template <int kCT>
 static void run_chained_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n) {
   hipStream_t s = b->ctx->stream;
   if (*(volatile unsigned*)b->ctx->kernel_error)
@@ -954,19 +917,15 @@ static void run_chained_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st,
   F.cols = cv->cols;
   F.hr = (b->size_map - 1) / 2;
   F.size_map = b->size_map;
-  const int side = 2 * F.hr + 1;
-  F.tiles_x = (side + kT - 1) / kT;
-  F.ntiles = F.tiles_x * F.tiles_x;
   F.pickup_rate = b->pickup_rate;
   F.dep_rate = b->dep_rate;
   F.cap = b->cap;
-  F.clk = DryClock{};  // a canvas with a drying clock stamps on the fused path
   // host plan of the whole list: roles, tickets, paints
   std::vector<int4> roles(n);
   std::vector<int> start(n + 1);
   std::vector<float> paint(6 * (size_t)n);
   const int64_t pick_floats = 7 * b->mstride;
-  const int nclear = (int)std::min<int64_t>((pick_floats + kT * kT * 4 - 1) / (kT * kT * 4), 256);
+  const int nclear = (int)std::min<int64_t>((pick_floats + kCT * kCT * 4 - 1) / (kCT * kCT * 4), 256);
   float pk[3] = {b->paintK[0], b->paintK[1], b->paintK[2]};
   float ps[3] = {b->paintS[0], b->paintS[1], b->paintS[2]};
   for (int64_t k = 0; k < n; ++k) {
@@ -982,8 +941,8 @@ static void run_chained_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st,
     }
     int4 r;
     r.x = (st[k].flags & PNT_STAMP_DIP) ? nclear : 0;
-    r.y = F.use_snap ? ring_blocks_for(p.box, kT * kT) : 0;
-    r.z = F.ntiles;
+    r.y = F.use_snap ? ring_blocks_for(p.box, kCT * kCT) : 0;
+    r.z = tile_count<kCT>(tile_window(stamp_geom(p, F.size_map, F.rows, F.cols), F.fb));
     r.w = (p.flags & (kStDupX | kStDupY)) && p.dl_nlev > 0 ? 1 : 0;
     roles[k] = r;
   }
@@ -1043,7 +1002,7 @@ static void run_chained_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st,
     A.long_sleep = std::getenv("PAINTY_CHAIN_SLEEP") != nullptr;
     PNT_HIP_CHECK(hipHostGetDevicePointer((void**)&A.host_err, b->ctx->kernel_error, 0));
     PNT_REQUIRE(total_blocks < ((int64_t)1 << 31), "stamp run too long for one launch");
-    k_stamp_chain<kT><<<(unsigned)total_blocks, kT * kT, 0, s>>>(A);
+    k_stamp_chain<kCT><<<(unsigned)total_blocks, kCT * kCT, 0, s>>>(A);
     PNT_HIP_CHECK(hipGetLastError());
     if (st[e].flags & PNT_STAMP_DRY_AFTER) {
       if (b->use_snap)
@@ -1140,30 +1099,10 @@ void run_fused_noalloc(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, in
   if (boff)
     PNT_HIP_CHECK(hipMemcpyAsync(loff, h_off.data(), (size_t)boff, hipMemcpyHostToDevice, s));
   PNT_HIP_CHECK(hipStreamSynchronize(s));
-  FArgs a;
-  a.st = reinterpret_cast<const PStamp*>(dev);
-  a.canvas = cv->layer();
-  a.snap = b->use_snap ? b->snap_planes() : cv->layer();
-  a.pick = b->pick_planes();
-  a.fp = b->fp;
-  a.fb = FpBox{b->fbox[0], b->fbox[1], b->fbox[2], b->fbox[3]};
-  a.dirty = b->dirty;
-  a.dl = reinterpret_cast<const int2*>(ldl);
-  a.dl_off = reinterpret_cast<const int*>(loff);
-  a.use_snap = b->use_snap ? 1 : 0;
-  a.rows = cv->rows;
-  a.cols = cv->cols;
-  a.hr = (b->size_map - 1) / 2;
-  a.size_map = b->size_map;
-  const int side = 2 * a.hr + 1;
-  a.tiles_x = (side + 15) / 16;
-  a.ntiles = a.tiles_x * a.tiles_x;
-  a.pickup_rate = b->pickup_rate;
-  a.dep_rate = b->dep_rate;
-  a.cap = b->cap;
-  a.clk = cv->clock != PNT_CLOCK_OFF && cv->tmap
-              ? DryClock{cv->tmap, 0, cv->drying_ms, cv->R0(), cv->h()}
-              : DryClock{};
+  const StampShared H = stamp_shared(b, cv, reinterpret_cast<const int2*>(ldl),
+                                     reinterpret_cast<const int*>(loff));
+  const FpBox dom = cell_domain(FpBox{b->fbox[0], b->fbox[1], b->fbox[2], b->fbox[3]}, b->size_map,
+                                H.tmap != nullptr);
   for (int64_t k = 0; k < n; ++k) {
     if (st[k].flags & PNT_STAMP_DIP) {  // dip(): clean() and the new paint
       launch_fill(b->pick, 7 * b->mstride, 0.0f, s);
@@ -1172,21 +1111,15 @@ void run_fused_noalloc(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, in
         b->paintS[c] = st[k].S[c];
       }
     }
-    for (int c = 0; c < 3; ++c) {
-      a.pk[c] = b->paintK[c];
-      a.ps[c] = b->paintS[c];
-    }
-    const PStamp& p = h_st[(size_t)k];
-    const int rb = a.use_snap ? ring_blocks_for(p.box, 256) : 0;
-    const int jk = (int)k;
-    k_stamp_fused<16><<<a.ntiles + rb + (dup_levels(p) ? 1 : 0), 256, 0, s>>>(a, jk, rb);
-    PNT_HIP_CHECK(hipGetLastError());
+    launch_slots(WArgs<1>{H, {stamp_slot(H, h_st[(size_t)k], b->fp, dom, b->size_map, b->pick,
+                                         b->mstride, b->paintK, b->paintS)}},
+                 1, s);
     if (st[k].flags & PNT_STAMP_DRY_AFTER) {
       if (b->use_snap)
         launch_dry_dirty(cv->n, cv->layer(), cv->R0(), cv->h(), b->dirty, s);
       else
         launch_dry(cv->n, cv->layer(), cv->R0(), cv->h(), s);
-      if (a.clk.tmap) launch_fill_i64(cv->tmap, cv->n, canvas_now_us(cv), s);
+      if (H.tmap) launch_fill_i64(cv->tmap, cv->n, canvas_now_us(cv), s);
     }
   }
   cv->epoch++;
@@ -1197,23 +1130,11 @@ void run_fused_noalloc(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, in
 }
 
 void run_fused_strokes(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* strokes, int64_t ns) {
-  int kT = 16;
-  if (const char* e = std::getenv("PAINTY_FUSED_TILE")) kT = std::atoi(e) == 32 ? 32 : 16;
-  if (kT == 32)
-    run_fused_strokes_t<32>(b, cv, strokes, ns);
-  else
-    run_fused_strokes_t<16>(b, cv, strokes, ns);
+  run_fused_strokes_t(b, cv, strokes, ns);
 }
 
 void run_fused(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains) {
-  if (n == 0) return;
-  // window tile side: 16 (256 threads), or 32 from PAINTY_FUSED_TILE
-  int kT = 16;
-  if (const char* e = std::getenv("PAINTY_FUSED_TILE")) kT = std::atoi(e) == 32 ? 32 : 16;
-  if (kT == 32)
-    run_fused_t<32>(b, cv, st, n, chains);
-  else
-    run_fused_t<16>(b, cv, st, n, chains);
+  if (n > 0) run_fused_t(b, cv, st, n, chains);
 }
 
 }  // namespace pnt

@@ -62,6 +62,26 @@ struct Rgb3 {
 template <class T>
 using gptr = __attribute__((address_space(1))) T*;
 
+// A record of device memory that no kernel writes (a plan or descriptor the
+// host copied in before the launch), read through the constant address space:
+// at a uniform address that is a few wide scalar loads, together.  Read as
+// ordinary memory, which the kernel's own stores might change, each field is
+// a vector load where it is used: a wave kernel spent 6 us on them one after
+// another (2100 canvases' stamps in waves: 14,400 cycles before its first
+// map cell, 1,500 with the same record in the kernel arguments).
+template <class T>
+__device__ __forceinline__ T load_const(const void* p) {
+  static_assert(sizeof(T) % 4 == 0 && alignof(T) >= 4, "whole words");
+  using word = const __attribute__((address_space(4))) uint32_t;
+  word* q = (word*)(uintptr_t)p;
+  uint32_t w[sizeof(T) / 4];
+#pragma unroll
+  for (size_t i = 0; i < sizeof(T) / 4; ++i) w[i] = q[i];
+  T v;
+  __builtin_memcpy(&v, w, sizeof(T));
+  return v;
+}
+
 // Brush state and parameters one imprint needs.
 struct BrushArgs {
   const float* fp;   // footprint, size_map^2
@@ -89,11 +109,6 @@ struct StampArgs {
   int dupx, dupy;    // canvas column / row 0 visited twice (see stamp_dup_axis)
   DryClock clk;
 };
-
-// 4-pixel groups a ring-scan thread takes per pass (ring_blocks_for).  More
-// groups per thread means fewer ring blocks per stamp but longer ones, and
-// a stamp launch lasts as long as its slowest block: two measured fastest.
-constexpr int kRingGroups = 2;
 
 // Snapshot ring of updateSnapshot(canvas, center), FootprintBrush.hxx:286-305.
 struct RingBox {

@@ -80,6 +80,17 @@ struct LdsPick {  // pickup map cell t of the block's tile, in LDS
   }
 };
 
+// One visit whose pickup cell lives in LDS; the pixels in one batch.
+template <class PickAcc>
+__device__ __forceinline__ void cached_visit(const VisitTarget& T, const PickAcc& pick, float fh,
+                                             int64_t ic, bool pull, const float pk[3],
+                                             const float ps[3]) {
+  CachedVisit<PickAcc> acc{pick, {}, {}, 0.0, 0.0, !T.use_snap, false};
+  load_pixel(T, T.use_snap, ic, pull, acc);
+  paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
+  store_pixel(T, T.use_snap, ic, pull, acc);
+}
+
 template <int kT>
 __global__ __launch_bounds__(kT* kT) void k_persistent(PArgs A) {
   constexpr int kCells = kT * kT;  // one map cell per thread

@@ -67,9 +67,7 @@ struct StampNeeds {
 };
 StampNeeds plan_stamp_needs(const std::vector<Unit>& U, const PStamp* h);
 // Blocks of `threads` threads that scan the snapshot ring of box b.
-// groups: 4-pixel groups per ring-scan thread (the ring_scan<groups> the
-// launch runs).
-int ring_blocks_for(const RingBox& b, int threads, int groups = kRingGroups);
+int ring_blocks_for(const RingBox& b, int threads);
 // Plans stamps [0, n) for a brush of footprint side size_map and radius on a
 // rows x cols canvas (FP64 geometry, ring boxes, shared-pixel levels).
 void plan_stamps_rc(int size_map, double radius, int rows, int cols, const pnt_stamp* st,
@@ -130,6 +128,7 @@ struct BWPlan {
   int64_t o_jobs = 0;
   std::vector<int64_t> wave_slots, wave_grp;
   std::vector<int> wave_blocks;
+  std::vector<char> wave_plain;  // runs the plain-stamps kernel (batchwave.hip)
   std::vector<int> job_first, job_last;  // each job's first and last wave (-1: none)
   int njobs = 0;
 };

@@ -74,7 +74,6 @@ namespace {
 constexpr int kPhases = 160;       // phases per wave
 constexpr int kChainsPerReq = 8;   // pickup maps of one request (concurrent units)
 constexpr int kAhead = 3;          // waves queued ahead of the engine
-constexpr int kT = kWT;            // window tile side
 constexpr int kT2 = kWT2;          // threads per block
 
 // What every phase of one admitted request shares: written to the device
@@ -90,7 +89,7 @@ struct SReq {
   const int* dl_off;
   const float* paint;  // 6 floats per stamp: the brush paint at that stamp
   float* out[3];
-  int cstride, mstride, dirty_bytes, rows, cols, hr, size_map, tiles_x, ntiles, use_snap;
+  int cstride, mstride, dirty_bytes, rows, cols, hr, size_map, use_snap;
   int fb[4];
   float bg[3];
   int pad;
@@ -109,7 +108,7 @@ struct SReqG {
   gptr<const int> dl_off;
   gptr<const float> paint;
   gptr<float> out[3];
-  int cstride, mstride, dirty_bytes, rows, cols, hr, size_map, tiles_x, ntiles, use_snap;
+  int cstride, mstride, dirty_bytes, rows, cols, hr, size_map, use_snap;
   int fb[4];
   float bg[3];
   int pad;
@@ -135,15 +134,21 @@ struct SPhase {
 struct SArgs {
   const SReqG* reqs;
   int nphases;
-  int pad;
+  int general;  // a phase is more than a plain stamp or a map clear (host only)
   SPhase ph[kPhases];
 };
 static_assert(sizeof(SArgs) <= 4000, "wave arguments must fit the kernel argument segment");
 
+// The stamps of most waves (no stamp on canvas column/row 0, snapshot on, no
+// streaming phase), and everything.
+using PlainStamps = StampKind<false, false, 1>;
+using AnyStamps = StampKind<false, true, 2>;
+
 // One wave of the server: its phases arrive as kernel arguments, each
 // request's shared fields from its device descriptor.
+template <class F, bool kStream>
 __global__ __launch_bounds__(kWT2, kWaveOccupancy) void k_serve_wave(SArgs A) {
-  __shared__ int sm[kWT + 2][kWT + 2];
+  __shared__ StampLds<kWT2> lds;
   int lo = 0, hi = A.nphases - 1;  // the last phase with start <= blockIdx.x
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -155,7 +160,7 @@ __global__ __launch_bounds__(kWT2, kWaveOccupancy) void k_serve_wave(SArgs A) {
   const SPhase& P = A.ph[lo];
   const int b = (int)blockIdx.x - P.start;
   if (b >= P.nblk) return;
-  const SReqG& Q = A.reqs[P.slot];
+  const SReqG Q = load_const<SReqG>(A.reqs + P.slot);
   SSlot S;
   S.st = (const PStamp*)(Q.st + P.k);
   S.canvas = (float*)Q.canvas;
@@ -176,7 +181,6 @@ __global__ __launch_bounds__(kWT2, kWaveOccupancy) void k_serve_wave(SArgs A) {
   S.kind = P.kind;
   S.start = P.start;
   S.nblk = P.nblk;
-  S.ntiles = Q.ntiles;
   // a streaming phase carries its part in rb: part | nparts << 16
   const bool streaming =
       P.kind == kSInit || P.kind == kSSnap || P.kind == kSDry || P.kind == kSCompose;
@@ -185,14 +189,17 @@ __global__ __launch_bounds__(kWT2, kWaveOccupancy) void k_serve_wave(SArgs A) {
   S.nparts = streaming ? (P.rb >> 16) : 1;
   S.hr = Q.hr;
   S.size_map = Q.size_map;
-  S.tiles_x = Q.tiles_x;
 #pragma unroll
   for (int c = 0; c < 4; ++c) S.fb[c] = Q.fb[c];
   const bool stamp_kind = P.kind == kSStamp;
+  struct Paint {
+    float v[6];
+  };
+  const Paint paint = stamp_kind ? load_const<Paint>((const float*)Q.paint + 6 * (int64_t)P.k) : Paint{};
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    S.pk[c] = stamp_kind ? Q.paint[6 * (int64_t)P.k + c] : 0.0f;
-    S.ps[c] = stamp_kind ? Q.paint[6 * (int64_t)P.k + 3 + c] : 0.0f;
+    S.pk[c] = paint.v[c];
+    S.ps[c] = paint.v[3 + c];
   }
   S.pickup_rate = Q.pickup_rate;
   S.dep_rate = Q.dep_rate;
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(kWT2, kWaveOccupancy) void k_serve_wave(SArgs A) {
   for (int c = 0; c < 3; ++c) S.bg[c] = Q.bg[c];
   S.tmap = nullptr;  // served canvases have no drying clock
   S.dry_ms = 0;
-  run_wave_slot(S, b, sm);
+  run_wave_slot<F, kStream>(S, b, lds);
 }
 
 // Blocks of one part of a streaming phase: at most 512, each thread taking
@@ -239,7 +246,7 @@ struct Req {
   bool done = false;
   // plan (planner thread)
   bool planned = false;
-  int size_map = 0, hr = 0, tiles_x = 0, ntiles = 0;
+  int size_map = 0, hr = 0;
   int64_t mstride = 0;
   int fbox[4] = {0, 0, -1, -1};
   std::vector<float> fp;  // padded footprint
@@ -250,7 +257,7 @@ struct Req {
   std::vector<std::vector<Phase>> ph;  // per unit
   std::vector<int> prev_on_chain;      // per unit
   std::vector<float> paint;            // 6 per stamp: the brush paint at that stamp
-  std::vector<int> rb;                 // ring-scan blocks per stamp
+  std::vector<int> rb, ntiles;                 // ring-scan blocks per stamp
   int64_t plan_bytes = 0;
   // engine
   int slot = -1;
@@ -382,9 +389,6 @@ void pnt_server_s::plan(Req* q) {
   const pnt_request& r = q->r;
   q->size_map = footprint_size_map(r.radius, q->footprint.data(), r.width);
   q->hr = (q->size_map - 1) / 2;
-  const int side = 2 * q->hr + 1;
-  q->tiles_x = (side + kT - 1) / kT;
-  q->ntiles = q->tiles_x * q->tiles_x;
   q->mstride = round_up((int64_t)q->size_map * q->size_map, 64);
   q->fp.assign((size_t)q->size_map * q->size_map, 0.0f);
   pad_footprint_into(q->footprint.data(), r.width, q->size_map, q->fp.data(), q->fbox);
@@ -398,12 +402,16 @@ void pnt_server_s::plan(Req* q) {
   const bool snap = r.use_snapshot != 0;
   q->ph.assign(q->U.size(), {});
   q->rb.assign((size_t)n, 0);
+  q->ntiles.assign((size_t)n, 1);
+  const FpBox dom{q->fbox[0], q->fbox[1], q->fbox[2], q->fbox[3]};
   for (size_t i = 0; i < q->U.size(); ++i)
     for (int64_t k = q->U[i].s0; k < q->U[i].s1; ++k) {
       if (clear[(size_t)k] || (q->stamps[(size_t)k].flags & PNT_STAMP_DIP))
         q->ph[i].push_back(Phase{k, kSClear});
       const PStamp& p = q->st[(size_t)k];
       q->rb[(size_t)k] = snap ? ring_blocks_for(p.box, kT2) : 0;
+      q->ntiles[(size_t)k] =
+          tile_count<kWT>(tile_window(stamp_geom(p, q->size_map, r.rows, r.cols), dom));
       q->ph[i].push_back(Phase{k, kSStamp});
     }
   q->prev_on_chain.assign(q->U.size(), -1);
@@ -725,8 +733,6 @@ void pnt_server_s::write_descriptor(Req* q, int64_t& o) {
   D.cols = R.cols;
   D.hr = q->hr;
   D.size_map = q->size_map;
-  D.tiles_x = q->tiles_x;
-  D.ntiles = q->ntiles;
   D.use_snap = snap ? 1 : 0;
   for (int k = 0; k < 4; ++k) D.fb[k] = q->fbox[k];
   for (int k = 0; k < 3; ++k) D.bg[k] = R.bg[k];
@@ -754,6 +760,7 @@ bool pnt_server_s::collect(Req* q, SArgs& A, int& start,
     P.slot = (int16_t)q->slot;
     P.kind = (int8_t)kind;
     P.start = start;
+    A.general |= kind != kSStamp && kind != kSClear;
     return P;
   };
   auto push = [&](SPhase& P, int unit) {
@@ -828,7 +835,8 @@ bool pnt_server_s::collect(Req* q, SArgs& A, int& start,
             break;
           default:  // kSStamp, + the shared-pixel levels' block of a dup stamp
             P.rb = rb;
-            P.nblk = q->ntiles + rb + (dup_levels(q->st[(size_t)f.k]) ? 1 : 0);
+            A.general |= !snap || (q->st[(size_t)f.k].flags & (kStDupX | kStDupY));
+            P.nblk = q->ntiles[(size_t)f.k] + rb + (dup_levels(q->st[(size_t)f.k]) ? 1 : 0);
             break;
         }
         if (P.nblk == 0) P.nblk = 1;  // an empty ring: the block returns at once
@@ -988,7 +996,8 @@ void pnt_server_s::run_engine() {
       }
       if (A.nphases == 0) continue;
       hipStream_t s = L.ctx->stream;
-      k_serve_wave<<<(unsigned)start, kT2, 0, s>>>(A);
+      const auto kernel = A.general ? k_serve_wave<AnyStamps, true> : k_serve_wave<PlainStamps, false>;
+      kernel<<<(unsigned)start, kT2, 0, s>>>(A);
       PNT_HIP_CHECK(hipGetLastError());
       PNT_HIP_CHECK(hipEventRecord(L.ev[L.waves % (kAhead + 1)], s));
       ++L.waves;

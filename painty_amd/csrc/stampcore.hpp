@@ -160,13 +160,6 @@ __device__ __forceinline__ void st_px(const Layer7& L, int64_t i, const float ks
   L.v[i] = v;
 }
 
-struct GlobalPick {  // pickup map cell in global memory
-  float* const* p;
-  int im;
-  __device__ float pick(int c) const { return p[c][im]; }
-  __device__ void set_pick(int c, float v) const { p[c][im] = v; }
-};
-
 // Where one visit reads and writes.
 struct VisitTarget {
   const Layer7* canvas;
@@ -175,27 +168,6 @@ struct VisitTarget {
   int use_snap;
   double pickup_rate, dep_rate, cap;
 };
-
-template <class PickAcc>
-__device__ __forceinline__ void cached_visit(const VisitTarget& T, const PickAcc& pick, float fh,
-                                             int64_t ic, bool pull, const float pk[3],
-                                             const float ps[3]) {
-  CachedVisit<PickAcc> acc{pick, {}, {}, 0.0, 0.0, !T.use_snap, false};
-  ld_px(*T.canvas, ic, acc.cv, acc.cvv);
-  if (T.use_snap && !pull)
-    ld_px(*T.src, ic, acc.sv, acc.svv);
-  else
-    acc.src_from_canvas();
-  paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
-  st_px(*T.canvas, ic, acc.cv, acc.cvv);
-  if (T.use_snap) {
-    if (pull)
-      st_px(*T.src, ic, acc.sv, acc.svv);
-    else if (acc.src_moved)
-      T.src->v[ic] = acc.svv;
-    T.dirty[ic] = 1;
-  }
-}
 
 // Tile of block b when blocks [0, ntiles) take one tile each: blocks go
 // round-robin to the 8 XCDs, so each XCD gets a contiguous run of tiles and
@@ -257,107 +229,138 @@ __device__ __forceinline__ bool on_window_border(const RingBox& b, int x, int y)
 }
 
 // Snapshot ring refresh of one stamp (updateSnapshot(canvas, center),
-// FootprintBrush.hxx:307-318) over `nthreads` threads.  The allowed box is
-// cut into 4-pixel groups at 4-aligned linear indices; a thread reads a
-// group's four dirty bytes (a set byte: snapshot differs from canvas), and
-// for the set pixels outside the window interior copies canvas -> snapshot
-// and clears the byte.  With `pull`, window-border pixels that a visit of
-// this stamp refreshes itself are left to that visit.  Each thread takes
-// kG groups per pass (so that a stamp's ring needs few blocks) with all
-// their dirty-word loads in flight together (the dirty
-// strip behind a moving window is contiguous, so a pixel-serial copy would
-// wait on one round trip per pixel).  Plane and dirty buffers are padded
-// past the last pixel to a multiple of 16, so a group never leaves them.
-template <int kG>
+// FootprintBrush.hxx:307-318) by block `blk` of `nblk`, kThreads threads
+// each (all of which must call it).  A set dirty byte says that the pixel's
+// snapshot differs from the canvas; for the set pixels of the allowed box
+// outside the window interior the block copies canvas -> snapshot and clears
+// the byte.  With `pull`, window-border pixels that a visit of this stamp
+// refreshes itself are left to that visit.
+//
+// A thread reads the 8 dirty bytes of 8 pixels at an 8-aligned linear
+// index in one load and lists the 4-pixel groups that hold work in LDS; then
+// the block shares the list out by pixel (which border pixels a visit
+// refreshes) and by plane (the copies).  The dirty strip behind a moving
+// window is contiguous: where a thread copied what it found itself, the few
+// that found the strip made one memory round trip per group, and the slowest
+// ring block held up its launch (16 us, beside tiles of 5.6 us on average).
+// Plane and dirty buffers are padded past the last pixel to a multiple of
+// 16, so a unit never leaves them.
+constexpr int kRingUnit = 8;                 // pixels per dirty load
+constexpr int kRingGroups = kRingUnit / 4;   // 4-pixel groups per thread and pass
+
+template <int kThreads>
+struct RingList {  // the groups of a pass: pixel base relative to the box's first, mask
+  unsigned n;
+  unsigned g[kRingGroups * kThreads];  // group number << 8 | border bits << 4 | copy bits
+};
+
+template <int kThreads>
 __device__ __forceinline__ void ring_scan(const Layer7& canvas, const Layer7& snap, uint8_t* dirty,
                                           const float* fp, const StampGeom& g, const RingBox& b,
-                                          bool pull, int tid, int nthreads,
+                                          bool pull, int blk, int nblk, RingList<kThreads>& list,
                                           bool clocked = false) {
   if (b.a_x1 < b.a_x0 || b.a_y1 < b.a_y0) return;
   const int rows = b.a_y1 - b.a_y0 + 1;
   const int span = b.a_x1 - b.a_x0 + 1;
-  const int per_row = (span + 3) / 4 + 1;  // +1: misaligned start
+  const int per_row = (span + kRingUnit - 1) / kRingUnit + 1;  // +1: misaligned start
   const int total = per_row * rows;
-  for (int e0 = tid; e0 < total; e0 += kG * nthreads) {
-    unsigned mask[kG];
-    int64_t base[kG];
-#pragma unroll
-    for (int u = 0; u < kG; ++u) {
-      mask[u] = 0u;
-      base[u] = 0;
-      const int e = e0 + u * nthreads;
-      if (e >= total) continue;
-      // group e: row a_y0 + e / per_row, pixels [base, base + 4) with
-      // base = (lo & ~3) + 4 * (e % per_row), lo = row*cols + a_x0
-      const int row = b.a_y0 + e / per_row;
-      const int64_t rowi = (int64_t)row * g.cols;
-      const int64_t lo = rowi + b.a_x0;
-      const int64_t bs = (lo & ~(int64_t)3) + 4 * (int64_t)(e % per_row);
-      if (bs >= lo + span) continue;
+  // pixel base of group q of unit e, and its canvas row and first column
+  const auto unit = [&](int e, int* row, int* x0) {
+    const int r = e / per_row;
+    *row = b.a_y0 + r;
+    const int64_t rowi = (int64_t)*row * g.cols, lo = rowi + b.a_x0;
+    const int64_t base = (lo & ~(int64_t)(kRingUnit - 1)) + kRingUnit * (int64_t)(e - r * per_row);
+    *x0 = (int)(base - rowi);
+    return base;
+  };
+  for (int p0 = blk * kThreads; p0 < total; p0 += nblk * kThreads) {
+    if (threadIdx.x == 0) list.n = 0;
+    __syncthreads();
+    const int e = p0 + (int)threadIdx.x;
+    if (e < total) {
+      int row, x0;
+      const int64_t base = unit(e, &row, &x0);
       const bool interior_row = row > b.tl_y && row < b.br_y;
-      const int x0 = (int)(bs - rowi);
-      if (interior_row && x0 > b.tl_x && x0 + 3 < b.br_x) continue;  // inside the window interior
-      const unsigned d = *reinterpret_cast<const unsigned*>(dirty + bs);
-      if (!d) continue;
-      unsigned m = 0u, border = 0u;
+      if (x0 <= b.a_x1 && !(interior_row && x0 > b.tl_x && x0 + kRingUnit - 1 < b.br_x)) {
+        const uint2 d2 = *reinterpret_cast<const uint2*>(dirty + base);
+        const unsigned d[kRingGroups] = {d2.x, d2.y};
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (!((d >> (8 * q)) & 0xffu)) continue;
-        const int64_t i = bs + q;
-        if (i < lo || i >= lo + span) continue;
-        const int col = x0 + q;
-        if (interior_row && col > b.tl_x && col < b.br_x) continue;
-        m |= 1u << q;
-        if (pull && on_window_border(b, col, row)) border |= 1u << q;
-      }
-      // window-border pixels a visit refreshes itself (few: one loop body)
-#pragma unroll 1
-      for (int q = 0; q < 4; ++q)
-        if (((border >> q) & 1u) && ring_pixel_visited(g, b, fp, x0 + q, row, clocked))
-          m &= ~(1u << q);
-      mask[u] = m;
-      base[u] = bs;
-    }
-    // the copies (few: the strip the last stamps left dirty), one group at a
-    // time: two groups' planes in registers at once set the register peak
-    // of every kernel that runs ring scans
-    constexpr int kC = 1;
+        for (int q = 0; q < kRingGroups; ++q) {
+          if (!d[q]) continue;
+          unsigned m = 0u, border = 0u;
 #pragma unroll
-    for (int u0 = 0; u0 < kG; u0 += kC) {
-      float4 v[kC][6];
-      double2 w[kC][2];  // the four volumes
-#pragma unroll
-      for (int h = 0; h < kC; ++h) {
-        const int u = u0 + h;
-        if (!mask[u]) continue;
-#pragma unroll
-        for (int c = 0; c < 6; ++c) v[h][c] = reinterpret_cast<const float4*>(canvas.ks[c])[base[u] >> 2];
-        w[h][0] = reinterpret_cast<const double2*>(canvas.v)[base[u] >> 1];
-        w[h][1] = reinterpret_cast<const double2*>(canvas.v)[(base[u] >> 1) + 1];
-      }
-#pragma unroll
-      for (int h = 0; h < kC; ++h) {
-        const int u = u0 + h;
-        if (!mask[u]) continue;
-        if (mask[u] == 0xfu) {
-#pragma unroll
-          for (int c = 0; c < 6; ++c) reinterpret_cast<float4*>(snap.ks[c])[base[u] >> 2] = v[h][c];
-          reinterpret_cast<double2*>(snap.v)[base[u] >> 1] = w[h][0];
-          reinterpret_cast<double2*>(snap.v)[(base[u] >> 1) + 1] = w[h][1];
-          *reinterpret_cast<unsigned*>(dirty + base[u]) = 0u;
-        } else {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            if (!((mask[u] >> q) & 1u)) continue;
-#pragma unroll
-            for (int c = 0; c < 6; ++c)
-              snap.ks[c][base[u] + q] = reinterpret_cast<const float*>(&v[h][c])[q];
-            snap.v[base[u] + q] = reinterpret_cast<const double*>(&w[h][0])[q];
-            dirty[base[u] + q] = 0;
+          for (int k = 0; k < 4; ++k) {
+            const int col = x0 + 4 * q + k;
+            const bool in = ((d[q] >> (8 * k)) & 0xffu) && col >= b.a_x0 && col <= b.a_x1 &&
+                            !(interior_row && col > b.tl_x && col < b.br_x);
+            m |= (in ? 1u : 0u) << k;
+            border |= (in && pull && on_window_border(b, col, row) ? 1u : 0u) << k;
           }
+          if (m)
+            list.g[atomicAdd(&list.n, 1u)] =
+                ((unsigned)(threadIdx.x * kRingGroups + q) << 8) | (border << 4) | m;
         }
       }
     }
+    __syncthreads();
+    const int n = (int)list.n;
+    // window-border pixels that a visit refreshes itself
+    for (int i = threadIdx.x; i < 4 * n; i += kThreads) {
+      const unsigned w = list.g[i >> 2];
+      if (!((w >> (4 + (i & 3))) & 1u)) continue;
+      int row, x0;
+      unit(p0 + (int)(w >> 8) / kRingGroups, &row, &x0);
+      const int col = x0 + 4 * ((int)(w >> 8) % kRingGroups) + (i & 3);
+      if (ring_pixel_visited(g, b, fp, col, row, clocked)) atomicAnd(&list.g[i >> 2], ~(1u << (i & 3)));
+    }
+    __syncthreads();
+    // the copies: a thread takes one plane (or half of the FP64 volumes) of a
+    // group, eight groups' loads in flight together
+    constexpr int kPer = kThreads / 8, kFlight = 8;
+    const int plane = (int)threadIdx.x & 7;
+    for (int i0 = (int)threadIdx.x >> 3; i0 < n; i0 += kFlight * kPer) {
+      float4 v[kFlight];
+      unsigned m[kFlight];
+      int64_t at[kFlight];
+#pragma unroll
+      for (int u = 0; u < kFlight; ++u) {
+        const int i = i0 + u * kPer;
+        const unsigned w = i < n ? list.g[i] : 0u;
+        m[u] = w & 0xfu;
+        at[u] = 0;
+        if (!m[u]) continue;
+        int row, x0;
+        at[u] = unit(p0 + (int)(w >> 8) / kRingGroups, &row, &x0) + 4 * ((int)(w >> 8) % kRingGroups);
+        v[u] = plane < 6 ? *reinterpret_cast<const float4*>(canvas.ks[0] + plane * (canvas.ks[1] - canvas.ks[0]) + at[u])
+                         : *reinterpret_cast<const float4*>(canvas.v + at[u] + 2 * (plane - 6));
+      }
+#pragma unroll
+      for (int u = 0; u < kFlight; ++u) {
+        if (!m[u]) continue;
+        if (plane < 6) {
+          float* dst = snap.ks[0] + plane * (snap.ks[1] - snap.ks[0]) + at[u];
+          if (m[u] == 0xfu) {
+            *reinterpret_cast<float4*>(dst) = v[u];
+          } else {
+            if (m[u] & 1u) dst[0] = v[u].x;
+            if (m[u] & 2u) dst[1] = v[u].y;
+            if (m[u] & 4u) dst[2] = v[u].z;
+            if (m[u] & 8u) dst[3] = v[u].w;
+          }
+        } else {
+          float2* dst = reinterpret_cast<float2*>(snap.v + at[u]) + 2 * (plane - 6);
+          const unsigned h = m[u] >> (2 * (plane - 6));
+          if (h & 1u) dst[0] = make_float2(v[u].x, v[u].y);
+          if (h & 2u) dst[1] = make_float2(v[u].z, v[u].w);
+        }
+        if (plane == 0) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if ((m[u] >> k) & 1u) dirty[at[u] + k] = 0;
+        }
+      }
+    }
+    __syncthreads();  // the list is rewritten by the next pass
   }
 }
 
@@ -374,29 +377,45 @@ __device__ __forceinline__ int64_t canvas_index(const StampGeom& g, int col, int
 }
 
 // Loads everything one visit reads: canvas and pickup-source pixel.
-__device__ __forceinline__ void load_pixel(const VisitTarget& T, int64_t ic, bool pull,
-                                           CachedVisit<RegPick>& acc) {
+template <class PickAcc>
+__device__ __forceinline__ void load_pixel(const VisitTarget& T, bool snap, int64_t ic, bool pull,
+                                           CachedVisit<PickAcc>& acc) {
   ld_px(*T.canvas, ic, acc.cv, acc.cvv);
-  if (T.use_snap && !pull)
+  if (snap && !pull)
     ld_px(*T.src, ic, acc.sv, acc.svv);
   else
     acc.src_from_canvas();
   acc.src_moved = false;
 }
 
-// Runs one visit on loaded values and stores the canvas / snapshot side.
-__device__ __forceinline__ void run_pixel(const VisitTarget& T, int64_t ic, bool pull, float fh,
-                                          const float pk[3], const float ps[3],
-                                          CachedVisit<RegPick>& acc) {
-  paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
+// Stores the canvas / snapshot side of a visit.
+template <class PickAcc>
+__device__ __forceinline__ void store_pixel(const VisitTarget& T, bool snap, int64_t ic, bool pull,
+                                            const CachedVisit<PickAcc>& acc) {
   st_px(*T.canvas, ic, acc.cv, acc.cvv);
-  if (T.use_snap) {
+  if (snap) {
     if (pull)
       st_px(*T.src, ic, acc.sv, acc.svv);
     else if (acc.src_moved)
       T.src->v[ic] = acc.svv;
     T.dirty[ic] = 1;
   }
+}
+
+// One whole visit of map cell m at canvas pixel ic: everything it reads in
+// one batch, the arithmetic, the stores.
+__device__ __forceinline__ void cached_visit(const VisitTarget& T, float* const* pick, int m,
+                                             float fh, int64_t ic, bool pull, const float pk[3],
+                                             const float ps[3]) {
+  CachedVisit<RegPick> acc;
+  acc.alias = !T.use_snap;
+#pragma unroll
+  for (int c = 0; c < 7; ++c) acc.v[c] = pick[c][m];
+  load_pixel(T, T.use_snap, ic, pull, acc);
+  paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
+  store_pixel(T, T.use_snap, ic, pull, acc);
+#pragma unroll
+  for (int c = 0; c < 7; ++c) pick[c][m] = acc.v[c];
 }
 
 // Canvas::checkDry (Canvas.hxx:123-155) of a visited pixel whose canvas
@@ -441,124 +460,243 @@ __device__ __forceinline__ void check_only(const VisitTarget& T, const DryClock&
   if (T.use_snap && v0 > 0.001 && T.canvas->v[ic] != v0) T.dirty[ic] = 1;
 }
 
+// The map cells a stamp's visits are run over: the footprint's nonzero box,
+// or, with a drying clock, the whole map (every visited pixel is checked,
+// whatever its footprint height).
+__host__ __device__ inline FpBox cell_domain(const FpBox& nonzero, int size_map, bool clocked) {
+  return clocked ? FpBox{0, 0, size_map - 1, size_map - 1} : nonzero;
+}
+
+// The window offsets that can fall on a box of map cells and on the canvas,
+// cut into tiles.
+struct TileWin {
+  int col0, row0, cols, rows;  // first offset, extent (<= 0: none)
+};
+
+// Rotating a cell's centre back gives a point within (|c| + |s|) / 2 <=
+// 0.70711 of its visitors along both axes, so the box's corners bound the
+// offsets.  Half of a window holds no footprint (its side is sqrt(2) times
+// the footprint's, so that every rotation fits): without the cut, half of
+// the workgroups of a stamp would find nothing to do.
+__host__ __device__ __forceinline__ TileWin tile_window(const StampGeom& g, const FpBox& dom) {
+#pragma clang fp contract(off)
+  const double hr = (double)g.hr;
+  const double u0 = (double)dom.x0 - hr, u1 = (double)dom.x1 - hr;
+  const double v0 = (double)dom.y0 - hr, v1 = (double)dom.y1 - hr;
+  // col = u c + v s, row = v c - u s
+  const double clo = (g.c >= 0.0 ? u0 : u1) * g.c + (g.s >= 0.0 ? v0 : v1) * g.s - 0.7072;
+  const double chi = (g.c >= 0.0 ? u1 : u0) * g.c + (g.s >= 0.0 ? v1 : v0) * g.s + 0.7072;
+  const double rlo = (g.c >= 0.0 ? v0 : v1) * g.c - (g.s >= 0.0 ? u1 : u0) * g.s - 0.7072;
+  const double rhi = (g.c >= 0.0 ? v1 : v0) * g.c - (g.s >= 0.0 ? u0 : u1) * g.s + 0.7072;
+  // offsets on the canvas: -1 < offset + centre < side
+  const int col0 = (int)fmax(fmax(floor(clo), -hr), floor(-g.cx) - 1.0);
+  const int col1 = (int)fmin(fmin(ceil(chi), hr), ceil((double)g.cols - g.cx));
+  const int row0 = (int)fmax(fmax(floor(rlo), -hr), floor(-g.cy) - 1.0);
+  const int row1 = (int)fmin(fmin(ceil(rhi), hr), ceil((double)g.rows - g.cy));
+  const bool any = dom.x1 >= dom.x0 && dom.y1 >= dom.y0;
+  return TileWin{col0, row0, any ? col1 - col0 + 1 : 0, any ? row1 - row0 + 1 : 0};
+}
+// Tiles of kT x kT offsets that cover the window (at least 1).
+template <int kT>
+__host__ __device__ inline int tile_count(const TileWin& w) {
+  if (w.cols <= 0 || w.rows <= 0) return 1;
+  return ((w.cols + kT - 1) / kT) * ((w.rows + kT - 1) / kT);
+}
+
+__host__ __device__ inline StampGeom stamp_geom(const PStamp& p, int size_map, int rows, int cols) {
+  return StampGeom{p.cx, p.cy, p.c, p.s, (size_map - 1) / 2, size_map, rows, cols};
+}
+
+// A window offset's visit and who shares its map cell.
+struct VisitCell {
+  int mm;    // map cell, -1: no visit (outside the window, canvas, map or box)
+  int x, y;  // canvas pixel
+  int shared;  // 0 alone, 1..4: with the left, upper, right, lower neighbour
+};
+
+// Is z, a map coordinate before rounding, rounded to cell m?  Round half
+// away from zero: m - 0.5 <= z < m + 0.5, the lower bound open for m = 0.
+__host__ __device__ __forceinline__ bool rounds_to(double z, int m) {
+  const double lo = (double)m - 0.5;
+  return (m == 0 ? z > lo : z >= lo) && z < (double)m + 0.5;
+}
+
+// The visit of window offset (col, row), with the index arithmetic of
+// stamp_visit, and the 4-neighbour that falls on the same cell: rotation
+// preserves distances and a half-open unit cell holds no two points a
+// distance >= 1 apart except 4-neighbours, so a cell has at most two
+// visitors.
+//
+// A neighbour lies (+-c, +-s) or (+-s, -+c) away on the map; FP32 places it
+// in or out of the cell unless it lies within 4e-6 of the cell's edge (the
+// FP32 error is below 2e-7), and only then is its own FP64 index arithmetic
+// run.  A stamp kernel is a chain of latencies, this test its longest
+// arithmetic one.
+__host__ __device__ __forceinline__ VisitCell visit_cell(const StampGeom& g, const FpBox& dom,
+                                                         int col, int row) {
+#pragma clang fp contract(off)
+  VisitCell V{-1, 0, 0, 0};
+  const double dc = (double)col, dr = (double)row, hr = (double)g.hr;
+  V.x = (int)(dc + g.cx);
+  V.y = (int)(dr + g.cy);
+  const double zx = (dc * g.c - dr * g.s) + hr, zy = (dc * g.s + dr * g.c) + hr;
+  // round half away from zero, for the z > -0.5 that can be a cell
+  const double fx = floor(zx), fy = floor(zy);
+  const int mx = (int)fx + (zx - fx >= 0.5 ? 1 : 0), my = (int)fy + (zy - fy >= 0.5 ? 1 : 0);
+  const bool ok = (unsigned)(col + g.hr) <= (unsigned)(2 * g.hr) &&
+                  (unsigned)(row + g.hr) <= (unsigned)(2 * g.hr) && V.x >= 0 && V.y >= 0 &&
+                  V.x < g.cols && V.y < g.rows && zx > -0.5 && zy > -0.5 && mx >= dom.x0 &&
+                  mx <= dom.x1 && my >= dom.y0 && my <= dom.y1;
+  if (!ok) return V;
+  V.mm = my * g.size_map + mx;
+  const float px = (float)(zx - (double)mx), py = (float)(zy - (double)my);
+  const float cf = (float)g.c, sf = (float)g.s;
+  constexpr float kEdge = 0.5f + 4e-6f;
+  bool near_edge = false;
+  int shared = 0;
+  const auto test = [&](float qx, float qy, int dir) {
+    const float m = fmaxf(fabsf(qx), fabsf(qy));
+    if (m < kEdge) {
+      shared = dir;
+      near_edge |= m > 0.5f - 4e-6f;
+    }
+  };
+  test(px - cf, py - sf, 1);
+  test(px + sf, py - cf, 2);
+  test(px + cf, py + sf, 3);
+  test(px - sf, py + cf, 4);
+  if (near_edge) {
+    shared = 0;
+    for (int d = 1; d <= 4; ++d) {
+      const double nc = dc + (double)(d == 3) - (double)(d == 1);
+      const double nr = dr + (double)(d == 4) - (double)(d == 2);
+      if (rounds_to((nc * g.c - nr * g.s) + hr, mx) && rounds_to((nc * g.s + nr * g.c) + hr, my))
+        shared = d;
+    }
+  }
+  if (shared) {  // a neighbour outside the window or the canvas is no visit
+    const int dx = (shared == 3) - (shared == 1), dy = (shared == 4) - (shared == 2);
+    const int x = (int)((dc + (double)dx) + g.cx), y = (int)((dr + (double)dy) + g.cy);
+    if ((unsigned)(col + dx + g.hr) <= (unsigned)(2 * g.hr) &&
+        (unsigned)(row + dy + g.hr) <= (unsigned)(2 * g.hr) && x >= 0 && y >= 0 && x < g.cols &&
+        y < g.rows)
+      V.shared = shared;
+  }
+  return V;
+}
+
 // The visits of one kT x kT tile of a stamp's window, by one workgroup of
-// kT*kT threads (all of which must call it).  The map cells of the tile and
-// a one-pixel halo go to LDS (`sm`); a visit whose left or upper neighbour
-// shares its cell is left to that neighbour, which runs both in row-major
-// order (a cell has at most two visitors, and they are 4-neighbours).
-// Visits on a duplicated canvas column/row 0 (and their partners) are left
-// out; they run afterwards by dependency level.  Each visit's pickup cell,
-// canvas pixel and source pixel are loaded in one batch.
+// kT*kT threads (all of which must call it), one visit per thread.
+//
+// A cell shared by two visits passes from the first to the second in
+// reference order (the left or upper one first) through LDS (`hand`: 8
+// floats per thread): every thread loads and stores its own pixel, in whole
+// rows, and none carries a second one in registers.  Only where the second
+// lies outside the tile does the first one's thread run both.  Visits on a
+// duplicated canvas column/row 0 (and the visits sharing their cells) are
+// left out; level_visits runs them.
+//
+// Bound: the L1's line lookups and the two memory round trips of a visit
+// (its cell's values, fetched with the pixel's, then the stores).  Map cells
+// are met along a rotated row, about 16 lines per 64 cells and plane.
 //
 // With a drying clock (clk.tmap != nullptr) every visited pixel -- in the canvas
 // and in the map, whatever its footprint height -- gets Canvas::checkDry
-// before its pickup and deposit (FootprintBrush.hxx:115), by the thread that
-// runs its visit: map cells are then taken without the footprint-box cut,
-// so the pairs are those of the plain kernel.
-
-template <int kT>
+// before its pickup and deposit (FootprintBrush.hxx:115).
+//
+// F: what the stamps of the launch may need (StampKind); code for what they
+// don't is left out, which shortens every wave's first pass over cold
+// instruction lines and frees registers.
+template <int kT, class F>
 __device__ __forceinline__ void window_tile(const VisitTarget& T, float* const* pick,
-                                            const float* fp, const FpBox& fb, const StampGeom& g,
+                                            const float* fp, const FpBox& dom, const StampGeom& g,
                                             const PStamp& st, bool dup, bool pull, int tile,
-                                            int tiles_x, int (*sm)[kT + 2], const float pk[3],
-                                            const float ps[3], const DryClock& clk = DryClock{}) {
-  const bool clocked = clk.tmap != nullptr;
+                                            const TileWin& win, float (*hand)[kT * kT],
+                                            const float pk[3], const float ps[3],
+                                            const DryClock& clk = DryClock{}) {
+  const bool clocked = F::clock && clk.tmap != nullptr;
+  const bool snap = F::snap(T.use_snap);
   const int t = threadIdx.x;
   const int lx = t % kT, ly = t / kT;
-  const int col0 = -g.hr + (tile % tiles_x) * kT;
-  const int row0 = -g.hr + (tile / tiles_x) * kT;
-  // map cells of the tile and its halo; without a clock, cells outside the
-  // footprint's nonzero box count as no visit (their visits have fh = 0)
-  for (int e = t; e < (kT + 2) * (kT + 2); e += kT * kT) {
-    const int hy = e / (kT + 2), hx = e % (kT + 2);
-    int64_t ic;
-    sm[hy][hx] = clocked ? stamp_visit(g, col0 + hx - 1, row0 + hy - 1, &ic)
-                     : stamp_visit_in(g, col0 + hx - 1, row0 + hy - 1, fb.x0, fb.y0, fb.x1,
-                                      fb.y1, &ic);
+  const int tiles_x = (win.cols + kT - 1) / kT;
+  // tile / tiles_x: at most 513 a side, so half a tile outweighs the rounding
+  const int ty = (int)(((float)tile + 0.5f) * __builtin_amdgcn_rcpf((float)tiles_x));
+  const int col = win.col0 + (tile - ty * tiles_x) * kT + lx;
+  const int row = win.row0 + ty * kT + ly;
+  const VisitCell V = visit_cell(g, dom, col, row);
+  bool act = V.mm >= 0;
+  const bool second = V.shared == 1 || V.shared == 2;  // runs after its neighbour
+  const bool inside = V.shared == 1   ? lx > 0
+                      : V.shared == 2 ? ly > 0
+                      : V.shared == 3 ? lx < kT - 1
+                                      : ly < kT - 1;
+  const int dx = V.shared == 1 ? -1 : (V.shared == 3 ? 1 : 0);
+  const int dy = V.shared == 2 ? -1 : (V.shared == 4 ? 1 : 0);
+  if (F::dup && dup && act && (on_dup_line(st, col, row) ||
+                     (V.shared && on_dup_line(st, col + dx, row + dy))))
+    act = false;
+  if (second && !inside) act = false;  // the neighbour's tile runs it
+  const bool first = act && !second;
+  float fh = 0.0f;
+  const int64_t ic = (int64_t)V.y * g.cols + V.x;
+  bool pv = false;
+  CachedVisit<RegPick> acc;
+  acc.alias = !snap;
+  if (act) {
+    pv = pull && on_window_border(st.box, V.x, V.y);
+    fh = fp[V.mm];
+    if (first)
+#pragma unroll
+      for (int c = 0; c < 7; ++c) acc.v[c] = pick[c][V.mm];
+    load_pixel(T, snap, ic, pv, acc);
+    if (clocked) {
+      if (fh > 0.0f) {
+        check_dry_regs(clk, acc.cv, acc.cvv, ic);
+        if (!snap) acc.src_from_canvas();  // the pickup source is the canvas itself
+      } else {
+        check_only(T, clk, ic, pv);
+      }
+    }
+  }
+  const bool paint = act && fh > 0.0f;
+  if (paint && first) {
+    paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
+    if (V.shared && inside)
+#pragma unroll
+      for (int c = 0; c < 7; ++c) hand[c][t] = acc.v[c];
   }
   __syncthreads();
-  const int mm = sm[ly + 1][lx + 1];
-  // Tiles of up to 16x16 threads also load the partner visit's pixel in the
-  // first batch (it is another canvas pixel, which no other visit of this
-  // stamp touches), saving a dependent round trip; larger tiles keep the
-  // registers and load it after the first visit.
-  constexpr bool kPre = kT <= 16;
-  bool act = false;
-  int pdir = 0;
-  int64_t ic = 0, pic = 0;
-  bool pv = false, ppull = false;
-  float fh = 0.0f;
-  CachedVisit<RegPick> acc;
-  float pcv[kPre ? 6 : 1], psv[kPre ? 6 : 1];
-  double pcvv = 0.0, psvv = 0.0;
-  if (mm >= 0 && sm[ly + 1][lx] != mm && sm[ly][lx + 1] != mm) {
-    const int col = col0 + lx, row = row0 + ly;
-    pdir = sm[ly + 1][lx + 2] == mm ? 1 : (sm[ly + 2][lx + 1] == mm ? 2 : 0);
-    if (!(dup && (on_dup_line(st, col, row) ||
-                  (pdir && on_dup_line(st, col + (pdir == 1), row + (pdir == 2)))))) {
-      act = true;
-      const int x = (int)(col + g.cx), y = (int)(row + g.cy);  // canvas_index's pixel
-      ic = (int64_t)y * g.cols + x;
-      pv = pull && on_window_border(st.box, x, y);
-      // the footprint height and every value the visits read go out in one
-      // batch (a visit with fh <= 0 then uses none of them)
-      fh = fp[mm];
+  if (paint && second) {
+    const int from = t + dx + dy * kT;
 #pragma unroll
-      for (int c = 0; c < 7; ++c) acc.v[c] = pick[c][mm];
-      acc.alias = !T.use_snap;
-      load_pixel(T, ic, pv, acc);
-      if (pdir) {  // the second visitor of the cell, right or below
-        const int px = (int)(col + (pdir == 1) + g.cx), py = (int)(row + (pdir == 2) + g.cy);
-        pic = (int64_t)py * g.cols + px;
-        ppull = pull && on_window_border(st.box, px, py);
-        if constexpr (kPre) {
-          ld_px(*T.canvas, pic, pcv, pcvv);
-          if (T.use_snap && !ppull) {
-            ld_px(*T.src, pic, psv, psvv);
-          } else {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) psv[c] = pcv[c];
-            psvv = pcvv;
-          }
-        }
-      }
-    }
+    for (int c = 0; c < 7; ++c) acc.v[c] = hand[c][from];
+    paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
   }
-  if (act && clocked && !(fh > 0.0f)) {  // visits that only check
-    check_only(T, clk, ic, pv);
-    if (pdir) check_only(T, clk, pic, ppull);
-  }
-  act = act && fh > 0.0f;
-  if (act) {
-    if (clocked) {
-      check_dry_regs(clk, acc.cv, acc.cvv, ic);
-      if (!T.use_snap) acc.src_from_canvas();  // the pickup source is the canvas itself
-    }
-    run_pixel(T, ic, pv, fh, pk, ps, acc);
-    if (pdir) {
-      acc.alias = !T.use_snap;
-      if constexpr (kPre) {
+  if (paint) {
+    store_pixel(T, snap, ic, pv, acc);
+    if (second || !V.shared)
 #pragma unroll
-        for (int c = 0; c < 6; ++c) {
-          acc.cv[c] = pcv[c];
-          acc.sv[c] = psv[c];
-        }
-        acc.cvv = pcvv;
-        acc.svv = psvv;
-        acc.src_moved = false;
-      } else {
-        load_pixel(T, pic, ppull, acc);  // the pickup cell stays in acc.v
-      }
+      for (int c = 0; c < 7; ++c) pick[c][V.mm] = acc.v[c];
+  }
+  if (first && V.shared && !inside) {  // the second visit lies in another tile
+    const int px = (int)(col + dx + g.cx), py = (int)(row + dy + g.cy);
+    const int64_t pic = (int64_t)py * g.cols + px;
+    const bool ppv = pull && on_window_border(st.box, px, py);
+    if (paint) {
+      load_pixel(T, snap, pic, ppv, acc);
       if (clocked) {
         check_dry_regs(clk, acc.cv, acc.cvv, pic);
-        if (!T.use_snap) acc.src_from_canvas();
+        if (!snap) acc.src_from_canvas();
       }
-      run_pixel(T, pic, ppull, fh, pk, ps, acc);
-    }
+      paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
+      store_pixel(T, snap, pic, ppv, acc);
 #pragma unroll
-    for (int c = 0; c < 7; ++c) pick[c][mm] = acc.v[c];
+      for (int c = 0; c < 7; ++c) pick[c][V.mm] = acc.v[c];
+    } else if (clocked) {
+      check_only(T, clk, pic, ppv);
+    }
   }
-  __syncthreads();  // sm is rewritten by the block's next tile
+  __syncthreads();  // hand is rewritten by the block's next tile
 }
 
 // Is visit (col, row), at canvas pixel ic on the window border of box b,
@@ -592,6 +730,12 @@ __device__ __forceinline__ bool first_acting_visit(const StampGeom& g, const Rin
 // pixel when it is the first visit of that pixel that acts (footprint
 // height > 0, or any visit with a clock) in reference order; the ring scan
 // leaves such pixels alone.
+//
+// The block is one chain of levels (3, rarely 4) beside tiles that take one
+// round trip each, so what a level needs besides the pixels and cells is
+// fetched for all levels first: the list entries, their geometry and
+// footprint heights.  A level is then one round trip (17 us to 10 us of the
+// launches that hold such a stamp).
 template <int kThreads>
 __device__ __forceinline__ void level_visits(const VisitTarget& T, float* const* pick,
                                              const float* fp, const StampGeom& g, const PStamp& st,
@@ -599,20 +743,96 @@ __device__ __forceinline__ void level_visits(const VisitTarget& T, float* const*
                                              const float ps[3],
                                              const DryClock& clk = DryClock{},
                                              bool pull = false) {
-  for (int L = 0; L < st.dl_nlev; ++L) {
-    const int e0 = dl_off[st.dl_lev + L], e1 = dl_off[st.dl_lev + L + 1];
-    for (int e = e0 + (int)threadIdx.x; e < e1; e += kThreads) {
-      const int2 v = dl[e];
-      int64_t ic;
-      const int m = stamp_visit(g, v.x, v.y, &ic);
-      if (m < 0) continue;
-      const bool pv = pull && first_acting_visit(g, st.box, fp, v.x, v.y, ic, clk.tmap != nullptr);
-      if (clk.tmap) check_only(T, clk, ic, pv);  // with pv, the refresh comes first
-      if (fp[m] > 0.0f)
-        cached_visit(T, GlobalPick{pick, m}, fp[m], ic, pv && !clk.tmap, pk, ps);
+  const bool clocked = clk.tmap != nullptr;
+  const int nlev = st.dl_nlev;
+  const int* off = dl_off + st.dl_lev;
+  struct Entry {
+    int m;  // map cell, -1: none
+    float fh;
+    int64_t ic;
+    bool pv;
+  };
+  const auto fetch = [&](int e) {
+    const int2 v = dl[e];
+    Entry E;
+    E.m = stamp_visit(g, v.x, v.y, &E.ic);
+    E.fh = 0.0f;
+    E.pv = false;
+    if (E.m >= 0) {
+      E.fh = fp[E.m];
+      E.pv = pull && first_acting_visit(g, st.box, fp, v.x, v.y, E.ic, clocked);
     }
+    return E;
+  };
+  const auto visit = [&](const Entry& E) {
+    if (E.m < 0) return;
+    if (clocked) check_only(T, clk, E.ic, E.pv);  // with pv, the refresh comes first
+    if (E.fh > 0.0f) cached_visit(T, pick, E.m, E.fh, E.ic, E.pv && !clocked, pk, ps);
+  };
+  constexpr int kPre = 4;
+  Entry pre[kPre];
+#pragma unroll
+  for (int L = 0; L < kPre; ++L) {
+    pre[L].m = -1;
+    if (L < nlev && off[L] + (int)threadIdx.x < off[L + 1]) pre[L] = fetch(off[L] + (int)threadIdx.x);
+  }
+#pragma unroll
+  for (int L = 0; L < kPre; ++L) {
+    if (L >= nlev) break;
+    visit(pre[L]);
+    for (int e = off[L] + kThreads + (int)threadIdx.x; e < off[L + 1]; e += kThreads) visit(fetch(e));
     __builtin_amdgcn_s_waitcnt(0);  // this level's stores before the next level's loads
     __syncthreads();
+  }
+  for (int L = kPre; L < nlev; ++L) {
+    for (int e = off[L] + (int)threadIdx.x; e < off[L + 1]; e += kThreads) visit(fetch(e));
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  }
+}
+
+// What the stamps of a launch may need.
+//   clock  Canvas::checkDry on every visited pixel
+//   dup    stamps that straddle canvas column/row 0 (shared-pixel levels)
+//   kSnap  the snapshot buffer: 0 off, 1 on, 2 per stamp
+template <bool kClock, bool kDup, int kSnap>
+struct StampKind {
+  static constexpr bool clock = kClock, dup = kDup;
+  static __device__ __forceinline__ bool snap(int use_snap) {
+    return kSnap == 2 ? use_snap != 0 : kSnap == 1;
+  }
+};
+
+// What a stamp's block keeps in LDS: cells handed from a tile's first to its
+// second visits, or the groups of a ring pass.
+template <int kThreads>
+union StampLds {
+  float hand[7][kThreads];
+  RingList<kThreads> ring;
+};
+
+// Block b of one imprint whose window tiles, ring scan and shared-pixel
+// levels run side by side: blocks [0, ntiles) take a 16 x 16 window tile
+// each, the next rb scan the snapshot ring, and one more runs the levels of
+// a stamp that has them.  Visits on the window border refresh their own
+// snapshot pixels (the ring scan leaves them).
+template <class F>
+__device__ __forceinline__ void stamp_block(const VisitTarget& T, float* const* pick,
+                                            const float* fp, const FpBox& dom, const StampGeom& g,
+                                            const PStamp& st, const TileWin& win, int ntiles, int rb,
+                                            int b, StampLds<256>& lds, const int2* dl,
+                                            const int* dl_off, const float pk[3],
+                                            const float ps[3], const DryClock& clk) {
+  const bool dup = F::dup && (st.flags & (kStDupX | kStDupY)) != 0;
+  const bool pull = F::snap(T.use_snap);
+  if (b < ntiles) {
+    window_tile<16, F>(T, pick, fp, dom, g, st, dup, pull, tile_of_block(b, ntiles), win, lds.hand, pk,
+                       ps, clk);
+  } else if (b < ntiles + rb) {
+    ring_scan<256>(*T.canvas, *T.src, T.dirty, fp, g, st.box, pull, b - ntiles, rb, lds.ring,
+                   F::clock && clk.tmap != nullptr);
+  } else if (F::dup && dup) {
+    level_visits<256>(T, pick, fp, g, st, dl, dl_off, pk, ps, F::clock ? clk : DryClock{}, pull);
   }
 }
 

@@ -24,8 +24,8 @@ namespace pnt {
 
 constexpr int kWT = 16;          // window tile side of wave phases
 constexpr int kWT2 = kWT * kWT;  // threads per block
-// Waves per SIMD the wave kernels keep (at most 128 VGPRs): four workgroups
-// of a launch per CU.  They need 108-112; five (at most 102) spills.
+// Waves per SIMD the wave kernels keep (at most 128 VGPRs): the kernel of
+// plain stamps needs 101, the general one 116.
 constexpr int kWaveOccupancy = 4;
 
 enum : int {
@@ -53,9 +53,9 @@ struct SSlot {
   float* out[3];    // composite planes
   int cstride, mstride, dirty_bytes;
   int rows, cols;
-  int kind, start, nblk, ntiles, rb, hr, size_map, tiles_x;
+  int kind, start, nblk, rb, hr, size_map;
   int part, nparts;  // streaming kinds: part `part` of `nparts` of every range they cover
-  int fb[4];
+  int fb[4];  // the cells visits run over (cell_domain)
   float pk[3], ps[3];
   double pickup_rate, dep_rate, cap;
   int use_snap;
@@ -119,8 +119,9 @@ __device__ __forceinline__ void wave_compose_pixel(const Layer7& L, const float*
 }
 
 // Block b (of S.nblk) of phase S; all kWT2 threads of the block call it.
-template <int kG = kRingGroups>
-__device__ __forceinline__ void run_wave_slot(const SSlot& S, int b, int (*sm)[kWT + 2]) {
+// kStream: the wave may hold phases other than stamps and map clears.
+template <class F, bool kStream>
+__device__ __forceinline__ void run_wave_slot(const SSlot& S, int b, StampLds<kWT2>& lds) {
   const int tid = b * kWT2 + (int)threadIdx.x, nth = S.nblk * kWT2;
   const int64_t cs = S.cstride;
   const Layer7 canvas = layer_at(S.canvas, cs);
@@ -133,7 +134,11 @@ __device__ __forceinline__ void run_wave_slot(const SSlot& S, int b, int (*sm)[k
   int64_t lo4, hi4, lod, hid;
   part_range(cs / 4, S.part, S.nparts, lo4, hi4);
   part_range(S.dirty_bytes / 16, S.part, S.nparts, lod, hid);
-  switch (S.kind) {
+  if (S.kind == kSClear) {
+    wave_fill4(S.pick, 0, 7 * (int64_t)S.mstride / 4, 0.0f, tid, nth);
+    return;
+  }
+  if (kStream) switch (S.kind) {
     case kSInit: {
       // zero bits are 0.0f and 0.0: the wet layer (8 strides) and h
       for (int p = 0; p < kCanvasStrides; ++p)
@@ -155,15 +160,12 @@ __device__ __forceinline__ void run_wave_slot(const SSlot& S, int b, int (*sm)[k
         reinterpret_cast<uint4*>(S.dirty)[q] = make_uint4(0u, 0u, 0u, 0u);
       return;
     }
-    case kSClear:
-      wave_fill4(S.pick, 0, 7 * (int64_t)S.mstride / 4, 0.0f, tid, nth);
-      return;
     case kSCopyPick:
       for (int64_t q = tid; q < 7 * (int64_t)S.mstride / 4; q += nth)
         reinterpret_cast<float4*>(S.pick_dst)[q] = reinterpret_cast<const float4*>(S.pick)[q];
       return;
     case kSDry: {  // with a clock, dryCanvas also stamps every pixel's time (its last imprint's)
-      const int64_t now = S.tmap ? S.st->now_us : 0;
+      const int64_t now = S.tmap ? load_const<PStamp>(S.st).now_us : 0;
       int64_t lo, hi;
       part_range(n, S.part, S.nparts, lo, hi);
       for (int64_t i = lo + tid; i < hi; i += nth) {
@@ -181,18 +183,8 @@ __device__ __forceinline__ void run_wave_slot(const SSlot& S, int b, int (*sm)[k
     default:
       break;
   }
-  const PStamp& st = *S.st;
-  StampGeom g;
-  g.cx = st.cx;
-  g.cy = st.cy;
-  g.c = st.c;
-  g.s = st.s;
-  g.hr = S.hr;
-  g.size_map = S.size_map;
-  g.rows = S.rows;
-  g.cols = S.cols;
-  const bool dup = (st.flags & (kStDupX | kStDupY)) != 0;
-  const bool pull = S.use_snap != 0;  // border visits refresh their own snapshot pixels
+  const PStamp st = load_const<PStamp>(S.st);
+  const StampGeom g = stamp_geom(st, S.size_map, S.rows, S.cols);
   const VisitTarget T{&canvas, &snap, S.dirty, S.use_snap, S.pickup_rate, S.dep_rate, S.cap};
   float* pick[7];
 #pragma unroll
@@ -200,16 +192,9 @@ __device__ __forceinline__ void run_wave_slot(const SSlot& S, int b, int (*sm)[k
   const FpBox fb{S.fb[0], S.fb[1], S.fb[2], S.fb[3]};
   // Canvas::checkDry on every visited pixel when the canvas has a clock
   const DryClock ck{S.tmap, st.now_us, S.dry_ms, Rgb3{{R0, R0 + cs, R0 + 2 * cs}}, hp};
-  const int win = S.ntiles;
-  if (b < win) {
-    window_tile<kWT>(T, pick, S.fp, fb, g, st, dup, pull, tile_of_block(b, S.ntiles), S.tiles_x,
-                     sm, S.pk, S.ps, ck);
-  } else if (b < win + S.rb) {
-    ring_scan<kG>(canvas, snap, S.dirty, S.fp, g, st.box, pull, (b - win) * kWT2 + (int)threadIdx.x,
-                 S.rb * kWT2, S.tmap != nullptr);
-  } else if (dup) {  // the shared-pixel visits, beside the tiles
-    level_visits<kWT2>(T, pick, S.fp, g, st, S.dl, S.dl_off, S.pk, S.ps, ck, pull);
-  }
+  const TileWin tw = tile_window(g, fb);
+  stamp_block<F>(T, pick, S.fp, fb, g, st, tw, tile_count<kWT>(tw), S.rb, b, lds, S.dl,
+                     S.dl_off, S.pk, S.ps, ck);
 }
 
 // Blocks of a streaming phase over `items` work items (at most 2048).
