@@ -485,8 +485,11 @@ int pnt_dev_compose2_wet(pnt_ctx ctx, int64_t n, pnt_dev_wet dry,
  * (PaintMixer.cxx:327-355) over an n_pig palette (palK/palS n_pig x 3), then
  * R = Renderer::compose (Renderer.hxx:26-41).  pnt_grad_backward gives the
  * gradient of <gR, R> w.r.t. the initial wet layer (K0..S2, V planes), the
- * substrate R0 and W (n_paint x n_pig, row-major), by recomputing the stamp
- * state from checkpoints taken every seg_len stamps (and at every dip).
+ * substrate R0 and W (n_paint x n_pig, row-major).  The forward keeps every
+ * visit's input on a tape while the list's tapes fit 1/8 of the free device
+ * memory and 16 GiB (or PAINTY_GRAD_TAPE_MB); a longer list keeps checkpoints
+ * every seg_len stamps (and at every dip) and the backward reruns it from
+ * them.  The brush keeps its geometry and snapshot switch in between.
  * Device planes are caller-owned, n = rows*cols floats each; the brush's
  * pickup map and snapshot are used as scratch by both calls. */
 typedef struct pnt_grad_s* pnt_grad;

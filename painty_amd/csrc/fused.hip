@@ -61,6 +61,7 @@ struct StampShared {
   int rows, cols, use_snap, pad;
   int64_t* tmap;    // the canvas' drying clock (nullptr: none)
   int64_t dry_ms;
+  int64_t tape_area, tape_m;  // pixels and cells of a tape record (0: no tape)
 };
 
 StampShared stamp_shared(pnt_brush_s* b, pnt_canvas_s* cv, const int2* dl, const int* dl_off) {
@@ -96,6 +97,7 @@ struct WSlot {
   int64_t mstride;
   const float* fp;
   float* pick;         // the unit's pickup map (7 planes of mstride)
+  float* tape;         // the stamp's tape record (launches that keep one)
   FpBox dom;           // the cells its visits run over (cell_domain)
   TileWin win;
   float pk[3], ps[3];  // the brush paint of this stamp
@@ -131,7 +133,9 @@ __global__ __launch_bounds__(kT2, F::clock || F::dup ? 4 : 5) void k_stamp_wave(
   const PStamp& st = S.stamp;
   const StampGeom g = stamp_geom(st, S.size_map, H.rows, H.cols);
   const Layer7 canvas = layer_at(H.canvas, H.cs), snap = layer_at(H.snap, H.ss);
-  const VisitTarget T{&canvas, &snap, H.dirty, H.use_snap, H.pickup_rate, H.dep_rate, H.cap};
+  const TapeRec tape =
+      F::tape ? tape_rec(S.tape, H.tape_area, H.tape_m, st.box, H.cols) : TapeRec{};
+  const VisitTarget T{&canvas, &snap, H.dirty, H.use_snap, H.pickup_rate, H.dep_rate, H.cap, &tape};
   float* pick[7];
 #pragma unroll
   for (int c = 0; c < 7; ++c) pick[c] = S.pick + c * S.mstride;
@@ -159,6 +163,11 @@ void launch_slots(const WArgs<kSlots>& A, int n, hipStream_t q) {
                         : k_stamp_wave<StampKind<false, true, 0>, kSlots>)
                 : (snap ? k_stamp_wave<StampKind<false, false, 1>, kSlots>
                         : k_stamp_wave<StampKind<false, false, 0>, kSlots>);
+  if (A.sh.tape_area)  // a differentiable list: no clock
+    kernel = dup ? (snap ? k_stamp_wave<StampKind<false, true, 1, true>, kSlots>
+                         : k_stamp_wave<StampKind<false, true, 0, true>, kSlots>)
+                 : (snap ? k_stamp_wave<StampKind<false, false, 1, true>, kSlots>
+                         : k_stamp_wave<StampKind<false, false, 0, true>, kSlots>);
   kernel<<<dim3((unsigned)round_up(widest, 8), (unsigned)n), kT2, 0, q>>>(A);
   PNT_HIP_CHECK(hipGetLastError());
 }
@@ -406,11 +415,27 @@ struct ListGeo {
 // geo[k]; clear[k] cleans the pickup map before it (a geometry change).
 void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n,
                     const PlanDev& D, const std::vector<ListGeo>& geos, const std::vector<int>& geo,
-                    const std::vector<uint8_t>& clear, int want_chains) {
+                    const std::vector<uint8_t>& clear, int want_chains, TapeRun* tape = nullptr) {
   hipStream_t s = b->ctx->stream;
   b->last_launches = 0;
   if (b->ktimer) b->ktimer->used = 0;
-  const StampShared H = stamp_shared(b, cv, D.dl, D.dl_off);
+  StampShared H = stamp_shared(b, cv, D.dl, D.dl_off);
+  if (tape) {
+    PNT_REQUIRE(!H.tmap, "a taped stamp list takes no drying clock");
+    H.tape_area = tape->area;
+    H.tape_m = tape->m;
+    tape->waves.clear();
+    tape->st.assign(D.host, D.host + n);
+    tape->n_visits.assign((size_t)n, 0);
+    for (int64_t k = 0; k < n; ++k)
+      if (D.host[k].dl_nlev > 0)
+        tape->n_visits[(size_t)k] = D.host_off[D.host[k].dl_lev + D.host[k].dl_nlev] -
+                                    D.host_off[D.host[k].dl_lev];
+    tape->dl = D.dl;
+    tape->dl_off = D.dl_off;
+    tape->n_dl = D.n_dl;
+    tape->n_off = D.n_off;
+  }
   std::vector<FpBox> gdom(geos.size());
   std::vector<int64_t> gstride(geos.size());
   int64_t max_stride = 0;
@@ -512,6 +537,7 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
         }
         if (ready.empty()) break;  // the phase is done
         const int nslots = (int)ready.size();
+        if (tape) tape->waves.emplace_back();
         for (int q = 0; q < nslots; ++q) {
           const int i = ready[(size_t)q];
           const Ph& f = ph[(size_t)i][next[(size_t)i]];
@@ -519,6 +545,11 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
           const float* p = &paint[6 * (size_t)f.k];
           W.slot[q] = f.kind == kPhClear ? clear_slot(map, gstride[(size_t)geo[(size_t)f.k]])
                                          : slot_of(f.k, map, p, p + 3);
+          if (tape) {
+            W.slot[q].tape = tape->base + tape->slot * f.k;
+            tape->waves.back().push_back(
+                TapeRun::Phase{(int)f.k, f.kind == kPhClear ? 1 : 0, U[(size_t)i].chain});
+          }
         }
         ktimer_mark(b, s);
         launch_slots(W, nslots, s);
@@ -540,10 +571,10 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
   const bool one_geo = geos.size() == 1 && !geos[0].core;
   const int nchains = fused_chains(want_chains);
   std::vector<Unit> U;
-  if (nchains > 1 || !one_geo) U = plan_units(st, D.host, clear.data(), n, nchains);
+  if (nchains > 1 || !one_geo || tape) U = plan_units(st, D.host, clear.data(), n, nchains);
   int used = 1;
   for (const Unit& u : U) used = std::max(used, u.chain + 1);
-  if (used <= 1 && one_geo) {  // one chain, the brush's own map: the list in stream order
+  if (used <= 1 && one_geo && !tape) {  // one chain, the brush's own map: the list in stream order
     for (int64_t k = 0; k < n; ++k) {
       launch_stamp(k, s, b->pick);
       if (st[k].flags & PNT_STAMP_DRY_AFTER) dry(s);
@@ -567,7 +598,7 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
       S[c] = c == 0 ? s : F.streams[c];
       pick[c] = F.pick[c];
     }
-    if (fused_waves()) {
+    if (fused_waves() || tape) {
       // a first unit that continues the brush's stroke starts from its map
       if (!clear[0] && !(st[0].flags & PNT_STAMP_DIP))
         PNT_HIP_CHECK(hipMemcpyAsync(pick[0], b->pick,
@@ -638,12 +669,13 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
   }
 }
 
-void run_fused_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains) {
+void run_fused_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains,
+                 TapeRun* tape) {
   const PlanDev D = upload_plan(b, cv, st, n);
   const std::vector<ListGeo> geos{ListGeo{b->fp, b->size_map, b->radius, nullptr, b->width,
                                           FpBox{b->fbox[0], b->fbox[1], b->fbox[2], b->fbox[3]}}};
   run_fused_list(b, cv, st, n, D, geos, std::vector<int>((size_t)n, 0),
-                     std::vector<uint8_t>((size_t)n, 0), chains);
+                     std::vector<uint8_t>((size_t)n, 0), chains, tape);
 }
 
 // A stroke list: each stroke is FootprintBrush::setRadius(radius) with its
@@ -1133,8 +1165,9 @@ void run_fused_strokes(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* strok
   run_fused_strokes_t(b, cv, strokes, ns);
 }
 
-void run_fused(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains) {
-  if (n > 0) run_fused_t(b, cv, st, n, chains);
+void run_fused(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains,
+               TapeRun* tape) {
+  if (n > 0) run_fused_t(b, cv, st, n, chains, tape);
 }
 
 }  // namespace pnt

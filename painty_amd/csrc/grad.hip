@@ -5,29 +5,38 @@
 // the initial wet layer K, S, V, the substrate R0 and the mixing weights.
 // The reference has no gradients; this is the extension it is measured on.
 //
-// Forward: the stamps run as PNT_EXEC_FUSED, split into segments of at most
-// `seg_len` stamps that never cross a dip.  Before each segment the state it
-// can touch is checkpointed: the canvas and snapshot inside the union of its
-// stamps' snapshot boxes, and the pickup map.
+// Forward: the stamps run as PNT_EXEC_FUSED (waves of independent strokes),
+// each visit leaving what it found -- its map cell, canvas pixel and pickup
+// source -- on a tape, one record per stamp (TapeRec, stampcore.hpp).
 //
-// Backward, segment by segment from the last: restore the checkpoint and
-// recompute the segment stamp by stamp (ring copy | tape | visits), where the
-// tape of a stamp holds what its visits read -- the canvas and snapshot of
-// its window box after the ring copy, and the pickup map.  Then, from the
-// last stamp of the segment to the first:
-//   visits   k_adj_visits: each cell's visits replayed from the tape (the
-//            forward arithmetic of visit.hpp, so branches resolve the same
-//            way) and their adjoints applied in reverse order;
-//   shared   k_adj_shared: visits on a duplicated canvas column/row 0,
-//            replayed on the tape and reversed level by level;
-//   ring     k_adj_ring: the ring copy canvas -> snapshot moves the snapshot
-//            adjoint onto the canvas;
-//   dip      the pickup map was cleared: its adjoint is dropped.
-// The state is recomputed, not stored: memory is the checkpoints (a few MB
-// per segment) plus one segment of tapes.
+// Backward: the waves again, in reverse, one launch each (k_adj_wave): the
+// stamps of a wave touch disjoint pixels and maps, so their adjoints run side
+// by side as they did.  Per stamp
+//   tiles    each cell's visits replayed from the tape (the forward
+//            arithmetic of visit.hpp, so branches resolve the same way) and
+//            their adjoints applied in reverse order;
+//   ring     the snapshot refresh's adjoint: the snapshot's adjoint of a ring
+//            pixel moves onto the canvas', found by dirty bytes; a window
+//            border pixel with a visit is moved by that visit;
+//   levels   visits on a duplicated canvas column/row 0, replayed on the tape
+//            and reversed level by level;
+// and where the pickup map was cleared its adjoint is dropped.
+//
+// The tapes of a whole list may take kTapeFree of the free device memory (0.8
+// MB per stamp at radius 32).  A longer list keeps checkpoints instead: it is
+// cut into segments of at most `seg_len` stamps that never cross a dip, the
+// canvas and snapshot inside a segment's snapshot boxes and the pickup map are
+// saved before it, and backward restores and reruns the segment onto its tape.
+//
+// Bound: the chain of launches, one per wave (108 for 500 stamps on 2048^2),
+// each as long as one tile's round trips and FP64 arithmetic (16.5 us).  500
+// stamps of radius 32 on 2048^2, forward and backward: 30.3 ms with every
+// segment recomputed stamp by stamp (six launches and 48 us a stamp in the
+// backward, one stroke at a time), 3.9 ms from the tape.
 #include <algorithm>
 #include <initializer_list>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <vector>
@@ -44,6 +53,9 @@ namespace {
 
 constexpr int kGT = 16;  // window tile of the adjoint kernel
 constexpr int kBlk = 256;
+constexpr int kAdjSlots = 8;          // stamps of one adjoint launch (a wave of the forward)
+constexpr int64_t kTapeFree = 8;      // tapes take at most 1/8 of the free memory,
+constexpr int64_t kTapeMost = 16ll << 30;  // and 16 GiB
 
 // ------------------------------------------------------ visit adjoint ----
 struct VState {
@@ -203,62 +215,63 @@ __device__ __forceinline__ void visit_fwd(VState& s, float fh, double pr, double
   s.X[6] = alias ? acc.cvv : acc.svv;
 }
 
-// One stamp's tape: canvas and snapshot of the window box as the visits
-// find them (7 FP64 planes of `area` each: K, S widened, V as stored), then
-// the pickup map (7 FP32 planes of m).
-struct Tape {
-  const double* C;
-  const double* X;
-  const float* P;
+// One phase of an adjoint launch: a stamp, or the clear of a map's adjoint
+// (the pickup map was cleared there).
+struct ASlot {
+  int nblk, clear, ntiles, rb;
+  float* tape;     // the stamp's tape record
+  float* gP;       // its chain's pickup-map adjoint, 7 planes of m
+  float* gB;       // 6 floats: the stamp's paint adjoint
+  float* scratch;  // records of the shared-pixel replay
+  TileWin win;
+  float pk[3], ps[3];
+  PStamp st;
+};
+
+struct AShared {
+  const float* fp;
+  FpBox dom;
+  int size_map, rows, cols, use_snap;
   int64_t area, m;
-  int bx0, by0, bw, bh;
+  Plane7 gC, gX;        // adjoints: canvas (caller's planes), snapshot
+  uint8_t* dirty;       // 0: the pixel's snapshot adjoint is zero
+  const int2* dl;       // shared-pixel visits (plan lists)
+  const int* dl_off;
+  double pr, dr, cap;
 };
 
 struct AArgs {
-  const PStamp* st;
-  int j;  // stamp index into st
-  int hr, size_map, rows, cols, tiles_x, ntiles, use_snap;
-  const float* fp;
-  Tape t;
-  Plane7 gC, gX, gP;  // adjoints: canvas (caller's planes), snapshot, pickup map
-  float* gB;          // 6 floats of this stamp's paint adjoint
-  double pr, dr, cap;
-  float pk[3], ps[3];
-  // shared-pixel visits of this stamp (plan lists) and their scratch
-  const int2* dl;
-  const int* dl_off;
-  float* scratch;  // per-visit records of the shared-pixel replay
+  AShared sh;
+  ASlot slot[kAdjSlots];
 };
+static_assert(sizeof(AArgs) <= 4000, "kernel arguments must fit the argument segment");
 
-__device__ __forceinline__ StampGeom geom_of(const AArgs& A, const PStamp& st) {
-  StampGeom g;
-  g.cx = st.cx;
-  g.cy = st.cy;
-  g.c = st.c;
-  g.s = st.s;
-  g.hr = A.hr;
-  g.size_map = A.size_map;
-  g.rows = A.rows;
-  g.cols = A.cols;
-  return g;
-}
-
-__device__ __forceinline__ int64_t tape_index(const Tape& t, int64_t ic, int cols) {
-  const int x = (int)(ic % cols), y = (int)(ic / cols);
-  return (int64_t)(y - t.by0) * t.bw + (x - t.bx0);
-}
-
-__device__ __forceinline__ void load_in(const AArgs& A, int64_t ic, int mm, VState& s) {
-  const int64_t k = tape_index(A.t, ic, A.cols);
+__device__ __forceinline__ void load_in(const TapeRec& t, bool snap, int64_t k, int mm, VState& s) {
 #pragma unroll
-  for (int c = 0; c < 7; ++c) {
-    s.P[c] = A.t.P[c * A.t.m + mm];
-    s.C[c] = A.t.C[c * A.t.area + k];
-    s.X[c] = A.use_snap ? A.t.X[c * A.t.area + k] : 0.0;
+  for (int c = 0; c < 7; ++c) s.P[c] = t.P[c * t.m + mm];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    s.C[c] = t.ck[c * t.area + k];
+    s.X[c] = snap ? t.xk[c * t.area + k] : 0.0f;
   }
+  s.C[6] = t.cv[k];
+  s.X[6] = snap ? t.xv[k] : 0.0;
 }
 
-__device__ __forceinline__ void load_g_pixel(const AArgs& A, int64_t ic, VState& g) {
+__device__ __forceinline__ void store_in(const TapeRec& t, bool snap, int64_t k, int mm,
+                                         const VState& s) {
+#pragma unroll
+  for (int c = 0; c < 7; ++c) t.P[c * t.m + mm] = s.P[c];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    t.ck[c * t.area + k] = (float)s.C[c];
+    if (snap) t.xk[c * t.area + k] = (float)s.X[c];
+  }
+  t.cv[k] = s.C[6];
+  if (snap) t.xv[k] = s.X[6];
+}
+
+__device__ __forceinline__ void load_g_pixel(const AShared& A, int64_t ic, VState& g) {
 #pragma unroll
   for (int c = 0; c < 7; ++c) {
     g.C[c] = A.gC.p[c][ic];
@@ -266,98 +279,143 @@ __device__ __forceinline__ void load_g_pixel(const AArgs& A, int64_t ic, VState&
   }
 }
 
-__device__ __forceinline__ void store_g_pixel(const AArgs& A, int64_t ic, const VState& g) {
+// `moved`: the stamp's ring refresh copied this pixel before its visits, so
+// the snapshot's adjoint goes on to the canvas.
+__device__ __forceinline__ void store_g_pixel(const AShared& A, int64_t ic, const VState& g,
+                                              bool moved) {
 #pragma unroll
   for (int c = 0; c < 7; ++c) {
-    A.gC.p[c][ic] = (float)g.C[c];
-    if (A.use_snap) A.gX.p[c][ic] = (float)g.X[c];
+    const float gc = (float)g.C[c], gx = (float)g.X[c];
+    A.gC.p[c][ic] = moved ? gc + gx : gc;
+    if (A.use_snap) A.gX.p[c][ic] = moved ? 0.0f : gx;
+  }
+  if (A.use_snap) A.dirty[ic] = moved ? 0 : 1;
+}
+
+// Adds the block's paint adjoints to out[6]: summed over each wave by
+// shuffles, over its waves in LDS, one atomic per value and block.
+__device__ __forceinline__ void flush_gB(float* out, const float gB[6]) {
+  __shared__ float s_gB[kBlk / 64][6];
+  float v[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    v[c] = gB[c];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v[c] += __shfl_xor(v[c], d);
+  }
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int c = 0; c < 6; ++c) s_gB[threadIdx.x >> 6][c] = v[c];
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    float t = 0.0f;
+    for (int w = 0; w < kBlk / 64; ++w) t += s_gB[w][threadIdx.x];
+    if (t != 0.0f) atomicAdd(&out[threadIdx.x], t);
   }
 }
 
-__device__ __forceinline__ void flush_gB(const AArgs& A, const float gB[6]) {
-  __shared__ float s_gB[6];
-  if (threadIdx.x < 6) s_gB[threadIdx.x] = 0.0f;
-  __syncthreads();
-#pragma unroll
-  for (int c = 0; c < 6; ++c)
-    if (gB[c] != 0.0f) atomicAdd(&s_gB[c], gB[c]);
-  __syncthreads();
-  if (threadIdx.x < 6 && s_gB[threadIdx.x] != 0.0f) atomicAdd(&A.gB[threadIdx.x], s_gB[threadIdx.x]);
-}
-
-// Adjoint of the visits of one stamp that do not share a canvas pixel, one
-// kGT x kGT window tile per block (cells and partners as window_tile).
-__global__ __launch_bounds__(kGT* kGT) void k_adj_visits(AArgs A) {
-  __shared__ int sm[kGT + 2][kGT + 2];
-  const PStamp& st = A.st[A.j];
-  const StampGeom g = geom_of(A, st);
-  const bool dup = (st.flags & (kStDupX | kStDupY)) != 0;
-  const int tile = blockIdx.x;
+// Adjoint of the visits of one kGT x kGT window tile that do not share a
+// canvas pixel; a cell's first visitor runs both its visits' adjoints.
+__device__ __forceinline__ void adj_tile(const AShared& A, const ASlot& S, const StampGeom& g,
+                                         const TapeRec& tape, bool dup, int tile) {
   const int t = threadIdx.x, lx = t % kGT, ly = t / kGT;
-  const int col0 = -g.hr + (tile % A.tiles_x) * kGT;
-  const int row0 = -g.hr + (tile / A.tiles_x) * kGT;
-  for (int e = t; e < (kGT + 2) * (kGT + 2); e += kGT * kGT) {
-    const int hy = e / (kGT + 2), hx = e % (kGT + 2);
-    int64_t ic;
-    sm[hy][hx] = stamp_visit(g, col0 + hx - 1, row0 + hy - 1, &ic);
-  }
-  __syncthreads();
+  const int tiles_x = (S.win.cols + kGT - 1) / kGT;
+  const int col = S.win.col0 + (tile % tiles_x) * kGT + lx;
+  const int row = S.win.row0 + (tile / tiles_x) * kGT + ly;
   float gB[6] = {0, 0, 0, 0, 0, 0};
-  const int mm = sm[ly + 1][lx + 1];
-  if (mm >= 0 && sm[ly + 1][lx] != mm && sm[ly][lx + 1] != mm) {
-    const int col = col0 + lx, row = row0 + ly;
-    const int pdir = sm[ly + 1][lx + 2] == mm ? 1 : (sm[ly + 2][lx + 1] == mm ? 2 : 0);
-    const bool skip = dup && (on_dup_line(st, col, row) ||
-                              (pdir && on_dup_line(st, col + (pdir == 1), row + (pdir == 2))));
-    const float fh = A.fp[mm];
-    if (!skip && fh > 0.0f) {
-      const bool alias = !A.use_snap;
-      const int64_t ic1 = canvas_index(g, col, row);
-      VState in1, gs;
-      load_in(A, ic1, mm, in1);
+  const VisitCell V = visit_cell(g, A.dom, col, row);
+  const int dx = V.shared == 3 ? 1 : 0, dy = V.shared == 4 ? 1 : 0;
+  const bool two = V.shared >= 3;
+  bool act = V.mm >= 0 && V.shared != 1 && V.shared != 2;
+  if (dup && act && (on_dup_line(S.st, col, row) || (two && on_dup_line(S.st, col + dx, row + dy))))
+    act = false;
+  const float fh = act ? A.fp[V.mm] : 0.0f;
+  if (fh > 0.0f) {
+    const bool snap = A.use_snap != 0, alias = !snap;
+    const int64_t ic1 = (int64_t)V.y * A.cols + V.x;
+    VState in1, gs;
+    load_in(tape, snap, tape.at(V.x, V.y), V.mm, in1);
 #pragma unroll
-      for (int c = 0; c < 7; ++c) gs.P[c] = A.gP.p[c][mm];
-      if (pdir) {
-        const int64_t ic2 = canvas_index(g, col + (pdir == 1), row + (pdir == 2));
-        VState in2 = in1;
-        visit_fwd(in2, fh, A.pr, A.dr, A.cap, A.pk, A.ps, alias);  // pickup cell after visit 1
-        const int64_t k2 = tape_index(A.t, ic2, A.cols);
+    for (int c = 0; c < 7; ++c) gs.P[c] = S.gP[c * A.m + V.mm];
+    if (two) {
+      const int x2 = (int)(col + dx + g.cx), y2 = (int)(row + dy + g.cy);
+      const int64_t ic2 = (int64_t)y2 * A.cols + x2;
+      VState in2 = in1;
+      visit_fwd(in2, fh, A.pr, A.dr, A.cap, S.pk, S.ps, alias);  // pickup cell after visit 1
+      float P2[7];
 #pragma unroll
-        for (int c = 0; c < 7; ++c) {
-          in2.C[c] = A.t.C[c * A.t.area + k2];
-          in2.X[c] = A.use_snap ? A.t.X[c * A.t.area + k2] : 0.0;
-        }
-        load_g_pixel(A, ic2, gs);
-        visit_adj(in2, gs, gB, fh, A.pr, A.dr, A.cap, A.pk, A.ps, alias);
-        store_g_pixel(A, ic2, gs);
+      for (int c = 0; c < 7; ++c) P2[c] = in2.P[c];
+      load_in(tape, snap, tape.at(x2, y2), V.mm, in2);
+#pragma unroll
+      for (int c = 0; c < 7; ++c) in2.P[c] = P2[c];
+      load_g_pixel(A, ic2, gs);
+      visit_adj(in2, gs, gB, fh, A.pr, A.dr, A.cap, S.pk, S.ps, alias);
+      store_g_pixel(A, ic2, gs, snap && on_window_border(S.st.box, x2, y2));
+    }
+    load_g_pixel(A, ic1, gs);
+    visit_adj(in1, gs, gB, fh, A.pr, A.dr, A.cap, S.pk, S.ps, alias);
+    store_g_pixel(A, ic1, gs, snap && on_window_border(S.st.box, V.x, V.y));
+#pragma unroll
+    for (int c = 0; c < 7; ++c) S.gP[c * A.m + V.mm] = gs.P[c];
+  }
+  flush_gB(S.gB, gB);
+}
+
+// Adjoint of the ring copy canvas -> snapshot (FootprintBrush.hxx:307-318) by
+// block `blk` of S.rb: the pixels of the allowed box, outside the window
+// interior, whose snapshot adjoint may be nonzero (dirty bytes, read eight at
+// a time) and that no visit of the stamp moves itself.
+__device__ __forceinline__ void adj_ring(const AShared& A, const ASlot& S, const StampGeom& g,
+                                         int blk) {
+  const RingBox& b = S.st.box;
+  const int span = b.a_x1 - b.a_x0 + 1;
+  const int per_row = (span + kRingUnit - 1) / kRingUnit + 1;
+  const int total = per_row * (b.a_y1 - b.a_y0 + 1);
+  for (int e = blk * kBlk + (int)threadIdx.x; e < total; e += S.rb * kBlk) {
+    const int r = e / per_row, row = b.a_y0 + r;
+    const int64_t rowi = (int64_t)row * A.cols, lo = rowi + b.a_x0;
+    const int64_t base = (lo & ~(int64_t)(kRingUnit - 1)) + kRingUnit * (int64_t)(e - r * per_row);
+    const int x0 = (int)(base - rowi);
+    const bool interior_row = row > b.tl_y && row < b.br_y;
+    if (x0 > b.a_x1 || (interior_row && x0 > b.tl_x && x0 + kRingUnit - 1 < b.br_x)) continue;
+    const uint2 d = *reinterpret_cast<const uint2*>(A.dirty + base);
+    if (!(d.x | d.y)) continue;
+    for (int q = 0; q < kRingUnit; ++q) {
+      if (!((((q < 4 ? d.x : d.y) >> (8 * (q & 3)))) & 0xffu)) continue;
+      const int col = x0 + q;
+      if (col < b.a_x0 || col > b.a_x1) continue;
+      if (interior_row && col > b.tl_x && col < b.br_x) continue;
+      if (on_window_border(b, col, row) && ring_pixel_visited(g, b, A.fp, col, row)) continue;
+      const int64_t i = base + q;
+      float c[7], x[7];
+#pragma unroll
+      for (int k = 0; k < 7; ++k) {
+        c[k] = A.gC.p[k][i];
+        x[k] = A.gX.p[k][i];
       }
-      load_g_pixel(A, ic1, gs);
-      visit_adj(in1, gs, gB, fh, A.pr, A.dr, A.cap, A.pk, A.ps, alias);
-      store_g_pixel(A, ic1, gs);
 #pragma unroll
-      for (int c = 0; c < 7; ++c) A.gP.p[c][mm] = gs.P[c];
+      for (int k = 0; k < 7; ++k) {
+        A.gC.p[k][i] = c[k] + x[k];
+        A.gX.p[k][i] = 0.0f;
+      }
+      A.dirty[i] = 0;
     }
   }
-  flush_gB(A, gB);
 }
 
 // Adjoint of a stamp's visits on a duplicated canvas column/row 0 and their
 // partners.  Only these visits touch those pixels and cells, so the tape
-// holds their true starting state; the tape of stamp j is not read after
-// its adjoint, so the replay runs on it in place.  Visits are replayed level
-// by level (a level's visits share no map cell and no canvas pixel, so each
-// level runs in parallel), each visit's input recorded; then the adjoints
-// run level by level in reverse.
-__global__ __launch_bounds__(kBlk) void k_adj_shared(AArgs A) {
-  const PStamp& st = A.st[A.j];
-  if (st.dl_nlev <= 0) return;
+// holds their true starting state, and the replay runs on it in place: visits
+// level by level (a level's visits share no map cell and no canvas pixel, so
+// each level runs in parallel), each visit's input recorded; then the adjoints
+// level by level in reverse, each putting its input back on the tape.
+// The first visit of a border pixel that acts moves its snapshot adjoint.
+__device__ __forceinline__ void adj_levels(const AShared& A, const ASlot& S, const StampGeom& g,
+                                           const TapeRec& t) {
+  const PStamp& st = S.st;
   const int base = A.dl_off[st.dl_lev];
-  VState* rec = reinterpret_cast<VState*>(A.scratch);
-  const StampGeom g = geom_of(A, st);
-  const bool alias = !A.use_snap;
-  double* wC = const_cast<double*>(A.t.C);  // C, X (7 planes of area each), P (7 of m)
-  double* wX = const_cast<double*>(A.t.X);
-  float* wP = const_cast<float*>(A.t.P);
+  VState* rec = reinterpret_cast<VState*>(S.scratch);
+  const bool snap = A.use_snap != 0, alias = !snap;
   for (int L = 0; L < st.dl_nlev; ++L) {  // replay in plan order, a level at a time
     const int e0 = A.dl_off[st.dl_lev + L], e1 = A.dl_off[st.dl_lev + L + 1];
     for (int e = e0 + (int)threadIdx.x; e < e1; e += kBlk) {
@@ -365,22 +423,12 @@ __global__ __launch_bounds__(kBlk) void k_adj_shared(AArgs A) {
       int64_t ic;
       const int mm = stamp_visit(g, v.x, v.y, &ic);
       if (mm < 0 || !(A.fp[mm] > 0.0f)) continue;
-      const int64_t k = tape_index(A.t, ic, A.cols);
+      const int64_t k = t.at((int)(ic % A.cols), (int)(ic / A.cols));
       VState sv;
-#pragma unroll
-      for (int c = 0; c < 7; ++c) {
-        sv.P[c] = wP[c * A.t.m + mm];
-        sv.C[c] = wC[c * A.t.area + k];
-        sv.X[c] = A.use_snap ? wX[c * A.t.area + k] : 0.0;
-      }
+      load_in(t, snap, k, mm, sv);
       rec[e - base] = sv;
-      visit_fwd(sv, A.fp[mm], A.pr, A.dr, A.cap, A.pk, A.ps, alias);
-#pragma unroll
-      for (int c = 0; c < 7; ++c) {
-        wP[c * A.t.m + mm] = sv.P[c];
-        wC[c * A.t.area + k] = sv.C[c];
-        if (A.use_snap) wX[c * A.t.area + k] = sv.X[c];
-      }
+      visit_fwd(sv, A.fp[mm], A.pr, A.dr, A.cap, S.pk, S.ps, alias);
+      store_in(t, snap, k, mm, sv);
     }
     __builtin_amdgcn_s_waitcnt(0);  // this level's stores before the next level's loads
     __syncthreads();
@@ -395,41 +443,61 @@ __global__ __launch_bounds__(kBlk) void k_adj_shared(AArgs A) {
       if (mm < 0 || !(A.fp[mm] > 0.0f)) continue;
       VState gs;
 #pragma unroll
-      for (int c = 0; c < 7; ++c) gs.P[c] = A.gP.p[c][mm];
+      for (int c = 0; c < 7; ++c) gs.P[c] = S.gP[c * A.m + mm];
       load_g_pixel(A, ic, gs);
-      visit_adj(rec[e - base], gs, gB, A.fp[mm], A.pr, A.dr, A.cap, A.pk, A.ps, alias);
-      store_g_pixel(A, ic, gs);
+      const VState in = rec[e - base];
+      store_in(t, snap, t.at((int)(ic % A.cols), (int)(ic / A.cols)), mm, in);
+      visit_adj(in, gs, gB, A.fp[mm], A.pr, A.dr, A.cap, S.pk, S.ps, alias);
+      store_g_pixel(A, ic, gs, snap && first_acting_visit(g, st.box, A.fp, v.x, v.y, ic, false));
 #pragma unroll
-      for (int c = 0; c < 7; ++c) A.gP.p[c][mm] = gs.P[c];
+      for (int c = 0; c < 7; ++c) S.gP[c * A.m + mm] = gs.P[c];
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
   }
-  flush_gB(A, gB);
+  flush_gB(S.gB, gB);
 }
 
-// Adjoint of the ring copy canvas -> snapshot (FootprintBrush.hxx:307-318).
-__global__ __launch_bounds__(kBlk) void k_adj_ring(RingBox b, int cols, Plane7 gC, Plane7 gX) {
-  const int w = b.a_x1 - b.a_x0 + 1;
-  const int64_t total = (int64_t)w * (b.a_y1 - b.a_y0 + 1);
-  for (int64_t e = (int64_t)blockIdx.x * kBlk + threadIdx.x; e < total;
-       e += (int64_t)gridDim.x * kBlk) {
-    const int row = b.a_y0 + (int)(e / w), col = b.a_x0 + (int)(e % w);
-    if (row > b.tl_y && row < b.br_y && col > b.tl_x && col < b.br_x) continue;
-    const int64_t i = (int64_t)row * cols + col;
-#pragma unroll
-    for (int c = 0; c < 7; ++c) {
-      gC.p[c][i] += gX.p[c][i];
-      gX.p[c][i] = 0.0f;
-    }
+// One wave of the forward, reversed: slot y of the grid's rows.
+template <bool kDup>
+__global__ __launch_bounds__(kBlk) void k_adj_wave(AArgs A) {
+  const ASlot& S = A.slot[blockIdx.y];
+  const int b = (int)blockIdx.x;
+  if (b >= S.nblk) return;
+  if (S.clear) {
+    for (int64_t i = (int64_t)b * kBlk + threadIdx.x; i < 7 * A.sh.m; i += (int64_t)S.nblk * kBlk)
+      S.gP[i] = 0.0f;
+    return;
   }
+  const StampGeom g = stamp_geom(S.st, A.sh.size_map, A.sh.rows, A.sh.cols);
+  const TapeRec tape = tape_rec(S.tape, A.sh.area, A.sh.m, S.st.box, A.sh.cols);
+  const bool dup = kDup && (S.st.flags & (kStDupX | kStDupY)) != 0;
+  if (b < S.ntiles)
+    adj_tile(A.sh, S, g, tape, dup, b);
+  else if (b < S.ntiles + S.rb)
+    adj_ring(A.sh, S, g, b - S.ntiles);
+  else if (dup)
+    adj_levels(A.sh, S, g, tape);
 }
 
-// Adjoint of the first imprint's full canvas -> snapshot copy.
-__global__ __launch_bounds__(kBlk) void k_adj_full_copy(int64_t n, Plane7 gC, Plane7 gX) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlk + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlk)
+// Adjoint of the first imprint's full canvas -> snapshot copy, where the
+// snapshot's adjoint may be nonzero; it ends all zero, and so do the dirty
+// bytes (the next backward starts from that).  A thread takes eight pixels.
+__global__ __launch_bounds__(kBlk) void k_adj_full_copy(int64_t n, Plane7 gC, Plane7 gX,
+                                                        uint8_t* dirty) {
+  const int64_t units = (n + 7) / 8;
+  for (int64_t u = (int64_t)blockIdx.x * kBlk + threadIdx.x; u < units; u += (int64_t)gridDim.x * kBlk) {
+    const uint2 d = reinterpret_cast<const uint2*>(dirty)[u];
+    if (!(d.x | d.y)) continue;
+    for (int64_t i = 8 * u; i < 8 * u + 8 && i < n; ++i)
+      if (dirty[i])
 #pragma unroll
-    for (int c = 0; c < 7; ++c) gC.p[c][i] += gX.p[c][i];
+        for (int c = 0; c < 7; ++c) {
+          gC.p[c][i] += gX.p[c][i];
+          gX.p[c][i] = 0.0f;
+        }
+    reinterpret_cast<uint2*>(dirty)[u] = make_uint2(0u, 0u);
+  }
 }
 
 // Adjoint of ComputeReflectance (KubelkaMunk.hxx:25-83) in the stable form
@@ -631,10 +699,18 @@ struct pnt_grad_s {
   int64_t ckpt_cap = 0;
   float* tape = nullptr;
   int64_t tape_cap = 0;
-  float* gX = nullptr;  // 7 planes of round_up(n, 64) (snapshot adjoint)
-  float* gP = nullptr;  // 7 planes of m (pickup adjoint)
+  bool full_tape = false;  // the last forward taped the whole list
+  TapeRun run;
+  int2* dl = nullptr;      // the taped list's shared-pixel visits (the brush may plan again)
+  int* dl_off = nullptr;
+  int64_t dl_cap = 0, dl_off_cap = 0;
+  int fwd_size_map = 0;    // the brush's geometry at the forward
+  bool fwd_snap = false;
+  float* gX = nullptr;  // 7 planes of round_up(n, 64) (snapshot adjoint); zero between calls
+  uint8_t* gdirty = nullptr;  // its dirty bytes; zero between calls
+  float* gP = nullptr;  // per chain: 7 planes of m (pickup adjoint)
   float* gB = nullptr;  // n_stamps x 6
-  int64_t gX_cap = 0, gP_cap = 0, gB_cap = 0;
+  int64_t gX_cap = 0, gdirty_cap = 0, gP_cap = 0, gB_cap = 0;
   float* scratch = nullptr;
   int64_t scratch_cap = 0;
   bool have_forward = false;
@@ -663,20 +739,101 @@ Plane7 dense7(float* base, int64_t stride) {
   return L;
 }
 
-// Window box of a stamp (canvas pixels its visits can touch), clipped.
-void window_box(const PStamp& p, int rows, int cols, int* x0, int* y0, int* w, int* h) {
-  const int a = std::max(p.box.tl_x, 0), c = std::min(p.box.br_x, cols - 1);
-  const int e = std::max(p.box.tl_y, 0), f = std::min(p.box.br_y, rows - 1);
-  *x0 = a;
-  *y0 = e;
-  *w = std::max(c - a + 1, 0);
-  *h = std::max(f - e + 1, 0);
-}
-
 }  // namespace
 
 static void check_status(int st) {
   if (st != PNT_OK) throw Error(st, pnt_last_error());
+}
+
+// The taped run's shared-pixel lists, copied: the brush's plan is its own.
+static void keep_lists(pnt_grad_s* g, hipStream_t s) {
+  TapeRun& R = g->run;
+  if (R.n_dl == 0) return;
+  ensure(g->dl, g->dl_cap, R.n_dl, s);
+  ensure(g->dl_off, g->dl_off_cap, R.n_off, s);
+  PNT_HIP_CHECK(hipMemcpyAsync(g->dl, R.dl, (size_t)R.n_dl * sizeof(int2), hipMemcpyDeviceToDevice, s));
+  PNT_HIP_CHECK(hipMemcpyAsync(g->dl_off, R.dl_off, (size_t)R.n_off * sizeof(int),
+                               hipMemcpyDeviceToDevice, s));
+}
+
+// The adjoint of the taped run (stamps s0 .. of the list), its waves in
+// reverse.  Every chain's map adjoint goes on from where it stands.
+static void adjoint_waves(pnt_grad_s* g, int s0, const Plane7& gC, const Plane7& gX, hipStream_t s) {
+  const TapeRun& R = g->run;
+  pnt_brush b = g->b;
+  AArgs A{};
+  A.sh.fp = b->fp;
+  A.sh.dom = FpBox{b->fbox[0], b->fbox[1], b->fbox[2], b->fbox[3]};
+  A.sh.size_map = b->size_map;
+  A.sh.rows = g->rows;
+  A.sh.cols = g->cols;
+  A.sh.use_snap = b->use_snap ? 1 : 0;
+  A.sh.area = R.area;
+  A.sh.m = R.m;
+  A.sh.gC = gC;
+  A.sh.gX = gX;
+  A.sh.dirty = g->gdirty;
+  A.sh.dl = g->dl;
+  A.sh.dl_off = g->dl_off;
+  A.sh.pr = b->pickup_rate;
+  A.sh.dr = b->dep_rate;
+  A.sh.cap = b->cap;
+  const int64_t rec = R.n_dl * (int64_t)(sizeof(VState) / sizeof(float));  // one per listed visit
+  if (rec) ensure(g->scratch, g->scratch_cap, rec, s);
+  std::vector<int> dl0;  // first listed visit of each stamp
+  if (R.n_dl) {
+    dl0.assign(R.st.size(), 0);
+    int at = 0;
+    for (size_t k = 0; k < R.st.size(); ++k) {
+      dl0[k] = at;
+      if (R.st[k].dl_nlev > 0) at += R.n_visits[k];
+    }
+  }
+  // the last dip up to every stamp (its paint is the brush's; stamp 0 dips)
+  int dip = s0;
+  while (!(g->st[(size_t)dip].flags & PNT_STAMP_DIP)) --dip;
+  std::vector<int> dip_of(R.st.size());
+  for (size_t k = 0; k < R.st.size(); ++k) {
+    if (g->st[(size_t)s0 + k].flags & PNT_STAMP_DIP) dip = s0 + (int)k;
+    dip_of[k] = dip;
+  }
+  for (size_t w = R.waves.size(); w-- > 0;) {
+    int ns = 0, widest = 1;
+    bool dup = false;
+    for (const TapeRun::Phase& f : R.waves[w]) {
+      ASlot& S = A.slot[ns++];
+      S = ASlot{};
+      S.clear = f.clear;
+      S.gP = g->gP + (int64_t)f.chain * 7 * R.m;
+      if (f.clear) {
+        S.nblk = (int)std::min<int64_t>(64, (7 * R.m + 4 * kBlk - 1) / (4 * kBlk));
+      } else {
+        const PStamp& st = R.st[(size_t)f.k];
+        S.st = st;
+        S.tape = R.base + R.slot * f.k;
+        S.gB = g->gB + 6 * (int64_t)(s0 + f.k);
+        S.scratch = R.n_dl ? g->scratch + dl0[(size_t)f.k] * (int64_t)(sizeof(VState) / sizeof(float))
+                           : nullptr;
+        S.win = tile_window(stamp_geom(st, b->size_map, g->rows, g->cols), A.sh.dom);
+        S.ntiles = tile_count<kGT>(S.win);
+        S.rb = b->use_snap ? ring_blocks_for(st.box, kBlk) : 0;
+        S.nblk = S.ntiles + S.rb + (dup_levels(st) ? 1 : 0);
+        for (int c = 0; c < 3; ++c) {
+          S.pk[c] = g->st[(size_t)dip_of[(size_t)f.k]].K[c];
+          S.ps[c] = g->st[(size_t)dip_of[(size_t)f.k]].S[c];
+        }
+        dup |= (st.flags & (kStDupX | kStDupY)) != 0;
+      }
+      widest = std::max(widest, S.nblk);
+    }
+    if (!ns) continue;
+    const dim3 grid((unsigned)widest, (unsigned)ns);
+    if (dup)
+      k_adj_wave<true><<<grid, kBlk, 0, s>>>(A);
+    else
+      k_adj_wave<false><<<grid, kBlk, 0, s>>>(A);
+    PNT_HIP_CHECK(hipGetLastError());
+  }
 }
 
 extern "C" {
@@ -733,6 +890,9 @@ int pnt_grad_destroy(pnt_grad g) {
     (void)hipFree(g->ckpt);
     (void)hipFree(g->tape);
     (void)hipFree(g->gX);
+    (void)hipFree(g->gdirty);
+    (void)hipFree(g->dl);
+    (void)hipFree(g->dl_off);
     (void)hipFree(g->gP);
     (void)hipFree(g->gB);
     (void)hipFree(g->scratch);
@@ -774,54 +934,86 @@ int pnt_grad_forward(pnt_grad g, pnt_dev_layer wet0, pnt_dev_rgb R0, const doubl
         g->st[i].S[c] = (float)S[c];
       }
     }
+    // the brush's calls run on its own context's stream
+    const bool other = b->ctx->stream != s;
+    if (other) PNT_HIP_CHECK(hipStreamSynchronize(s));
     // the first imprint on a canvas copies it whole into the snapshot
     if (b->use_snap) brush_full_snapshot(b, cv);
-    // segments (at most seg_len stamps, a dip starts a new one) and their
-    // checkpoint boxes: the union of their snapshot boxes (window boxes
-    // without the snapshot)
     g->segs.clear();
     const int ns = (int)g->st.size();
-    int64_t total = 0;
-    const int64_t m = b->m;
-    for (int s0 = 0; s0 < ns;) {
-      int s1 = s0 + 1;
-      while (s1 < ns && s1 - s0 < g->seg_len && !(g->st[s1].flags & PNT_STAMP_DIP)) ++s1;
-      int x0 = cv->cols, y0 = cv->rows, x1 = -1, y1 = -1;
-      for (int i = s0; i < s1; ++i) {
-        const StampArgs a = stamp_args(b, cv, g->st[i].cx, g->st[i].cy, g->st[i].theta);
-        const RingBox rb = ring_box(a.g, b->radius);
-        int bx0 = rb.a_x0, by0 = rb.a_y0, bx1 = rb.a_x1, by1 = rb.a_y1;
-        if (!b->use_snap) {
-          bx0 = std::max(rb.tl_x, 0);
-          by0 = std::max(rb.tl_y, 0);
-          bx1 = std::min(rb.br_x, cv->cols - 1);
-          by1 = std::min(rb.br_y, cv->rows - 1);
-        }
-        if (bx1 < bx0 || by1 < by0) continue;
-        x0 = std::min(x0, bx0);
-        y0 = std::min(y0, by0);
-        x1 = std::max(x1, bx1);
-        y1 = std::max(y1, by1);
-      }
-      pnt_grad_s::Seg sg{s0, s1, x0, y0, std::max(x1 - x0 + 1, 0), std::max(y1 - y0 + 1, 0), total};
-      // canvas and snapshot boxes as 7 FP64 planes (14 floats per pixel
-      // each), the pickup map as 7 FP32 planes; offsets kept 8-byte aligned
-      total += round_up((int64_t)sg.w * sg.h * (b->use_snap ? 28 : 14) + 7 * m, 2);
-      g->segs.push_back(sg);
-      s0 = s1;
+    const int64_t m = b->m, side = 2 * (int64_t)((b->size_map - 1) / 2) + 2;
+    g->run.area = side * side;
+    g->run.m = m;
+    g->run.slot = tape_floats(g->run.area, m);
+    g->fwd_size_map = b->size_map;
+    g->fwd_snap = b->use_snap;
+    g->have_forward = false;
+    const int64_t whole = g->run.slot * ns;
+    g->full_tape = whole <= g->tape_cap;
+    // PAINTY_GRAD_TAPE_MB bounds the tapes instead (0: always checkpoints)
+    const char* bound = std::getenv("PAINTY_GRAD_TAPE_MB");
+    if (bound) {
+      g->full_tape = whole * (int64_t)sizeof(float) <= ((int64_t)std::atoll(bound) << 20);
+    } else if (!g->full_tape) {
+      size_t mem_free = 0, mem_total = 0;
+      PNT_HIP_CHECK(hipMemGetInfo(&mem_free, &mem_total));
+      g->full_tape = whole * (int64_t)sizeof(float) <=
+                     std::min((int64_t)mem_free / kTapeFree, kTapeMost);
     }
-    ensure(g->ckpt, g->ckpt_cap, std::max<int64_t>(total, 1), s);
-    const Plane7 pick = b->pick_planes();
-    for (const auto& sg : g->segs) {
-      const int64_t area = (int64_t)sg.w * sg.h;
-      float* c0 = g->ckpt + sg.off;
-      box_copy({layer_box(L, cv->cols, sg.x0, sg.y0, sg.w, sg.h, reinterpret_cast<double*>(c0), area),
-                layer_box(b->snap_planes(), cv->cols, sg.x0, sg.y0, b->use_snap ? sg.w : 0, sg.h,
-                          reinterpret_cast<double*>(c0 + 14 * area), area),
-                plane_box(pick, b->size_map, 0, 0, b->size_map, b->size_map,
-                          c0 + (b->use_snap ? 28 : 14) * area, m)},
-               true, s);
-      run_fused(b, cv, g->st.data() + sg.s0, sg.s1 - sg.s0);
+    if (g->full_tape) {
+      ensure(g->tape, g->tape_cap, whole, s);
+      g->run.base = g->tape;
+      run_fused(b, cv, g->st.data(), ns, 0, &g->run);
+      if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
+      keep_lists(g, s);
+    } else {
+      if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
+      // segments (at most seg_len stamps, a dip starts a new one) and their
+      // checkpoint boxes: the union of their snapshot boxes (window boxes
+      // without the snapshot)
+      int64_t total = 0;
+      for (int s0 = 0; s0 < ns;) {
+        int s1 = s0 + 1;
+        while (s1 < ns && s1 - s0 < g->seg_len && !(g->st[s1].flags & PNT_STAMP_DIP)) ++s1;
+        int x0 = cv->cols, y0 = cv->rows, x1 = -1, y1 = -1;
+        for (int i = s0; i < s1; ++i) {
+          const StampArgs a = stamp_args(b, cv, g->st[i].cx, g->st[i].cy, g->st[i].theta);
+          const RingBox rb = ring_box(a.g, b->radius);
+          int bx0 = rb.a_x0, by0 = rb.a_y0, bx1 = rb.a_x1, by1 = rb.a_y1;
+          if (!b->use_snap) {
+            bx0 = std::max(rb.tl_x, 0);
+            by0 = std::max(rb.tl_y, 0);
+            bx1 = std::min(rb.br_x, cv->cols - 1);
+            by1 = std::min(rb.br_y, cv->rows - 1);
+          }
+          if (bx1 < bx0 || by1 < by0) continue;
+          x0 = std::min(x0, bx0);
+          y0 = std::min(y0, by0);
+          x1 = std::max(x1, bx1);
+          y1 = std::max(y1, by1);
+        }
+        pnt_grad_s::Seg sg{s0, s1, x0, y0, std::max(x1 - x0 + 1, 0), std::max(y1 - y0 + 1, 0), total};
+        // canvas and snapshot boxes as 7 FP64 planes (14 floats per pixel
+        // each), the pickup map as 7 FP32 planes; offsets kept 8-byte aligned
+        total += round_up((int64_t)sg.w * sg.h * (b->use_snap ? 28 : 14) + 7 * m, 2);
+        g->segs.push_back(sg);
+        s0 = s1;
+      }
+      ensure(g->ckpt, g->ckpt_cap, std::max<int64_t>(total, 1), s);
+      const Plane7 pick = b->pick_planes();
+      for (const auto& sg : g->segs) {
+        const int64_t area = (int64_t)sg.w * sg.h;
+        float* c0 = g->ckpt + sg.off;
+        box_copy({layer_box(L, cv->cols, sg.x0, sg.y0, sg.w, sg.h, reinterpret_cast<double*>(c0), area),
+                  layer_box(b->snap_planes(), cv->cols, sg.x0, sg.y0, b->use_snap ? sg.w : 0, sg.h,
+                            reinterpret_cast<double*>(c0 + 14 * area), area),
+                  plane_box(pick, b->size_map, 0, 0, b->size_map, b->size_map,
+                            c0 + (b->use_snap ? 28 : 14) * area, m)},
+                 true, s);
+        if (other) PNT_HIP_CHECK(hipStreamSynchronize(s));
+        run_fused(b, cv, g->st.data() + sg.s0, sg.s1 - sg.s0);
+        if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
+      }
     }
     launch_compose(n, L, R0c, Rgb3{{R.p[0], R.p[1], R.p[2]}}, s);
     g->have_forward = true;
@@ -839,8 +1031,10 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
     pnt_brush b = g->b;
     pnt_canvas cv = g->cv;
     hipStream_t s = g->ctx->stream;
+    PNT_REQUIRE(b->size_map == g->fwd_size_map && b->use_snap == g->fwd_snap,
+                "the brush's geometry or snapshot switch changed since the forward");
     const int64_t n = cv->n, m = b->m;
-    const int sm = b->size_map, hr = (sm - 1) / 2;
+    const int sm = b->size_map;
     const int ns = (int)g->st.size();
     const Layer7 L = cv->layer();
     const Plane7 gC{{gwet.p[0], gwet.p[1], gwet.p[2], gwet.p[3], gwet.p[4], gwet.p[5], gwet.p[6]}};
@@ -850,145 +1044,58 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
     PNT_HIP_CHECK(hipGetLastError());
     const int64_t nst = round_up(n, 64);
     if (b->use_snap) {
-      ensure(g->gX, g->gX_cap, 7 * nst, s);
-      launch_fill(g->gX, 7 * nst, 0.0f, s);
+      if (7 * nst > g->gX_cap) {  // zero to begin with; every call leaves it zero
+        ensure(g->gX, g->gX_cap, 7 * nst, s);
+        launch_fill(g->gX, 7 * nst, 0.0f, s);
+        ensure(g->gdirty, g->gdirty_cap, nst + 16, s);
+        launch_fill_u8(g->gdirty, nst + 16, 0, s);
+      }
     }
-    ensure(g->gP, g->gP_cap, 7 * m, s);
+    ensure(g->gP, g->gP_cap, kAdjSlots * 7 * m, s);
     ensure(g->gB, g->gB_cap, 6 * (int64_t)ns, s);
-    launch_fill(g->gP, 7 * m, 0.0f, s);
+    launch_fill(g->gP, kAdjSlots * 7 * m, 0.0f, s);
     launch_fill(g->gB, 6 * (int64_t)ns, 0.0f, s);
     const Plane7 gXL = b->use_snap ? dense7(g->gX, nst) : gC;
-    const Plane7 gPL = dense7(g->gP, m);
-    // tapes of one segment
-    const int64_t bwmax = 2 * (int64_t)hr + 2;
-    const int64_t area = bwmax * bwmax;
-    // per stamp: C and X as 7 FP64 planes of area (28 floats per pixel),
-    // then P as 7 FP32 planes of m
-    const int64_t slot = round_up(28 * area + 7 * m, 2);
-    ensure(g->tape, g->tape_cap, slot * g->seg_len, s);
-    const int side = 2 * hr + 1;
-    const int tiles_x = (side + kGT - 1) / kGT;
-    const Plane7 pick = b->pick_planes();
-    std::vector<float> paints(6 * (size_t)g->seg_len);
-    for (int k = (int)g->segs.size() - 1; k >= 0; --k) {
-      const auto& sg = g->segs[k];
-      const int cnt = sg.s1 - sg.s0;
-      const PlanDev D = upload_plan(b, cv, g->st.data() + sg.s0, cnt);
-      // scratch of the shared-pixel replay: one record per visit
-      int64_t max_list = 0;
-      for (int q = 0; q < cnt; ++q)
-        if (D.host[q].dl_nlev > 0)
-          max_list = std::max<int64_t>(
-              max_list, D.host_off[D.host[q].dl_lev + D.host[q].dl_nlev] - D.host_off[D.host[q].dl_lev]);
-      if (max_list)
-        ensure(g->scratch, g->scratch_cap, max_list * (int64_t)(sizeof(VState) / sizeof(float)), s);
-      // ---- restore the segment's checkpoint
-      const int64_t carea = (int64_t)sg.w * sg.h;
-      float* c0 = g->ckpt + sg.off;
-      box_copy({layer_box(L, cv->cols, sg.x0, sg.y0, sg.w, sg.h, reinterpret_cast<double*>(c0), carea),
-                layer_box(b->snap_planes(), cv->cols, sg.x0, sg.y0, b->use_snap ? sg.w : 0, sg.h,
-                          reinterpret_cast<double*>(c0 + 14 * carea), carea),
-                plane_box(pick, sm, 0, 0, sm, sm, c0 + (b->use_snap ? 28 : 14) * carea, m)},
-               false, s);
-      {  // brush paint at the segment start: its last dip (stamp 0 dips)
-        int i = sg.s0;
+    if (g->full_tape) {
+      adjoint_waves(g, 0, gC, gXL, s);
+    } else {
+      const Plane7 pick = b->pick_planes();
+      for (int k = (int)g->segs.size() - 1; k >= 0; --k) {
+        const auto& sg = g->segs[k];
+        // restore the segment's checkpoint: the snapshot's dirty bytes no
+        // longer hold
+        const int64_t carea = (int64_t)sg.w * sg.h;
+        float* c0 = g->ckpt + sg.off;
+        box_copy({layer_box(L, cv->cols, sg.x0, sg.y0, sg.w, sg.h, reinterpret_cast<double*>(c0), carea),
+                  layer_box(b->snap_planes(), cv->cols, sg.x0, sg.y0, b->use_snap ? sg.w : 0, sg.h,
+                            reinterpret_cast<double*>(c0 + 14 * carea), carea),
+                  plane_box(pick, sm, 0, 0, sm, sm, c0 + (b->use_snap ? 28 : 14) * carea, m)},
+                 false, s);
+        cv->epoch++;
+        b->dirty_canvas = nullptr;
+        int i = sg.s0;  // brush paint at the segment start: its last dip (stamp 0 dips)
         while (!(g->st[i].flags & PNT_STAMP_DIP)) --i;
         for (int c = 0; c < 3; ++c) {
           b->paintK[c] = g->st[i].K[c];
           b->paintS[c] = g->st[i].S[c];
         }
+        // run it again onto its tape, then reverse it
+        ensure(g->tape, g->tape_cap, g->run.slot * g->seg_len, s);
+        g->run.base = g->tape;
+        const bool other = b->ctx->stream != s;
+        if (other) PNT_HIP_CHECK(hipStreamSynchronize(s));
+        run_fused(b, cv, g->st.data() + sg.s0, sg.s1 - sg.s0, 0, &g->run);
+        if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
+        keep_lists(g, s);
+        adjoint_waves(g, sg.s0, gC, gXL, s);
       }
-      // ---- recompute the segment, taping each stamp
-      std::vector<Tape> tapes(cnt);
-      for (int q = 0; q < cnt; ++q) {
-        const pnt_stamp& sq = g->st[sg.s0 + q];
-        if (sq.flags & PNT_STAMP_DIP) {
-          launch_fill(b->pick, 7 * b->mstride, 0.0f, s);
-          for (int c = 0; c < 3; ++c) {
-            b->paintK[c] = sq.K[c];
-            b->paintS[c] = sq.S[c];
-          }
-        }
-        for (int c = 0; c < 3; ++c) {
-          paints[6 * q + c] = b->paintK[c];
-          paints[6 * q + 3 + c] = b->paintS[c];
-        }
-        const StampArgs a = stamp_args(b, cv, sq.cx, sq.cy, sq.theta);
-        const PStamp& p = D.host[q];
-        if (b->use_snap) launch_ring_refresh(p.box, cv->cols, L, b->snap_planes(), s);
-        Tape& t = tapes[q];
-        float* base = g->tape + slot * q;
-        double* tC = reinterpret_cast<double*>(base);
-        double* tX = reinterpret_cast<double*>(base + 14 * area);
-        float* tP = base + 28 * area;
-        t.C = tC;
-        t.X = tX;
-        t.P = tP;
-        t.area = area;
-        t.m = m;
-        window_box(p, cv->rows, cv->cols, &t.bx0, &t.by0, &t.bw, &t.bh);
-        box_copy({layer_box(L, cv->cols, t.bx0, t.by0, t.bw, t.bh, tC, area),
-                  layer_box(b->snap_planes(), cv->cols, t.bx0, t.by0, b->use_snap ? t.bw : 0, t.bh,
-                            tX, area),
-                  plane_box(pick, sm, 0, 0, sm, sm, tP, m)},
-                 true, s);
-        launch_stamp_main(a, s);
-        if (p.dl_nlev > 0) launch_stamp_serial(a, D.dl, D.dl_off + p.dl_lev, p.dl_nlev, s);
-      }
-      // ---- adjoints, last stamp first
-      for (int q = cnt - 1; q >= 0; --q) {
-        const int i = sg.s0 + q;
-        const PStamp& p = D.host[q];
-        AArgs A;
-        A.st = D.st;
-        A.j = q;
-        A.hr = hr;
-        A.size_map = sm;
-        A.rows = cv->rows;
-        A.cols = cv->cols;
-        A.tiles_x = tiles_x;
-        A.ntiles = tiles_x * tiles_x;
-        A.use_snap = b->use_snap ? 1 : 0;
-        A.fp = b->fp;
-        A.t = tapes[q];
-        A.gC = gC;
-        A.gX = gXL;
-        A.gP = gPL;
-        A.gB = g->gB + 6 * (int64_t)i;
-        A.pr = b->pickup_rate;
-        A.dr = b->dep_rate;
-        A.cap = b->cap;
-        for (int c = 0; c < 3; ++c) {
-          A.pk[c] = paints[6 * q + c];
-          A.ps[c] = paints[6 * q + 3 + c];
-        }
-        A.dl = D.dl;
-        A.dl_off = D.dl_off;
-        A.scratch = g->scratch;
-        if (A.t.bw > 0 && A.t.bh > 0) {
-          k_adj_visits<<<(unsigned)A.ntiles, kGT * kGT, 0, s>>>(A);
-          PNT_HIP_CHECK(hipGetLastError());
-          if (p.dl_nlev > 0) {
-            k_adj_shared<<<1, kBlk, 0, s>>>(A);
-            PNT_HIP_CHECK(hipGetLastError());
-          }
-        }
-        if (b->use_snap && p.box.a_x1 >= p.box.a_x0 && p.box.a_y1 >= p.box.a_y0) {
-          const int64_t tot = (int64_t)(p.box.a_x1 - p.box.a_x0 + 1) * (p.box.a_y1 - p.box.a_y0 + 1);
-          k_adj_ring<<<grid_for(tot), kBlk, 0, s>>>(p.box, cv->cols, gC, gXL);
-          PNT_HIP_CHECK(hipGetLastError());
-        }
-        if (g->st[i].flags & PNT_STAMP_DIP) launch_fill(g->gP, 7 * m, 0.0f, s);
-      }
-      PNT_HIP_CHECK(hipStreamSynchronize(s));  // tapes and the plan are reused next segment
+      cv->epoch++;
+      b->dirty_canvas = nullptr;
     }
     if (b->use_snap) {
-      k_adj_full_copy<<<grid_for(n), kBlk, 0, s>>>(n, gC, gXL);
+      k_adj_full_copy<<<grid_for((n + 7) / 8), kBlk, 0, s>>>(n, gC, gXL, g->gdirty);
       PNT_HIP_CHECK(hipGetLastError());
     }
-    // the recompute ran kernels that do not keep the snapshot dirty bytes
-    cv->epoch++;
-    b->dirty_canvas = nullptr;
     // ---- mixing weights: dB/dW of mixSinglePaint (PaintMixer.cxx:327-355)
     std::vector<float> hB(6 * (size_t)ns);
     PNT_HIP_CHECK(hipMemcpyAsync(hB.data(), g->gB, hB.size() * sizeof(float), hipMemcpyDeviceToHost, s));

@@ -533,7 +533,8 @@ PlanDev upload_plan_parts(pnt_brush_s* b, pnt_canvas_s* cv, const PlanPart* part
   }
   if (d_fp) *d_fp = P.d_fp;
   PNT_HIP_CHECK(hipEventRecord(P.uploaded, s));
-  return PlanDev{P.d_st, P.d_dl, P.d_off, P.h_st.data(), P.h_off.data()};
+  return PlanDev{P.d_st,          P.d_dl, P.d_off, P.h_st.data(), P.h_off.data(),
+                 (int64_t)P.h_dl.size(), (int64_t)P.h_off.size()};
 }
 
 void run_persistent(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n) {

@@ -11,6 +11,7 @@
 
 #include "painty_hip.h"
 #include "internal.hpp"
+#include "stampcore.hpp"
 
 struct pnt_brush_s;
 struct pnt_canvas_s;
@@ -18,7 +19,6 @@ struct pnt_canvas_s;
 namespace pnt {
 
 struct PersistentState;
-struct PStamp;
 
 // A stamp list's plan on the device, and its host copy (valid until the
 // brush plans again).
@@ -28,6 +28,7 @@ struct PlanDev {
   const int* dl_off;
   const PStamp* host;
   const int* host_off;  // host copy of dl_off
+  int64_t n_dl, n_off;  // entries of dl, dl_off
 };
 PlanDev upload_plan(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n);
 // A list cut into parts that each have their own brush geometry (padded
@@ -74,8 +75,26 @@ void plan_stamps_rc(int size_map, double radius, int rows, int cols, const pnt_s
                     int64_t n, std::vector<PStamp>& h_st, std::vector<int2>& h_dl,
                     std::vector<int>& h_off);
 
-// chains: concurrent stroke chains at most (0: PAINTY_FUSED_CHAINS or 4)
-void run_fused(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains = 0);
+// The tape of a stamp list's visits, for its adjoint (grad.hip): what every
+// visit found, stamp k's record at base + k * slot (TapeRec, stampcore.hpp),
+// and the waves that ran the list.
+struct TapeRun {
+  float* base = nullptr;
+  int64_t slot = 0, area = 0, m = 0;  // floats per stamp, pixels and map cells of a record
+  struct Phase {
+    int k, clear, chain;  // stamp k, or the clear of the chain's map before it
+  };
+  std::vector<std::vector<Phase>> waves;
+  std::vector<PStamp> st;
+  std::vector<int> n_visits;  // listed shared-pixel visits of each stamp
+  const int2* dl = nullptr;  // the plan's lists (the brush's, until it plans again)
+  const int* dl_off = nullptr;
+  int64_t n_dl = 0, n_off = 0;
+};
+// chains: concurrent stroke chains at most (0: PAINTY_FUSED_CHAINS or 8);
+// tape (optional): keep the visits' tape and the schedule.
+void run_fused(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains = 0,
+               TapeRun* tape = nullptr);
 void run_fused_strokes(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* strokes, int64_t ns);
 // The fused stamps of a list in stream order with the plan in a file-scope
 // device array (pnt_imprint_stamps_noalloc).

@@ -160,6 +160,36 @@ __device__ __forceinline__ void st_px(const Layer7& L, int64_t i, const float ks
   L.v[i] = v;
 }
 
+// One stamp's tape record: the canvas and pickup-source pixels as its visits
+// find them, by pixel of its window box clipped to the canvas, and the map
+// cells before their first visits.  Only the visited entries are written.
+struct TapeRec {
+  double *cv, *xv;  // volumes
+  float *ck, *xk;   // K, S: 6 planes of `area`
+  float* P;         // 7 planes of `m`
+  int64_t area, m;
+  int bx0, by0, bw;
+  __host__ __device__ int64_t at(int x, int y) const { return (int64_t)(y - by0) * bw + (x - bx0); }
+};
+__host__ __device__ inline int64_t tape_floats(int64_t area, int64_t m) {
+  return (16 * area + 7 * m + 3) / 4 * 4;
+}
+__host__ __device__ inline TapeRec tape_rec(float* base, int64_t area, int64_t m, const RingBox& b,
+                                            int cols) {
+  TapeRec t;
+  t.cv = reinterpret_cast<double*>(base);
+  t.xv = t.cv + area;
+  t.ck = base + 4 * area;
+  t.xk = t.ck + 6 * area;
+  t.P = t.xk + 6 * area;
+  t.area = area;
+  t.m = m;
+  t.bx0 = b.tl_x > 0 ? b.tl_x : 0;
+  t.by0 = b.tl_y > 0 ? b.tl_y : 0;
+  t.bw = (b.br_x < cols - 1 ? b.br_x : cols - 1) - t.bx0 + 1;
+  return t;
+}
+
 // Where one visit reads and writes.
 struct VisitTarget {
   const Layer7* canvas;
@@ -167,6 +197,7 @@ struct VisitTarget {
   uint8_t* dirty;
   int use_snap;
   double pickup_rate, dep_rate, cap;
+  const TapeRec* tape = nullptr;  // StampKind::tape
 };
 
 // Tile of block b when blocks [0, ntiles) take one tile each: blocks go
@@ -399,6 +430,21 @@ __device__ __forceinline__ void store_pixel(const VisitTarget& T, bool snap, int
     else if (acc.src_moved)
       T.src->v[ic] = acc.svv;
     T.dirty[ic] = 1;
+  }
+}
+
+// The pixel (x, y) as a visit finds it, into the tape.
+__device__ __forceinline__ void tape_pixel(const TapeRec& t, bool snap, int x, int y,
+                                           const float cv[6], double cvv, const float sv[6],
+                                           double svv) {
+  const int64_t k = t.at(x, y);
+#pragma unroll
+  for (int c = 0; c < 6; ++c) t.ck[c * t.area + k] = cv[c];
+  t.cv[k] = cvv;
+  if (snap) {
+#pragma unroll
+    for (int c = 0; c < 6; ++c) t.xk[c * t.area + k] = sv[c];
+    t.xv[k] = svv;
   }
 }
 
@@ -659,6 +705,12 @@ __device__ __forceinline__ void window_tile(const VisitTarget& T, float* const* 
     }
   }
   const bool paint = act && fh > 0.0f;
+  if (F::tape && paint) {
+    tape_pixel(*T.tape, snap, V.x, V.y, acc.cv, acc.cvv, acc.sv, acc.svv);
+    if (first)
+#pragma unroll
+      for (int c = 0; c < 7; ++c) T.tape->P[c * T.tape->m + V.mm] = acc.v[c];
+  }
   if (paint && first) {
     paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
     if (V.shared && inside)
@@ -688,6 +740,7 @@ __device__ __forceinline__ void window_tile(const VisitTarget& T, float* const* 
         check_dry_regs(clk, acc.cv, acc.cvv, pic);
         if (!snap) acc.src_from_canvas();
       }
+      if (F::tape) tape_pixel(*T.tape, snap, px, py, acc.cv, acc.cvv, acc.sv, acc.svv);
       paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
       store_pixel(T, snap, pic, ppv, acc);
 #pragma unroll
@@ -795,9 +848,10 @@ __device__ __forceinline__ void level_visits(const VisitTarget& T, float* const*
 //   clock  Canvas::checkDry on every visited pixel
 //   dup    stamps that straddle canvas column/row 0 (shared-pixel levels)
 //   kSnap  the snapshot buffer: 0 off, 1 on, 2 per stamp
-template <bool kClock, bool kDup, int kSnap>
+//   tape   every visit's input is kept (VisitTarget::tape)
+template <bool kClock, bool kDup, int kSnap, bool kTape = false>
 struct StampKind {
-  static constexpr bool clock = kClock, dup = kDup;
+  static constexpr bool clock = kClock, dup = kDup, tape = kTape;
   static __device__ __forceinline__ bool snap(int use_snap) {
     return kSnap == 2 ? use_snap != 0 : kSnap == 1;
   }
@@ -832,6 +886,23 @@ __device__ __forceinline__ void stamp_block(const VisitTarget& T, float* const* 
     ring_scan<256>(*T.canvas, *T.src, T.dirty, fp, g, st.box, pull, b - ntiles, rb, lds.ring,
                    F::clock && clk.tmap != nullptr);
   } else if (F::dup && dup) {
+    if (F::tape) {  // the pixels and cells the levels start from
+      const bool snap = F::snap(T.use_snap);
+      for (int e = dl_off[st.dl_lev] + (int)threadIdx.x; e < dl_off[st.dl_lev + st.dl_nlev]; e += 256) {
+        const int2 v = dl[e];
+        int64_t ic;
+        const int m = stamp_visit(g, v.x, v.y, &ic);
+        if (m < 0 || !(fp[m] > 0.0f)) continue;
+        const int x = (int)(ic % g.cols), y = (int)(ic / g.cols);
+        CachedVisit<RegPick> acc;
+        load_pixel(T, snap, ic, pull && on_window_border(st.box, x, y), acc);
+        tape_pixel(*T.tape, snap, x, y, acc.cv, acc.cvv, acc.sv, acc.svv);
+#pragma unroll
+        for (int c = 0; c < 7; ++c) T.tape->P[c * T.tape->m + m] = pick[c][m];
+      }
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+    }
     level_visits<256>(T, pick, fp, g, st, dl, dl_off, pk, ps, F::clock ? clk : DryClock{}, pull);
   }
 }
