@@ -4,7 +4,9 @@ composite within 1e-5 relative per channel; the 8- and 16-bit encodings
 bit for bit (the encode runs in FP64 on the float input)."""
 import numpy as np
 import pytest
+import torch
 
+from painty_amd import _lib
 from painty_amd import workload as W
 from tests.parity import assert_close, run_gpu, run_oracle
 
@@ -55,3 +57,30 @@ def test_encode_bit_exact(hip, oracle, bits, to_srgb):
     ref = oracle.encode(x.astype(np.float64), to_srgb=to_srgb, bits=bits)
     assert got.dtype == (np.uint16 if bits == 16 else np.uint8)
     np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("bits", [8, 16])
+@pytest.mark.parametrize("n", [1, 4, 7, 65535])
+def test_encode_at_rounding_edges(hip, oracle, bits, n):
+    """Floats around every place where the encoded value changes, in lengths
+    that leave 0..3 pixels past the four-pixel groups."""
+    scale = 65535.0 if bits == 16 else 255.0
+    edge = (np.arange(int(scale)) + 0.5) / scale  # sRGB values halfway between two codes
+    lin = np.where(edge <= 0.04045, edge / 12.92, ((edge + 0.055) / 1.055) ** 2.4).astype(np.float32)
+    x = np.concatenate([lin, np.nextafter(lin, np.float32(0)), np.nextafter(lin, np.float32(2)),
+                        np.float32([0.0031306684, 0.0031307, 1.0, np.nextafter(np.float32(1), 0)])])
+    x = np.resize(x, (n, 3)) if n < 65535 else np.resize(x, (-(-x.size // 3), 3))
+    ref = oracle.encode(x.astype(np.float64), to_srgb=True, bits=bits)
+    np.testing.assert_array_equal(hip.encode(x, to_srgb=True, bits=bits), ref)
+    # on the device: planes on 4-byte boundaries, and an image off its word
+    m = len(x)
+    planes = torch.from_numpy(np.ascontiguousarray(x.T)).cuda()
+    buf = torch.zeros(3 * m + 1, device="cuda", dtype=torch.int16 if bits == 16 else torch.uint8)
+    for off in (0, 1):
+        torch.cuda.synchronize()
+        _lib.call("pnt_dev_encode", hip.default_context().h, m,
+                  _lib.DevRgb((_lib.C.c_void_p * 3)(*[planes[c].data_ptr() for c in range(3)])), 1,
+                  bits, buf[off:].data_ptr(), None)
+        hip.default_context().synchronize()
+        got = buf[off:off + 3 * m].cpu().numpy().view(ref.dtype).reshape(m, 3)
+        np.testing.assert_array_equal(got, ref)
