@@ -456,42 +456,11 @@ void brush_dip(pnt_brush b, const float K[3], const float S[3]) {
 
 // FootprintBrush::imprint (FootprintBrush.hxx:73-143) as kernel launches.
 void imprint_plain(pnt_brush b, pnt_canvas cv, double cx, double cy, double theta) {
-  hipStream_t s = b->ctx->stream;
   cv->epoch++;
   b->dirty_canvas = nullptr;
-  if (b->use_snap) {
-    if (b->snap_rows != cv->rows || b->snap_cols != cv->cols) brush_full_snapshot(b, cv);
-  }
-  StampArgs a = stamp_args(b, cv, cx, cy, theta);
-  if (cv->tmap)  // Canvas::checkDry on every visit (FootprintBrush.hxx:86, 115)
-    a.clk = DryClock{cv->tmap, canvas_now_us(cv), cv->drying_ms, cv->R0(), cv->h()};
-  if (b->use_snap) launch_ring_refresh(ring_box(a.g, b->radius), cv->cols, cv->layer(), b->snap_planes(), s);
-  launch_stamp_main(a, s);
-  if (a.dupx || a.dupy) {
-    std::vector<int2> list;
-    std::vector<int> off;
-    plan_shared_visits(a, list, off);
-    if (!list.empty()) {
-      const int64_t need = (int64_t)list.size();
-      if (need > b->d_cap || (int64_t)off.size() > b->d_cap + 1) {
-        PNT_HIP_CHECK(hipStreamSynchronize(s));
-        dev_free(b->d_list);
-        dev_free(b->d_off);
-        b->d_list = nullptr;
-        b->d_off = nullptr;
-        const int64_t cap = std::max<int64_t>(need, (int64_t)off.size()) * 2;
-        PNT_HIP_CHECK(hipMalloc(&b->d_list, cap * sizeof(int2)));
-        PNT_HIP_CHECK(hipMalloc(&b->d_off, (cap + 1) * sizeof(int)));
-        b->d_cap = cap;
-      }
-      PNT_HIP_CHECK(hipMemcpyAsync(b->d_list, list.data(), need * sizeof(int2),
-                                   hipMemcpyHostToDevice, s));
-      PNT_HIP_CHECK(hipMemcpyAsync(b->d_off, off.data(), off.size() * sizeof(int),
-                                   hipMemcpyHostToDevice, s));
-      launch_stamp_serial(a, b->d_list, b->d_off, (int)off.size() - 1, s);
-      PNT_HIP_CHECK(hipStreamSynchronize(s));  // host lists die here
-    }
-  }
+  if (b->use_snap && (b->snap_rows != cv->rows || b->snap_cols != cv->cols))
+    brush_full_snapshot(b, cv);
+  run_plain_stamp(b, cv, cx, cy, theta);
 }
 
 void check_layout(int layout) {
@@ -1804,6 +1773,7 @@ int pnt_paint_stroke(pnt_brush b, pnt_canvas cv, const double* p, int64_t n) {
     canvas_tick(cv);
     if (cv->ctx->stream != b->ctx->stream) PNT_HIP_CHECK(hipStreamSynchronize(cv->ctx->stream));
     // FootprintBrush.hxx:251-267
+    std::vector<pnt_stamp> path;
     for (int64_t i = 0; i + 1 < n; ++i) {
       const int64_t ipre = i > 0 ? i - 1 : 0;
       const int64_t inext = (i + 2 < n) ? i + 2 : n - 1;
@@ -1818,10 +1788,20 @@ int pnt_paint_stroke(pnt_brush b, pnt_canvas cv, const double* p, int64_t n) {
         const double t = (double)pd / dist;
         const double ddx = catmull_rom_d1(pp[0], p0[0], p1[0], pn[0], t);
         const double ddy = catmull_rom_d1(pp[1], p0[1], p1[1], pn[1], t);
-        imprint_plain(b, cv, catmull_rom(pp[0], p0[0], p1[0], pn[0], t),
-                      catmull_rom(pp[1], p0[1], p1[1], pn[1], t), std::atan2(ddy, ddx));
+        pnt_stamp st{};
+        st.cx = catmull_rom(pp[0], p0[0], p1[0], pn[0], t);
+        st.cy = catmull_rom(pp[1], p0[1], p1[1], pn[1], t);
+        st.theta = std::atan2(ddy, ddx);
+        path.push_back(st);
       }
     }
+    if (path.empty()) return;
+    // the imprints as one planned list; the dirty bytes are begun anew (all
+    // set) and not kept past it, as after single imprints
+    cv->epoch++;
+    b->dirty_canvas = nullptr;
+    run_fused(b, cv, path.data(), (int64_t)path.size(), 1);
+    b->dirty_canvas = nullptr;
     if (cv->ctx->stream != b->ctx->stream) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
   });
 }

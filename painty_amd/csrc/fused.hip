@@ -168,6 +168,10 @@ void launch_slots(const WArgs<kSlots>& A, int n, hipStream_t q) {
                          : k_stamp_wave<StampKind<false, true, 0, true>, kSlots>)
                  : (snap ? k_stamp_wave<StampKind<false, false, 1, true>, kSlots>
                          : k_stamp_wave<StampKind<false, false, 0, true>, kSlots>);
+  if (snap && !A.sh.dirty)  // an imprint on its own (run_plain_stamp)
+    kernel = A.sh.tmap ? k_stamp_wave<StampKind<true, true, 1, false, true>, kSlots>
+             : dup     ? k_stamp_wave<StampKind<false, true, 1, false, true>, kSlots>
+                       : k_stamp_wave<StampKind<false, false, 1, false, true>, kSlots>;
   kernel<<<dim3((unsigned)round_up(widest, 8), (unsigned)n), kT2, 0, q>>>(A);
   PNT_HIP_CHECK(hipGetLastError());
 }
@@ -1159,6 +1163,58 @@ void run_fused_noalloc(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, in
     b->dirty_canvas = cv;
     b->dirty_epoch = cv->epoch;
   }
+}
+
+// One imprint on its own: the stamp's launch with the ring copied whole
+// instead of by dirty bytes (they are kept per planned list; between single
+// imprints the caller may have written the canvas' device planes).
+void run_plain_stamp(pnt_brush_s* b, pnt_canvas_s* cv, double cx, double cy, double theta) {
+  hipStream_t s = b->ctx->stream;
+  pnt_stamp st{};
+  st.cx = cx;
+  st.cy = cy;
+  st.theta = theta;
+  thread_local std::vector<PStamp> h_st;
+  thread_local std::vector<int2> h_dl;
+  thread_local std::vector<int> h_off;
+  h_st.clear();
+  h_dl.clear();
+  h_off.clear();
+  plan_stamps(b, cv, &st, 1, h_st, h_dl, h_off);
+  if (!h_dl.empty()) {
+    const int64_t need = (int64_t)std::max(h_dl.size(), h_off.size());
+    if (need > b->d_cap) {
+      PNT_HIP_CHECK(hipStreamSynchronize(s));
+      dev_free(b->d_list);
+      dev_free(b->d_off);
+      b->d_list = nullptr;
+      b->d_off = nullptr;
+      b->d_cap = 0;
+      PNT_HIP_CHECK(hipMalloc(&b->d_list, 2 * need * sizeof(int2)));
+      PNT_HIP_CHECK(hipMalloc(&b->d_off, (2 * need + 1) * sizeof(int)));
+      b->d_cap = 2 * need;
+    }
+    PNT_HIP_CHECK(hipMemcpyAsync(b->d_list, h_dl.data(), h_dl.size() * sizeof(int2),
+                                 hipMemcpyHostToDevice, s));
+    PNT_HIP_CHECK(hipMemcpyAsync(b->d_off, h_off.data(), h_off.size() * sizeof(int),
+                                 hipMemcpyHostToDevice, s));
+  }
+  StampShared H = stamp_shared(b, cv, b->d_list, b->d_off);
+  H.dirty = nullptr;
+  const PStamp& p = h_st[0];
+  const FpBox dom = cell_domain(FpBox{b->fbox[0], b->fbox[1], b->fbox[2], b->fbox[3]}, b->size_map,
+                                H.tmap != nullptr);
+  WArgs<1> A{H, {stamp_slot(H, p, b->fp, dom, b->size_map, b->pick, b->mstride, b->paintK, b->paintS)}};
+  if (H.use_snap) {  // one ring pixel a thread
+    WSlot& S = A.slot[0];
+    const int64_t px = (int64_t)std::max(p.box.a_x1 - p.box.a_x0 + 1, 0) *
+                       std::max(p.box.a_y1 - p.box.a_y0 + 1, 0);
+    const int rb = (int)std::min<int64_t>((px + kT2 - 1) / kT2, 4096);
+    S.nblk += rb - S.rb;
+    S.rb = rb;
+  }
+  launch_slots(A, 1, s);
+  if (!h_dl.empty()) PNT_HIP_CHECK(hipStreamSynchronize(s));  // the copies read pageable lists
 }
 
 void run_fused_strokes(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* strokes, int64_t ns) {

@@ -152,15 +152,6 @@ void launch_copy_layer(int64_t n, const Layer7& src, const Layer7& dst, hipStrea
 void launch_layer_from_planes(int64_t n, const Plane7& src, const Layer7& dst, hipStream_t s);
 void launch_planes_from_layer(int64_t n, const Layer7& src, const Plane7& dst, hipStream_t s);
 
-// ---- stamping (kernels.hip) ----
-void launch_ring_refresh(const RingBox& box, int cols, const Layer7& canvas, const Layer7& snap,
-                         hipStream_t s);
-void launch_stamp_main(const StampArgs& a, hipStream_t s);
-// Visits that share a canvas pixel at column/row 0 (and their map-cell
-// partners), listed in reference order and grouped by dependency level.
-void launch_stamp_serial(const StampArgs& a, const int2* list, const int* level_off, int nlevels,
-                         hipStream_t s);
-
 RingBox ring_box(const StampGeom& g, double radius);
 
 }  // namespace pnt

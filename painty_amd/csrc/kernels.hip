@@ -3,8 +3,6 @@
 // Composite and dry are streaming kernels over the layer planes (FP32 K/S,
 // FP64 V; HBM-bound): one thread handles four consecutive pixels with
 // 16-byte loads from every FP32 plane and 32 bytes of volumes.
-// Stamping follows renderer/FootprintBrush.hxx:73-143 visit by visit; see the
-// comment above k_stamp_main for how the reference's serial order is kept.
 #include <algorithm>
 
 #include "internal.hpp"
@@ -296,131 +294,9 @@ __global__ __launch_bounds__(kBlock) void k_planes_from_layer(int64_t n, Layer7 
   dst.p[6][i] = (float)src.v[i];
 }
 
-// ------------------------------------------------------------ stamping ---
-// One visit of an imprint for canvas pixel ic and map cell im: the shared
-// visit arithmetic (visit.hpp) on the pickup map in global memory.
-struct GlobalVisit {
-  const StampArgs& a;
-  int64_t ic;
-  int im;
-  __device__ float pick(int c) const { return a.b.pick.p[c][im]; }
-  __device__ void set_pick(int c, float v) const { a.b.pick.p[c][im] = v; }
-  __device__ float src(int c) const { return a.src.ks[c][ic]; }
-  __device__ double src_v() const { return a.src.v[ic]; }
-  __device__ void set_src_v(double v) const { a.src.v[ic] = v; }
-  __device__ float canvas(int c) const { return a.canvas.ks[c][ic]; }
-  __device__ double canvas_v() const { return a.canvas.v[ic]; }
-  __device__ void set_canvas(int c, float v) const { a.canvas.ks[c][ic] = v; }
-  __device__ void set_canvas_v(double v) const { a.canvas.v[ic] = v; }
-};
-
 // Canvas::checkDry of one pixel, called directly (Canvas.hxx:123-155).
 __global__ __launch_bounds__(64) void k_check_dry_pixel(DryClock c, Layer7 canvas, int64_t ic) {
   if (threadIdx.x == 0) check_dry(c, canvas, ic);
-}
-
-__device__ __forceinline__ void paint_visit(const StampArgs& a, int64_t ic, int im) {
-  const float fh = a.b.fp[im];
-  if (!(fh > 0.0f)) return;
-  GlobalVisit acc{a, ic, im};
-  paint_visit_math(acc, fh, a.b.pickup_rate, a.b.dep_rate, a.b.cap, a.b.paintK, a.b.paintS);
-}
-
-// updateSnapshot(canvas, center), FootprintBrush.hxx:307-318: copy the wet
-// layer into the snapshot over the allowed box except the window interior.
-__global__ __launch_bounds__(kBlock) void k_ring_refresh(RingBox b, int cols, Layer7 canvas,
-                                                         Layer7 snap) {
-  const int w = b.a_x1 - b.a_x0 + 1;
-  const int hgt = b.a_y1 - b.a_y0 + 1;
-  const int64_t total = (int64_t)w * hgt;
-  for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < total;
-       e += (int64_t)gridDim.x * kBlock) {
-    const int row = b.a_y0 + (int)(e / w);
-    const int col = b.a_x0 + (int)(e % w);
-    if (row > b.tl_y && row < b.br_y && col > b.tl_x && col < b.br_x) continue;
-    const int64_t i = (int64_t)row * cols + col;
-#pragma unroll
-    for (int c = 0; c < 6; ++c) snap.ks[c][i] = canvas.ks[c][i];
-    snap.v[i] = canvas.v[i];
-  }
-}
-
-// One imprint's visits, spread over the GPU.
-//
-// The reference visits window pixels in row-major order.  Two visits can
-// touch the same state only when
-//   (a) they round to the same pickup-map cell: rotation preserves distances
-//       and a half-open unit cell holds no two points >= 1 apart except at
-//       distance exactly 1, so such pairs are 4-neighbours in the window and a
-//       cell has at most two visitors; or
-//   (b) they truncate to the same canvas pixel: only column 0 / row 0 when the
-//       stamp straddles the left / top edge with a fractional centre.
-// Each workgroup takes a 16x16 tile of the window and computes the map cells
-// of the tile plus a one-pixel halo in LDS.  A visit whose earlier neighbour
-// (left or up) shares its cell is skipped; the earlier one runs both, in
-// order.  Under (b), visits on canvas column/row 0 and their partners are
-// left to k_stamp_serial, which runs them in reference order by dependency
-// level.  No other visit shares state with them, so the two kernels commute.
-constexpr int kTile = 16;
-
-__device__ __forceinline__ bool on_dup_line(const StampArgs& a, int col, int row) {
-  return (a.dupx && (int)(col + a.g.cx) == 0) || (a.dupy && (int)(row + a.g.cy) == 0);
-}
-
-__global__ __launch_bounds__(kTile* kTile) void k_stamp_main(StampArgs a, int tiles_x) {
-  __shared__ int sm[kTile + 2][kTile + 2];
-  const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
-  const int col0 = -a.g.hr + tx * kTile, row0 = -a.g.hr + ty * kTile;
-  for (int e = threadIdx.x; e < (kTile + 2) * (kTile + 2); e += kTile * kTile) {
-    const int ly = e / (kTile + 2), lx = e % (kTile + 2);
-    int64_t ic;
-    sm[ly][lx] = stamp_visit(a.g, col0 + lx - 1, row0 + ly - 1, &ic);
-  }
-  __syncthreads();
-  const int lx = threadIdx.x % kTile, ly = threadIdx.x / kTile;
-  const int m = sm[ly + 1][lx + 1];
-  if (m < 0) return;
-  if (sm[ly + 1][lx] == m || sm[ly][lx + 1] == m) return;  // earlier visitor owns the cell
-  const int col = col0 + lx, row = row0 + ly;
-  int pcol = col, prow = row;
-  bool partner = false;
-  if (sm[ly + 1][lx + 2] == m) {
-    pcol = col + 1;
-    partner = true;
-  } else if (sm[ly + 2][lx + 1] == m) {
-    prow = row + 1;
-    partner = true;
-  }
-  if ((a.dupx | a.dupy) && (on_dup_line(a, col, row) || (partner && on_dup_line(a, pcol, prow))))
-    return;
-  int64_t ic, pic = 0;
-  stamp_visit(a.g, col, row, &ic);
-  if (partner) stamp_visit(a.g, pcol, prow, &pic);
-  if (a.clk.tmap) check_dry(a.clk, a.canvas, ic);
-  paint_visit(a, ic, m);
-  if (partner) {
-    if (a.clk.tmap) check_dry(a.clk, a.canvas, pic);
-    paint_visit(a, pic, m);
-  }
-}
-
-// Visits listed in reference order, grouped by level: a visit's level is one
-// more than the highest level of the earlier visits sharing its map cell or
-// canvas pixel.  One workgroup; levels are separated by barriers.
-__global__ __launch_bounds__(kBlock) void k_stamp_serial(StampArgs a, const int2* list,
-                                                         const int* level_off, int nlevels) {
-  for (int L = 0; L < nlevels; ++L) {
-    for (int k = level_off[L] + threadIdx.x; k < level_off[L + 1]; k += kBlock) {
-      const int2 v = list[k];
-      int64_t ic;
-      const int m = stamp_visit(a.g, v.x, v.y, &ic);
-      if (m >= 0) {
-        if (a.clk.tmap) check_dry(a.clk, a.canvas, ic);
-        paint_visit(a, ic, m);
-      }
-    }
-    __syncthreads();
-  }
 }
 
 inline unsigned blocks_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -561,29 +437,6 @@ RingBox ring_box(const StampGeom& g, double radius) {
   b.a_x1 = std::min((int)(g.cx + g.hr + radius), g.cols - 1);
   b.a_y1 = std::min((int)(g.cy + g.hr + radius), g.rows - 1);
   return b;
-}
-
-void launch_ring_refresh(const RingBox& box, int cols, const Layer7& canvas, const Layer7& snap,
-                         hipStream_t s) {
-  if (box.a_x1 < box.a_x0 || box.a_y1 < box.a_y0) return;
-  const int64_t total = (int64_t)(box.a_x1 - box.a_x0 + 1) * (box.a_y1 - box.a_y0 + 1);
-  const unsigned grid = (unsigned)std::min<int64_t>(blocks_for(total), 4096);
-  k_ring_refresh<<<grid, kBlock, 0, s>>>(box, cols, canvas, snap);
-  PNT_HIP_CHECK(hipGetLastError());
-}
-
-void launch_stamp_main(const StampArgs& a, hipStream_t s) {
-  const int side = 2 * a.g.hr + 1;
-  const int tiles = (side + kTile - 1) / kTile;
-  k_stamp_main<<<(unsigned)(tiles * tiles), kTile * kTile, 0, s>>>(a, tiles);
-  PNT_HIP_CHECK(hipGetLastError());
-}
-
-void launch_stamp_serial(const StampArgs& a, const int2* list, const int* level_off, int nlevels,
-                         hipStream_t s) {
-  if (nlevels <= 0) return;
-  k_stamp_serial<<<1, kBlock, 0, s>>>(a, list, level_off, nlevels);
-  PNT_HIP_CHECK(hipGetLastError());
 }
 
 }  // namespace pnt

@@ -95,6 +95,8 @@ struct TapeRun {
 // tape (optional): keep the visits' tape and the schedule.
 void run_fused(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains = 0,
                TapeRun* tape = nullptr);
+// One imprint, the ring copied whole (pnt_imprint, PNT_EXEC_PLAIN).
+void run_plain_stamp(pnt_brush_s* b, pnt_canvas_s* cv, double cx, double cy, double theta);
 void run_fused_strokes(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* strokes, int64_t ns);
 // The fused stamps of a list in stream order with the plan in a file-scope
 // device array (pnt_imprint_stamps_noalloc).

@@ -395,6 +395,27 @@ __device__ __forceinline__ void ring_scan(const Layer7& canvas, const Layer7& sn
   }
 }
 
+// The same refresh without dirty bytes: every pixel of the ring is copied,
+// one a thread, except the border pixels left to their visits.
+template <int kThreads>
+__device__ __forceinline__ void ring_copy(const Layer7& canvas, const Layer7& snap,
+                                          const float* fp, const StampGeom& g, const RingBox& b,
+                                          int blk, int nblk, bool clocked) {
+  const int w = b.a_x1 - b.a_x0 + 1, h = b.a_y1 - b.a_y0 + 1;
+  if (w <= 0 || h <= 0) return;
+  const int64_t total = (int64_t)w * h;
+  for (int64_t e = (int64_t)blk * kThreads + threadIdx.x; e < total; e += (int64_t)nblk * kThreads) {
+    const int r = (int)(e / w), row = b.a_y0 + r, col = b.a_x0 + (int)(e - (int64_t)r * w);
+    if (row > b.tl_y && row < b.br_y && col > b.tl_x && col < b.br_x) continue;
+    const int64_t i = (int64_t)row * g.cols + col;
+    float ks[6];
+    double v;
+    ld_px(canvas, i, ks, v);
+    if (on_window_border(b, col, row) && ring_pixel_visited(g, b, fp, col, row, clocked)) continue;
+    st_px(snap, i, ks, v);
+  }
+}
+
 // Pickup map cell held in registers between its load and its store.
 struct RegPick {
   float v[7];
@@ -429,7 +450,7 @@ __device__ __forceinline__ void store_pixel(const VisitTarget& T, bool snap, int
       st_px(*T.src, ic, acc.sv, acc.svv);
     else if (acc.src_moved)
       T.src->v[ic] = acc.svv;
-    T.dirty[ic] = 1;
+    if (T.dirty) T.dirty[ic] = 1;
   }
 }
 
@@ -499,11 +520,11 @@ __device__ __forceinline__ void check_only(const VisitTarget& T, const DryClock&
     double v;
     ld_px(*T.canvas, ic, ks, v);
     st_px(*T.src, ic, ks, v);
-    T.dirty[ic] = 0;
+    if (T.dirty) T.dirty[ic] = 0;
   }
   const double v0 = T.canvas->v[ic];
   check_dry(c, *T.canvas, ic);
-  if (T.use_snap && v0 > 0.001 && T.canvas->v[ic] != v0) T.dirty[ic] = 1;
+  if (T.use_snap && T.dirty && v0 > 0.001 && T.canvas->v[ic] != v0) T.dirty[ic] = 1;
 }
 
 // The map cells a stamp's visits are run over: the footprint's nonzero box,
@@ -849,9 +870,10 @@ __device__ __forceinline__ void level_visits(const VisitTarget& T, float* const*
 //   dup    stamps that straddle canvas column/row 0 (shared-pixel levels)
 //   kSnap  the snapshot buffer: 0 off, 1 on, 2 per stamp
 //   tape   every visit's input is kept (VisitTarget::tape)
-template <bool kClock, bool kDup, int kSnap, bool kTape = false>
+//   whole  no dirty bytes are kept: the ring is copied whole
+template <bool kClock, bool kDup, int kSnap, bool kTape = false, bool kWhole = false>
 struct StampKind {
-  static constexpr bool clock = kClock, dup = kDup, tape = kTape;
+  static constexpr bool clock = kClock, dup = kDup, tape = kTape, whole = kWhole;
   static __device__ __forceinline__ bool snap(int use_snap) {
     return kSnap == 2 ? use_snap != 0 : kSnap == 1;
   }
@@ -883,8 +905,12 @@ __device__ __forceinline__ void stamp_block(const VisitTarget& T, float* const* 
     window_tile<16, F>(T, pick, fp, dom, g, st, dup, pull, tile_of_block(b, ntiles), win, lds.hand, pk,
                        ps, clk);
   } else if (b < ntiles + rb) {
-    ring_scan<256>(*T.canvas, *T.src, T.dirty, fp, g, st.box, pull, b - ntiles, rb, lds.ring,
-                   F::clock && clk.tmap != nullptr);
+    if (F::whole)
+      ring_copy<256>(*T.canvas, *T.src, fp, g, st.box, b - ntiles, rb,
+                     F::clock && clk.tmap != nullptr);
+    else
+      ring_scan<256>(*T.canvas, *T.src, T.dirty, fp, g, st.box, pull, b - ntiles, rb, lds.ring,
+                     F::clock && clk.tmap != nullptr);
   } else if (F::dup && dup) {
     if (F::tape) {  // the pixels and cells the levels start from
       const bool snap = F::snap(T.use_snap);

@@ -17,10 +17,11 @@
 //                  turned (updateOrientation, resampled at the rotated
 //                  positions into the other of two FP64 buffers), then the
 //                  cell's exchange with the canvas pixel under it;
+//   k_smudge_steps several spine positions in one launch;
 //   k_tex_deposit  the volume-weighted mix.
-// The smudge runs one step per unit of stroke length, in stream order.  A
-// step is independent per cell: a cell reads the previous map and writes
-// only itself, and a map cell meets one canvas pixel at a time.
+// The smudge runs one step per unit of stroke length.  A step is independent
+// per cell: a cell reads the previous map and writes only itself, and a map
+// cell meets one canvas pixel at a time.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -48,6 +49,9 @@ constexpr int kBlock = 256;
 // 64-thread workgroups spread a step over four times the CUs (6.7 against
 // 7.3 us per launch at radius 40).
 constexpr int kStepBlock = 64;
+// Maps up to this side go several steps a launch: the blocks then fit the
+// device at once.
+constexpr int kSmudgeMost = 128;
 constexpr double kPi = 3.141592653589793238462643383279502884;  // Math.hxx:21-22
 
 __host__ __device__ __forceinline__ int reflect_index(int p, int len) {
@@ -237,6 +241,37 @@ struct TradeArgs {
   double maxD;
 };
 
+// The exchange of Smudge::smudge (Smudge.hxx:94-157) between a map cell and
+// the canvas pixel under it, texture thickness Dv > 0.
+__device__ __forceinline__ void smudge_trade(double pK[3], double pS[3], double& pV, float cK[3],
+                                             float cS[3], double& cV, double Dv, double maxD) {
+  constexpr double pickupRate = 0.1, depositionRate = 0.1, MinVolume = 0.001;
+  const double md = maxD;
+  const double cVl = cV * depositionRate * Dv / md, cVr = cV - cVl;
+  const double pVl = pV * pickupRate * Dv / md, pVr = pV - pVl;
+  const double K[3] = {cK[0], cK[1], cK[2]}, S[3] = {cS[0], cS[1], cS[2]};
+  const double cVnew = cVr + pVl;
+  if (cVnew > MinVolume) {
+    const double inv = 1. / cVnew;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      cK[c] = (float)(inv * (cVr * K[c] + pVl * pK[c]));
+      cS[c] = (float)(inv * (cVr * S[c] + pVl * pS[c]));
+    }
+    cV = fmax(cVnew, 0.0);
+  }
+  const double pVnew = pVr + cVl;
+  if (pVnew > MinVolume) {
+    const double inv = 1.0 / pVnew;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      pK[c] = inv * (pVr * pK[c] + cVl * K[c]);
+      pS[c] = inv * (pVr * pS[c] + cVl * S[c]);
+    }
+    pV = fmax(pVnew, 0.0);
+  }
+}
+
 // One spine position of Smudge::smudge (Smudge.hxx:49-157), for map cell
 // ip = y * n + x:
 //  - updateOrientation (Smudge.hxx:164-198): dst(x, y) = src at (x, y)
@@ -283,40 +318,21 @@ __global__ __launch_bounds__(kStepBlock) void k_smudge_step(SMap src, SMap dst, 
     trade = !(Dv <= 0.0);
   }
   if (trade) {
-    constexpr double pickupRate = 0.1, depositionRate = 0.1, MinVolume = 0.001;
-    const double md = T.maxD;
     const int64_t ic = (int64_t)cpy * T.cols + cpx;
-    const double cV = T.canvas.v[ic];
-    const double cVl = cV * depositionRate * Dv / md, cVr = cV - cVl;
-    const double pVl = pV * pickupRate * Dv / md, pVr = pV - pVl;
-    double cK[3], cS[3];
+    float cK[3], cS[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       cK[c] = T.canvas.ks[c][ic];
       cS[c] = T.canvas.ks[3 + c][ic];
     }
-    const double cVnew = cVr + pVl;
-    if (cVnew > MinVolume) {
-      const double inv = 1. / cVnew;
+    double cV = T.canvas.v[ic];
+    smudge_trade(pK, pS, pV, cK, cS, cV, Dv, T.maxD);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        T.canvas.ks[c][ic] = (float)(inv * (cVr * cK[c] + pVl * pK[c]));
-        T.canvas.ks[3 + c][ic] = (float)(inv * (cVr * cS[c] + pVl * pS[c]));
-      }
-      T.canvas.v[ic] = fmax(cVnew, 0.0);
+    for (int c = 0; c < 3; ++c) {
+      T.canvas.ks[c][ic] = cK[c];
+      T.canvas.ks[3 + c][ic] = cS[c];
     }
-    const double pVnew = pVr + cVl;
-    if (pVnew > MinVolume) {
-      const double inv = 1.0 / pVnew;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const double k = inv * (pVr * pK[c] + cVl * cK[c]);
-        const double q = inv * (pVr * pS[c] + cVl * cS[c]);
-        pK[c] = k;
-        pS[c] = q;
-      }
-      pV = fmax(pVnew, 0.0);
-    }
+    T.canvas.v[ic] = cV;
   }
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
@@ -324,6 +340,242 @@ __global__ __launch_bounds__(kStepBlock) void k_smudge_step(SMap src, SMap dst, 
     dst.S[3 * ip + c] = pS[c];
   }
   dst.V[ip] = pV;
+}
+
+// Several spine positions in one launch.  A step is a few microseconds of
+// latency over a map of a few thousand cells: one launch a step waits on its
+// launch and two round trips to memory each time.  Here a block owns a kSB x
+// kSB tile of the map and carries, in LDS, all that the tile depends on
+// through `steps` turns: the cells whose turned positions reach into it and
+// the canvas pixels those cells meet, a border that shrinks step by step to the
+// tile.  Border cells and pixels are computed by every block that needs them,
+// with the same arithmetic (the results are those of k_smudge_step to the
+// bit), and written only by the block that owns them.
+//
+// A step's region is a rectangle of map cells: step t needs, of step t - 1,
+// the cells within the turn's largest displacement (and one more, the
+// bilinear neighbour) and the cells that met its pixels then (the map moves a
+// pixel or so along the stroke).  Rectangles may reach outside the map: such
+// places have a pixel and no cell.
+//
+// The canvas pixels the blocks own go to a staging buffer (the pixels under the map
+// during the launch), since other blocks still read them; the next launch
+// reads them there, and writes back those it no longer covers.
+constexpr int kSB = 8;        // tile side
+constexpr int kSSide = 40;    // side of the region in LDS: 96 B a place, 150 KB
+constexpr int kSMax = 8;      // steps of a launch
+constexpr int kSThreads = 1024;
+constexpr int kSPer = (kSSide * kSSide + kSThreads - 1) / kSThreads;
+
+struct SBox {  // [x0, x1) x [y0, y1)
+  int x0, y0, x1, y1;
+};
+struct Staged {  // canvas pixels of a box: K, S planes and V
+  SBox box;      // x1 <= x0: nothing staged
+  float* ks;     // 6 planes of `stride`
+  double* v;
+  int64_t stride;
+};
+struct SStep {
+  double sn, cs, ctr_x, ctr_y;
+  int roi_x, roi_y;
+  int lo_x, lo_y, hi_x, hi_y;  // how far the step before reaches beyond this one's region
+};
+struct SArgs {
+  SMap src, dst;
+  int n, tiles, steps;
+  double cx, cy;
+  TradeArgs T;         // roi, ctr unused
+  int ext[4];          // pixels beyond the map at the last step: left, top, right, bottom
+  Staged prev, cur;
+  SStep st[kSMax];
+};
+static_assert(sizeof(SArgs) <= 4000, "kernel arguments must fit the argument segment");
+
+__device__ __forceinline__ bool in_box(const SBox& b, int x, int y) {
+  return x >= b.x0 && x < b.x1 && y >= b.y0 && y < b.y1;
+}
+__device__ __forceinline__ int64_t staged_at(const Staged& s, int x, int y) {
+  return (int64_t)(y - s.box.y0) * (s.box.x1 - s.box.x0) + (x - s.box.x0);
+}
+
+__global__ __launch_bounds__(kSThreads) void k_smudge_steps(SArgs A) {
+  constexpr int kN = kSSide * kSSide;
+  __shared__ double M[7][kN];   // map cells: K, S, V
+  __shared__ float C[6][kN];    // canvas pixels: K, S
+  __shared__ double CV[kN], D[kN];  // their volume and texture thickness (0: no trade)
+  const TradeArgs& T = A.T;
+  const int t = threadIdx.x, n = A.n;
+  // regions: R[i] of step i (1-based; 0: the source map), in cells
+  SBox own;
+  {
+    const int bx = (int)blockIdx.x % A.tiles, by = (int)blockIdx.x / A.tiles;
+    own.x0 = bx * kSB - (bx == 0 ? A.ext[0] : 0);
+    own.y0 = by * kSB - (by == 0 ? A.ext[1] : 0);
+    own.x1 = min((bx + 1) * kSB, n) + (bx == A.tiles - 1 ? A.ext[2] : 0);
+    own.y1 = min((by + 1) * kSB, n) + (by == A.tiles - 1 ? A.ext[3] : 0);
+  }
+  SBox r0 = own;
+  for (int i = A.steps - 1; i >= 0; --i) {
+    r0.x0 -= A.st[i].lo_x;
+    r0.y0 -= A.st[i].lo_y;
+    r0.x1 += A.st[i].hi_x;
+    r0.y1 += A.st[i].hi_y;
+  }
+  SBox reg = r0;  // region of the step before, shrinking
+  const int w0 = r0.x1 - r0.x0;
+  // step 1's region: the pixels of the launch
+  const SBox r1{r0.x0 + A.st[0].lo_x, r0.y0 + A.st[0].lo_y, r0.x1 - A.st[0].hi_x,
+                r0.y1 - A.st[0].hi_y};
+  const int pw = r1.x1 - r1.x0, ph = r1.y1 - r1.y0;
+  const int px0 = r1.x0 + A.st[0].roi_x, py0 = r1.y0 + A.st[0].roi_y;
+  // ---- load
+  for (int e = t; e < w0 * (r0.y1 - r0.y0); e += kSThreads) {
+    const int x = r0.x0 + e % w0, y = r0.y0 + e / w0;
+    if (x < 0 || y < 0 || x >= n || y >= n) continue;
+    const int64_t ip = (int64_t)y * n + x;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      M[c][e] = A.src.K[3 * ip + c];
+      M[3 + c][e] = A.src.S[3 * ip + c];
+    }
+    M[6][e] = A.src.V[ip];
+  }
+  for (int e = t; e < pw * ph; e += kSThreads) {
+    const int x = px0 + e % pw, y = py0 + e / pw;
+    double d = 0.0;
+    if (x >= 0 && y >= 0 && x < T.cols && y < T.rows) {
+      if (in_box(A.prev.box, x, y)) {
+        const int64_t k = staged_at(A.prev, x, y);
+#pragma unroll
+        for (int c = 0; c < 6; ++c) C[c][e] = A.prev.ks[c * A.prev.stride + k];
+        CV[e] = A.prev.v[k];
+      } else {
+        const int64_t ic = (int64_t)y * T.cols + x;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) C[c][e] = T.canvas.ks[c][ic];
+        CV[e] = T.canvas.v[ic];
+      }
+      const int tpx = (int)(x - T.bmin_x), tpy = (int)(y - T.bmin_y);
+      if (!(tpx < 0 || tpy < 0 || tpx >= T.tcols || tpy >= T.trows)) {
+        d = T.tmap[(int64_t)tpy * T.tcols + tpx];
+        if (d <= 0.0) d = 0.0;
+      }
+    }
+    D[e] = d;
+  }
+  // the staged pixels that leave: back to the canvas (nobody reads them there)
+  {
+    const int sw = A.prev.box.x1 - A.prev.box.x0, sh = A.prev.box.y1 - A.prev.box.y0;
+    for (int e = (int)blockIdx.x * kSThreads + t; sw > 0 && e < sw * sh; e += (int)gridDim.x * kSThreads) {
+      const int x = A.prev.box.x0 + e % sw, y = A.prev.box.y0 + e / sw;
+      if (in_box(A.cur.box, x, y) || x < 0 || y < 0 || x >= T.cols || y >= T.rows) continue;
+      const int64_t ic = (int64_t)y * T.cols + x;
+#pragma unroll
+      for (int c = 0; c < 6; ++c) T.canvas.ks[c][ic] = A.prev.ks[c * A.prev.stride + e];
+      T.canvas.v[ic] = A.prev.v[e];
+    }
+  }
+  __syncthreads();
+  // ---- steps
+  for (int i = 0; i < A.steps; ++i) {
+    const SStep& S = A.st[i];
+    const SBox b{reg.x0 + S.lo_x, reg.y0 + S.lo_y, reg.x1 - S.hi_x, reg.y1 - S.hi_y};
+    reg = b;
+    const int w = b.x1 - b.x0, cells = w * (b.y1 - b.y0);
+    double p[kSPer][7];
+    int at[kSPer];
+#pragma unroll
+    for (int u = 0; u < kSPer; ++u) {
+      const int e = t + u * kSThreads;
+      at[u] = -1;
+      if (e >= cells) continue;
+      const int x = b.x0 + e % w, y = b.y0 + e / w;
+      if (x < 0 || y < 0 || x >= n || y >= n) continue;
+      at[u] = (y - r0.y0) * w0 + (x - r0.x0);
+      const double ox = x - A.cx, oy = y - A.cy;
+      const double rx = ox * S.cs - oy * S.sn + A.cx, ry = ox * S.sn + oy * S.cs + A.cy;
+      if (rx < 0 || ry < 0 || rx >= n || ry >= n) {
+#pragma unroll
+        for (int c = 0; c < 7; ++c) p[u][c] = M[c][at[u]];
+      } else {  // interp (bilinear, reflected border) on the region
+        const int xi = (int)floor(rx), yi = (int)floor(ry);
+        const int x0 = reflect_index(xi, n) - r0.x0, x1 = reflect_index(xi + 1, n) - r0.x0;
+        const int y0 = reflect_index(yi, n) - r0.y0, y1 = reflect_index(yi + 1, n) - r0.y0;
+        const double fa = rx - (double)xi, fc = ry - (double)yi;
+        const int i00 = y0 * w0 + x0, i01 = y0 * w0 + x1, i10 = y1 * w0 + x0, i11 = y1 * w0 + x1;
+#pragma unroll
+        for (int c = 0; c < 7; ++c)
+          p[u][c] = (M[c][i00] * (1.0 - fa) + M[c][i01] * fa) * (1.0 - fc) +
+                    (M[c][i10] * (1.0 - fa) + M[c][i11] * fa) * fc;
+      }
+      const int cpx = x + S.roi_x, cpy = y + S.roi_y;
+      const int q = (cpy - py0) * pw + (cpx - px0);
+      const double Dv = D[q];
+      const double dx = S.ctr_x - (double)cpx, dy = S.ctr_y - (double)cpy;
+      if (Dv > 0.0 && !(sqrt(dx * dx + dy * dy) > T.radius)) {
+        float cK[3], cS[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          cK[c] = C[c][q];
+          cS[c] = C[3 + c][q];
+        }
+        double cV = CV[q];
+        smudge_trade(&p[u][0], &p[u][3], p[u][6], cK, cS, cV, Dv, T.maxD);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          C[c][q] = cK[c];
+          C[3 + c][q] = cS[c];
+        }
+        CV[q] = cV;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kSPer; ++u)
+      if (at[u] >= 0)
+#pragma unroll
+        for (int c = 0; c < 7; ++c) M[c][at[u]] = p[u][c];
+    __syncthreads();
+  }
+  // ---- store what the block owns
+  const SStep& L = A.st[A.steps - 1];
+  const int ow = own.x1 - own.x0;
+  for (int e = t; e < ow * (own.y1 - own.y0); e += kSThreads) {
+    const int x = own.x0 + e % ow, y = own.y0 + e / ow;
+    if (x >= 0 && y >= 0 && x < n && y < n) {
+      const int64_t ip = (int64_t)y * n + x;
+      const int k = (y - r0.y0) * w0 + (x - r0.x0);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        A.dst.K[3 * ip + c] = M[c][k];
+        A.dst.S[3 * ip + c] = M[3 + c][k];
+      }
+      A.dst.V[ip] = M[6][k];
+    }
+    const int cpx = x + L.roi_x, cpy = y + L.roi_y;
+    if (cpx >= 0 && cpy >= 0 && cpx < T.cols && cpy < T.rows) {
+      const int q = (cpy - py0) * pw + (cpx - px0);
+      const int64_t k = staged_at(A.cur, cpx, cpy);
+#pragma unroll
+      for (int c = 0; c < 6; ++c) A.cur.ks[c * A.cur.stride + k] = C[c][q];
+      A.cur.v[k] = CV[q];
+    }
+  }
+}
+
+// The staged pixels back to the canvas.
+__global__ __launch_bounds__(kBlock) void k_smudge_unstage(Staged s, Layer7 canvas, int rows,
+                                                           int cols) {
+  const int w = s.box.x1 - s.box.x0;
+  const int e = (int)blockIdx.x * kBlock + (int)threadIdx.x;
+  if (e >= w * (s.box.y1 - s.box.y0)) return;
+  const int x = s.box.x0 + e % w, y = s.box.y0 + e / w;
+  if (x < 0 || y < 0 || x >= cols || y >= rows) return;
+  const int64_t ic = (int64_t)y * cols + x;
+#pragma unroll
+  for (int c = 0; c < 6; ++c) canvas.ks[c][ic] = s.ks[c * s.stride + e];
+  canvas.v[ic] = s.v[e];
 }
 
 inline unsigned blocks_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -398,6 +650,9 @@ struct pnt_tbrush_s {
   int64_t geo_cap = 0;
   double* tmap = nullptr;
   int64_t tmap_cap = 0;
+  // staged canvas pixels of the smudge's launches (two, ping-pong)
+  double* staged[2] = {nullptr, nullptr};
+  int64_t staged_px = 0;   // pixels each holds
   SMap maps(int k) const {
     const int64_t m = (int64_t)map * map;
     return SMap{smap[k], smap[k] + 3 * m, smap[k] + 6 * m};
@@ -422,6 +677,111 @@ void tb_smudge_reset(pnt_tbrush_s* b, int size) {
   }
   b->cur = 0;
   b->cur_rot = 0.0;
+}
+// A spine position of the smudge: the map's turn, centre and top-left pixel.
+struct Spine {
+  double sn, cs, x, y, dtheta;
+  int roi_x, roi_y;
+};
+
+// The smudge along the spine: as many positions per launch of k_smudge_steps
+// as its region holds, single ones (a sharp turn: the region would not hold
+// even that) through k_smudge_step.
+void smudge_spine(pnt_tbrush_s* b, TradeArgs T, const std::vector<Spine>& spine, hipStream_t s) {
+  const int n = b->map;
+  const int64_t m = (int64_t)n * n;
+  const double ctr = b->max_size / 2.0;
+  // cells lie at most this far from the turning point
+  const double far = std::sqrt(2.0) * std::max(ctr, std::fabs(n - 1 - ctr));
+  const int tiles = (n + kSB - 1) / kSB;
+  const bool blocked = n <= kSmudgeMost;
+  const int64_t px = (int64_t)(n + 2 * kSSide) * (n + 2 * kSSide);
+  if (blocked && px > b->staged_px) {
+    PNT_HIP_CHECK(hipStreamSynchronize(s));
+    for (double*& p : b->staged) {
+      dev_free(p);
+      p = nullptr;
+    }
+    b->staged_px = 0;
+    for (double*& p : b->staged) p = reinterpret_cast<double*>(dev_alloc(2 * 4 * px));
+    b->staged_px = px;
+  }
+  Staged prev{};
+  int which = 0;
+  const auto unstage = [&] {
+    const int w = prev.box.x1 - prev.box.x0, h = prev.box.y1 - prev.box.y0;
+    if (w <= 0 || h <= 0) return;
+    k_smudge_unstage<<<blocks_for((int64_t)w * h), kBlock, 0, s>>>(prev, T.canvas, T.rows, T.cols);
+    PNT_HIP_CHECK(hipGetLastError());
+    prev = Staged{};
+  };
+  SArgs A{};
+  A.n = n;
+  A.tiles = tiles;
+  A.cx = A.cy = ctr;
+  A.T = T;
+  for (size_t i = 0; i < spine.size();) {
+    // steps i .. i + k - 1 of one launch: the widest block's region must fit
+    int k = 0, grow_x = 0, grow_y = 0;
+    int min_x = INT_MAX, min_y = INT_MAX, max_x = INT_MIN, max_y = INT_MIN;
+    while (blocked && k < kSMax && i + k < spine.size()) {
+      const Spine& q = spine[i + k];
+      const int64_t jump = k ? std::max(std::llabs((long long)q.roi_x - spine[i + k - 1].roi_x),
+                                        std::llabs((long long)q.roi_y - spine[i + k - 1].roi_y))
+                             : 0;
+      const double turn = 2.0 * far * std::fabs(std::sin(0.5 * q.dtheta)) + 1e-6;
+      if (jump > kSSide || !(turn <= kSSide)) break;
+      const int d = (int)std::ceil(turn);
+      const int sx = k ? q.roi_x - spine[i + k - 1].roi_x : 0;
+      const int sy = k ? q.roi_y - spine[i + k - 1].roi_y : 0;
+      SStep S{q.sn, q.cs, q.x, q.y, q.roi_x, q.roi_y, std::max(d, -sx), std::max(d, -sy),
+              std::max(d + 1, sx), std::max(d + 1, sy)};
+      const int gx = grow_x + S.lo_x + S.hi_x, gy = grow_y + S.lo_y + S.hi_y;
+      const int nx0 = std::min(min_x, q.roi_x), nx1 = std::max(max_x, q.roi_x);
+      const int ny0 = std::min(min_y, q.roi_y), ny1 = std::max(max_y, q.roi_y);
+      // a tile and, at the map's edges, the pixels the map has left
+      if (kSB + gx + (nx1 - nx0) > kSSide || kSB + gy + (ny1 - ny0) > kSSide) break;
+      grow_x = gx;
+      grow_y = gy;
+      min_x = nx0;
+      max_x = nx1;
+      min_y = ny0;
+      max_y = ny1;
+      A.st[k++] = S;
+    }
+    if (k < 2) {
+      unstage();
+      const Spine& q = spine[i];
+      T.roi_x = q.roi_x;
+      T.roi_y = q.roi_y;
+      T.ctr_x = q.x;
+      T.ctr_y = q.y;
+      k_smudge_step<<<step_blocks_for(m), kStepBlock, 0, s>>>(b->maps(b->cur), b->maps(1 - b->cur), n,
+                                                              ctr, ctr, q.sn, q.cs, T);
+      k = 1;
+    } else {
+      const SStep& L = A.st[k - 1];
+      A.steps = k;
+      A.ext[0] = L.roi_x - min_x;
+      A.ext[1] = L.roi_y - min_y;
+      A.ext[2] = max_x - L.roi_x;
+      A.ext[3] = max_y - L.roi_y;
+      A.src = b->maps(b->cur);
+      A.dst = b->maps(1 - b->cur);
+      A.prev = prev;
+      A.cur.box = SBox{min_x, min_y, max_x + n, max_y + n};
+      A.cur.stride = b->staged_px;
+      A.cur.v = b->staged[which];
+      A.cur.ks = reinterpret_cast<float*>(b->staged[which] + b->staged_px);
+      which = 1 - which;
+      k_smudge_steps<<<(unsigned)(tiles * tiles), kSThreads, 0, s>>>(A);
+      prev = A.cur;
+    }
+    PNT_HIP_CHECK(hipGetLastError());
+    b->cur = 1 - b->cur;
+    i += (size_t)k;
+  }
+  unstage();
 }
 }  // namespace
 }  // namespace pnt
@@ -456,6 +816,7 @@ int pnt_tbrush_destroy(pnt_tbrush b) {
     dev_free(b->thick);
     dev_free(b->geo);
     dev_free(b->tmap);
+    for (double* p : b->staged) dev_free(p);
     delete b;
     ctx_release(ctx);
   });
@@ -666,6 +1027,8 @@ int pnt_tbrush_paint_stroke(pnt_tbrush b, pnt_canvas cv, const double* xy, int64
       T.trows = trows;
       T.tcols = tcols;
       T.maxD = maxD_h;
+      // the spine positions
+      std::vector<Spine> spine;
       for (double u = 0.0; maxD_h > 0.0 && u <= 1.0; u += 1. / length) {
         double center[2], t[2];
         spline_cr(v, u, false, center);
@@ -674,16 +1037,14 @@ int pnt_tbrush_paint_stroke(pnt_tbrush b, pnt_canvas cv, const double* xy, int64
         const double theta = std::atan2(t[1], t[0]);
         const double dtheta = normalize_angle(theta - b->cur_rot);
         b->cur_rot = theta;
-        T.roi_x = (int)(center[0] - b->map / 2.0);
-        T.roi_y = (int)(center[1] - b->map / 2.0);
-        T.ctr_x = center[0];
-        T.ctr_y = center[1];
-        k_smudge_step<<<step_blocks_for(m), kStepBlock, 0, s>>>(
-            b->maps(b->cur), b->maps(1 - b->cur), b->map, b->max_size / 2.0, b->max_size / 2.0,
-            std::sin(dtheta), std::cos(dtheta), T);
-        PNT_HIP_CHECK(hipGetLastError());
-        b->cur = 1 - b->cur;
+        spine.push_back(Spine{std::sin(dtheta), std::cos(dtheta), center[0], center[1], dtheta,
+                              (int)(center[0] - b->map / 2.0), (int)(center[1] - b->map / 2.0)});
+        if (spine.size() == 65536) {
+          smudge_spine(b, T, spine, s);
+          spine.clear();
+        }
       }
+      smudge_spine(b, T, spine, s);
     }
     k_tex_deposit<<<blocks_for(npx), kBlock, 0, s>>>(A);
     PNT_HIP_CHECK(hipGetLastError());

@@ -163,3 +163,21 @@ def test_short_stroke_and_errors(hip, oracle):
         gb.setThicknessMap(np.full((4, 4), np.nan))
     gb.setThicknessMap(np.ones((4, 4)))
     compare_canvas("texture/no-op", gc, oc)
+
+
+# Maps of less than one tile, of whole tiles, of a tile and a bit, and past the
+# side that goes one step a launch; hairpins turn the map too far for a region.
+@pytest.mark.parametrize("radius", [1.5, 4.0, 12.3, 40.0, 70.0])
+@pytest.mark.parametrize("path", ["diagonal", "hairpin", "wave"])
+def test_smudge_over_map_sizes_and_turns(hip, oracle, radius, path):
+    rows, cols = 150, 190
+    oc, gc = _canvases(hip, oracle, rows, cols, int(10 * radius))
+    ob, gb = _brushes(hip, oracle, radius, sample_thickness(), True)
+    strokes = {"diagonal": [[[5.2, 140.7], [180.3, 12.1]], [[185.0, 140.0], [20.0, 20.0]]],
+               "hairpin": [[[20.1, 60.3], [150.4, 66.2], [150.9, 72.8], [22.3, 78.1]]],
+               "wave": [[[4.3, 75.0], [50.2, 40.1], [100.7, 110.4], [150.2, 44.6], [188.0, 80.3]],
+                        [[180.0, 30.0], [90.5, 32.0], [10.0, 120.0]]]}[path]
+    for k, xy in enumerate(strokes):
+        ob.paint_stroke(np.array(xy), oc)
+        gb.paintStroke(np.array(xy), gc)
+        _compare("texture/r%g/%s/%d" % (radius, path, k), gc, oc, gb, ob)
