@@ -353,8 +353,8 @@ __global__ __launch_bounds__(kStepBlock) void k_smudge_step(SMap src, SMap dst, 
 // bit), and written only by the block that owns them.
 //
 // A step's region is a rectangle of map cells: step t needs, of step t - 1,
-// the cells within the turn's largest displacement (and one more, the
-// bilinear neighbour) and the cells that met its pixels then (the map moves a
+// the cells within the turn's largest displacement rounded up (x + d with
+// |d| < D: floor(x + d) >= x - D, and its right neighbour <= x + D) and the cells that met its pixels then (the map moves a
 // pixel or so along the stroke).  Rectangles may reach outside the map: such
 // places have a pixel and no cell.
 //
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(kStepBlock) void k_smudge_step(SMap src, SMap dst, 
 // reads them there, and writes back those it no longer covers.
 constexpr int kSB = 8;        // tile side
 constexpr int kSSide = 40;    // side of the region in LDS: 96 B a place, 150 KB
-constexpr int kSMax = 8;      // steps of a launch
+constexpr int kSMax = 10;     // steps of a launch
 constexpr int kSThreads = 1024;
 constexpr int kSPer = (kSSide * kSSide + kSThreads - 1) / kSThreads;
 
@@ -483,6 +483,7 @@ __global__ __launch_bounds__(kSThreads) void k_smudge_steps(SArgs A) {
     const SBox b{reg.x0 + S.lo_x, reg.y0 + S.lo_y, reg.x1 - S.hi_x, reg.y1 - S.hi_y};
     reg = b;
     const int w = b.x1 - b.x0, cells = w * (b.y1 - b.y0);
+    const float iw = __builtin_amdgcn_rcpf((float)w);
     double p[kSPer][7];
     int at[kSPer];
 #pragma unroll
@@ -490,7 +491,8 @@ __global__ __launch_bounds__(kSThreads) void k_smudge_steps(SArgs A) {
       const int e = t + u * kSThreads;
       at[u] = -1;
       if (e >= cells) continue;
-      const int x = b.x0 + e % w, y = b.y0 + e / w;
+      const int ey = (int)(((float)e + 0.5f) * iw);  // e / w (w <= 40, e < 1600)
+      const int x = b.x0 + e - ey * w, y = b.y0 + ey;
       if (x < 0 || y < 0 || x >= n || y >= n) continue;
       at[u] = (y - r0.y0) * w0 + (x - r0.x0);
       const double ox = x - A.cx, oy = y - A.cy;
@@ -731,11 +733,11 @@ void smudge_spine(pnt_tbrush_s* b, TradeArgs T, const std::vector<Spine>& spine,
                              : 0;
       const double turn = 2.0 * far * std::fabs(std::sin(0.5 * q.dtheta)) + 1e-6;
       if (jump > kSSide || !(turn <= kSSide)) break;
-      const int d = (int)std::ceil(turn);
+      const int d = (int)std::ceil(turn);  // a turned position and its right neighbour lie within d
       const int sx = k ? q.roi_x - spine[i + k - 1].roi_x : 0;
       const int sy = k ? q.roi_y - spine[i + k - 1].roi_y : 0;
       SStep S{q.sn, q.cs, q.x, q.y, q.roi_x, q.roi_y, std::max(d, -sx), std::max(d, -sy),
-              std::max(d + 1, sx), std::max(d + 1, sy)};
+              std::max(d, sx), std::max(d, sy)};
       const int gx = grow_x + S.lo_x + S.hi_x, gy = grow_y + S.lo_y + S.hi_y;
       const int nx0 = std::min(min_x, q.roi_x), nx1 = std::max(max_x, q.roi_x);
       const int ny0 = std::min(min_y, q.roi_y), ny1 = std::max(max_y, q.roi_y);
