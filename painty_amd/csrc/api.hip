@@ -190,10 +190,10 @@ void brush_set_geometry(pnt_brush b, double radius, const float* core, int width
   // would wait for the whole device)
   float* fp = b->fp;
   float* pick = b->pick;
-  if (m > b->fp_cap || 7 * mstride > b->pick_cap) {
+  if (m > b->fp_cap || kCell * mstride > b->pick_cap) {
     fp = dev_alloc(m);
     try {
-      pick = dev_alloc(7 * mstride);
+      pick = dev_alloc(kCell * mstride);
     } catch (...) {
       dev_free(fp);
       throw;
@@ -201,7 +201,7 @@ void brush_set_geometry(pnt_brush b, double radius, const float* core, int width
   }
   try {
     PNT_HIP_CHECK(hipMemcpyAsync(fp, full.data(), m * sizeof(float), hipMemcpyHostToDevice, s));
-    launch_fill(pick, 7 * mstride, 0.0f, s);
+    launch_fill(pick, kCell * mstride, 0.0f, s);
     PNT_HIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
     if (fp != b->fp) {  // the new buffers are not the brush's yet
@@ -214,7 +214,7 @@ void brush_set_geometry(pnt_brush b, double radius, const float* core, int width
     dev_free(b->fp);
     dev_free(b->pick);
     b->fp_cap = m;
-    b->pick_cap = 7 * mstride;
+    b->pick_cap = kCell * mstride;
   }
   b->fp = fp;
   footprint_box(full, size_map, b->fbox);
@@ -267,12 +267,8 @@ StampArgs stamp_args(pnt_brush b, pnt_canvas cv, double cx, double cy, double th
   a.g.size_map = b->size_map;
   a.g.rows = cv->rows;
   a.g.cols = cv->cols;
-  a.b = b->args();
-  a.canvas = cv->layer();
-  a.src = b->use_snap ? b->snap_planes() : cv->layer();
   a.dupx = stamp_dup_axis(cx, a.g.hr) ? 1 : 0;
   a.dupy = stamp_dup_axis(cy, a.g.hr) ? 1 : 0;
-  a.clk = DryClock{};
   return a;
 }
 
@@ -517,7 +513,7 @@ void plan_shared_visits(const StampArgs& a, std::vector<int2>& list, std::vector
 namespace {
 
 void brush_dip(pnt_brush b, const float K[3], const float S[3]) {
-  launch_fill(b->pick, 7 * b->mstride, 0.0f, b->ctx->stream);
+  launch_fill(b->pick, kCell * b->mstride, 0.0f, b->ctx->stream);
   for (int c = 0; c < 3; ++c) {
     b->paintK[c] = K[c];
     b->paintS[c] = S[c];
@@ -1458,10 +1454,21 @@ int pnt_brush_get_pickup_map(pnt_brush b, float* K, float* S, float* V, int layo
     PNT_REQUIRE(b, "NULL brush");
     check_layout(layout);
     b->ctx->use();
-    const Plane7 P = b->pick_planes();
-    if (K) download_planes(K, 3, P.p, b->m, layout, b->ctx->stream);
-    if (S) download_planes(S, 3, P.p + 3, b->m, layout, b->ctx->stream);
-    if (V) download_planes(V, 1, P.p + 6, b->m, layout, b->ctx->stream);
+    if (!K && !S && !V) return;
+    std::vector<float> cells((size_t)(kCell * b->m));
+    PNT_HIP_CHECK(hipMemcpyAsync(cells.data(), b->pick, cells.size() * sizeof(float),
+                                 hipMemcpyDeviceToHost, b->ctx->stream));
+    PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
+    const bool planar = layout == PNT_PLANAR;
+    for (int64_t i = 0; i < b->m; ++i) {
+      const float* c = &cells[(size_t)(kCell * i)];
+      for (int k = 0; k < 3; ++k) {
+        const int64_t at = planar ? k * b->m + i : 3 * i + k;
+        if (K) K[at] = c[k];
+        if (S) S[at] = c[3 + k];
+      }
+      if (V) V[i] = c[6];
+    }
   });
 }
 
@@ -1514,7 +1521,7 @@ int pnt_brush_clean(pnt_brush b) {
   return guard([&] {
     PNT_REQUIRE(b, "NULL brush");
     b->ctx->use();
-    launch_fill(b->pick, 7 * b->mstride, 0.0f, b->ctx->stream);
+    launch_fill(b->pick, kCell * b->mstride, 0.0f, b->ctx->stream);
   });
 }
 

@@ -48,7 +48,7 @@ constexpr int64_t kComposeItem = 1 << 18;  // pixels per composite work item
 
 struct BJob {
   Layer7 canvas, snap;
-  Plane7 pick;
+  float* pick;
   Rgb3 R0, out;
   float* h;
   const float* fp;
@@ -158,9 +158,9 @@ __global__ __launch_bounds__(kWT* kWT) void k_batch(BArgs A) {
           pk[c] = st.K[c];
           ps[c] = st.S[c];
         }
+        const float clean[7] = {};
         for (int64_t i = gtid; i < m; i += gthreads)
-#pragma unroll
-          for (int c = 0; c < 7; ++c) J.pick.p[c][i] = 0.0f;
+          st_cell(J.pick, (int)i, clean);
         if (!group_sync(bar, nb, rank, A.host_err)) {
           alive = false;
           break;
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kWT* kWT) void k_batch(BArgs A) {
       const TileWin win = tile_window(g, J.fb);
       const int ntiles = tile_count<kWT>(win);
       for (int tile = rank; tile < ntiles; tile += (int)nb)
-        window_tile<kWT, StampKind<false, true, 2>>(T, J.pick.p, J.fp, J.fb, g, st, dup, pull, tile,
+        window_tile<kWT, StampKind<false, true, 2>>(T, J.pick, J.fp, J.fb, g, st, dup, pull, tile,
                                                     win, lds.hand, pk, ps);
       // ---- visits sharing canvas column/row 0, level by level
       for (int L = 0; L < st.dl_nlev; ++L) {
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(kWT* kWT) void k_batch(BArgs A) {
           int64_t ic;
           const int mm2 = stamp_visit(g, v.x, v.y, &ic);
           if (mm2 >= 0 && J.fp[mm2] > 0.0f)
-            cached_visit(T, J.pick.p, mm2, J.fp[mm2], ic, false, pk, ps);
+            cached_visit(T, J.pick, mm2, J.fp[mm2], ic, false, pk, ps);
         }
       }
       if (!alive) break;
@@ -519,7 +519,7 @@ static BatchPlan plan_batch(pnt_ctx ctx, const pnt_batch_job* jobs, int n,
     BJob& J = h_jobs[j];
     J = BJob{};
     J.canvas = cv->layer();
-    J.pick = b->pick_planes();
+    J.pick = b->pick;
     J.snap = b->use_snap ? b->snap_planes() : cv->layer();
     J.R0 = cv->R0();
     J.h = cv->h();
@@ -773,8 +773,8 @@ pnt_batch_config get_batch_config(pnt_ctx ctx) { return batch_state(ctx)->cfg; }
 // as it found them.
 struct SavedJob {
   float* canvas = nullptr;  // 11 planes
-  float* pick = nullptr;    // 7 planes
-  float* snap = nullptr;    // 7 planes
+  float* pick = nullptr;    // mstride cells
+  float* snap = nullptr;    // mstride cells
   uint8_t* dirty = nullptr;
   int64_t canvas_n = 0, pick_n = 0, snap_n = 0, dirty_n = 0;
   float paintK[3], paintS[3];
@@ -793,7 +793,7 @@ static void save_or_restore(const pnt_batch_job* jobs, int n, std::vector<SavedJ
     SavedJob& S = sv[j];
     if (save) {
       S.canvas_n = kCanvasStrides * cv->stride;
-      S.pick_n = 7 * b->mstride;
+      S.pick_n = kCell * b->mstride;
       S.snap_n = b->snap ? kLayerStrides * b->snap_stride : 0;
       S.dirty_n = b->dirty ? b->dirty_cap : 0;
       S.canvas = dev_alloc(S.canvas_n);

@@ -287,7 +287,7 @@ static std::vector<int> job_chunks(const pnt_batch_job* jobs, int n, int chunk) 
 int64_t plan_waves_pool(const pnt_batch_job* jobs, int n, int chunk) {
   const std::vector<int> c = job_chunks(jobs, n, chunk);
   int64_t need = 0;
-  for (int j = 0; j < n; ++j) need += (int64_t)(c[(size_t)j] - 1) * 7 * jobs[j].brush->mstride;
+  for (int j = 0; j < n; ++j) need += (int64_t)(c[(size_t)j] - 1) * kCell * jobs[j].brush->mstride;
   return need;
 }
 
@@ -363,7 +363,7 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
             int nblk = 1;
             switch (f.kind) {
               case kSClear:
-                nblk = (int)std::min<int64_t>(64, (7 * b->mstride + 4 * kWT2 - 1) / (4 * kWT2));
+                nblk = (int)std::min<int64_t>(64, (kCell * b->mstride + 4 * kWT2 - 1) / (4 * kWT2));
                 break;
               case kSStamp:  // + the shared-pixel levels' block of a dup stamp
                 plain &= b->use_snap && !(J.st[(size_t)f.k].flags & (kStDupX | kStDupY)) &&
@@ -457,7 +457,7 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
     for (int c = 1; c < kMaxChunk; ++c) {
       if (c < J.chains) {
         d.pick[c] = pool + pool_at;
-        pool_at += 7 * b->mstride;
+        pool_at += kCell * b->mstride;
       } else {
         d.pick[c] = b->pick;
       }

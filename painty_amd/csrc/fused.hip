@@ -96,7 +96,7 @@ struct WSlot {
   int size_map, pad;
   int64_t mstride;
   const float* fp;
-  float* pick;         // the unit's pickup map (7 planes of mstride)
+  float* pick;         // the unit's pickup map (mstride cells)
   float* tape;         // the stamp's tape record (launches that keep one)
   FpBox dom;           // the cells its visits run over (cell_domain)
   TileWin win;
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kT2, F::clock || F::dup ? 4 : 5) void k_stamp_wave(
   const int b = (int)blockIdx.x;
   if (b >= S.nblk) return;
   if (S.kind == kPhClear) {  // dip() / setRadius: a clean pickup map
-    const int64_t total = 7 * S.mstride;
+    const int64_t total = kCell * S.mstride;
     for (int64_t i = (int64_t)b * kT2 + threadIdx.x; i < total; i += (int64_t)S.nblk * kT2)
       S.pick[i] = 0.0f;
     return;
@@ -136,13 +136,10 @@ __global__ __launch_bounds__(kT2, F::clock || F::dup ? 4 : 5) void k_stamp_wave(
   const TapeRec tape =
       F::tape ? tape_rec(S.tape, H.tape_area, H.tape_m, st.box, H.cols) : TapeRec{};
   const VisitTarget T{&canvas, &snap, H.dirty, H.use_snap, H.pickup_rate, H.dep_rate, H.cap, &tape};
-  float* pick[7];
-#pragma unroll
-  for (int c = 0; c < 7; ++c) pick[c] = S.pick + c * S.mstride;
   float* R0 = H.canvas + 8 * H.cs;
   const DryClock clk{F::clock ? H.tmap : nullptr, st.now_us, H.dry_ms,
                      Rgb3{{R0, R0 + H.cs, R0 + 2 * H.cs}}, H.canvas + 11 * H.cs};
-  stamp_block<F>(T, pick, S.fp, S.dom, g, st, S.win, S.ntiles, S.rb, b, lds, H.dl,
+  stamp_block<F>(T, S.pick, S.fp, S.dom, g, st, S.win, S.ntiles, S.rb, b, lds, H.dl,
                               H.dl_off, S.pk, S.ps, clk);
 }
 
@@ -203,7 +200,7 @@ WSlot clear_slot(float* pick, int64_t mstride) {
   S.kind = kPhClear;
   S.pick = pick;
   S.mstride = mstride;
-  S.nblk = (int)std::min<int64_t>(64, (7 * mstride + 4 * kT2 - 1) / (4 * kT2));
+  S.nblk = (int)std::min<int64_t>(64, (kCell * mstride + 4 * kT2 - 1) / (4 * kT2));
   return S;
 }
 
@@ -454,10 +451,10 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
     return stamp_slot(H, D.host[k], geos[i].fp, gdom[i], geos[i].size_map, pick, gstride[i], pk, ps);
   };
 
-  // one stamp on stream `q` with pickup map `pick` (7 planes of its stride)
+  // one stamp on stream `q` with pickup map `pick` (cells)
   auto launch_stamp = [&](int64_t k, hipStream_t q, float* pick) {
     if (clear[k] || (st[k].flags & PNT_STAMP_DIP))  // setRadius / dip(): a clean pickup map
-      launch_fill(pick, 7 * gstride[(size_t)geo[(size_t)k]], 0.0f, q);
+      launch_fill(pick, kCell * gstride[(size_t)geo[(size_t)k]], 0.0f, q);
     if (st[k].flags & PNT_STAMP_DIP)
       for (int c = 0; c < 3; ++c) {
         b->paintK[c] = st[k].K[c];
@@ -591,13 +588,13 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
     for (int c = 0; c < used; ++c) {
       if (c > 0 && !F.streams[c])
         PNT_HIP_CHECK(hipStreamCreateWithFlags(&F.streams[c], hipStreamNonBlocking));
-      if (F.pick_cap[c] < 7 * max_stride) {
+      if (F.pick_cap[c] < kCell * max_stride) {
         if (c > 0) PNT_HIP_CHECK(hipStreamSynchronize(F.streams[c]));
         PNT_HIP_CHECK(hipStreamSynchronize(s));
         dev_free(F.pick[c]);
         F.pick[c] = nullptr;
-        F.pick[c] = dev_alloc(7 * max_stride);
-        F.pick_cap[c] = 7 * max_stride;
+        F.pick[c] = dev_alloc(kCell * max_stride);
+        F.pick_cap[c] = kCell * max_stride;
       }
       S[c] = c == 0 ? s : F.streams[c];
       pick[c] = F.pick[c];
@@ -606,12 +603,12 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
       // a first unit that continues the brush's stroke starts from its map
       if (!clear[0] && !(st[0].flags & PNT_STAMP_DIP))
         PNT_HIP_CHECK(hipMemcpyAsync(pick[0], b->pick,
-                                     7 * gstride[(size_t)geo[0]] * sizeof(float),
+                                     kCell * gstride[(size_t)geo[0]] * sizeof(float),
                                      hipMemcpyDeviceToDevice, s));
       run_waves(U, used, pick);
       finish_geometry();
       PNT_HIP_CHECK(hipMemcpyAsync(b->pick, pick[U.back().chain],
-                                   7 * gstride[(size_t)geo[(size_t)n - 1]] * sizeof(float),
+                                   kCell * gstride[(size_t)geo[(size_t)n - 1]] * sizeof(float),
                                    hipMemcpyDeviceToDevice, s));
       cv->epoch++;
       if (b->use_snap) {
@@ -634,7 +631,7 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
     };
     // a first unit that continues the brush's stroke starts from its map
     if (!clear[0] && !(st[0].flags & PNT_STAMP_DIP))
-      PNT_HIP_CHECK(hipMemcpyAsync(pick[0], b->pick, 7 * gstride[(size_t)geo[0]] * sizeof(float),
+      PNT_HIP_CHECK(hipMemcpyAsync(pick[0], b->pick, kCell * gstride[(size_t)geo[0]] * sizeof(float),
                                    hipMemcpyDeviceToDevice, s));
     // the plan and everything before this call are on s
     const hipEvent_t ready = record(s);
@@ -663,7 +660,7 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
     finish_geometry();
     // the pickup map of the list's last stroke is the brush's from now on
     PNT_HIP_CHECK(hipMemcpyAsync(b->pick, pick[U.back().chain],
-                                 7 * gstride[(size_t)geo[(size_t)n - 1]] * sizeof(float),
+                                 kCell * gstride[(size_t)geo[(size_t)n - 1]] * sizeof(float),
                                  hipMemcpyDeviceToDevice, s));
   }
   cv->epoch++;
@@ -780,7 +777,7 @@ void run_fused_strokes_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* S, 
 struct FArgs {
   const PStamp* st;
   Layer7 canvas, snap;  // snap == canvas planes when the snapshot is off
-  Plane7 pick;
+  float* pick;
   const float* fp;
   FpBox fb;  // nonzero footprint cells
   uint8_t* dirty;
@@ -800,7 +797,7 @@ struct CArgs {
   unsigned* ticket;
   unsigned* abort;
   unsigned* host_err;
-  float* pick;          // pickup map base (7 planes of mstride)
+  float* pick;          // pickup map base (mstride cells)
   int64_t pick_floats;
   int long_sleep;       // poll every ~1 us instead of ~0.1 us
 };
@@ -872,7 +869,7 @@ __global__ __launch_bounds__(kCT* kCT) void k_stamp_chain(CArgs A) {
     const VisitTarget T{&A.f.canvas, &A.f.snap, A.f.dirty, A.f.use_snap, A.f.pickup_rate,
                         A.f.dep_rate, A.f.cap};
     float pkr[3] = {pk[0], pk[1], pk[2]}, psr[3] = {ps[0], ps[1], ps[2]};
-    window_tile<kCT, StampKind<false, true, 2>>(T, A.f.pick.p, A.f.fp, A.f.fb, g, st, dup, pull, off - r.x - r.y,
+    window_tile<kCT, StampKind<false, true, 2>>(T, A.f.pick, A.f.fp, A.f.fb, g, st, dup, pull, off - r.x - r.y,
                     tile_window(g, A.f.fb), lds.hand, pkr, psr);
   } else {  // visits sharing canvas column/row 0, by dependency level
     const VisitTarget T{&A.f.canvas, &A.f.snap, A.f.dirty, A.f.use_snap, A.f.pickup_rate,
@@ -885,7 +882,7 @@ __global__ __launch_bounds__(kCT* kCT) void k_stamp_chain(CArgs A) {
         int64_t ic;
         const int m = stamp_visit(g, vv.x, vv.y, &ic);
         if (m >= 0 && A.f.fp[m] > 0.0f)
-          cached_visit(T, A.f.pick.p, m, A.f.fp[m], ic, false, pkr, psr);
+          cached_visit(T, A.f.pick, m, A.f.fp[m], ic, false, pkr, psr);
       }
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
@@ -942,7 +939,7 @@ static void run_chained_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st,
   F.st = D.st;
   F.canvas = cv->layer();
   F.snap = b->use_snap ? b->snap_planes() : cv->layer();
-  F.pick = b->pick_planes();
+  F.pick = b->pick;
   F.fp = b->fp;
   F.fb = FpBox{b->fbox[0], b->fbox[1], b->fbox[2], b->fbox[3]};
   F.dirty = b->dirty;
@@ -960,7 +957,7 @@ static void run_chained_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st,
   std::vector<int4> roles(n);
   std::vector<int> start(n + 1);
   std::vector<float> paint(6 * (size_t)n);
-  const int64_t pick_floats = 7 * b->mstride;
+  const int64_t pick_floats = kCell * b->mstride;
   const int nclear = (int)std::min<int64_t>((pick_floats + kCT * kCT * 4 - 1) / (kCT * kCT * 4), 256);
   float pk[3] = {b->paintK[0], b->paintK[1], b->paintK[2]};
   float ps[3] = {b->paintS[0], b->paintS[1], b->paintS[2]};
@@ -1141,7 +1138,7 @@ void run_fused_noalloc(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, in
                                 H.tmap != nullptr);
   for (int64_t k = 0; k < n; ++k) {
     if (st[k].flags & PNT_STAMP_DIP) {  // dip(): clean() and the new paint
-      launch_fill(b->pick, 7 * b->mstride, 0.0f, s);
+      launch_fill(b->pick, kCell * b->mstride, 0.0f, s);
       for (int c = 0; c < 3; ++c) {
         b->paintK[c] = st[k].K[c];
         b->paintS[c] = st[k].S[c];

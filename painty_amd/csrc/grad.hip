@@ -220,7 +220,7 @@ __device__ __forceinline__ void visit_fwd(VState& s, float fh, double pr, double
 struct ASlot {
   int nblk, clear, ntiles, rb;
   float* tape;     // the stamp's tape record
-  float* gP;       // its chain's pickup-map adjoint, 7 planes of m
+  float* gP;       // its chain's pickup-map adjoint, m cells
   float* gB;       // 6 floats: the stamp's paint adjoint
   float* scratch;  // records of the shared-pixel replay
   TileWin win;
@@ -247,8 +247,7 @@ struct AArgs {
 static_assert(sizeof(AArgs) <= 4000, "kernel arguments must fit the argument segment");
 
 __device__ __forceinline__ void load_in(const TapeRec& t, bool snap, int64_t k, int mm, VState& s) {
-#pragma unroll
-  for (int c = 0; c < 7; ++c) s.P[c] = t.P[c * t.m + mm];
+  ld_cell(t.P, mm, s.P);
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
     s.C[c] = t.ck[c * t.area + k];
@@ -260,8 +259,7 @@ __device__ __forceinline__ void load_in(const TapeRec& t, bool snap, int64_t k, 
 
 __device__ __forceinline__ void store_in(const TapeRec& t, bool snap, int64_t k, int mm,
                                          const VState& s) {
-#pragma unroll
-  for (int c = 0; c < 7; ++c) t.P[c * t.m + mm] = s.P[c];
+  st_cell(t.P, mm, s.P);
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
     t.ck[c * t.area + k] = (float)s.C[c];
@@ -335,8 +333,7 @@ __device__ __forceinline__ void adj_tile(const AShared& A, const ASlot& S, const
     const int64_t ic1 = (int64_t)V.y * A.cols + V.x;
     VState in1, gs;
     load_in(tape, snap, tape.at(V.x, V.y), V.mm, in1);
-#pragma unroll
-    for (int c = 0; c < 7; ++c) gs.P[c] = S.gP[c * A.m + V.mm];
+    ld_cell(S.gP, V.mm, gs.P);
     if (two) {
       const int x2 = (int)(col + dx + g.cx), y2 = (int)(row + dy + g.cy);
       const int64_t ic2 = (int64_t)y2 * A.cols + x2;
@@ -355,8 +352,7 @@ __device__ __forceinline__ void adj_tile(const AShared& A, const ASlot& S, const
     load_g_pixel(A, ic1, gs);
     visit_adj(in1, gs, gB, fh, A.pr, A.dr, A.cap, S.pk, S.ps, alias);
     store_g_pixel(A, ic1, gs, snap && on_window_border(S.st.box, V.x, V.y));
-#pragma unroll
-    for (int c = 0; c < 7; ++c) S.gP[c * A.m + V.mm] = gs.P[c];
+    st_cell(S.gP, V.mm, gs.P);
   }
   flush_gB(S.gB, gB);
 }
@@ -442,15 +438,13 @@ __device__ __forceinline__ void adj_levels(const AShared& A, const ASlot& S, con
       const int mm = stamp_visit(g, v.x, v.y, &ic);
       if (mm < 0 || !(A.fp[mm] > 0.0f)) continue;
       VState gs;
-#pragma unroll
-      for (int c = 0; c < 7; ++c) gs.P[c] = S.gP[c * A.m + mm];
+      ld_cell(S.gP, mm, gs.P);
       load_g_pixel(A, ic, gs);
       const VState in = rec[e - base];
       store_in(t, snap, t.at((int)(ic % A.cols), (int)(ic / A.cols)), mm, in);
       visit_adj(in, gs, gB, A.fp[mm], A.pr, A.dr, A.cap, S.pk, S.ps, alias);
       store_g_pixel(A, ic, gs, snap && first_acting_visit(g, st.box, A.fp, v.x, v.y, ic, false));
-#pragma unroll
-      for (int c = 0; c < 7; ++c) S.gP[c * A.m + mm] = gs.P[c];
+      st_cell(S.gP, mm, gs.P);
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -465,7 +459,7 @@ __global__ __launch_bounds__(kBlk) void k_adj_wave(AArgs A) {
   const int b = (int)blockIdx.x;
   if (b >= S.nblk) return;
   if (S.clear) {
-    for (int64_t i = (int64_t)b * kBlk + threadIdx.x; i < 7 * A.sh.m; i += (int64_t)S.nblk * kBlk)
+    for (int64_t i = (int64_t)b * kBlk + threadIdx.x; i < kCell * A.sh.m; i += (int64_t)S.nblk * kBlk)
       S.gP[i] = 0.0f;
     return;
   }
@@ -578,10 +572,10 @@ __global__ __launch_bounds__(kBlk) void k_km_adj(int64_t n, Layer7 L, Rgb3 R0, R
 // A w x h box at (x0, y0) of a layer's planes (row stride `cols`) <-> a
 // dense buffer of 7 planes (plane stride `stride`): FP64 planes for a
 // canvas or snapshot layer (K, S widened exactly, V as stored), FP32 planes
-// for the pickup map.  Up to three boxes per launch.
+// for the pickup map's cells.  Up to three boxes per launch.
 struct BoxRegion {
   Layer7 L;   // when layer
-  Plane7 P;   // otherwise
+  float* P;   // otherwise: cells
   int layer;
   int cols, x0, y0, w, h;
   void* buf;  // double* (layer) or float*
@@ -603,7 +597,7 @@ inline BoxRegion layer_box(const Layer7& L, int cols, int x0, int y0, int w, int
   return r;
 }
 
-inline BoxRegion plane_box(const Plane7& P, int cols, int x0, int y0, int w, int h, float* buf,
+inline BoxRegion cell_box(float* P, int cols, int x0, int y0, int w, int h, float* buf,
                            int64_t stride) {
   BoxRegion r{};
   r.P = P;
@@ -643,9 +637,9 @@ __global__ __launch_bounds__(kBlk) void k_box_copy(BoxRegion r0, BoxRegion r1, B
 #pragma unroll
       for (int c = 0; c < 7; ++c) {
         if (to_buf)
-          b[c * r.stride + e] = r.P.p[c][i];
+          b[c * r.stride + e] = r.P[kCell * i + c];
         else
-          r.P.p[c][i] = b[c * r.stride + e];
+          r.P[kCell * i + c] = b[c * r.stride + e];
       }
     }
   }
@@ -708,7 +702,7 @@ struct pnt_grad_s {
   bool fwd_snap = false;
   float* gX = nullptr;  // 7 planes of round_up(n, 64) (snapshot adjoint); zero between calls
   uint8_t* gdirty = nullptr;  // its dirty bytes; zero between calls
-  float* gP = nullptr;  // per chain: 7 planes of m (pickup adjoint)
+  float* gP = nullptr;  // per chain: m cells (pickup adjoint)
   float* gB = nullptr;  // n_stamps x 6
   int64_t gX_cap = 0, gdirty_cap = 0, gP_cap = 0, gB_cap = 0;
   float* scratch = nullptr;
@@ -804,9 +798,9 @@ static void adjoint_waves(pnt_grad_s* g, int s0, const Plane7& gC, const Plane7&
       ASlot& S = A.slot[ns++];
       S = ASlot{};
       S.clear = f.clear;
-      S.gP = g->gP + (int64_t)f.chain * 7 * R.m;
+      S.gP = g->gP + (int64_t)f.chain * kCell * R.m;
       if (f.clear) {
-        S.nblk = (int)std::min<int64_t>(64, (7 * R.m + 4 * kBlk - 1) / (4 * kBlk));
+        S.nblk = (int)std::min<int64_t>(64, (kCell * R.m + 4 * kBlk - 1) / (4 * kBlk));
       } else {
         const PStamp& st = R.st[(size_t)f.k];
         S.st = st;
@@ -1000,14 +994,13 @@ int pnt_grad_forward(pnt_grad g, pnt_dev_layer wet0, pnt_dev_rgb R0, const doubl
         s0 = s1;
       }
       ensure(g->ckpt, g->ckpt_cap, std::max<int64_t>(total, 1), s);
-      const Plane7 pick = b->pick_planes();
       for (const auto& sg : g->segs) {
         const int64_t area = (int64_t)sg.w * sg.h;
         float* c0 = g->ckpt + sg.off;
         box_copy({layer_box(L, cv->cols, sg.x0, sg.y0, sg.w, sg.h, reinterpret_cast<double*>(c0), area),
                   layer_box(b->snap_planes(), cv->cols, sg.x0, sg.y0, b->use_snap ? sg.w : 0, sg.h,
                             reinterpret_cast<double*>(c0 + 14 * area), area),
-                  plane_box(pick, b->size_map, 0, 0, b->size_map, b->size_map,
+                  cell_box(b->pick, b->size_map, 0, 0, b->size_map, b->size_map,
                             c0 + (b->use_snap ? 28 : 14) * area, m)},
                  true, s);
         if (other) PNT_HIP_CHECK(hipStreamSynchronize(s));
@@ -1051,15 +1044,14 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
         launch_fill_u8(g->gdirty, nst + 16, 0, s);
       }
     }
-    ensure(g->gP, g->gP_cap, kAdjSlots * 7 * m, s);
+    ensure(g->gP, g->gP_cap, kAdjSlots * kCell * m, s);
     ensure(g->gB, g->gB_cap, 6 * (int64_t)ns, s);
-    launch_fill(g->gP, kAdjSlots * 7 * m, 0.0f, s);
+    launch_fill(g->gP, kAdjSlots * kCell * m, 0.0f, s);
     launch_fill(g->gB, 6 * (int64_t)ns, 0.0f, s);
     const Plane7 gXL = b->use_snap ? dense7(g->gX, nst) : gC;
     if (g->full_tape) {
       adjoint_waves(g, 0, gC, gXL, s);
     } else {
-      const Plane7 pick = b->pick_planes();
       for (int k = (int)g->segs.size() - 1; k >= 0; --k) {
         const auto& sg = g->segs[k];
         // restore the segment's checkpoint: the snapshot's dirty bytes no
@@ -1069,7 +1061,7 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
         box_copy({layer_box(L, cv->cols, sg.x0, sg.y0, sg.w, sg.h, reinterpret_cast<double*>(c0), carea),
                   layer_box(b->snap_planes(), cv->cols, sg.x0, sg.y0, b->use_snap ? sg.w : 0, sg.h,
                             reinterpret_cast<double*>(c0 + 14 * carea), carea),
-                  plane_box(pick, sm, 0, 0, sm, sm, c0 + (b->use_snap ? 28 : 14) * carea, m)},
+                  cell_box(b->pick, sm, 0, 0, sm, sm, c0 + (b->use_snap ? 28 : 14) * carea, m)},
                  false, s);
         cv->epoch++;
         b->dirty_canvas = nullptr;

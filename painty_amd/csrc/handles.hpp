@@ -115,7 +115,7 @@ struct pnt_brush_s {
   int64_t fp_cap = 0, pick_cap = 0;  // floats allocated at fp / pick
   std::vector<float> fp_host;  // same footprint on the host (traffic replay)
   int fbox[4] = {0, 0, 1 << 30, 1 << 30};  // nonzero footprint cells: x0 y0 x1 y1
-  float* pick = nullptr;       // pickup map: 7 FP32 planes of mstride
+  float* pick = nullptr;       // pickup map: mstride cells of kCell floats
   float* snap = nullptr;       // snapshot: a layer (8 strides of snap_stride)
   int snap_rows = 0, snap_cols = 0;
   int64_t snap_stride = 0, snap_cap = 0;  // floats allocated at snap
@@ -138,25 +138,7 @@ struct pnt_brush_s {
   int64_t last_launches = 0;  // stamp-kernel launches of the last fused stamp-list call
   pnt::KernelTimer* ktimer = nullptr;  // per-launch event pairs (pnt_brush_set_kernel_timing)
 
-  pnt::Plane7 pick_planes() const {
-    pnt::Plane7 L;
-    for (int i = 0; i < 7; ++i) L.p[i] = pick + i * mstride;
-    return L;
-  }
   pnt::Layer7 snap_planes() const { return pnt::layer_at(snap, snap_stride); }
-  pnt::BrushArgs args() const {
-    pnt::BrushArgs b;
-    b.fp = fp;
-    b.pick = pick_planes();
-    b.pickup_rate = pickup_rate;
-    b.dep_rate = dep_rate;
-    b.cap = cap;
-    for (int c = 0; c < 3; ++c) {
-      b.paintK[c] = paintK[c];
-      b.paintS[c] = paintS[c];
-    }
-    return b;
-  }
 };
 
 namespace pnt {

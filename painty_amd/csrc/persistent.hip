@@ -43,7 +43,7 @@ struct PArgs {
   int n;
   int hr, size_map, rows, cols, tiles_x, ntiles;
   const float* fp;
-  Plane7 pick;
+  float* pick;
   Layer7 canvas, src;
   uint8_t* dirty;
   int use_snap;
@@ -105,12 +105,14 @@ __global__ __launch_bounds__(kT* kT) void k_persistent(PArgs A) {
     const int mx = mx0 + t % kT, my = my0 + t / kT;
     const bool own = mx < A.size_map && my < A.size_map;
     const int m = my * A.size_map + mx;
+    float cell[7] = {};
+    if (own) ld_cell(A.pick, m, cell);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      P.K[c][t] = own ? A.pick.p[c][m] : 0.0f;
-      P.S[c][t] = own ? A.pick.p[3 + c][m] : 0.0f;
+      P.K[c][t] = cell[c];
+      P.S[c][t] = cell[3 + c];
     }
-    P.V[t] = own ? A.pick.p[6][m] : 0.0f;
+    P.V[t] = cell[6];
     P.F[t] = own ? A.fp[m] : 0.0f;
   }
   float pk[3], ps[3];
@@ -252,12 +254,9 @@ __global__ __launch_bounds__(kT* kT) void k_persistent(PArgs A) {
     const int mx = mx0 + t % kT, my = my0 + t / kT;
     if (mx < A.size_map && my < A.size_map) {
       const int m = my * A.size_map + mx;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        A.pick.p[c][m] = P.K[c][t];
-        A.pick.p[3 + c][m] = P.S[c][t];
-      }
-      A.pick.p[6][m] = P.V[t];
+      const float cell[7] = {P.K[0][t], P.K[1][t], P.K[2][t], P.S[0][t],
+                             P.S[1][t], P.S[2][t], P.V[t]};
+      st_cell(A.pick, m, cell);
     }
   }
 }
@@ -576,7 +575,7 @@ void run_persistent(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
   A.tiles_x = tiles_x;
   A.ntiles = ntiles;
   A.fp = b->fp;
-  A.pick = b->pick_planes();
+  A.pick = b->pick;
   A.canvas = cv->layer();
   A.src = b->use_snap ? b->snap_planes() : cv->layer();
   A.dirty = b->dirty;

@@ -89,7 +89,7 @@ struct SReq {
   float* canvas;
   float* snap;      // the canvas itself when the snapshot is off
   uint8_t* dirty;
-  float* pick;      // chain c's map at pick + c * 7 * mstride
+  float* pick;      // chain c's map at pick + c * kCell * mstride
   const float* fp;
   const int2* dl;
   const int* dl_off;
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(kWT2, kWaveOccupancy) void k_serve_wave(SArgs A) {
   S.canvas = (float*)Q.canvas;
   S.snap = (float*)Q.snap;
   S.dirty = (uint8_t*)Q.dirty;
-  S.pick = (float*)(Q.pick + (int64_t)P.chain * 7 * Q.mstride);
+  S.pick = (float*)(Q.pick + (int64_t)P.chain * kCell * Q.mstride);
   S.pick_dst = S.pick;
   S.fp = (const float*)Q.fp;
   S.dl = (const int2*)Q.dl;
@@ -685,7 +685,7 @@ void pnt_server_s::setup(Req* q) {
       PNT_HIP_CHECK(hipMalloc((void**)&S.dirty, (size_t)S.dirty_cap));
     }
   }
-  grow_f(S.pick, S.pick_cap, kChainsPerReq * 7 * q->mstride);
+  grow_f(S.pick, S.pick_cap, kChainsPerReq * kCell * q->mstride);
   if (q->plan_bytes > S.plan_cap) {
     dev_free(S.plan);
     S.plan = nullptr;
@@ -844,7 +844,7 @@ bool pnt_server_s::collect(Req* q, SArgs& A, int& start,
         const int rb = q->rb[(size_t)f.k];
         switch (f.kind) {
           case kSClear:
-            P.nblk = (int)std::min<int64_t>(64, (7 * q->mstride + 4 * kT2 - 1) / (4 * kT2));
+            P.nblk = (int)std::min<int64_t>(64, (kCell * q->mstride + 4 * kT2 - 1) / (4 * kT2));
             break;
           default:  // kSStamp, + the shared-pixel levels' block of a dup stamp
             P.rb = rb;

@@ -166,13 +166,13 @@ __device__ __forceinline__ void st_px(const Layer7& L, int64_t i, const float ks
 struct TapeRec {
   double *cv, *xv;  // volumes
   float *ck, *xk;   // K, S: 6 planes of `area`
-  float* P;         // 7 planes of `m`
+  float* P;         // `m` cells (kCell)
   int64_t area, m;
   int bx0, by0, bw;
   __host__ __device__ int64_t at(int x, int y) const { return (int64_t)(y - by0) * bw + (x - bx0); }
 };
 __host__ __device__ inline int64_t tape_floats(int64_t area, int64_t m) {
-  return (16 * area + 7 * m + 3) / 4 * 4;
+  return 16 * area + kCell * m;
 }
 __host__ __device__ inline TapeRec tape_rec(float* base, int64_t area, int64_t m, const RingBox& b,
                                             int cols) {
@@ -423,6 +423,24 @@ struct RegPick {
   __device__ void set_pick(int c, float x) { v[c] = x; }
 };
 
+// Cell m of a pickup map.
+__device__ __forceinline__ void ld_cell(const float* pick, int m, float v[7]) {
+  const float4* p = reinterpret_cast<const float4*>(pick) + 2 * (int64_t)m;
+  const float4 a = p[0], b = p[1];
+  v[0] = a.x;
+  v[1] = a.y;
+  v[2] = a.z;
+  v[3] = a.w;
+  v[4] = b.x;
+  v[5] = b.y;
+  v[6] = b.z;
+}
+__device__ __forceinline__ void st_cell(float* pick, int m, const float v[7]) {
+  float4* p = reinterpret_cast<float4*>(pick) + 2 * (int64_t)m;
+  p[0] = make_float4(v[0], v[1], v[2], v[3]);
+  p[1] = make_float4(v[4], v[5], v[6], 0.0f);
+}
+
 __device__ __forceinline__ int64_t canvas_index(const StampGeom& g, int col, int row) {
 #pragma clang fp contract(off)
   return (int64_t)(int)(row + g.cy) * g.cols + (int)(col + g.cx);
@@ -471,18 +489,16 @@ __device__ __forceinline__ void tape_pixel(const TapeRec& t, bool snap, int x, i
 
 // One whole visit of map cell m at canvas pixel ic: everything it reads in
 // one batch, the arithmetic, the stores.
-__device__ __forceinline__ void cached_visit(const VisitTarget& T, float* const* pick, int m,
+__device__ __forceinline__ void cached_visit(const VisitTarget& T, float* pick, int m,
                                              float fh, int64_t ic, bool pull, const float pk[3],
                                              const float ps[3]) {
   CachedVisit<RegPick> acc;
   acc.alias = !T.use_snap;
-#pragma unroll
-  for (int c = 0; c < 7; ++c) acc.v[c] = pick[c][m];
+  ld_cell(pick, m, acc.v);
   load_pixel(T, T.use_snap, ic, pull, acc);
   paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
   store_pixel(T, T.use_snap, ic, pull, acc);
-#pragma unroll
-  for (int c = 0; c < 7; ++c) pick[c][m] = acc.v[c];
+  st_cell(pick, m, acc.v);
 }
 
 // Canvas::checkDry (Canvas.hxx:123-155) of a visited pixel whose canvas
@@ -662,8 +678,9 @@ __host__ __device__ __forceinline__ VisitCell visit_cell(const StampGeom& g, con
 // left out; level_visits runs them.
 //
 // Bound: the L1's line lookups and the two memory round trips of a visit
-// (its cell's values, fetched with the pixel's, then the stores).  Map cells
-// are met along a rotated row, about 16 lines per 64 cells and plane.
+// (its cell, fetched with the pixel's values, then the stores).  Map cells
+// are met along a rotated row, 64 of them on about 16 rows of the map, and
+// are kept whole (kCell) for that.
 //
 // With a drying clock (clk.tmap != nullptr) every visited pixel -- in the canvas
 // and in the map, whatever its footprint height -- gets Canvas::checkDry
@@ -673,7 +690,7 @@ __host__ __device__ __forceinline__ VisitCell visit_cell(const StampGeom& g, con
 // don't is left out, which shortens every wave's first pass over cold
 // instruction lines and frees registers.
 template <int kT, class F>
-__device__ __forceinline__ void window_tile(const VisitTarget& T, float* const* pick,
+__device__ __forceinline__ void window_tile(const VisitTarget& T, float* pick,
                                             const float* fp, const FpBox& dom, const StampGeom& g,
                                             const PStamp& st, bool dup, bool pull, int tile,
                                             const TileWin& win, float (*hand)[kT * kT],
@@ -710,9 +727,7 @@ __device__ __forceinline__ void window_tile(const VisitTarget& T, float* const* 
   if (act) {
     pv = pull && on_window_border(st.box, V.x, V.y);
     fh = fp[V.mm];
-    if (first)
-#pragma unroll
-      for (int c = 0; c < 7; ++c) acc.v[c] = pick[c][V.mm];
+    if (first) ld_cell(pick, V.mm, acc.v);
     load_pixel(T, snap, ic, pv, acc);
     if (clocked) {
       if (fh > 0.0f) {
@@ -726,9 +741,7 @@ __device__ __forceinline__ void window_tile(const VisitTarget& T, float* const* 
   const bool paint = act && fh > 0.0f;
   if (F::tape && paint) {
     tape_pixel(*T.tape, snap, V.x, V.y, acc.cv, acc.cvv, acc.sv, acc.svv);
-    if (first)
-#pragma unroll
-      for (int c = 0; c < 7; ++c) T.tape->P[c * T.tape->m + V.mm] = acc.v[c];
+    if (first) st_cell(T.tape->P, V.mm, acc.v);
   }
   if (paint && first) {
     paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
@@ -745,9 +758,7 @@ __device__ __forceinline__ void window_tile(const VisitTarget& T, float* const* 
   }
   if (paint) {
     store_pixel(T, snap, ic, pv, acc);
-    if (second || !V.shared)
-#pragma unroll
-      for (int c = 0; c < 7; ++c) pick[c][V.mm] = acc.v[c];
+    if (second || !V.shared) st_cell(pick, V.mm, acc.v);
   }
   if (first && V.shared && !inside) {  // the second visit lies in another tile
     const int px = (int)(col + dx + g.cx), py = (int)(row + dy + g.cy);
@@ -762,8 +773,7 @@ __device__ __forceinline__ void window_tile(const VisitTarget& T, float* const* 
       if (F::tape) tape_pixel(*T.tape, snap, px, py, acc.cv, acc.cvv, acc.sv, acc.svv);
       paint_visit_math(acc, fh, T.pickup_rate, T.dep_rate, T.cap, pk, ps);
       store_pixel(T, snap, pic, ppv, acc);
-#pragma unroll
-      for (int c = 0; c < 7; ++c) pick[c][V.mm] = acc.v[c];
+      st_cell(pick, V.mm, acc.v);
     } else if (clocked) {
       check_only(T, clk, pic, ppv);
     }
@@ -809,7 +819,7 @@ __device__ __forceinline__ bool first_acting_visit(const StampGeom& g, const Rin
 // footprint heights.  A level is then one round trip (17 us to 10 us of the
 // launches that hold such a stamp).
 template <int kThreads>
-__device__ __forceinline__ void level_visits(const VisitTarget& T, float* const* pick,
+__device__ __forceinline__ void level_visits(const VisitTarget& T, float* pick,
                                              const float* fp, const StampGeom& g, const PStamp& st,
                                              const int2* dl, const int* dl_off, const float pk[3],
                                              const float ps[3],
@@ -891,7 +901,7 @@ union StampLds {
 // a stamp that has them.  Visits on the window border refresh their own
 // snapshot pixels (the ring scan leaves them).
 template <class F>
-__device__ __forceinline__ void stamp_block(const VisitTarget& T, float* const* pick,
+__device__ __forceinline__ void stamp_block(const VisitTarget& T, float* pick,
                                             const float* fp, const FpBox& dom, const StampGeom& g,
                                             const PStamp& st, const TileWin& win, int ntiles, int rb,
                                             int b, StampLds<256>& lds, const int2* dl,
@@ -921,8 +931,8 @@ __device__ __forceinline__ void stamp_block(const VisitTarget& T, float* const* 
         CachedVisit<RegPick> acc;
         load_pixel(T, snap, ic, pull && on_window_border(st.box, x, y), acc);
         tape_pixel(*T.tape, snap, x, y, acc.cv, acc.cvv, acc.sv, acc.svv);
-#pragma unroll
-        for (int c = 0; c < 7; ++c) T.tape->P[c * T.tape->m + m] = pick[c][m];
+        ld_cell(pick, m, acc.v);
+        st_cell(T.tape->P, m, acc.v);
       }
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();

@@ -45,7 +45,7 @@ struct SSlot {
   float* canvas;
   float* snap;      // a layer of cstride (the canvas itself when the snapshot is off)
   uint8_t* dirty;   // snapshot dirty bytes (dirty_bytes of them)
-  float* pick;      // the chain's pickup map: 7 planes of mstride
+  float* pick;      // the chain's pickup map: mstride cells
   float* pick_dst;  // kSCopyPick target
   const float* fp;  // padded footprint, size_map^2
   const int2* dl;   // shared-pixel visit lists
@@ -135,7 +135,7 @@ __device__ __forceinline__ void run_wave_slot(const SSlot& S, int b, StampLds<kW
   part_range(cs / 4, S.part, S.nparts, lo4, hi4);
   part_range(S.dirty_bytes / 16, S.part, S.nparts, lod, hid);
   if (S.kind == kSClear) {
-    wave_fill4(S.pick, 0, 7 * (int64_t)S.mstride / 4, 0.0f, tid, nth);
+    wave_fill4(S.pick, 0, kCell * (int64_t)S.mstride / 4, 0.0f, tid, nth);
     return;
   }
   if (kStream) switch (S.kind) {
@@ -161,7 +161,7 @@ __device__ __forceinline__ void run_wave_slot(const SSlot& S, int b, StampLds<kW
       return;
     }
     case kSCopyPick:
-      for (int64_t q = tid; q < 7 * (int64_t)S.mstride / 4; q += nth)
+      for (int64_t q = tid; q < kCell * (int64_t)S.mstride / 4; q += nth)
         reinterpret_cast<float4*>(S.pick_dst)[q] = reinterpret_cast<const float4*>(S.pick)[q];
       return;
     case kSDry: {  // with a clock, dryCanvas also stamps every pixel's time (its last imprint's)
@@ -186,14 +186,11 @@ __device__ __forceinline__ void run_wave_slot(const SSlot& S, int b, StampLds<kW
   const PStamp st = load_const<PStamp>(S.st);
   const StampGeom g = stamp_geom(st, S.size_map, S.rows, S.cols);
   const VisitTarget T{&canvas, &snap, S.dirty, S.use_snap, S.pickup_rate, S.dep_rate, S.cap};
-  float* pick[7];
-#pragma unroll
-  for (int c = 0; c < 7; ++c) pick[c] = S.pick + c * (int64_t)S.mstride;
   const FpBox fb{S.fb[0], S.fb[1], S.fb[2], S.fb[3]};
   // Canvas::checkDry on every visited pixel when the canvas has a clock
   const DryClock ck{S.tmap, st.now_us, S.dry_ms, Rgb3{{R0, R0 + cs, R0 + 2 * cs}}, hp};
   const TileWin tw = tile_window(g, fb);
-  stamp_block<F>(T, pick, S.fp, fb, g, st, tw, tile_count<kWT>(tw), S.rb, b, lds, S.dl,
+  stamp_block<F>(T, S.pick, S.fp, fb, g, st, tw, tile_count<kWT>(tw), S.rb, b, lds, S.dl,
                      S.dl_off, S.pk, S.ps, ck);
 }
 
