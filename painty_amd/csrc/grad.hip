@@ -29,10 +29,13 @@
 // saved before it, and backward restores and reruns the segment onto its tape.
 //
 // Bound: the chain of launches, one per wave (108 for 500 stamps on 2048^2),
-// each as long as one tile's round trips and FP64 arithmetic (16.5 us).  500
+// each as long as one tile's round trips and FP64 arithmetic.  500
 // stamps of radius 32 on 2048^2, forward and backward: 30.3 ms with every
 // segment recomputed stamp by stamp (six launches and 48 us a stamp in the
-// backward, one stroke at a time), 3.9 ms from the tape.
+// backward, one stroke at a time), 3.9 ms from a tape in planes, 3.3 ms with a
+// tape's pixels and cells each in one piece, every load of a thread's visits
+// issued before the first one's arithmetic, and the ring's pixels moved one a
+// thread.
 #include <algorithm>
 #include <initializer_list>
 #include <cmath>
@@ -97,9 +100,10 @@ __device__ __forceinline__ void visit_adj(const VState& in, VState& g, float gB[
     const double vt1 = vP + vLeave;
     bb = vt1 > kMinVolume;
     if (bb) {
-      iv1 = 1.0 / vt1;
+      iv1 = rcpd(vt1);
 #pragma unroll
-      for (int c = 0; c < 6; ++c) P1[c] = (float)blendd(vP, P[c], vLeave, X[c], iv1);
+      for (int c = 0; c < 6; ++c)
+        P1[c] = (float)__builtin_fma(vP * iv1, P[c], (vLeave * iv1) * X[c]);
     }
     P1[6] = (float)(vP + vLeave);
   }
@@ -108,26 +112,27 @@ __device__ __forceinline__ void visit_adj(const VState& in, VState& g, float gB[
   const double vFree = fmax(0.0, cap - u);
   const double vt2 = u + vFree;
   const bool d = vt2 > kMinVolume;
-  const double iv2 = d ? 1.0 / vt2 : 0.0;
+  const double iv2 = d ? rcpd(vt2) : 0.0;
   double src[6];
 #pragma unroll
-  for (int c = 0; c < 6; ++c) src[c] = d ? blendd(u, P1[c], vFree, B[c], iv2) : P1[c];
+  for (int c = 0; c < 6; ++c)
+    src[c] = d ? __builtin_fma(u * iv2, P1[c], (vFree * iv2) * B[c]) : P1[c];
   double Cd[7];  // the canvas pixel as depositPaint reads it
 #pragma unroll
   for (int c = 0; c < 6; ++c) Cd[c] = C[c];
   Cd[6] = alias ? X6n : C[6];
   const double vB = cap * fh, vCc = Cd[6], vt3 = vB + vCc;
   const bool e = vt3 > kMinVolume;
-  const double iv3 = e ? 1.0 / vt3 : 0.0;
+  const double iv3 = e ? rcpd(vt3) : 0.0;
   // ---- depositPaint
   double gCd[7], gsrc[6];
   double gvCc = g.C[6];
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
     if (e) {
-      const double C1 = blendd(vB, src[c], vCc, Cd[c], iv3);
-      gsrc[c] = g.C[c] * vB * iv3;
-      gCd[c] = g.C[c] * vCc * iv3;
+      const double C1 = __builtin_fma(vB * iv3, src[c], (vCc * iv3) * Cd[c]);
+      gsrc[c] = g.C[c] * (vB * iv3);
+      gCd[c] = g.C[c] * (vCc * iv3);
       gvCc += g.C[c] * (Cd[c] - C1) * iv3;
     } else {
       gsrc[c] = g.C[c];
@@ -141,8 +146,8 @@ __device__ __forceinline__ void visit_adj(const VState& in, VState& g, float gB[
     double gvFree = 0.0;
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
-      gP1[c] = g.P[c] + gsrc[c] * u * iv2;
-      gB[c] += (float)(gsrc[c] * vFree * iv2);
+      gP1[c] = g.P[c] + gsrc[c] * (u * iv2);
+      gB[c] += (float)(gsrc[c] * (vFree * iv2));
       gu += gsrc[c] * (P1[c] - src[c]) * iv2;
       gvFree += gsrc[c] * (B[c] - src[c]) * iv2;
     }
@@ -164,8 +169,8 @@ __device__ __forceinline__ void visit_adj(const VState& in, VState& g, float gB[
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
       if (bb) {
-        gPin[c] = gP1[c] * vP * iv1;
-        gXin[c] += gP1[c] * vLeave * iv1;
+        gPin[c] = gP1[c] * (vP * iv1);
+        gXin[c] += gP1[c] * (vLeave * iv1);
         gvP += gP1[c] * (P[c] - P1[c]) * iv1;
         gvLeave += gP1[c] * (X[c] - P1[c]) * iv1;
       } else {
@@ -246,27 +251,35 @@ struct AArgs {
 };
 static_assert(sizeof(AArgs) <= 4000, "kernel arguments must fit the argument segment");
 
+__device__ __forceinline__ void load_px(const TapeRec& t, bool snap, int64_t k, VState& s) {
+  const TapePx c = t.c[k], x = snap ? t.x[k] : TapePx{};
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    s.C[i] = c.ks[i];
+    s.X[i] = x.ks[i];
+  }
+  s.C[6] = c.v;
+  s.X[6] = x.v;
+}
+
 __device__ __forceinline__ void load_in(const TapeRec& t, bool snap, int64_t k, int mm, VState& s) {
   ld_cell(t.P, mm, s.P);
-#pragma unroll
-  for (int c = 0; c < 6; ++c) {
-    s.C[c] = t.ck[c * t.area + k];
-    s.X[c] = snap ? t.xk[c * t.area + k] : 0.0f;
-  }
-  s.C[6] = t.cv[k];
-  s.X[6] = snap ? t.xv[k] : 0.0;
+  load_px(t, snap, k, s);
 }
 
 __device__ __forceinline__ void store_in(const TapeRec& t, bool snap, int64_t k, int mm,
                                          const VState& s) {
   st_cell(t.P, mm, s.P);
+  TapePx p;
 #pragma unroll
-  for (int c = 0; c < 6; ++c) {
-    t.ck[c * t.area + k] = (float)s.C[c];
-    if (snap) t.xk[c * t.area + k] = (float)s.X[c];
-  }
-  t.cv[k] = s.C[6];
-  if (snap) t.xv[k] = s.X[6];
+  for (int i = 0; i < 6; ++i) p.ks[i] = (float)s.C[i];
+  p.v = s.C[6];
+  t.c[k] = p;
+  if (!snap) return;
+#pragma unroll
+  for (int i = 0; i < 6; ++i) p.ks[i] = (float)s.X[i];
+  p.v = s.X[6];
+  t.x[k] = p;
 }
 
 __device__ __forceinline__ void load_g_pixel(const AShared& A, int64_t ic, VState& g) {
@@ -331,25 +344,29 @@ __device__ __forceinline__ void adj_tile(const AShared& A, const ASlot& S, const
   if (fh > 0.0f) {
     const bool snap = A.use_snap != 0, alias = !snap;
     const int64_t ic1 = (int64_t)V.y * A.cols + V.x;
+    // everything the visits read, in one round trip
     VState in1, gs;
     load_in(tape, snap, tape.at(V.x, V.y), V.mm, in1);
     ld_cell(S.gP, V.mm, gs.P);
+    load_g_pixel(A, ic1, gs);
     if (two) {
       const int x2 = (int)(col + dx + g.cx), y2 = (int)(row + dy + g.cy);
       const int64_t ic2 = (int64_t)y2 * A.cols + x2;
+      VState at2, g2;
+      load_px(tape, snap, tape.at(x2, y2), at2);
+      load_g_pixel(A, ic2, g2);
       VState in2 = in1;
       visit_fwd(in2, fh, A.pr, A.dr, A.cap, S.pk, S.ps, alias);  // pickup cell after visit 1
-      float P2[7];
 #pragma unroll
-      for (int c = 0; c < 7; ++c) P2[c] = in2.P[c];
-      load_in(tape, snap, tape.at(x2, y2), V.mm, in2);
+      for (int c = 0; c < 7; ++c) {
+        at2.P[c] = in2.P[c];
+        g2.P[c] = gs.P[c];
+      }
+      visit_adj(at2, g2, gB, fh, A.pr, A.dr, A.cap, S.pk, S.ps, alias);
+      store_g_pixel(A, ic2, g2, snap && on_window_border(S.st.box, x2, y2));
 #pragma unroll
-      for (int c = 0; c < 7; ++c) in2.P[c] = P2[c];
-      load_g_pixel(A, ic2, gs);
-      visit_adj(in2, gs, gB, fh, A.pr, A.dr, A.cap, S.pk, S.ps, alias);
-      store_g_pixel(A, ic2, gs, snap && on_window_border(S.st.box, x2, y2));
+      for (int c = 0; c < 7; ++c) gs.P[c] = g2.P[c];
     }
-    load_g_pixel(A, ic1, gs);
     visit_adj(in1, gs, gB, fh, A.pr, A.dr, A.cap, S.pk, S.ps, alias);
     store_g_pixel(A, ic1, gs, snap && on_window_border(S.st.box, V.x, V.y));
     st_cell(S.gP, V.mm, gs.P);
@@ -360,29 +377,44 @@ __device__ __forceinline__ void adj_tile(const AShared& A, const ASlot& S, const
 // Adjoint of the ring copy canvas -> snapshot (FootprintBrush.hxx:307-318) by
 // block `blk` of S.rb: the pixels of the allowed box, outside the window
 // interior, whose snapshot adjoint may be nonzero (dirty bytes, read eight at
-// a time) and that no visit of the stamp moves itself.
+// a time) and that no visit of the stamp moves itself.  The pixels found are
+// listed in LDS and moved one a thread: a thread that moved its own eight one
+// after another took eight round trips, longer than any tile.
 __device__ __forceinline__ void adj_ring(const AShared& A, const ASlot& S, const StampGeom& g,
                                          int blk) {
   const RingBox& b = S.st.box;
   const int span = b.a_x1 - b.a_x0 + 1;
   const int per_row = (span + kRingUnit - 1) / kRingUnit + 1;
   const int total = per_row * (b.a_y1 - b.a_y0 + 1);
-  for (int e = blk * kBlk + (int)threadIdx.x; e < total; e += S.rb * kBlk) {
-    const int r = e / per_row, row = b.a_y0 + r;
+  __shared__ int s_n, s_list[kRingUnit * kBlk];  // e * kRingUnit + q
+  for (int e0 = blk * kBlk; e0 < total; e0 += S.rb * kBlk) {
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    const int e = e0 + (int)threadIdx.x, r = e / per_row, row = b.a_y0 + r;
     const int64_t rowi = (int64_t)row * A.cols, lo = rowi + b.a_x0;
     const int64_t base = (lo & ~(int64_t)(kRingUnit - 1)) + kRingUnit * (int64_t)(e - r * per_row);
     const int x0 = (int)(base - rowi);
     const bool interior_row = row > b.tl_y && row < b.br_y;
-    if (x0 > b.a_x1 || (interior_row && x0 > b.tl_x && x0 + kRingUnit - 1 < b.br_x)) continue;
-    const uint2 d = *reinterpret_cast<const uint2*>(A.dirty + base);
-    if (!(d.x | d.y)) continue;
-    for (int q = 0; q < kRingUnit; ++q) {
-      if (!((((q < 4 ? d.x : d.y) >> (8 * (q & 3)))) & 0xffu)) continue;
-      const int col = x0 + q;
-      if (col < b.a_x0 || col > b.a_x1) continue;
-      if (interior_row && col > b.tl_x && col < b.br_x) continue;
-      if (on_window_border(b, col, row) && ring_pixel_visited(g, b, A.fp, col, row)) continue;
-      const int64_t i = base + q;
+    if (e < total && x0 <= b.a_x1 &&
+        !(interior_row && x0 > b.tl_x && x0 + kRingUnit - 1 < b.br_x)) {
+      const uint2 d = *reinterpret_cast<const uint2*>(A.dirty + base);
+      if (d.x | d.y)
+        for (int q = 0; q < kRingUnit; ++q) {
+          if (!((((q < 4 ? d.x : d.y) >> (8 * (q & 3)))) & 0xffu)) continue;
+          const int col = x0 + q;
+          if (col < b.a_x0 || col > b.a_x1) continue;
+          if (interior_row && col > b.tl_x && col < b.br_x) continue;
+          s_list[atomicAdd(&s_n, 1)] = e * kRingUnit + q;
+        }
+    }
+    __syncthreads();
+    for (int j = (int)threadIdx.x; j < s_n; j += kBlk) {
+      const int id = s_list[j], e2 = id / kRingUnit, r2 = e2 / per_row, y = b.a_y0 + r2;
+      const int64_t rowj = (int64_t)y * A.cols, lo2 = rowj + b.a_x0;
+      const int64_t i = (lo2 & ~(int64_t)(kRingUnit - 1)) +
+                        kRingUnit * (int64_t)(e2 - r2 * per_row) + id % kRingUnit;
+      const int x2 = (int)(i - rowj);
+      if (on_window_border(b, x2, y) && ring_pixel_visited(g, b, A.fp, x2, y)) continue;
       float c[7], x[7];
 #pragma unroll
       for (int k = 0; k < 7; ++k) {
@@ -396,6 +428,7 @@ __device__ __forceinline__ void adj_ring(const AShared& A, const ASlot& S, const
       }
       A.dirty[i] = 0;
     }
+    __syncthreads();  // the list is rewritten by the next pass
   }
 }
 

@@ -163,10 +163,14 @@ __device__ __forceinline__ void st_px(const Layer7& L, int64_t i, const float ks
 // One stamp's tape record: the canvas and pickup-source pixels as its visits
 // find them, by pixel of its window box clipped to the canvas, and the map
 // cells before their first visits.  Only the visited entries are written.
+// A pixel's values lie together, as a cell's do: two 16-byte accesses.
+struct alignas(16) TapePx {
+  float ks[6];
+  double v;
+};
 struct TapeRec {
-  double *cv, *xv;  // volumes
-  float *ck, *xk;   // K, S: 6 planes of `area`
-  float* P;         // `m` cells (kCell)
+  TapePx *c, *x;  // canvas, pickup source: `area` pixels each
+  float* P;       // `m` cells (kCell)
   int64_t area, m;
   int bx0, by0, bw;
   __host__ __device__ int64_t at(int x, int y) const { return (int64_t)(y - by0) * bw + (x - bx0); }
@@ -177,11 +181,9 @@ __host__ __device__ inline int64_t tape_floats(int64_t area, int64_t m) {
 __host__ __device__ inline TapeRec tape_rec(float* base, int64_t area, int64_t m, const RingBox& b,
                                             int cols) {
   TapeRec t;
-  t.cv = reinterpret_cast<double*>(base);
-  t.xv = t.cv + area;
-  t.ck = base + 4 * area;
-  t.xk = t.ck + 6 * area;
-  t.P = t.xk + 6 * area;
+  t.c = reinterpret_cast<TapePx*>(base);
+  t.x = t.c + area;
+  t.P = base + 16 * area;
   t.area = area;
   t.m = m;
   t.bx0 = b.tl_x > 0 ? b.tl_x : 0;
@@ -477,14 +479,16 @@ __device__ __forceinline__ void tape_pixel(const TapeRec& t, bool snap, int x, i
                                            const float cv[6], double cvv, const float sv[6],
                                            double svv) {
   const int64_t k = t.at(x, y);
+  TapePx p;
 #pragma unroll
-  for (int c = 0; c < 6; ++c) t.ck[c * t.area + k] = cv[c];
-  t.cv[k] = cvv;
-  if (snap) {
+  for (int c = 0; c < 6; ++c) p.ks[c] = cv[c];
+  p.v = cvv;
+  t.c[k] = p;
+  if (!snap) return;
 #pragma unroll
-    for (int c = 0; c < 6; ++c) t.xk[c * t.area + k] = sv[c];
-    t.xv[k] = svv;
-  }
+  for (int c = 0; c < 6; ++c) p.ks[c] = sv[c];
+  p.v = svv;
+  t.x[k] = p;
 }
 
 // One whole visit of map cell m at canvas pixel ic: everything it reads in

@@ -1,10 +1,9 @@
 // The arithmetic of one imprint visit, shared by every stamp kernel.
 //
 // pickupPaint (renderer/FootprintBrush.hxx:349-384), then depositPaint
-// (:393-431), with blend() (:331-340) as blendd below.  Storage is reached
-// through an accessor so the plain kernel (pickup map in global memory) and
-// the persistent kernel (pickup map in LDS) execute the same instructions and
-// produce the same bits.
+// (:393-431), with blend() (:331-340).  Storage is reached through an accessor
+// so the kernels that keep the pickup map in global memory and the persistent
+// one (map in LDS) execute the same instructions and produce the same bits.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -28,9 +27,6 @@ constexpr double kMinVolume = 0.001;
 // va/vt and vb/vt, through one reciprocal: two operations a channel (a
 // product and a fused multiply-add).  The result is within 2e-16 relative of
 // the quotient, before it is rounded to FP32 for storage.
-__device__ __forceinline__ double blendd(double va, double a, double vb, double b, double inv_vt) {
-  return (va * a + vb * b) * inv_vt;
-}
 
 // 1/v for a normal v > MinVolume: the hardware's estimate (2^-23 or better)
 // and two Newton steps, within an ulp; no scaling for denormals or infinities.
@@ -38,11 +34,6 @@ __device__ __forceinline__ double rcpd(double v) {
   double r = __builtin_amdgcn_rcp(v);
   r = __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
   return __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
-}
-
-// Kept for the FP32 adjoint (grad.hip): the FP32 form of blend.
-__device__ __forceinline__ float blendf(float va, float a, float vb, float b, float inv_vt) {
-  return __builtin_fmaf(va, a, vb * b) * inv_vt;
 }
 
 __device__ __forceinline__ float rcpf(float x) { return __builtin_amdgcn_rcpf(x); }
