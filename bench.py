@@ -401,7 +401,7 @@ def leg_single(args, wl):
 
     stamps_s = len(wl.stamps) / (ms_per_step * 1e-3)
     waves = one_call and os.environ.get("PAINTY_FUSED_SCHED", "waves") != "streams"
-    kernel = {"plain": "k_stamp_main+k_ring_refresh", "persistent": "k_persistent",
+    kernel = {"plain": "k_stamp_wave", "persistent": "k_persistent",
               "fused": "k_stamp_wave",
               "chained": "k_stamp_chain<16>"}[args.mode]
     if kern_n:

@@ -389,7 +389,7 @@ int pnt_brush_stamp_traffic(pnt_brush brush, int rows, int cols,
                             int64_t* active_visits, int64_t* ring_pixels);
 
 /* Measurement helper (no reference counterpart): the number of stamp-kernel
- * launches (k_stamp_fused, k_stamp_levels, k_stamp_wave) the brush's last
+ * launches (k_stamp_wave) the brush's last
  * PNT_EXEC_FUSED stamp-list call issued; 0 after other modes. */
 int pnt_brush_last_launches(pnt_brush brush, int64_t* launches);
 /* Per-launch kernel timing of a brush's stamp-list calls (measurement; no

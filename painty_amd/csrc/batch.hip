@@ -9,13 +9,13 @@
 // barrier of stampcore.hpp.  Blocks of one group sit in one XCD lane
 // (block index = lane mod 8), so a job's window stays in one L2.
 //
-// Visit order within a stamp is kept as in k_stamp_main (kernels.hip): a map
-// cell has at most two visitors, which are 4-neighbours in the window; the
-// earlier one runs both, found through the map indices of the tile and a
-// one-pixel halo in LDS.  Visits on canvas column/row 0 that share a pixel
+// Visit order within a stamp is kept as in every stamp kernel: a map cell has
+// at most two visitors, which are 4-neighbours in the window; the earlier one
+// hands the cell to the later one through LDS, or runs both where a tile edge
+// parts them (window_tile, stampcore.hpp).  Visits on canvas column/row 0 that share a pixel
 // run after the others by dependency level.
 //
-// Snapshot ring: per-pixel dirty bytes (persistent.hip) scanned 16 at a time;
+// Snapshot ring: per-pixel dirty bytes (persistent.hip) scanned 8 a thread;
 // visits on the window border refresh their own pixel.
 //
 // Composite: after its jobs, every block takes composite tiles from a shared

@@ -67,7 +67,7 @@ using gptr = __attribute__((address_space(1))) T*;
 // at a uniform address that is a few wide scalar loads, together.  Read as
 // ordinary memory, which the kernel's own stores might change, each field is
 // a vector load where it is used: a wave kernel spent 6 us on them one after
-// another (2100 canvases' stamps in waves: 14,400 cycles before its first
+// another (a batch of 32 canvases: 14,400 cycles before its first
 // map cell, 1,500 with the same record in the kernel arguments).
 template <class T>
 __device__ __forceinline__ T load_const(const void* p) {

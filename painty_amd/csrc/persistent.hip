@@ -10,7 +10,7 @@
 //     mapped forward with the reference's exact FP64 formula), at most two
 //     per cell, and runs each cell's visits in row-major order.  Visits of
 //     different cells touch different canvas pixels, except on canvas
-//     column/row 0 (see k_stamp_main in kernels.hip): those visits and their
+//     column/row 0, which two window columns/rows share: those visits and their
 //     partners run afterwards by dependency level, one barrier per level.
 //   * Snapshot ring (updateSnapshot(canvas, center), :278-319): a copy of
 //     canvas into snapshot over the ring around the window.  A per-pixel

@@ -820,8 +820,8 @@ __device__ __forceinline__ bool first_acting_visit(const StampGeom& g, const Rin
 // The block is one chain of levels (3, rarely 4) beside tiles that take one
 // round trip each, so what a level needs besides the pixels and cells is
 // fetched for all levels first: the list entries, their geometry and
-// footprint heights.  A level is then one round trip (17 us to 10 us of the
-// launches that hold such a stamp).
+// footprint heights.  A level is then one round trip (17 us to 14.5 us of the
+// launches that hold such a stamp).  Starting the block first gave 0 to 2 %.
 template <int kThreads>
 __device__ __forceinline__ void level_visits(const VisitTarget& T, float* pick,
                                              const float* fp, const StampGeom& g, const PStamp& st,

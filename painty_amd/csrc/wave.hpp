@@ -25,7 +25,8 @@ namespace pnt {
 constexpr int kWT = 16;          // window tile side of wave phases
 constexpr int kWT2 = kWT * kWT;  // threads per block
 // Waves per SIMD the wave kernels keep (at most 128 VGPRs): the kernel of
-// plain stamps needs 101, the general one 116.
+// plain stamps needs 100 to 108, the general one 110 to 114.  Five waves
+// measured the same, six (with spills) 10 to 15 % slower.
 constexpr int kWaveOccupancy = 4;
 
 enum : int {
