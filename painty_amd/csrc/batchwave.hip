@@ -82,10 +82,9 @@ struct BWSlot {
   int64_t o_stamp, o_paint;
 };
 
-// The stamps of most waves: no clock, no stamp on canvas column/row 0, the
-// snapshot on, and no phase but stamps and map clears.  Waves with anything
-// else run the general kernel.
+// The kernels of kNeedPlain, kNeedDup and kNeedAny.
 using PlainStamps = StampKind<false, false, 1>;
+using DupStamps = StampKind<false, true, 1>;
 using AnyStamps = StampKind<true, true, 2>;
 
 // One wave: the group table gives the slot of every 8 blocks (slots start on
@@ -304,13 +303,13 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
   std::vector<int> grp;
   std::vector<int64_t> ws, wg;
   std::vector<int> wb;
-  std::vector<char> wp;  // the wave's phases are plain stamps and map clears
+  std::vector<char> wp;  // WaveNeed
   std::vector<std::pair<int, int>> took;  // (job, unit or -1 dry / -2 copy / -3 compose)
   std::vector<int> jfirst((size_t)n, -1), jlast((size_t)n, -1);
   for (;;) {
     const int64_t s0 = (int64_t)slots.size(), g0 = (int64_t)grp.size();
     int start = 0;
-    bool plain = true;
+    int need = kNeedPlain;
     took.clear();
     auto add = [&](int j, int64_t k, int kind, int nblk, int rb, int chain, int tag) {
       BWSlot d{j, (int)std::max<int64_t>(k, 0), kind, start, std::max(nblk, 1), rb, chain, 0, 0, 0};
@@ -319,7 +318,7 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
       slots.push_back(d);
       start += span;
       took.push_back({j, tag});
-      plain &= kind == kSStamp || kind == kSClear;
+      if (kind != kSStamp && kind != kSClear) need = kNeedAny;
     };
     for (int j = 0; j < n; ++j) {
       JobPlan& J = P[(size_t)j];
@@ -366,8 +365,10 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
                 nblk = (int)std::min<int64_t>(64, (kCell * b->mstride + 4 * kWT2 - 1) / (4 * kWT2));
                 break;
               case kSStamp:  // + the shared-pixel levels' block of a dup stamp
-                plain &= b->use_snap && !(J.st[(size_t)f.k].flags & (kStDupX | kStDupY)) &&
-                         job.canvas->clock == PNT_CLOCK_OFF;
+                if (!b->use_snap || job.canvas->clock != PNT_CLOCK_OFF)
+                  need = kNeedAny;
+                else if (J.st[(size_t)f.k].flags & (kStDupX | kStDupY))
+                  need = std::max<int>(need, kNeedDup);
                 nblk = ntiles + rb + (dup_levels(J.st[(size_t)f.k]) ? 1 : 0);
                 break;
               default: nblk = 1; break;
@@ -392,7 +393,7 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
     ws.push_back(s0);
     wg.push_back(g0);
     wb.push_back(start);
-    wp.push_back(plain ? 1 : 0);
+    wp.push_back((char)need);
     for (const auto& t : took) {
       JobPlan& J = P[(size_t)t.first];
       if (jfirst[(size_t)t.first] < 0) jfirst[(size_t)t.first] = (int)ws.size() - 1;
@@ -504,7 +505,7 @@ BWPlan plan_waves(const pnt_batch_job* jobs, int n, int chunk, float* pool, hipS
     W.wave_grp.push_back(o_grp + wg[w] * (int64_t)sizeof(int));
   }
   W.wave_blocks = wb;
-  W.wave_plain = std::move(wp);
+  W.wave_need = std::move(wp);
   W.job_first = std::move(jfirst);
   W.job_last = std::move(jlast);
   return W;
@@ -517,7 +518,9 @@ void enqueue_waves(const BWPlan& W, const char* stage, char* dev, hipStream_t s,
   if (ev) PNT_HIP_CHECK(hipEventRecord(ev[0], s));
   const BWJobG* jobs = reinterpret_cast<const BWJobG*>(dev + W.o_jobs);
   for (size_t w = 0; w < W.wave_blocks.size(); ++w) {
-    const auto kernel = W.wave_plain[w] ? k_batch_wave<PlainStamps, false> : k_batch_wave<AnyStamps, true>;
+    const auto kernel = W.wave_need[w] == kNeedPlain ? k_batch_wave<PlainStamps, false>
+                        : W.wave_need[w] == kNeedDup ? k_batch_wave<DupStamps, false>
+                                                     : k_batch_wave<AnyStamps, true>;
     kernel<<<(unsigned)W.wave_blocks[w], kWT2, 0, s>>>(
         dev, jobs, reinterpret_cast<const BWSlot*>(dev + W.wave_slots[w]),
         reinterpret_cast<const int*>(dev + W.wave_grp[w]));

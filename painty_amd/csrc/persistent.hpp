@@ -149,7 +149,7 @@ struct BWPlan {
   int64_t o_jobs = 0;
   std::vector<int64_t> wave_slots, wave_grp;
   std::vector<int> wave_blocks;
-  std::vector<char> wave_plain;  // runs the plain-stamps kernel (batchwave.hip)
+  std::vector<char> wave_need;  // WaveNeed (wave.hpp): its kernel
   std::vector<int> job_first, job_last;  // each job's first and last wave (-1: none)
   int njobs = 0;
 };

@@ -140,14 +140,14 @@ struct SPhase {
 struct SArgs {
   const SReqG* reqs;
   int nphases;
-  int general;  // a phase is more than a plain stamp or a map clear (host only)
+  int need;     // WaveNeed of its phases (host only)
   SPhase ph[kPhases];
 };
 static_assert(sizeof(SArgs) <= 4000, "wave arguments must fit the kernel argument segment");
 
-// The stamps of most waves (no stamp on canvas column/row 0, snapshot on, no
-// streaming phase), and everything.
+// The kernels of kNeedPlain, kNeedDup and kNeedAny.
 using PlainStamps = StampKind<false, false, 1>;
+using DupStamps = StampKind<false, true, 1>;
 using AnyStamps = StampKind<false, true, 2>;
 
 // One wave of the server: its phases arrive as kernel arguments, each
@@ -773,7 +773,7 @@ bool pnt_server_s::collect(Req* q, SArgs& A, int& start,
     P.slot = (int16_t)q->slot;
     P.kind = (int8_t)kind;
     P.start = start;
-    A.general |= kind != kSStamp && kind != kSClear;
+    if (kind != kSStamp && kind != kSClear) A.need = kNeedAny;
     return P;
   };
   auto push = [&](SPhase& P, int unit) {
@@ -848,7 +848,10 @@ bool pnt_server_s::collect(Req* q, SArgs& A, int& start,
             break;
           default:  // kSStamp, + the shared-pixel levels' block of a dup stamp
             P.rb = rb;
-            A.general |= !snap || (q->st[(size_t)f.k].flags & (kStDupX | kStDupY));
+            if (!snap)
+              A.need = kNeedAny;
+            else if (q->st[(size_t)f.k].flags & (kStDupX | kStDupY))
+              A.need = std::max<int>(A.need, kNeedDup);
             P.nblk = q->ntiles[(size_t)f.k] + rb + (dup_levels(q->st[(size_t)f.k]) ? 1 : 0);
             break;
         }
@@ -999,6 +1002,7 @@ void pnt_server_s::run_engine() {
       }
       A.reqs = reinterpret_cast<const SReqG*>(d_reqs);
       A.nphases = 0;
+      A.need = kNeedPlain;
       int start = 0;
       used.clear();
       for (Req* q : active) {
@@ -1008,7 +1012,9 @@ void pnt_server_s::run_engine() {
       }
       if (A.nphases == 0) continue;
       hipStream_t s = L.ctx->stream;
-      const auto kernel = A.general ? k_serve_wave<AnyStamps, true> : k_serve_wave<PlainStamps, false>;
+      const auto kernel = A.need == kNeedPlain ? k_serve_wave<PlainStamps, false>
+                          : A.need == kNeedDup ? k_serve_wave<DupStamps, false>
+                                               : k_serve_wave<AnyStamps, true>;
       kernel<<<(unsigned)start, kT2, 0, s>>>(A);
       PNT_HIP_CHECK(hipGetLastError());
       if (++L.waves % kMark == 0)

@@ -29,6 +29,14 @@ constexpr int kWT2 = kWT * kWT;  // threads per block
 // measured the same, six (with spills) 10 to 15 % slower.
 constexpr int kWaveOccupancy = 4;
 
+// What a wave's phases need, and so its kernel: plain stamps and map clears
+// with the snapshot on; the same with stamps on canvas column/row 0; anything.
+// A wave runs the smallest kernel that holds all its phases: code that is not
+// there is not fetched, and an edge stamp alone does not bring the streaming
+// phases, the clock and the snapshot switch along (sixteen served requests:
+// 7.94 to 7.40 ms; a batch of 32 canvases: 11.2 to 10.8 ms with its host work).
+enum WaveNeed : int { kNeedPlain = 0, kNeedDup, kNeedAny };
+
 enum : int {
   kSInit = 0,  // canvas planes: no paint, R0 = bg, h = 0 (and the snapshot of it)
   kSSnap,      // snapshot = canvas, dirty bytes 0
