@@ -1537,7 +1537,8 @@ int pnt_brush_update_snapshot(pnt_brush b, pnt_canvas cv) {
       PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
       dev_free(b->dirty);
       b->dirty = nullptr;
-      PNT_HIP_CHECK(hipMalloc((void**)&b->dirty, (size_t)need));
+      b->dirty_cap = 0;
+      b->dirty = reinterpret_cast<uint8_t*>(dev_alloc((need + 3) / 4));
       b->dirty_cap = need;
     }
     b->dirty_n = cv->n;

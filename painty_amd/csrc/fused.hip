@@ -595,6 +595,7 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
         PNT_HIP_CHECK(hipStreamSynchronize(s));
         dev_free(F.pick[c]);
         F.pick[c] = nullptr;
+        F.pick_cap[c] = 0;
         F.pick[c] = dev_alloc(kCell * max_stride);
         F.pick_cap[c] = kCell * max_stride;
       }

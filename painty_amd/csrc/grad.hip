@@ -733,8 +733,9 @@ struct pnt_grad_s {
   int64_t dl_cap = 0, dl_off_cap = 0;
   int fwd_size_map = 0;    // the brush's geometry at the forward
   bool fwd_snap = false;
-  float* gX = nullptr;  // 7 planes of round_up(n, 64) (snapshot adjoint); zero between calls
-  uint8_t* gdirty = nullptr;  // its dirty bytes; zero between calls
+  float* gX = nullptr;  // 7 planes of round_up(n, 64) (snapshot adjoint)
+  uint8_t* gdirty = nullptr;  // its dirty bytes
+  bool adj_zero = false;  // both are zero: a backward that runs to its end leaves them so
   float* gP = nullptr;  // per chain: m cells (pickup adjoint)
   float* gB = nullptr;  // n_stamps x 6
   int64_t gX_cap = 0, gdirty_cap = 0, gP_cap = 0, gB_cap = 0;
@@ -750,13 +751,15 @@ int guard_call(const std::function<void()>& f);  // api.hip: status + pnt_last_e
 
 namespace {
 
+// At least `need` elements at p; a failed allocation leaves none (cap 0).
 template <class T>
 void ensure(T*& p, int64_t& cap, int64_t need, hipStream_t s) {
   if (need <= cap) return;
   PNT_HIP_CHECK(hipStreamSynchronize(s));
-  if (p) PNT_HIP_CHECK(hipFree(p));
+  dev_free(p);
   p = nullptr;
-  PNT_HIP_CHECK(hipMalloc((void**)&p, (size_t)need * sizeof(T)));
+  cap = 0;
+  p = reinterpret_cast<T*>(dev_alloc((need * (int64_t)sizeof(T) + 3) / 4));
   cap = need;
 }
 
@@ -1070,12 +1073,13 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
     PNT_HIP_CHECK(hipGetLastError());
     const int64_t nst = round_up(n, 64);
     if (b->use_snap) {
-      if (7 * nst > g->gX_cap) {  // zero to begin with; every call leaves it zero
+      if (!g->adj_zero) {  // the first call, or the last one did not reach its end
         ensure(g->gX, g->gX_cap, 7 * nst, s);
-        launch_fill(g->gX, 7 * nst, 0.0f, s);
         ensure(g->gdirty, g->gdirty_cap, nst + 16, s);
+        launch_fill(g->gX, 7 * nst, 0.0f, s);
         launch_fill_u8(g->gdirty, nst + 16, 0, s);
       }
+      g->adj_zero = false;
     }
     ensure(g->gP, g->gP_cap, kAdjSlots * kCell * m, s);
     ensure(g->gB, g->gB_cap, 6 * (int64_t)ns, s);
@@ -1120,6 +1124,7 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
     if (b->use_snap) {
       k_adj_full_copy<<<grid_for((n + 7) / 8), kBlk, 0, s>>>(n, gC, gXL, g->gdirty);
       PNT_HIP_CHECK(hipGetLastError());
+      g->adj_zero = true;
     }
     // ---- mixing weights: dB/dW of mixSinglePaint (PaintMixer.cxx:327-355)
     std::vector<float> hB(6 * (size_t)ns);

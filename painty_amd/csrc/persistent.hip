@@ -392,7 +392,8 @@ void brush_prepare_snapshot(pnt_brush b, pnt_canvas cv, hipStream_t s) {
       PNT_HIP_CHECK(hipStreamSynchronize(s));
       dev_free(b->dirty);
       b->dirty = nullptr;
-      PNT_HIP_CHECK(hipMalloc((void**)&b->dirty, (size_t)need));
+      b->dirty_cap = 0;
+      b->dirty = reinterpret_cast<uint8_t*>(dev_alloc((need + 3) / 4));
       b->dirty_cap = need;
     }
     b->dirty_n = cv->n;
@@ -439,23 +440,27 @@ void persistent_release(PersistentState*& p) {
   p = nullptr;
 }
 
+// A failed allocation leaves no buffer (cap 0), and no error for a later call.
 template <class T>
 static void ensure_dev(T*& p, int64_t& cap, int64_t need, hipStream_t s) {
   if (need <= cap) return;
   PNT_HIP_CHECK(hipStreamSynchronize(s));  // the old buffer may still be read
-  if (p) PNT_HIP_CHECK(hipFree(p));
-  p = nullptr;
   const int64_t c = std::max<int64_t>(need, 2 * cap);
-  PNT_HIP_CHECK(hipMalloc((void**)&p, (size_t)c * sizeof(T)));
+  dev_free(p);
+  p = nullptr;
+  cap = 0;
+  p = reinterpret_cast<T*>(dev_alloc((c * (int64_t)sizeof(T) + 3) / 4));
   cap = c;
 }
 
 static PersistentState& plan_state(pnt_brush_s* b) {
   if (!b->pers) {
-    auto* P = new PersistentState;
-    b->pers = P;
-    PNT_HIP_CHECK(hipMalloc((void**)&P->d_bar, kBarWords * sizeof(unsigned)));
-    PNT_HIP_CHECK(hipEventCreateWithFlags(&P->uploaded, hipEventDisableTiming));
+    PersistentState P;
+    P.d_bar = reinterpret_cast<unsigned*>(dev_alloc(kBarWords));
+    const hipError_t e = hipEventCreateWithFlags(&P.uploaded, hipEventDisableTiming);
+    if (e != hipSuccess) dev_free(P.d_bar);
+    PNT_HIP_CHECK(e);
+    b->pers = new PersistentState(std::move(P));
   }
   return *b->pers;
 }
@@ -506,9 +511,10 @@ PlanDev upload_plan_parts(pnt_brush_s* b, pnt_canvas_s* cv, const PlanPart* part
   const int64_t need = (int64_t)(bst + bdl + boff + bfp);
   PNT_HIP_CHECK(hipEventSynchronize(P.uploaded));  // previous plan has been read
   if (need > P.stage_cap) {
+    const int64_t c = std::max<int64_t>(need, 2 * P.stage_cap);
     if (P.stage) PNT_HIP_CHECK(hipHostFree(P.stage));
     P.stage = nullptr;
-    const int64_t c = std::max<int64_t>(need, 2 * P.stage_cap);
+    P.stage_cap = 0;
     PNT_HIP_CHECK(hipHostMalloc((void**)&P.stage, (size_t)c));
     P.stage_cap = c;
   }
