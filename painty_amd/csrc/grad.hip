@@ -775,9 +775,12 @@ static void check_status(int st) {
   if (st != PNT_OK) throw Error(st, pnt_last_error());
 }
 
-// The taped run's shared-pixel lists, copied: the brush's plan is its own.
-static void keep_lists(pnt_grad_s* g, hipStream_t s) {
+// The taped run's shared-pixel lists, copied on the brush's stream, behind the
+// run and before the brush plans again; nothing else may be reading the lists
+// kept before.
+static void keep_lists(pnt_grad_s* g) {
   TapeRun& R = g->run;
+  hipStream_t s = g->b->ctx->stream;
   if (R.n_dl == 0) return;
   ensure(g->dl, g->dl_cap, R.n_dl, s);
   ensure(g->dl_off, g->dl_off_cap, R.n_off, s);
@@ -994,8 +997,8 @@ int pnt_grad_forward(pnt_grad g, pnt_dev_layer wet0, pnt_dev_rgb R0, const doubl
       ensure(g->tape, g->tape_cap, whole, s);
       g->run.base = g->tape;
       run_fused(b, cv, g->st.data(), ns, 0, &g->run);
+      keep_lists(g);
       if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
-      keep_lists(g, s);
     } else {
       if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
       // segments (at most seg_len stamps, a dip starts a new one) and their
@@ -1062,6 +1065,9 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
     hipStream_t s = g->ctx->stream;
     PNT_REQUIRE(b->size_map == g->fwd_size_map && b->use_snap == g->fwd_snap,
                 "the brush's geometry or snapshot switch changed since the forward");
+    // the brush's calls run on its own context's stream; segments use its buffers
+    const bool other = b->ctx->stream != s;
+    if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
     const int64_t n = cv->n, m = b->m;
     const int sm = b->size_map;
     const int ns = (int)g->st.size();
@@ -1111,11 +1117,10 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
         // run it again onto its tape, then reverse it
         ensure(g->tape, g->tape_cap, g->run.slot * g->seg_len, s);
         g->run.base = g->tape;
-        const bool other = b->ctx->stream != s;
         if (other) PNT_HIP_CHECK(hipStreamSynchronize(s));
         run_fused(b, cv, g->st.data() + sg.s0, sg.s1 - sg.s0, 0, &g->run);
+        keep_lists(g);
         if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
-        keep_lists(g, s);
         adjoint_waves(g, sg.s0, gC, gXL, s);
       }
       cv->epoch++;

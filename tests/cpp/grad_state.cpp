@@ -5,6 +5,9 @@
 //             allocations, the next one succeeds, its backward starts from
 //             cleared adjoint planes and no kernel or copy gets a buffer that is
 //             not there
+//   streams   a runner and a brush on two contexts: the runner's copies of the
+//             brush's plan are done when the forward returns, and a backward
+//             that touches the brush's buffers waits for the brush's stream
 #include "host_hip.hpp"
 
 #include <cmath>
@@ -30,6 +33,7 @@ constexpr size_t kAdjHead = 216;                     // bytes of k_adj_wave's sh
 struct Seen {
   int gX_filled, dirty_filled;  // clears of the whole adjoint planes / their dirty bytes
   int adj, adj_dirty_unset, adj_uncleared, stamps;
+  int box_early;  // checkpoint copies beside copies queued on another stream
   std::string order;  // 'k' composite adjoint, 's' stamps, 'a' adjoint wave
 } seen;
 
@@ -39,6 +43,8 @@ static void on_launch(const std::string& name, void** args) {
   if (is("6k_fillE") && *(int64_t*)args[1] == 7 * kStride) ++seen.gX_filled;
   if (is("k_stamp_wave")) ++seen.stamps, seen.order += 's';
   if (is("k_km_adj")) seen.order += 'k';
+  if (is("k_box_copy"))
+    for (const auto& o : state().queued) seen.box_early += o.stream != state().call.stream;
   if (is("k_adj_wave")) {
     seen.order += 'a';
     ++seen.adj;
@@ -151,11 +157,31 @@ static void check_failures() {
   }
 }
 
+static void check_streams() {
+  for (const char* mode : {"0", "64"}) {
+    setenv("PAINTY_GRAD_TAPE_MB", mode, 1);
+    Runner r(true);
+    pnt_canvas cv = nullptr;
+    Runner::ok(pnt_canvas_create(r.bctx, kRows, kCols, &cv));
+    for (int k = 0; k < 2; ++k) {
+      Runner::ok(r.forward());
+      // the brush plans the same stamps for another canvas, on its own stream
+      Runner::ok(pnt_imprint_stamps(r.b, cv, r.st.data(), (int64_t)r.st.size(), PNT_EXEC_FUSED));
+      Runner::ok(r.backward());
+      CHECK(seen.box_early == 0, "tape %s: checkpoints restored beside the brush's stream", mode);
+    }
+    CHECK(state().hazards.empty(), "tape %s: copies on two streams", mode);
+    pnt_canvas_destroy(cv);
+  }
+}
+
 int main(int argc, char** argv) {
   state().on_launch = on_launch;
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "failures")
     check_failures();
+  else if (what == "streams")
+    check_streams();
   else
     return 2;
   CHECK(state().hazards.empty(), "%s", state().hazards.empty() ? "" : state().hazards[0].c_str());
