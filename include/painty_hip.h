@@ -489,7 +489,9 @@ int pnt_dev_compose2_wet(pnt_ctx ctx, int64_t n, pnt_dev_wet dry,
  * visit's input on a tape while the list's tapes fit 1/8 of the free device
  * memory and 16 GiB (or PAINTY_GRAD_TAPE_MB); a longer list keeps checkpoints
  * every seg_len stamps (and at every dip) and the backward reruns it from
- * them.  The brush keeps its geometry and snapshot switch in between.
+ * them.  The brush keeps its map side (the radius' footprint, padded) and
+ * snapshot switch in between; the backward uses the rates, capacity and
+ * footprint that the forward found, whatever the brush has been given since.
  * Device planes are caller-owned, n = rows*cols floats each; the brush's
  * pickup map and snapshot are used as scratch by both calls. */
 typedef struct pnt_grad_s* pnt_grad;

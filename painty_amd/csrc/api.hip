@@ -219,6 +219,7 @@ void brush_set_geometry(pnt_brush b, double radius, const float* core, int width
   b->fp = fp;
   footprint_box(full, size_map, b->fbox);
   b->fp_host.swap(full);
+  ++b->geo_gen;
   b->pick = pick;
   b->radius = radius;
   b->width = w;

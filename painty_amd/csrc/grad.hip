@@ -731,8 +731,16 @@ struct pnt_grad_s {
   int2* dl = nullptr;      // the taped list's shared-pixel visits (the brush may plan again)
   int* dl_off = nullptr;
   int64_t dl_cap = 0, dl_off_cap = 0;
-  int fwd_size_map = 0;    // the brush's geometry at the forward
+  // the brush as the forward found it: a backward is of that forward, whatever
+  // rates or footprint the brush has been given since
+  int fwd_size_map = 0;
   bool fwd_snap = false;
+  uint64_t fwd_gen = 0;         // its geo_gen, for which fwd_fp was copied
+  std::vector<float> fwd_fp;    // padded footprint
+  double fwd_radius = 0.0, fwd_pr = 0.0, fwd_dr = 0.0, fwd_cap = 0.0;
+  int fwd_fbox[4] = {0, 0, -1, -1};
+  float* fp = nullptr;          // that footprint on the device, once the brush has another
+  int64_t fp_cap = 0;
   float* gX = nullptr;  // 7 planes of round_up(n, 64) (snapshot adjoint)
   uint8_t* gdirty = nullptr;  // its dirty bytes
   bool adj_zero = false;  // both are zero: a backward that runs to its end leaves them so
@@ -788,6 +796,51 @@ static void keep_lists(pnt_grad_s* g) {
   PNT_HIP_CHECK(hipMemcpyAsync(g->dl_off, R.dl_off, (size_t)R.n_off * sizeof(int),
                                hipMemcpyDeviceToDevice, s));
 }
+
+// The runner's brush with the values of the forward, for as long as this lives
+// (its map side and snapshot switch are the same).
+namespace {
+struct BrushAsForward {
+  pnt_grad_s* g;
+  float* fp;
+  double radius, pr, dr, cap;
+  int fbox[4];
+  explicit BrushAsForward(pnt_grad_s* g_) : g(g_) {
+    pnt_brush b = g->b;
+    hipStream_t s = b->ctx->stream;
+    fp = b->fp;
+    float* mine = b->fp;
+    if (b->geo_gen != g->fwd_gen && b->fp_host != g->fwd_fp) {
+      ensure(g->fp, g->fp_cap, b->m, s);
+      PNT_HIP_CHECK(hipMemcpyAsync(g->fp, g->fwd_fp.data(), (size_t)b->m * sizeof(float),
+                                   hipMemcpyHostToDevice, s));
+      PNT_HIP_CHECK(hipStreamSynchronize(s));
+      mine = g->fp;
+    }
+    radius = b->radius;
+    pr = b->pickup_rate;
+    dr = b->dep_rate;
+    cap = b->cap;
+    std::copy(b->fbox, b->fbox + 4, fbox);
+    b->fp = mine;
+    b->radius = g->fwd_radius;
+    b->pickup_rate = g->fwd_pr;
+    b->dep_rate = g->fwd_dr;
+    b->cap = g->fwd_cap;
+    std::copy(g->fwd_fbox, g->fwd_fbox + 4, b->fbox);
+  }
+  BrushAsForward(const BrushAsForward&) = delete;
+  ~BrushAsForward() {
+    pnt_brush b = g->b;
+    b->fp = fp;
+    b->radius = radius;
+    b->pickup_rate = pr;
+    b->dep_rate = dr;
+    b->cap = cap;
+    std::copy(fbox, fbox + 4, b->fbox);
+  }
+};
+}  // namespace
 
 // The adjoint of the taped run (stamps s0 .. of the list), its waves in
 // reverse.  Every chain's map adjoint goes on from where it stands.
@@ -929,6 +982,7 @@ int pnt_grad_destroy(pnt_grad g) {
     (void)hipFree(g->gP);
     (void)hipFree(g->gB);
     (void)hipFree(g->scratch);
+    (void)hipFree(g->fp);
     pnt_ctx ctx = g->ctx;
     delete g;
     ctx_release(ctx);
@@ -980,6 +1034,13 @@ int pnt_grad_forward(pnt_grad g, pnt_dev_layer wet0, pnt_dev_rgb R0, const doubl
     g->run.slot = tape_floats(g->run.area, m);
     g->fwd_size_map = b->size_map;
     g->fwd_snap = b->use_snap;
+    if (g->fwd_gen != b->geo_gen || g->fwd_fp.empty()) g->fwd_fp = b->fp_host;
+    g->fwd_gen = b->geo_gen;
+    g->fwd_radius = b->radius;
+    g->fwd_pr = b->pickup_rate;
+    g->fwd_dr = b->dep_rate;
+    g->fwd_cap = b->cap;
+    std::copy(b->fbox, b->fbox + 4, g->fwd_fbox);
     g->have_forward = false;
     const int64_t whole = g->run.slot * ns;
     g->full_tape = whole <= g->tape_cap;
@@ -1068,6 +1129,7 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
     // the brush's calls run on its own context's stream; segments use its buffers
     const bool other = b->ctx->stream != s;
     if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
+    const BrushAsForward as_forward(g);
     const int64_t n = cv->n, m = b->m;
     const int sm = b->size_map;
     const int ns = (int)g->st.size();

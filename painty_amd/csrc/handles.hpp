@@ -114,6 +114,7 @@ struct pnt_brush_s {
   float* fp = nullptr;         // footprint, size_map^2
   int64_t fp_cap = 0, pick_cap = 0;  // floats allocated at fp / pick
   std::vector<float> fp_host;  // same footprint on the host (traffic replay)
+  uint64_t geo_gen = 0;        // bumped with every new footprint
   int fbox[4] = {0, 0, 1 << 30, 1 << 30};  // nonzero footprint cells: x0 y0 x1 y1
   float* pick = nullptr;       // pickup map: mstride cells of kCell floats
   float* snap = nullptr;       // snapshot: a layer (8 strides of snap_stride)

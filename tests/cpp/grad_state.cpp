@@ -8,6 +8,8 @@
 //   streams   a runner and a brush on two contexts: the runner's copies of the
 //             brush's plan are done when the forward returns, and a backward
 //             that touches the brush's buffers waits for the brush's stream
+//   brush     rates and footprint changed after the forward: the backward (and
+//             its rerun of segments) has the forward's, the brush keeps the new
 #include "host_hip.hpp"
 
 #include <cmath>
@@ -27,12 +29,18 @@ static int g_fail = 0;
 
 constexpr int kRows = 60, kCols = 64;
 constexpr int64_t kN = kRows * kCols, kStride = kN;  // a multiple of 64
-constexpr size_t kAdjHead = 216;                     // bytes of k_adj_wave's shared arguments
+constexpr size_t kAdjHead = 216;  // bytes of k_adj_wave's shared arguments
+
+constexpr size_t kStampHead = 128;  // of k_stamp_wave's
+constexpr double kOldRate = 0.625, kNewRate = 0.375;  // pickup rates
+constexpr float kOldMid = 0.5f, kNewMid = 0.75f;      // the footprint's middle
+constexpr int kSide = 13;                             // map side at radius 4
 
 // What the launches since `reset` did.
 struct Seen {
   int gX_filled, dirty_filled;  // clears of the whole adjoint planes / their dirty bytes
   int adj, adj_dirty_unset, adj_uncleared, stamps;
+  int rate_old, rate_new, fp_old, fp_new;  // launches with either's value
   int box_early;  // checkpoint copies beside copies queued on another stream
   std::string order;  // 'k' composite adjoint, 's' stamps, 'a' adjoint wave
 } seen;
@@ -42,6 +50,18 @@ static void on_launch(const std::string& name, void** args) {
   if (is("9k_fill_u8") && *(int64_t*)args[1] == kStride + 16) ++seen.dirty_filled;
   if (is("6k_fillE") && *(int64_t*)args[1] == 7 * kStride) ++seen.gX_filled;
   if (is("k_stamp_wave")) ++seen.stamps, seen.order += 's';
+  if (is("k_stamp_wave") || is("k_adj_wave")) {
+    const size_t head = is("k_adj_wave") ? kAdjHead : kStampHead;
+    seen.rate_old += host_hip::holds(args[0], head, kOldRate);
+    seen.rate_new += host_hip::holds(args[0], head, kNewRate);
+    // the padded footprint on the device, by its content
+    for (const auto& a : state().dev)
+      if (host_hip::holds(args[0], kAdjHead, a.first) && a.second == kSide * kSide * sizeof(float)) {
+        const float mid = ((const float*)a.first)[kSide * (kSide / 2) + kSide / 2];
+        seen.fp_old += mid == kOldMid && is("k_adj_wave");
+        seen.fp_new += mid == kNewMid;
+      }
+  }
   if (is("k_km_adj")) seen.order += 'k';
   if (is("k_box_copy"))
     for (const auto& o : state().queued) seen.box_early += o.stream != state().call.stream;
@@ -67,6 +87,7 @@ struct Runner {
     const int w = (int)(2.0 * std::ceil(r) + 1.0);
     std::vector<float> f((size_t)w * w);
     for (int i = 0; i < w * w; ++i) f[(size_t)i] = 0.2f + 0.01f * (float)(i % 7);
+    f[f.size() / 2] = kOldMid;
     return f;
   }
   static int ok(int st) {
@@ -79,6 +100,7 @@ struct Runner {
     if (other_ctx) ok(pnt_ctx_create(0, &bctx));
     fp = footprint(radius);
     ok(pnt_brush_create(bctx, radius, fp.data(), (int)(2 * std::ceil(radius) + 1), &b));
+    ok(pnt_brush_set_pickup_rate(b, kOldRate));
     std::vector<int32_t> paint_of;
     for (int i = 0; i < 24; ++i) {
       pnt_stamp s{};
@@ -175,6 +197,30 @@ static void check_streams() {
   }
 }
 
+static void check_brush() {
+  for (const char* mode : {"0", "64"}) {
+    setenv("PAINTY_GRAD_TAPE_MB", mode, 1);
+    Runner r;
+    Runner::ok(r.forward());
+    Runner::ok(pnt_brush_set_pickup_rate(r.b, kNewRate));
+    std::vector<float> other = r.fp;
+    other[other.size() / 2] = kNewMid;
+    Runner::ok(pnt_brush_set_radius(r.b, 8.0, Runner::footprint(8.0).data(), 17));
+    Runner::ok(pnt_brush_set_radius(r.b, 4.0, other.data(), 9));
+    Runner::ok(r.backward());
+    CHECK(seen.adj > 0 && seen.rate_new == 0 && seen.rate_old == seen.adj + seen.stamps,
+          "tape %s: the forward's rate in %d + %d launches: %d, the new one in %d", mode, seen.adj,
+          seen.stamps, seen.rate_old, seen.rate_new);
+    CHECK(seen.fp_new == 0 && seen.fp_old == seen.adj, "tape %s: the forward's footprint", mode);
+    pnt_canvas cv = nullptr;
+    Runner::ok(pnt_canvas_create(r.ctx, kRows, kCols, &cv));
+    seen = Seen{};
+    Runner::ok(pnt_imprint(r.b, cv, 30.0, 30.0, 0.1));
+    CHECK(seen.rate_new == 1 && seen.rate_old == 0, "tape %s: the brush's own rate", mode);
+    pnt_canvas_destroy(cv);
+  }
+}
+
 int main(int argc, char** argv) {
   state().on_launch = on_launch;
   const std::string what = argc > 1 ? argv[1] : "";
@@ -182,6 +228,8 @@ int main(int argc, char** argv) {
     check_failures();
   else if (what == "streams")
     check_streams();
+  else if (what == "brush")
+    check_brush();
   else
     return 2;
   CHECK(state().hazards.empty(), "%s", state().hazards.empty() ? "" : state().hazards[0].c_str());

@@ -1,6 +1,6 @@
 """What a gradient runner may count on between its calls: a brush on another
-context that stamps elsewhere between the forward and the backward.  Every
-gradient against the FP64 oracle's, with the bound of test_gpu_grad.py."""
+context that stamps elsewhere between the forward and the backward, a brush
+whose rates and footprint change in between.  Every gradient against the FP64 oracle's, with the bound of test_gpu_grad.py."""
 import numpy as np
 import pytest
 
@@ -48,3 +48,16 @@ def test_brush_of_another_context(hip, oracle, tape):
     st["cx"], st["cy"] = st["cy"] + 3.25, st["cx"] + 2.5  # another plan in the same buffers
     br.imprintStamps(st, cv)
     check("other/" + tape, run, gR, ref)
+
+
+def test_brush_changed_after_the_forward(hip, oracle, tape):
+    c = edge_case(True)
+    gR = np.random.default_rng(8).normal(size=c["R0"].shape)
+    ref = oracle_gradient(oracle, c, gR)[1]
+    br, run = make(c)
+    core = c["core"].astype(np.float32)
+    br.setRadius(c["radius"] + 5, np.ones((2 * (int(np.ceil(c["radius"])) + 5) + 1,) * 2, np.float32))
+    br.setRadius(c["radius"], np.ascontiguousarray(core[::-1] * np.float32(0.5)))
+    br.setPickupRate(0.3)
+    br.setDepositionRate(0.6)
+    check("changed/" + tape, run, gR, ref)
