@@ -727,6 +727,7 @@ struct pnt_grad_s {
   float* tape = nullptr;
   int64_t tape_cap = 0;
   bool full_tape = false;  // the last forward taped the whole list
+  bool canvas_final = false;  // cv is as the forward left it (segments rerun change it)
   TapeRun run;
   int2* dl = nullptr;      // the taped list's shared-pixel visits (the brush may plan again)
   int* dl_off = nullptr;
@@ -841,6 +842,37 @@ struct BrushAsForward {
   }
 };
 }  // namespace
+
+// Segment sg again, from its checkpoint: canvas and snapshot in its box and the
+// pickup map as before it, the brush paint of its last dip (stamp 0 dips), and
+// its stamps, onto `tape` if given.  In list order over all segments this ends
+// in the forward's final state.
+static void rerun_segment(pnt_grad_s* g, const pnt_grad_s::Seg& sg, TapeRun* tape) {
+  pnt_brush b = g->b;
+  pnt_canvas cv = g->cv;
+  hipStream_t s = g->ctx->stream;
+  const int64_t area = (int64_t)sg.w * sg.h, m = b->m;
+  const int sm = b->size_map;
+  float* c0 = g->ckpt + sg.off;
+  box_copy({layer_box(cv->layer(), cv->cols, sg.x0, sg.y0, sg.w, sg.h, reinterpret_cast<double*>(c0), area),
+            layer_box(b->snap_planes(), cv->cols, sg.x0, sg.y0, b->use_snap ? sg.w : 0, sg.h,
+                      reinterpret_cast<double*>(c0 + 14 * area), area),
+            cell_box(b->pick, sm, 0, 0, sm, sm, c0 + (b->use_snap ? 28 : 14) * area, m)},
+           false, s);
+  cv->epoch++;
+  b->dirty_canvas = nullptr;  // the snapshot's dirty bytes no longer hold
+  int i = sg.s0;
+  while (!(g->st[(size_t)i].flags & PNT_STAMP_DIP)) --i;
+  for (int c = 0; c < 3; ++c) {
+    b->paintK[c] = g->st[(size_t)i].K[c];
+    b->paintS[c] = g->st[(size_t)i].S[c];
+  }
+  const bool other = b->ctx->stream != s;
+  if (other) PNT_HIP_CHECK(hipStreamSynchronize(s));
+  run_fused(b, cv, g->st.data() + sg.s0, sg.s1 - sg.s0, 0, tape);
+  if (tape) keep_lists(g);
+  if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
+}
 
 // The adjoint of the taped run (stamps s0 .. of the list), its waves in
 // reverse.  Every chain's map adjoint goes on from where it stands.
@@ -1109,7 +1141,7 @@ int pnt_grad_forward(pnt_grad g, pnt_dev_layer wet0, pnt_dev_rgb R0, const doubl
       }
     }
     launch_compose(n, L, R0c, Rgb3{{R.p[0], R.p[1], R.p[2]}}, s);
-    g->have_forward = true;
+    g->have_forward = g->canvas_final = true;
   });
 }
 
@@ -1136,6 +1168,17 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
     const Layer7 L = cv->layer();
     const Plane7 gC{{gwet.p[0], gwet.p[1], gwet.p[2], gwet.p[3], gwet.p[4], gwet.p[5], gwet.p[6]}};
     // ---- composite adjoint at the final state
+    if (!g->full_tape) {
+      // the snapshot has this canvas' size again, should the brush have
+      // stamped another since; the segments restore what they read of it
+      if (b->use_snap && (b->snap_rows != cv->rows || b->snap_cols != cv->cols)) {
+        brush_full_snapshot(b, cv);
+        if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
+      }
+      if (!g->canvas_final)  // a backward was here before: every segment again, in order
+        for (const auto& sg : g->segs) rerun_segment(g, sg, nullptr);
+      g->canvas_final = true;
+    }
     k_km_adj<<<grid_for(n), kBlk, 0, s>>>(n, L, cv->R0(), Rgb3{{gR.p[0], gR.p[1], gR.p[2]}}, gC,
                                           Rgb3{{gR0.p[0], gR0.p[1], gR0.p[2]}});
     PNT_HIP_CHECK(hipGetLastError());
@@ -1157,33 +1200,12 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
     if (g->full_tape) {
       adjoint_waves(g, 0, gC, gXL, s);
     } else {
-      for (int k = (int)g->segs.size() - 1; k >= 0; --k) {
-        const auto& sg = g->segs[k];
-        // restore the segment's checkpoint: the snapshot's dirty bytes no
-        // longer hold
-        const int64_t carea = (int64_t)sg.w * sg.h;
-        float* c0 = g->ckpt + sg.off;
-        box_copy({layer_box(L, cv->cols, sg.x0, sg.y0, sg.w, sg.h, reinterpret_cast<double*>(c0), carea),
-                  layer_box(b->snap_planes(), cv->cols, sg.x0, sg.y0, b->use_snap ? sg.w : 0, sg.h,
-                            reinterpret_cast<double*>(c0 + 14 * carea), carea),
-                  cell_box(b->pick, sm, 0, 0, sm, sm, c0 + (b->use_snap ? 28 : 14) * carea, m)},
-                 false, s);
-        cv->epoch++;
-        b->dirty_canvas = nullptr;
-        int i = sg.s0;  // brush paint at the segment start: its last dip (stamp 0 dips)
-        while (!(g->st[i].flags & PNT_STAMP_DIP)) --i;
-        for (int c = 0; c < 3; ++c) {
-          b->paintK[c] = g->st[i].K[c];
-          b->paintS[c] = g->st[i].S[c];
-        }
-        // run it again onto its tape, then reverse it
-        ensure(g->tape, g->tape_cap, g->run.slot * g->seg_len, s);
-        g->run.base = g->tape;
-        if (other) PNT_HIP_CHECK(hipStreamSynchronize(s));
-        run_fused(b, cv, g->st.data() + sg.s0, sg.s1 - sg.s0, 0, &g->run);
-        keep_lists(g);
-        if (other) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
-        adjoint_waves(g, sg.s0, gC, gXL, s);
+      ensure(g->tape, g->tape_cap, g->run.slot * g->seg_len, s);
+      g->run.base = g->tape;
+      g->canvas_final = false;
+      for (int k = (int)g->segs.size() - 1; k >= 0; --k) {  // rerun onto the tape, then reversed
+        rerun_segment(g, g->segs[(size_t)k], &g->run);
+        adjoint_waves(g, g->segs[(size_t)k].s0, gC, gXL, s);
       }
       cv->epoch++;
       b->dirty_canvas = nullptr;

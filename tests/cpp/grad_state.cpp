@@ -10,6 +10,8 @@
 //             that touches the brush's buffers waits for the brush's stream
 //   brush     rates and footprint changed after the forward: the backward (and
 //             its rerun of segments) has the forward's, the brush keeps the new
+//   again     a second backward of one forward begins with the final state: from
+//             checkpoints it reruns every segment before the composite's adjoint
 #include "host_hip.hpp"
 
 #include <cmath>
@@ -221,6 +223,23 @@ static void check_brush() {
   }
 }
 
+static void check_again() {
+  for (const char* mode : {"0", "64"}) {
+    setenv("PAINTY_GRAD_TAPE_MB", mode, 1);
+    Runner r;
+    Runner::ok(r.forward());
+    const int stamps = seen.stamps;
+    Runner::ok(r.backward());
+    CHECK(seen.order.find('k') == 0, "tape %s: first backward %s", mode, seen.order.c_str());
+    for (int k = 0; k < 2; ++k) {
+      Runner::ok(r.backward());
+      const int before = (int)seen.order.find('k');
+      CHECK(before == (mode[0] == '0' ? stamps : 0), "tape %s: another backward: %s", mode,
+            seen.order.c_str());
+    }
+  }
+}
+
 int main(int argc, char** argv) {
   state().on_launch = on_launch;
   const std::string what = argc > 1 ? argv[1] : "";
@@ -230,6 +249,8 @@ int main(int argc, char** argv) {
     check_streams();
   else if (what == "brush")
     check_brush();
+  else if (what == "again")
+    check_again();
   else
     return 2;
   CHECK(state().hazards.empty(), "%s", state().hazards.empty() ? "" : state().hazards[0].c_str());

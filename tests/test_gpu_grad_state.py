@@ -1,6 +1,7 @@
 """What a gradient runner may count on between its calls: a brush on another
 context that stamps elsewhere between the forward and the backward, a brush
-whose rates and footprint change in between.  Every gradient against the FP64 oracle's, with the bound of test_gpu_grad.py."""
+whose rates and footprint change in between, and a second backward of one
+forward, the brush having stamped canvases of other sizes.  Every gradient against the FP64 oracle's, with the bound of test_gpu_grad.py."""
 import numpy as np
 import pytest
 
@@ -61,3 +62,14 @@ def test_brush_changed_after_the_forward(hip, oracle, tape):
     br.setPickupRate(0.3)
     br.setDepositionRate(0.6)
     check("changed/" + tape, run, gR, ref)
+
+
+def test_backward_again(hip, oracle, tape):
+    c = edge_case(True)
+    gR = np.random.default_rng(9).normal(size=c["R0"].shape)
+    ref = oracle_gradient(oracle, c, gR)[1]
+    br, run = make(c)
+    for k, side in enumerate((None, 40, 130)):
+        if side:
+            br.imprintStamps(c["stamps"], H.Canvas(side, side + 3))
+        check("again%d/%s" % (k, tape), run, gR, ref)
