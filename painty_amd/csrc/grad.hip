@@ -1087,7 +1087,14 @@ int pnt_grad_forward(pnt_grad g, pnt_dev_layer wet0, pnt_dev_rgb R0, const doubl
                      std::min((int64_t)mem_free / kTapeFree, kTapeMost);
     }
     if (g->full_tape) {
-      ensure(g->tape, g->tape_cap, whole, s);
+      try {
+        ensure(g->tape, g->tape_cap, whole, s);
+      } catch (const Error& e) {  // less memory in one piece than free: checkpoints
+        if (e.code != PNT_ENOMEM) throw;
+        g->full_tape = false;
+      }
+    }
+    if (g->full_tape) {
       g->run.base = g->tape;
       run_fused(b, cv, g->st.data(), ns, 0, &g->run);
       keep_lists(g);

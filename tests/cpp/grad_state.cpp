@@ -12,6 +12,7 @@
 //             its rerun of segments) has the forward's, the brush keeps the new
 //   again     a second backward of one forward begins with the final state: from
 //             checkpoints it reruns every segment before the composite's adjoint
+//   no-tape   a forward whose tape cannot be allocated keeps checkpoints
 #include "host_hip.hpp"
 
 #include <cmath>
@@ -96,12 +97,12 @@ struct Runner {
     if (st) std::fprintf(stderr, "status %d: %s\n", st, pnt_last_error()), std::abort();
     return st;
   }
-  explicit Runner(bool other_ctx = false, double radius = 4.0) {
+  explicit Runner(bool other_ctx = false) {
     ok(pnt_ctx_create(0, &ctx));
     bctx = ctx;
     if (other_ctx) ok(pnt_ctx_create(0, &bctx));
-    fp = footprint(radius);
-    ok(pnt_brush_create(bctx, radius, fp.data(), (int)(2 * std::ceil(radius) + 1), &b));
+    fp = footprint(4.0);
+    ok(pnt_brush_create(bctx, 4.0, fp.data(), 9, &b));
     ok(pnt_brush_set_pickup_rate(b, kOldRate));
     std::vector<int32_t> paint_of;
     for (int i = 0; i < 24; ++i) {
@@ -240,6 +241,24 @@ static void check_again() {
   }
 }
 
+static void check_no_tape() {
+  unsetenv("PAINTY_GRAD_TAPE_MB");
+  int refused = 0;
+  for (int at = 1;; ++at) {
+    Runner r;
+    state().fail_in = at;
+    const int first = r.forward();
+    const bool hit = state().fail_in == 0;
+    state().fail_in = 0;
+    if (!hit) break;
+    if (first) continue;  // another allocation than the tape's
+    ++refused;
+    Runner::ok(r.backward());
+    CHECK(seen.stamps > 0, "a backward without a tape reruns segments: %s", seen.order.c_str());
+  }
+  CHECK(refused == 1, "%d allocations a forward does without", refused);
+}
+
 int main(int argc, char** argv) {
   state().on_launch = on_launch;
   const std::string what = argc > 1 ? argv[1] : "";
@@ -251,6 +270,8 @@ int main(int argc, char** argv) {
     check_brush();
   else if (what == "again")
     check_again();
+  else if (what == "no-tape")
+    check_no_tape();
   else
     return 2;
   CHECK(state().hazards.empty(), "%s", state().hazards.empty() ? "" : state().hazards[0].c_str());
