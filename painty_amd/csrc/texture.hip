@@ -38,7 +38,8 @@
 #include "internal.hpp"
 #include "visit.hpp"
 
-// FP64 expressions evaluate as written (no fused multiply-adds), as the
+// FP64 expressions evaluate as written (no fused multiply-adds but inside
+// quot and recip, whose results are rounded as the operators' are), as the
 // reference's do: the texture coordinates decide which pixels a stroke
 // covers, and the smudge's map offsets are truncations.
 #pragma clang fp contract(off)
@@ -240,27 +241,39 @@ struct TradeArgs {
   double bmin_x, bmin_y, ctr_x, ctr_y, radius;
   const double* tmap;
   int trows, tcols;
-  double maxD;
+  double maxD, inv_maxD;  // the largest thickness and 1 / it
 };
 
-// The share of its volume that either side gives where the texture thickness
-// is Dv: the pickup and deposition rates of Smudge.hxx:94-157 are both 0.1.
-// 0 or less: the pixel is not textured.
-__device__ __forceinline__ double smudge_share(double Dv, double maxD) {
-  return Dv <= 0.0 ? 0.0 : 0.1 * Dv / maxD;
+// a / d and 1 / v, correctly rounded as the division operator's are, without
+// its scaling and fix-up: `r` is 1 / d rounded (made on the host), and a
+// quotient q within an ulp becomes the rounded one by q + (a - q d) r
+// (Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", 1990).  Quotients above 2^-960; an infinite one stays infinite.
+__device__ __forceinline__ double quot(double a, double d, double r) {
+  const double q0 = a * r;
+  const double q1 = __builtin_fma(__builtin_fma(-q0, d, a), r, q0);
+  const double q = __builtin_fma(__builtin_fma(-q1, d, a), r, q1);
+  return __builtin_isinf(q0) ? q0 : q;
+}
+__device__ __forceinline__ double recip(double v) {
+  const double r = rcpd(v);
+  return __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
 }
 
 // The exchange of Smudge::smudge (Smudge.hxx:94-157) between a map cell and
-// the canvas pixel under it.
+// the canvas pixel under it, where the texture thickness is Dv: both rates are
+// 0.1 of the thickness' share of the largest.  Volumes decide the branches:
+// they, and all else here, are the reference's expressions as written.
 __device__ __forceinline__ void smudge_trade(double pK[3], double pS[3], double& pV, float cK[3],
-                                             float cS[3], double& cV, double share) {
-  constexpr double MinVolume = 0.001;
-  const double cVl = cV * share, cVr = cV - cVl;
-  const double pVl = pV * share, pVr = pV - pVl;
+                                             float cS[3], double& cV, double Dv,
+                                             const TradeArgs& T) {
+  constexpr double MinVolume = 0.001, rate = 0.1;
+  const double cVl = quot(cV * rate * Dv, T.maxD, T.inv_maxD), cVr = cV - cVl;
+  const double pVl = quot(pV * rate * Dv, T.maxD, T.inv_maxD), pVr = pV - pVl;
   const double K[3] = {cK[0], cK[1], cK[2]}, S[3] = {cS[0], cS[1], cS[2]};
   const double cVnew = cVr + pVl;
   if (cVnew > MinVolume) {
-    const double inv = rcpd(cVnew);
+    const double inv = recip(cVnew);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       cK[c] = (float)(inv * (cVr * K[c] + pVl * pK[c]));
@@ -270,7 +283,7 @@ __device__ __forceinline__ void smudge_trade(double pK[3], double pS[3], double&
   }
   const double pVnew = pVr + cVl;
   if (pVnew > MinVolume) {
-    const double inv = rcpd(pVnew);
+    const double inv = recip(pVnew);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       pK[c] = inv * (pVr * pK[c] + cVl * K[c]);
@@ -334,7 +347,7 @@ __global__ __launch_bounds__(kStepBlock) void k_smudge_step(SMap src, SMap dst, 
       cS[c] = T.canvas.ks[3 + c][ic];
     }
     double cV = T.canvas.v[ic];
-    smudge_trade(pK, pS, pV, cK, cS, cV, smudge_share(Dv, T.maxD));
+    smudge_trade(pK, pS, pV, cK, cS, cV, Dv, T);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       T.canvas.ks[c][ic] = cK[c];
@@ -371,9 +384,10 @@ __global__ __launch_bounds__(kStepBlock) void k_smudge_step(SMap src, SMap dst, 
 // reads them there, and writes back those it no longer covers.
 //
 // A step is bound by the FP64 chain of its cells (bilinear turn, trade): with
-// reciprocals in place of divisions, the radius test on squares and the
-// bilinear neighbours clamped instead of reflected, a stroke of 1177 steps
-// took 3.05 ms (3.7 before, 8.2 with a launch a step).
+// correctly rounded quotients by Newton steps in place of the division
+// operator's scaling and fix-up, the radius test on squares and the bilinear
+// neighbours clamped instead of reflected, a stroke of 1177 steps takes 3.14 ms
+// (3.7 before, 8.2 with a launch a step; 3.06 with quotients an ulp off).
 constexpr int kSB = 8;        // tile side
 constexpr int kSSide = 40;    // side of the region in LDS: 96 B a place, 150 KB
 constexpr int kSMax = 10;     // steps of a launch
@@ -417,7 +431,7 @@ __global__ __launch_bounds__(kSThreads) void k_smudge_steps(SArgs A) {
   constexpr int kN = kSSide * kSSide;
   __shared__ double M[7][kN];   // map cells: K, S, V
   __shared__ float C[6][kN];    // canvas pixels: K, S
-  __shared__ double CV[kN], D[kN];  // their volume and smudge_share (0: no trade)
+  __shared__ double CV[kN], D[kN];  // their volume and the texture's thickness (0: no trade)
   const TradeArgs& T = A.T;
   const int t = threadIdx.x, n = A.n;
   // regions: R[i] of step i (1-based; 0: the source map), in cells
@@ -472,7 +486,7 @@ __global__ __launch_bounds__(kSThreads) void k_smudge_steps(SArgs A) {
       }
       const int tpx = (int)(x - T.bmin_x), tpy = (int)(y - T.bmin_y);
       if (!(tpx < 0 || tpy < 0 || tpx >= T.tcols || tpy >= T.trows)) {
-        d = smudge_share(T.tmap[(int64_t)tpy * T.tcols + tpx], T.maxD);
+        d = T.tmap[(int64_t)tpy * T.tcols + tpx];
       }
     }
     D[e] = d;
@@ -527,10 +541,10 @@ __global__ __launch_bounds__(kSThreads) void k_smudge_steps(SArgs A) {
       }
       const int cpx = x + S.roi_x, cpy = y + S.roi_y;
       const int q = (cpy - py0) * pw + (cpx - px0);
-      const double share = D[q];
+      const double Dv = D[q];
       const double dx = S.ctr_x - (double)cpx, dy = S.ctr_y - (double)cpy, dd = dx * dx + dy * dy;
       // !(sqrt(dd) > radius), the root taken only within 1e-12 of the edge
-      if (!(share <= 0.0) && !(dd > A.rr_hi) &&
+      if (!(Dv <= 0.0) && !(dd > A.rr_hi) &&
           (dd < A.rr_lo || !(sqrt(dd) > T.radius))) {
         float cK[3], cS[3];
 #pragma unroll
@@ -539,7 +553,7 @@ __global__ __launch_bounds__(kSThreads) void k_smudge_steps(SArgs A) {
           cS[c] = C[3 + c][q];
         }
         double cV = CV[q];
-        smudge_trade(&p[u][0], &p[u][3], p[u][6], cK, cS, cV, share);
+        smudge_trade(&p[u][0], &p[u][3], p[u][6], cK, cS, cV, Dv, T);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
           C[c][q] = cK[c];
@@ -1051,6 +1065,7 @@ int pnt_tbrush_paint_stroke(pnt_tbrush b, pnt_canvas cv, const double* xy, int64
       T.trows = trows;
       T.tcols = tcols;
       T.maxD = maxD_h;
+      T.inv_maxD = 1.0 / maxD_h;
       // the spine positions
       std::vector<Spine> spine;
       for (double u = 0.0; maxD_h > 0.0 && u <= 1.0; u += 1. / length) {

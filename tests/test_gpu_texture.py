@@ -181,3 +181,24 @@ def test_smudge_over_map_sizes_and_turns(hip, oracle, radius, path):
         ob.paint_stroke(np.array(xy), oc)
         gb.paintStroke(np.array(xy), gc)
         _compare("texture/r%g/%s/%d" % (radius, path, k), gc, oc, gb, ob)
+
+
+# Volumes decide the MinVolume branches, and nothing FP32 feeds them: the trade
+# is evaluated as the reference writes it, so canvas and map volumes are the
+# oracle's to the bit -- blocked steps, single ones (radius 70), sharp turns.
+# The canvas' volumes lie near the threshold in part.
+@pytest.mark.parametrize("radius", [5.6, 12.3, 70.0])
+def test_smudge_volumes_are_the_oracles(hip, oracle, radius):
+    rows, cols = 150, 190
+    oc, gc = _canvases(hip, oracle, rows, cols, 3)
+    V = np.random.default_rng(4).uniform(0.0, 1.1, (rows, cols))
+    V[::3] *= 0.002
+    gc.getPaintLayer().setBuffers(V=V)
+    oc.V[...] = V
+    ob, gb = _brushes(hip, oracle, radius, sample_thickness(), True)
+    for xy in ([[5.2, 140.7], [90.0, 60.2], [180.3, 12.1]],
+               [[20.1, 60.3], [150.4, 66.2], [150.9, 72.8], [22.3, 78.1]]):
+        ob.paint_stroke(np.array(xy), oc)
+        gb.paintStroke(np.array(xy), gc)
+        np.testing.assert_array_equal(gc.getPaintLayer().getV_buffer(), oc.V)
+        np.testing.assert_array_equal(gb.getSmudgeMap()[2], ob.smudge_map()[2])
