@@ -772,9 +772,9 @@ pnt_batch_config get_batch_config(pnt_ctx ctx) { return batch_state(ctx)->cfg; }
 // saved first and restored after each candidate, so tuning leaves the jobs
 // as it found them.
 struct SavedJob {
-  float* canvas = nullptr;  // 11 planes
+  float* canvas = nullptr;  // kCanvasStrides of the canvas stride
   float* pick = nullptr;    // mstride cells
-  float* snap = nullptr;    // mstride cells
+  float* snap = nullptr;    // a layer (kLayerStrides of snap_stride)
   uint8_t* dirty = nullptr;
   int64_t canvas_n = 0, pick_n = 0, snap_n = 0, dirty_n = 0;
   float paintK[3], paintS[3];

@@ -1,6 +1,8 @@
-// Device pieces shared by the launch-per-list stamp kernels (persistent.hip,
-// batch.hip): the planned stamp descriptor, the bounded group barrier, the
-// one-round-trip visit, and the snapshot-ring helpers.
+// Device pieces shared by every stamp kernel (fused.hip, batch.hip,
+// batchwave.hip, serve.hip, persistent.hip) and the adjoint (grad.hip): the
+// planned stamp descriptor, the window tiles and their visits, the tape record,
+// the snapshot ring, the shared-pixel levels, and the bounded group barrier of
+// the kernels that run many stamps a launch.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -443,11 +445,6 @@ __device__ __forceinline__ void st_cell(float* pick, int m, const float v[7]) {
   p[1] = make_float4(v[4], v[5], v[6], 0.0f);
 }
 
-__device__ __forceinline__ int64_t canvas_index(const StampGeom& g, int col, int row) {
-#pragma clang fp contract(off)
-  return (int64_t)(int)(row + g.cy) * g.cols + (int)(col + g.cx);
-}
-
 // Loads everything one visit reads: canvas and pickup-source pixel.
 template <class PickAcc>
 __device__ __forceinline__ void load_pixel(const VisitTarget& T, bool snap, int64_t ic, bool pull,
@@ -590,6 +587,14 @@ __host__ __device__ inline int tile_count(const TileWin& w) {
   return ((w.cols + kT - 1) / kT) * ((w.rows + kT - 1) / kT);
 }
 
+// tile / tiles_x by r, 1 / tiles_x within an ulp: the half keeps the product at
+// least 0.5 / tiles_x from a whole number.  The largest map (a footprint of
+// radius 4095, 11587 cells a side) has 725 tiles a side: 6.9e-4 there, beside a
+// rounding of at most 1.3e-4.
+__host__ __device__ __forceinline__ int tile_row(int tile, float r) {
+  return (int)(((float)tile + 0.5f) * r);
+}
+
 __host__ __device__ inline StampGeom stamp_geom(const PStamp& p, int size_map, int rows, int cols) {
   return StampGeom{p.cx, p.cy, p.c, p.s, (size_map - 1) / 2, size_map, rows, cols};
 }
@@ -705,8 +710,7 @@ __device__ __forceinline__ void window_tile(const VisitTarget& T, float* pick,
   const int t = threadIdx.x;
   const int lx = t % kT, ly = t / kT;
   const int tiles_x = (win.cols + kT - 1) / kT;
-  // tile / tiles_x: at most 513 a side, so half a tile outweighs the rounding
-  const int ty = (int)(((float)tile + 0.5f) * __builtin_amdgcn_rcpf((float)tiles_x));
+  const int ty = tile_row(tile, __builtin_amdgcn_rcpf((float)tiles_x));
   const int col = win.col0 + (tile - ty * tiles_x) * kT + lx;
   const int row = win.row0 + ty * kT + ly;
   const VisitCell V = visit_cell(g, dom, col, row);

@@ -14,19 +14,20 @@ namespace pnt {
 constexpr double kMinVolume = 0.001;
 
 // The arithmetic runs in FP64, as the reference's does (vec3 is Eigen's
-// double vector): loads widen the stored FP32 values, every product, sum,
-// quotient and threshold test is the reference's own in double precision,
-// and each K/S result is rounded to FP32 once, when it is stored (canvas
-// and snapshot volumes are stored in FP64).  Over the
-// hundreds of dependent visits a pixel and a pickup cell take in a long
-// stamp list, only that storage rounding accumulates (an FP32 chain would
-// add the rounding of every intermediate step as well).
+// double vector): loads widen the stored FP32 values, every volume and
+// threshold test is the reference's own expression in double precision, and
+// each K/S result is rounded to FP32 once, when it is stored (canvas and
+// snapshot volumes are stored in FP64).  Over the hundreds of dependent visits
+// a pixel and a pickup cell take in a long stamp list, only that storage
+// rounding accumulates (an FP32 chain would add the rounding of every
+// intermediate step as well).
 //
 // blend(va, a, vb, b) = vt > MinVolume ? (va*a + vb*b) / vt : a with
-// vt = va + vb (FootprintBrush.hxx:331-340).  Its channels share the weights
-// va/vt and vb/vt, through one reciprocal: two operations a channel (a
-// product and a fused multiply-add).  The result is within 2e-16 relative of
-// the quotient, before it is rounded to FP32 for storage.
+// vt = va + vb (FootprintBrush.hxx:331-340) is not rounded step by step as
+// there: its channels share the weights va/vt and vb/vt, through one
+// reciprocal, two operations a channel (a product and a fused multiply-add).
+// The result is within 5e-16 relative of the quotient, before it is rounded to
+// FP32 for storage, and no volume or test depends on it.
 
 // 1/v for a normal v > MinVolume: the hardware's estimate (2^-23 or better)
 // and two Newton steps, within an ulp; no scaling for denormals or infinities.
@@ -46,7 +47,7 @@ __device__ __forceinline__ float rcpf(float x) { return __builtin_amdgcn_rcpf(x)
 //   void set_canvas(int c, float) (c < 6) / void set_canvas_v(double)
 // Canvas and source volumes are FP64 in memory, so every volume that a
 // MinVolume test sees is the reference's own number; contraction is off so
-// that each product and sum rounds as the reference's does.
+// that the volumes' products and sums round as the reference's do.
 template <class Acc>
 __device__ __forceinline__ void paint_visit_math(Acc& a, float fh_f, double pickup_rate,
                                                  double dep_rate, double cap, const float pK[3],

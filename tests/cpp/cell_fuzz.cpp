@@ -1,10 +1,10 @@
 // visit_cell and tile_window (stampcore.hpp) against the window walk they
 // stand for, on the CPU: for random imprint geometries and cell boxes, every
-// window offset that stamp_visit_in sends to a cell of the box gets the same
-// cell and pixel and lies in the tile window, and the neighbour it names is
-// exactly the other visitor of its cell -- any angle (multiples of 45 and 90
-// degrees among them), whole, half and fractional centres, stamps across
-// every canvas edge.
+// window offset that falls on a cell of the box gets the same cell and pixel
+// and lies in the tile window, and the neighbour it names is exactly the other
+// visitor of its cell -- any angle (multiples of 45 and 90 degrees among them),
+// whole, half and fractional centres, stamps across every canvas edge.  And
+// tile_row against the division, for every tile of up to 725 x 725.
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -19,7 +19,7 @@
 using namespace pnt;
 
 // The reference's index math (FootprintBrush.hxx:90-113) as written there,
-// with std::round: stamp_visit and stamp_visit_in must give the same.
+// with std::round: stamp_visit must give the same.
 static int walk_visit(const StampGeom& g, int col, int row, const FpBox& b, int64_t* ic) {
 #pragma clang fp contract(off)
   if (col < -g.hr || col > g.hr || row < -g.hr || row > g.hr) return -1;
@@ -77,7 +77,8 @@ int main(int argc, char** argv) {
         const int m = walk_visit(g, col, row, box, &ic);
         const VisitCell V = visit_cell(g, box, col, row);
         int64_t i2 = -1;
-        bool ok = V.mm == m && stamp_visit_in(g, col, row, box.x0, box.y0, box.x1, box.y1, &i2) == m &&
+        const FpBox all{0, 0, g.size_map - 1, g.size_map - 1};
+        bool ok = V.mm == m && stamp_visit(g, col, row, &i2) == walk_visit(g, col, row, all, &ic) &&
                   (m < 0 || i2 == ic);
         if (ok && m >= 0) {
           const auto& c = want[(size_t)m];
@@ -98,6 +99,14 @@ int main(int argc, char** argv) {
                        col, row, side, V.mm, m, V.shared);
       }
     if (seen != visits) ++fail;
+  }
+  // the rows' first and last tiles: tile_row rises with the tile; the
+  // hardware's reciprocal is within an ulp
+  for (int tx = 1; tx <= 725; ++tx) {
+    const float r0 = 1.0f / (float)tx;
+    for (const float r : {std::nextafter(r0, 0.0f), r0, std::nextafter(r0, 2.0f)})
+      for (int ty = 0; ty < 725; ++ty)
+        if (tile_row(ty * tx, r) != ty || tile_row(ty * tx + tx - 1, r) != ty) ++fail;
   }
   std::printf("%d stamps, %ld offsets, %ld shared cells: %ld failures\n", cases, cells,
               pairs, fail);
