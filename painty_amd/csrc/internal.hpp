@@ -54,6 +54,22 @@ struct Rgb3 {
   float* p[3];
 };
 
+// Division of any 32-bit number by one d >= 1 as a product and shifts
+// (Granlund and Montgomery, "Division by invariant integers using
+// multiplication", 1994, figure 4.1).
+struct Divisor {
+  uint32_t mul, sh1, sh2;
+  static Divisor of(uint32_t d) {
+    const uint32_t l = d > 1 ? 32 - (uint32_t)__builtin_clz(d - 1) : 0;  // ceil(log2 d)
+    const uint64_t m = (((uint64_t)1 << l) - d << 32) / d + 1;
+    return Divisor{(uint32_t)m, l > 0 ? 1u : 0u, l > 0 ? l - 1 : 0};
+  }
+  __host__ __device__ uint32_t div(uint32_t n) const {
+    const uint32_t t = (uint32_t)(((uint64_t)mul * n) >> 32);
+    return (t + ((n - t) >> sh1)) >> sh2;
+  }
+};
+
 // A pointer in the global address space.  Kernels that read device-memory
 // records holding pointers view them through a mirror record with these
 // fields: a pointer loaded as global keeps that address space through the

@@ -4,7 +4,8 @@
 // and lies in the tile window, and the neighbour it names is exactly the other
 // visitor of its cell -- any angle (multiples of 45 and 90 degrees among them),
 // whole, half and fractional centres, stamps across every canvas edge.  And
-// tile_row against the division, for every tile of up to 725 x 725.
+// tile_row against the division, for every tile of up to 725 x 725, and Divisor
+// (internal.hpp) around the multiples of every kind of divisor.
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -107,6 +108,15 @@ int main(int argc, char** argv) {
     for (const float r : {std::nextafter(r0, 0.0f), r0, std::nextafter(r0, 2.0f)})
       for (int ty = 0; ty < 725; ++ty)
         if (tile_row(ty * tx, r) != ty || tile_row(ty * tx + tx - 1, r) != ty) ++fail;
+  }
+  for (int it = 0; it < 20000; ++it) {
+    const uint32_t d = it < 3000 ? 1u + (uint32_t)it : 1u + (uint32_t)(rng() >> (1 + rng() % 31 + 32));
+    const Divisor D = Divisor::of(d);
+    for (int k = 0; k < 64; ++k) {
+      const uint32_t n = k < 4 ? 0xffffffffu - (uint32_t)k : (uint32_t)(rng() >> (32 + rng() % 31));
+      for (const uint32_t v : {n, n / d * d, n / d * d - 1u, n / d * d + d - 1u})
+        if (D.div(v) != v / d) ++fail;
+    }
   }
   std::printf("%d stamps, %ld offsets, %ld shared cells: %ld failures\n", cases, cells,
               pairs, fail);

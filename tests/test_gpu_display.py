@@ -84,3 +84,11 @@ def test_encode_at_rounding_edges(hip, oracle, bits, n):
         hip.default_context().synchronize()
         got = buf[off:off + 3 * m].cpu().numpy().view(ref.dtype).reshape(m, 3)
         np.testing.assert_array_equal(got, ref)
+
+
+# A column, a few, a wavefront's width and one more, a row: pixels are numbered
+# through, so widths only meet the division by the row's length.
+@pytest.mark.parametrize("rows,cols", [(9001, 1), (300, 3), (33, 64), (21, 65), (1, 129), (2, 2)])
+def test_render_of_any_width(hip, oracle, rows, cols):
+    cv, arrays = _canvas(hip, rows, cols, rows + cols)
+    assert_close("render/%dx%d" % (rows, cols), hip.Renderer.render(cv), oracle.render(*arrays))
