@@ -116,7 +116,9 @@ __device__ __forceinline__ void render_pixel(const RenderArgs& a, int i, int j) 
     const float G = g < 1.0f ? g : 1.0f;  // std::min(1.0, g)
     spec = (A * B * G) * rcp1(NdotL * NdotV);
   }
-  constexpr float beta = lightPower * (1.0f / (4.0f * kPiF));
+  // a volume that is no number has no light direction: as its squared length
+  // would, it makes the pixel NaN, which the clamp below makes 0
+  const float beta = __builtin_isfinite(s11) ? lightPower * (1.0f / (4.0f * kPiF)) : NAN;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     const float r = (beta * NdotL) * ((1.0f - s) * Kd[c] + s * spec) + (Kd[c] * 0.2f) * Kd[c];

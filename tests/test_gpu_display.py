@@ -92,3 +92,17 @@ def test_encode_at_rounding_edges(hip, oracle, bits, n):
 def test_render_of_any_width(hip, oracle, rows, cols):
     cv, arrays = _canvas(hip, rows, cols, rows + cols)
     assert_close("render/%dx%d" % (rows, cols), hip.Renderer.render(cv), oracle.render(*arrays))
+
+
+def test_render_of_volumes_that_are_no_numbers(hip, oracle):
+    """Infinite and NaN volumes, alone and as neighbours, come out as the
+    reference's NaN arithmetic and its clamp have them."""
+    cv, (K, S, V, R0) = _canvas(hip, 24, 30, 9)
+    for i, v in enumerate((np.inf, -np.inf, np.nan)):
+        V[4 + 7 * i, 3:28:5] = v
+        V[5 + 7 * i, 8] = v
+    cv.getPaintLayer().setBuffers(K, S, V)
+    got, ref = hip.Renderer.render(cv), oracle.render(K, S, V, R0)
+    own = ~np.isfinite(V)
+    np.testing.assert_array_equal(got[own], ref[own])
+    assert_close("render/non-finite", got, ref)
