@@ -1851,8 +1851,23 @@ int pnt_paint_stroke(pnt_brush b, pnt_canvas cv, const double* p, int64_t n) {
     b->ctx->use();
     canvas_tick(cv);
     if (cv->ctx->stream != b->ctx->stream) PNT_HIP_CHECK(hipStreamSynchronize(cv->ctx->stream));
-    // FootprintBrush.hxx:251-267
+    // FootprintBrush.hxx:251-267: the imprints as planned lists of at most
+    // kStrokePart (a stroke may be of any length, and the plan is pinned memory
+    // that the brush keeps); the dirty bytes are begun anew (all set) and not
+    // kept past the stroke, as after single imprints
+    constexpr size_t kStrokePart = 4096;
     std::vector<pnt_stamp> path;
+    const auto run = [&] {
+      if (path.empty()) return;
+      run_fused(b, cv, path.data(), (int64_t)path.size(), 1);
+      path.clear();
+    };
+    const struct Forget {
+      pnt_brush b;
+      ~Forget() { b->dirty_canvas = nullptr; }
+    } forget{b};
+    cv->epoch++;
+    b->dirty_canvas = nullptr;
     for (int64_t i = 0; i + 1 < n; ++i) {
       const int64_t ipre = i > 0 ? i - 1 : 0;
       const int64_t inext = (i + 2 < n) ? i + 2 : n - 1;
@@ -1872,15 +1887,10 @@ int pnt_paint_stroke(pnt_brush b, pnt_canvas cv, const double* p, int64_t n) {
         st.cy = catmull_rom(pp[1], p0[1], p1[1], pn[1], t);
         st.theta = std::atan2(ddy, ddx);
         path.push_back(st);
+        if (path.size() == kStrokePart) run();
       }
     }
-    if (path.empty()) return;
-    // the imprints as one planned list; the dirty bytes are begun anew (all
-    // set) and not kept past it, as after single imprints
-    cv->epoch++;
-    b->dirty_canvas = nullptr;
-    run_fused(b, cv, path.data(), (int64_t)path.size(), 1);
-    b->dirty_canvas = nullptr;
+    run();
     if (cv->ctx->stream != b->ctx->stream) PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
   });
 }

@@ -123,6 +123,29 @@ def test_paint_stroke_placement(hip, oracle):
     compare_canvas("paintStroke", gcv, ocv, pickup=(gb, ob))
 
 
+def test_long_paint_stroke_equals_its_imprints(hip, oracle):
+    """A stroke of more imprints than one planned part holds (4096), doubling
+    back and along column 0, against the imprints one by one, to the bit."""
+    wl = _wl(40, 90, 5, 12)
+    path = [(0.4 + 80.0 * (k % 2) * (k // 8 % 2), 3.3 + (k * 7) % 30) for k in range(1, 130)]
+    st = oracle.stroke_stamps(path)
+    assert len(st) > 4200
+    out = []
+    for whole in (True, False):
+        gcv, _ = run_gpu(wl, _stamp_array([]))
+        gb = hip.FootprintBrush(wl.radii[0], wl.cores[0])
+        gb.dip(PA)
+        if whole:
+            gb.paintStroke(path, gcv)
+        else:
+            for cx, cy, th in st:
+                gb.imprint((cx, cy), th, gcv)
+        L = gcv.getPaintLayer()
+        out.append([L.getK_buffer(), L.getS_buffer(), L.getV_buffer()] + list(gb.getPickupMap()))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_brush_accessors(hip):
     core = W.gaussian_core(65, 16.0)
     b = hip.FootprintBrush(32.0, core)
