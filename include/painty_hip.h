@@ -265,10 +265,10 @@ int pnt_imprint_stamps(pnt_brush brush, pnt_canvas canvas,
  * memory -- code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc: the same stamps and results as
  * pnt_imprint_stamps(PNT_EXEC_FUSED) (stamps in stream order on the brush's
- * own pickup map), with the stamp plan in a fixed 4 MiB device array of the
- * library instead of library-allocated buffers; the call allocates no device
- * or pinned memory.  Limits: at most 24576 stamps per call (and 1 MiB of
- * shared-pixel visit lists), else PNT_EINVAL.  The brush's snapshot buffers
+ * own pickup map), with the plan's shared-pixel visit lists in a fixed 1 MiB
+ * device array of the library instead of library-allocated buffers; the call
+ * allocates no device or pinned memory.  Limits: at most 24576 stamps per call
+ * and lists that fit the array, else PNT_EINVAL.  The brush's snapshot buffers
  * must already fit the canvas (a previous stamp call on a canvas at least as
  * large, or pnt_brush_update_snapshot), else PNT_EINVAL; so is a canvas
  * with a drying clock (pnt_canvas_set_clock).  Returns once the

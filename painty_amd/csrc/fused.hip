@@ -675,7 +675,7 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
 
 void run_fused_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, int chains,
                  TapeRun* tape) {
-  const PlanDev D = upload_plan(b, cv, st, n);
+  const PlanDev D = upload_plan(b, cv, st, n, false);  // a stamp's plan goes with its launch
   const std::vector<ListGeo> geos{ListGeo{b->fp, b->size_map, b->radius, nullptr, b->width,
                                           FpBox{b->fbox[0], b->fbox[1], b->fbox[2], b->fbox[3]}}};
   run_fused_list(b, cv, st, n, D, geos, std::vector<int>((size_t)n, 0),
@@ -752,7 +752,7 @@ void run_fused_strokes_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stroke* S, 
         if (e) std::rethrow_exception(e);
     };
     const PlanDev D =
-        upload_plan_parts(b, cv, parts.data(), (int)parts.size(), fp_floats, fill, &d_fp);
+        upload_plan_parts(b, cv, parts.data(), (int)parts.size(), fp_floats, fill, &d_fp, false);
     for (size_t g = 1; g < geos.size(); ++g) geos[g].fp = d_fp + fp_off[g];
     run_fused_list(b, cv, all.data(), n, D, geos, geo, clear, 0);
   }
@@ -937,7 +937,7 @@ static void run_chained_t(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st,
   hipStream_t s = b->ctx->stream;
   if (*(volatile unsigned*)b->ctx->kernel_error)
     throw Error(PNT_EKERNEL, "an earlier stamp kernel aborted");
-  const PlanDev D = upload_plan(b, cv, st, n);
+  const PlanDev D = upload_plan(b, cv, st, n, true);
   FArgs F;
   F.st = D.st;
   F.canvas = cv->layer();
@@ -1072,14 +1072,14 @@ void run_chained(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t 
 
 // ------------------------------------------------------ no-allocation call --
 // pnt_imprint_stamps_noalloc: the stamps of a list in stream order on the
-// brush's own pickup map (PNT_EXEC_FUSED, one chain), with the plan -- the
-// stamp descriptors and shared-pixel visit lists the kernels read -- in a
-// file-scope device array instead of library-allocated buffers, so the call
-// allocates no device or pinned memory.  Each GPU holds its own copy of the
-// array; its address is looked up once per device with hipGetSymbolAddress
-// and kept here, and only that address is handed to kernels and copies.
-constexpr int64_t kScratchBytes = 4 << 20;
-constexpr int64_t kScratchStampBytes = 3 << 20;  // stamp descriptors; visit lists after
+// brush's own pickup map (PNT_EXEC_FUSED, one chain).  A stamp's plan goes with
+// its launch; the shared-pixel visit lists are in a file-scope device array
+// instead of library-allocated buffers, so the call allocates no device or
+// pinned memory.  Each GPU holds its own copy of the array; its address is
+// looked up once per device with hipGetSymbolAddress and kept here, and only
+// that address is handed to kernels and copies.
+constexpr int64_t kScratchBytes = 1 << 20;
+constexpr int64_t kNoallocStamps = 24576;  // a call's limit, part of the interface
 __device__ __align__(256) char scratch[kScratchBytes];
 
 namespace {
@@ -1111,12 +1111,11 @@ void run_fused_noalloc(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, in
   h_dl.clear();
   h_off.clear();
   plan_stamps(b, cv, st, n, h_st, h_dl, h_off);
-  const int64_t bst = (int64_t)(h_st.size() * sizeof(PStamp));
   const int64_t bdl = (int64_t)(h_dl.size() * sizeof(int2));
   const int64_t boff = (int64_t)(h_off.size() * sizeof(int));
-  PNT_REQUIRE(bst <= kScratchStampBytes,
+  PNT_REQUIRE(n <= kNoallocStamps,
               "stamp list too long for the no-allocation call (at most 24576 stamps)");
-  PNT_REQUIRE(round_up(bdl, 256) + boff <= kScratchBytes - kScratchStampBytes,
+  PNT_REQUIRE(round_up(bdl, 256) + boff <= kScratchBytes,
               "shared-pixel visit lists too long for the no-allocation call");
   // the brush's snapshot and dirty bytes must already fit this canvas
   if (b->use_snap) {
@@ -1126,10 +1125,9 @@ void run_fused_noalloc(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, in
                 "call); stamp this canvas once with pnt_imprint_stamps first");
     brush_prepare_snapshot(b, cv, s);  // copies or marks; allocates nothing at these sizes
   }
-  // the plan into the array, then the kernels read it (the copy is waited for
-  // before returning control of the host buffers)
-  if (bst) PNT_HIP_CHECK(hipMemcpyAsync(dev, h_st.data(), (size_t)bst, hipMemcpyHostToDevice, s));
-  char* ldl = dev + kScratchStampBytes;
+  // the lists into the array, then the kernels read them (the copy is waited
+  // for before returning control of the host buffers)
+  char* ldl = dev;
   char* loff = ldl + round_up(bdl, 256);
   if (bdl) PNT_HIP_CHECK(hipMemcpyAsync(ldl, h_dl.data(), (size_t)bdl, hipMemcpyHostToDevice, s));
   if (boff)

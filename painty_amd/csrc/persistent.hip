@@ -468,14 +468,15 @@ static PersistentState& plan_state(pnt_brush_s* b) {
 // Plans stamps [0, n) on the host, readies the snapshot and dirty bytes,
 // and uploads the plan through pinned staging.  The host copy of the plan
 // stays in the brush's state until the next call.
-PlanDev upload_plan(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n) {
+PlanDev upload_plan(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n,
+                    bool stamps) {
   const PlanPart part{b->size_map, b->radius, st, n};
-  return upload_plan_parts(b, cv, &part, 1, 0, nullptr, nullptr);
+  return upload_plan_parts(b, cv, &part, 1, 0, nullptr, nullptr, stamps);
 }
 
 PlanDev upload_plan_parts(pnt_brush_s* b, pnt_canvas_s* cv, const PlanPart* parts, int np,
                           int64_t fp_floats, const std::function<void(float*)>& fill_fp,
-                          const float** d_fp) {
+                          const float** d_fp, bool stamps) {
   hipStream_t s = b->ctx->stream;
   PersistentState& P = plan_state(b);
   P.h_st.clear();
@@ -504,7 +505,7 @@ PlanDev upload_plan_parts(pnt_brush_s* b, pnt_canvas_s* cv, const PlanPart* part
     }
   }
   brush_prepare_snapshot(b, cv, s);
-  const size_t bst = P.h_st.size() * sizeof(PStamp);
+  const size_t bst = stamps ? P.h_st.size() * sizeof(PStamp) : 0;
   const size_t bdl = P.h_dl.size() * sizeof(int2);
   const size_t boff = P.h_off.size() * sizeof(int);
   const size_t bfp = (size_t)fp_floats * sizeof(float);
@@ -518,15 +519,15 @@ PlanDev upload_plan_parts(pnt_brush_s* b, pnt_canvas_s* cv, const PlanPart* part
     PNT_HIP_CHECK(hipHostMalloc((void**)&P.stage, (size_t)c));
     P.stage_cap = c;
   }
-  std::memcpy(P.stage, P.h_st.data(), bst);
+  if (bst) std::memcpy(P.stage, P.h_st.data(), bst);
   if (bdl) std::memcpy(P.stage + bst, P.h_dl.data(), bdl);
   if (boff) std::memcpy(P.stage + bst + bdl, P.h_off.data(), boff);
   if (bfp) fill_fp(reinterpret_cast<float*>(P.stage + bst + bdl + boff));
-  const int64_t n = (int64_t)P.h_st.size();
-  ensure_dev(P.d_st, P.st_cap, std::max<int64_t>(n, 1), s);
+  if (stamps) ensure_dev(P.d_st, P.st_cap, std::max<int64_t>((int64_t)P.h_st.size(), 1), s);
   ensure_dev(P.d_dl, P.dl_cap, std::max<int64_t>((int64_t)P.h_dl.size(), 1), s);
   ensure_dev(P.d_off, P.off_cap, std::max<int64_t>((int64_t)P.h_off.size(), 1), s);
-  PNT_HIP_CHECK(hipMemcpyAsync(P.d_st, P.stage, bst, hipMemcpyHostToDevice, s));
+  if (bst)
+    PNT_HIP_CHECK(hipMemcpyAsync(P.d_st, P.stage, bst, hipMemcpyHostToDevice, s));
   if (bdl)
     PNT_HIP_CHECK(hipMemcpyAsync(P.d_dl, P.stage + bst, bdl, hipMemcpyHostToDevice, s));
   if (boff)
@@ -538,7 +539,7 @@ PlanDev upload_plan_parts(pnt_brush_s* b, pnt_canvas_s* cv, const PlanPart* part
   }
   if (d_fp) *d_fp = P.d_fp;
   PNT_HIP_CHECK(hipEventRecord(P.uploaded, s));
-  return PlanDev{P.d_st,          P.d_dl, P.d_off, P.h_st.data(), P.h_off.data(),
+  return PlanDev{stamps ? P.d_st : nullptr, P.d_dl, P.d_off, P.h_st.data(), P.h_off.data(),
                  (int64_t)P.h_dl.size(), (int64_t)P.h_off.size()};
 }
 
@@ -571,7 +572,7 @@ void run_persistent(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
     throw Error(PNT_ESTATE, "brush map of " + std::to_string(b->size_map) +
                                 " cells per side needs more co-resident workgroups than the "
                                 "device holds; use PNT_EXEC_PLAIN");
-  upload_plan(b, cv, st, n);
+  upload_plan(b, cv, st, n, true);
 
   PArgs A;
   A.hr = (b->size_map - 1) / 2;

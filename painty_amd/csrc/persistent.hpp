@@ -30,7 +30,9 @@ struct PlanDev {
   const int* host_off;  // host copy of dl_off
   int64_t n_dl, n_off;  // entries of dl, dl_off
 };
-PlanDev upload_plan(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n);
+// stamps: with the descriptors (PlanDev::st), for kernels that run a list in one
+// launch; the others take a stamp's plan with its launch.
+PlanDev upload_plan(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64_t n, bool stamps);
 // A list cut into parts that each have their own brush geometry (padded
 // footprint side, radius).  The footprints of the list's geometries
 // (fp_floats floats) travel with the plan, to *d_fp: fill_fp writes them
@@ -43,7 +45,7 @@ struct PlanPart {
 };
 PlanDev upload_plan_parts(pnt_brush_s* b, pnt_canvas_s* cv, const PlanPart* parts, int np,
                           int64_t fp_floats, const std::function<void(float*)>& fill_fp,
-                          const float** d_fp);
+                          const float** d_fp, bool stamps);
 
 // A run of stamps of one stroke (from a dip to the next dip) within one
 // drying phase, and the earlier units of its phase whose snapshot boxes meet
