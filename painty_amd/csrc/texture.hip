@@ -52,9 +52,13 @@ constexpr int kBlock = 256;
 // 64-thread workgroups spread a step over four times the CUs (6.7 against
 // 7.3 us per launch at radius 40).
 constexpr int kStepBlock = 64;
-// Maps up to this side go several steps a launch: the blocks then fit the
-// device at once.
-constexpr int kSmudgeMost = 128;
+// Maps up to this side go several steps a launch.  A block takes a CU's LDS, so
+// a launch of ten steps runs in rounds of 256 blocks of 8 x 8 cells: 26 us for
+// one (up to side 128), 40 for two, more where a step's region grows.  Measured
+// us a step on a curved stroke, several a launch against one a launch: side 130
+// 4.0 and 7.1, 160 4.6 and 7.4, 200 6.4 and 8.2, 250 9.0 and 9.4, 260 10.4 and 9.6,
+// 360 16.9 and 11.3: the line lies where four rounds are full.
+constexpr int kSmudgeMost = 256;
 constexpr double kPi = 3.141592653589793238462643383279502884;  // Math.hxx:21-22
 
 __host__ __device__ __forceinline__ int reflect_index(int p, int len) {

@@ -165,8 +165,9 @@ def test_short_stroke_and_errors(hip, oracle):
     compare_canvas("texture/no-op", gc, oc)
 
 
-# Maps of less than one tile, of whole tiles, of a tile and a bit, and past the
-# side that goes one step a launch; hairpins turn the map too far for a region.
+# Maps of less than one tile, of whole tiles, of a tile and a bit, and of more
+# blocks than a round of the device holds; hairpins turn the map too far for a
+# region.
 @pytest.mark.parametrize("radius", [1.5, 4.0, 12.3, 40.0, 70.0])
 @pytest.mark.parametrize("path", ["diagonal", "hairpin", "wave"])
 def test_smudge_over_map_sizes_and_turns(hip, oracle, radius, path):
@@ -187,7 +188,7 @@ def test_smudge_over_map_sizes_and_turns(hip, oracle, radius, path):
 # is evaluated as the reference writes it, so canvas and map volumes are the
 # oracle's to the bit -- blocked steps, single ones (radius 70), sharp turns.
 # The canvas' volumes lie near the threshold in part.
-@pytest.mark.parametrize("radius", [5.6, 12.3, 70.0])
+@pytest.mark.parametrize("radius", [5.6, 12.3, 70.0, 128.0, 129.0])
 def test_smudge_volumes_are_the_oracles(hip, oracle, radius):
     rows, cols = 150, 190
     oc, gc = _canvases(hip, oracle, rows, cols, 3)
