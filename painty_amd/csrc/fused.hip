@@ -112,7 +112,6 @@ struct WArgs {
   StampShared sh;
   WSlot slot[kSlots];
 };
-constexpr int kWaveSlots = 8;
 static_assert(sizeof(WArgs<kWaveSlots>) <= 4000, "wave arguments must fit the kernel argument segment");
 
 // Slot y of the grid's rows, blocks along x: a block knows its slot without
@@ -577,6 +576,7 @@ void run_fused_list(pnt_brush_s* b, pnt_canvas_s* cv, const pnt_stamp* st, int64
   if (nchains > 1 || !one_geo || tape) U = plan_units(st, D.host, clear.data(), n, nchains);
   int used = 1;
   for (const Unit& u : U) used = std::max(used, u.chain + 1);
+  if (tape) tape->chains = used;
   if (used <= 1 && one_geo && !tape) {  // one chain, the brush's own map: the list in stream order
     for (int64_t k = 0; k < n; ++k) {
       launch_stamp(k, s, b->pick);

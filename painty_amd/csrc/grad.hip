@@ -56,7 +56,7 @@ namespace {
 
 constexpr int kGT = 16;  // window tile of the adjoint kernel
 constexpr int kBlk = 256;
-constexpr int kAdjSlots = 8;          // stamps of one adjoint launch (a wave of the forward)
+constexpr int kAdjSlots = kWaveSlots;  // stamps of one adjoint launch (a wave of the forward)
 constexpr int64_t kTapeFree = 8;      // tapes take at most 1/8 of the free memory,
 constexpr int64_t kTapeMost = 16ll << 30;  // and 16 GiB
 
@@ -745,7 +745,7 @@ struct pnt_grad_s {
   float* gX = nullptr;  // 7 planes of round_up(n, 64) (snapshot adjoint)
   uint8_t* gdirty = nullptr;  // its dirty bytes
   bool adj_zero = false;  // both are zero: a backward that runs to its end leaves them so
-  float* gP = nullptr;  // per chain: m cells (pickup adjoint)
+  float* gP = nullptr;  // per chain of the waves: m cells (pickup adjoint)
   float* gB = nullptr;  // n_stamps x 6
   int64_t gX_cap = 0, gdirty_cap = 0, gP_cap = 0, gB_cap = 0;
   float* scratch = nullptr;
@@ -1199,9 +1199,11 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
       }
       g->adj_zero = false;
     }
-    ensure(g->gP, g->gP_cap, kAdjSlots * kCell * m, s);
+    // a map adjoint per chain; a segment is one stroke's stamps, one chain
+    const int64_t gp_floats = (g->full_tape ? g->run.chains : 1) * kCell * m;
+    ensure(g->gP, g->gP_cap, gp_floats, s);
     ensure(g->gB, g->gB_cap, 6 * (int64_t)ns, s);
-    launch_fill(g->gP, kAdjSlots * kCell * m, 0.0f, s);
+    launch_fill(g->gP, gp_floats, 0.0f, s);
     launch_fill(g->gB, 6 * (int64_t)ns, 0.0f, s);
     const Plane7 gXL = b->use_snap ? dense7(g->gX, nst) : gC;
     if (g->full_tape) {
@@ -1212,6 +1214,7 @@ int pnt_grad_backward(pnt_grad g, pnt_dev_rgb gR, pnt_dev_layer gwet, pnt_dev_rg
       g->canvas_final = false;
       for (int k = (int)g->segs.size() - 1; k >= 0; --k) {  // rerun onto the tape, then reversed
         rerun_segment(g, g->segs[(size_t)k], &g->run);
+        PNT_REQUIRE(g->run.chains == 1, "a segment on more than one chain");
         adjoint_waves(g, g->segs[(size_t)k].s0, gC, gXL, s);
       }
       cv->epoch++;

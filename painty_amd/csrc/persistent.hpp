@@ -77,6 +77,9 @@ void plan_stamps_rc(int size_map, double radius, int rows, int cols, const pnt_s
                     int64_t n, std::vector<PStamp>& h_st, std::vector<int2>& h_dl,
                     std::vector<int>& h_off);
 
+// Phases of one wave of a stamp list, at most (fused.hip, grad.hip).
+constexpr int kWaveSlots = 8;
+
 // The tape of a stamp list's visits, for its adjoint (grad.hip): what every
 // visit found, stamp k's record at base + k * slot (TapeRec, stampcore.hpp),
 // and the waves that ran the list.
@@ -87,6 +90,7 @@ struct TapeRun {
     int k, clear, chain;  // stamp k, or the clear of the chain's map before it
   };
   std::vector<std::vector<Phase>> waves;
+  int chains = 1;  // chains the waves use
   std::vector<PStamp> st;
   std::vector<int> n_visits;  // listed shared-pixel visits of each stamp
   const int2* dl = nullptr;  // the plan's lists (the brush's, until it plans again)

@@ -13,8 +13,10 @@
 //   again     a second backward of one forward begins with the final state: from
 //             checkpoints it reruns every segment before the composite's adjoint
 //   no-tape   a forward whose tape cannot be allocated keeps checkpoints
+//   maps      a map adjoint is held and cleared for each chain that the waves use
 #include "host_hip.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 #include "painty_hip.h"
@@ -44,12 +46,15 @@ struct Seen {
   int gX_filled, dirty_filled;  // clears of the whole adjoint planes / their dirty bytes
   int adj, adj_dirty_unset, adj_uncleared, stamps;
   int rate_old, rate_new, fp_old, fp_new;  // launches with either's value
+  int64_t map_floats;  // the largest clear of whole map adjoints
   int box_early;  // checkpoint copies beside copies queued on another stream
   std::string order;  // 'k' composite adjoint, 's' stamps, 'a' adjoint wave
 } seen;
 
 static void on_launch(const std::string& name, void** args) {
   const auto is = [&](const char* k) { return name.find(k) != std::string::npos; };
+  if (is("6k_fillE") && *(int64_t*)args[1] % (8 * kSide * kSide) == 0)
+    seen.map_floats = std::max(seen.map_floats, *(int64_t*)args[1]);
   if (is("9k_fill_u8") && *(int64_t*)args[1] == kStride + 16) ++seen.dirty_filled;
   if (is("6k_fillE") && *(int64_t*)args[1] == 7 * kStride) ++seen.gX_filled;
   if (is("k_stamp_wave")) ++seen.stamps, seen.order += 's';
@@ -97,7 +102,7 @@ struct Runner {
     if (st) std::fprintf(stderr, "status %d: %s\n", st, pnt_last_error()), std::abort();
     return st;
   }
-  explicit Runner(bool other_ctx = false) {
+  explicit Runner(bool other_ctx = false, int strokes = 3) {
     ok(pnt_ctx_create(0, &ctx));
     bctx = ctx;
     if (other_ctx) ok(pnt_ctx_create(0, &bctx));
@@ -110,9 +115,9 @@ struct Runner {
       s.cx = i < 16 ? 20.3 + i : 1.4 + 0.7 * (i - 16);
       s.cy = i < 8 ? 30.2 : 2.6 + 0.3 * (i - 8);
       s.theta = 0.2 * i;
-      s.flags = i % 8 == 0 ? PNT_STAMP_DIP : 0;
+      s.flags = i % (24 / strokes) == 0 ? PNT_STAMP_DIP : 0;
       st.push_back(s);
-      paint_of.push_back(i % 8 == 0 ? 0 : -1);
+      paint_of.push_back(s.flags ? 0 : -1);
     }
     const double palK[6] = {.1, .2, .3, .4, .5, .6}, palS[6] = {.6, .5, .4, .3, .2, .1};
     ok(pnt_grad_create(ctx, kRows, kCols, b, st.data(), (int64_t)st.size(), paint_of.data(), 2, palK,
@@ -241,6 +246,22 @@ static void check_again() {
   }
 }
 
+static void check_maps() {
+  for (const char* mode : {"0", "64"}) {
+    setenv("PAINTY_GRAD_TAPE_MB", mode, 1);
+    Runner one(false, 1);
+    Runner::ok(one.forward());
+    Runner::ok(one.backward());
+    CHECK(seen.map_floats == 8 * kSide * kSide, "tape %s: %lld floats of map adjoint for one stroke",
+          mode, (long long)seen.map_floats);
+  }
+  Runner far(false, 24);  // strokes of one stamp: several run at once
+  Runner::ok(far.forward());
+  Runner::ok(far.backward());
+  CHECK(seen.map_floats >= 16 * kSide * kSide && seen.map_floats <= 64 * kSide * kSide,
+        "%lld floats of map adjoint for many strokes", (long long)seen.map_floats);
+}
+
 static void check_no_tape() {
   unsetenv("PAINTY_GRAD_TAPE_MB");
   int refused = 0;
@@ -272,6 +293,8 @@ int main(int argc, char** argv) {
     check_again();
   else if (what == "no-tape")
     check_no_tape();
+  else if (what == "maps")
+    check_maps();
   else
     return 2;
   CHECK(state().hazards.empty(), "%s", state().hazards.empty() ? "" : state().hazards[0].c_str());

@@ -30,7 +30,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.skipif(not shutil.which("g++"), reason="needs a C++ compiler")
-@pytest.mark.parametrize("check", ["failures", "streams", "brush", "again", "no-tape"])
+@pytest.mark.parametrize("check", ["failures", "streams", "brush", "again", "no-tape", "maps"])
 def test_runner_state(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
