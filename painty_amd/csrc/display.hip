@@ -167,9 +167,9 @@ __device__ __forceinline__ double encode_fast(float xf, int to_srgb, double scal
 }
 
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_encode(int64_t p0, int64_t n, Rgb3 in, int to_srgb,
-                                                   double scale, T* out) {
-  const int64_t p = p0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
+__global__ __launch_bounds__(kBlock) void k_encode(int64_t n, Rgb3 in, int to_srgb, double scale,
+                                                   T* out) {
+  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (p >= n) return;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
@@ -182,13 +182,23 @@ __global__ __launch_bounds__(kBlock) void k_encode(int64_t p0, int64_t n, Rgb3 i
 
 // Four pixels a thread: 16-byte loads of the planes (a plane of odd size
 // leaves the next one on a 4-byte boundary, which these loads allow), and
-// their twelve values in three words.
+// their twelve values in three words.  The last n % 4 pixels go one a thread,
+// behind the fours (a launch of their own took 3 us more).
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_encode_vec(int64_t n4, Rgb3 in, int to_srgb,
+__global__ __launch_bounds__(kBlock) void k_encode_vec(int64_t n, Rgb3 in, int to_srgb,
                                                        double scale, T* out) {
   using Word = typename std::conditional<sizeof(T) == 1, uint32_t, uint64_t>::type;
-  const int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (q >= n4) return;
+  const int64_t q = (int64_t)blockIdx.x * kBlock + threadIdx.x, n4 = n / 4;
+  if (q >= n4) {
+    const int64_t p = 3 * n4 + q;
+    if (p < n)
+#pragma unroll 1
+      for (int c = 0; c < 3; ++c) {
+        const float* plane = c == 0 ? in.p[0] : (c == 1 ? in.p[1] : in.p[2]);
+        out[3 * p + c] = (T)encode_exact(plane[p], to_srgb, scale);
+      }
+    return;
+  }
   typedef float Float4 __attribute__((ext_vector_type(4), aligned(4)));
   Float4 v[3];
 #pragma unroll
@@ -217,17 +227,14 @@ __global__ __launch_bounds__(kBlock) void k_encode_vec(int64_t n4, Rgb3 in, int 
 
 inline unsigned blocks_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
-// The image word-aligned: four pixels a thread, the last n % 4 one a thread;
-// otherwise all one a thread (single-value stores).
+// The image word-aligned: four pixels a thread; otherwise one a thread
+// (single-value stores).
 template <class T>
 void launch_encode_t(int64_t n, const Rgb3& in, int to_srgb, double scale, T* out, hipStream_t s) {
-  int64_t done = 0;
-  if (((uintptr_t)out & (4 * sizeof(T) - 1)) == 0 && n >= 4) {
-    k_encode_vec<T><<<blocks_for(n / 4), kBlock, 0, s>>>(n / 4, in, to_srgb, scale, out);
-    done = n / 4 * 4;
-  }
-  if (done < n)
-    k_encode<T><<<blocks_for(n - done), kBlock, 0, s>>>(done, n, in, to_srgb, scale, out);
+  if (((uintptr_t)out & (4 * sizeof(T) - 1)) == 0)
+    k_encode_vec<T><<<blocks_for(n / 4 + n % 4), kBlock, 0, s>>>(n, in, to_srgb, scale, out);
+  else
+    k_encode<T><<<blocks_for(n), kBlock, 0, s>>>(n, in, to_srgb, scale, out);
   PNT_HIP_CHECK(hipGetLastError());
 }
 
