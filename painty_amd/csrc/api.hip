@@ -1413,6 +1413,8 @@ int pnt_brush_destroy(pnt_brush b) {
     ktimer_release(b->ktimer);
     dev_free(b->fp);
     dev_free(b->pick);
+    dev_free(b->unpack);
+    if (b->unpack_host) (void)hipHostFree(b->unpack_host);
     dev_free(b->snap);
     dev_free(b->d_list);
     dev_free(b->d_off);
@@ -1456,19 +1458,54 @@ int pnt_brush_get_pickup_map(pnt_brush b, float* K, float* S, float* V, int layo
     check_layout(layout);
     b->ctx->use();
     if (!K && !S && !V) return;
-    std::vector<float> cells((size_t)(kCell * b->m));
-    PNT_HIP_CHECK(hipMemcpyAsync(cells.data(), b->pick, cells.size() * sizeof(float),
-                                 hipMemcpyDeviceToHost, b->ctx->stream));
-    PNT_HIP_CHECK(hipStreamSynchronize(b->ctx->stream));
-    const bool planar = layout == PNT_PLANAR;
-    for (int64_t i = 0; i < b->m; ++i) {
-      const float* c = &cells[(size_t)(kCell * i)];
-      for (int k = 0; k < 3; ++k) {
-        const int64_t at = planar ? k * b->m + i : 3 * i + k;
-        if (K) K[at] = c[k];
-        if (S) S[at] = c[3 + k];
+    // unpacked by a kernel, kUnpack cells at a time, into what the caller asked
+    // for, K, then S, then V: small maps straight into pinned memory (a copy
+    // waits for the kernel by way of another queue, 14 us), others into device
+    // staging that is copied to the caller
+    constexpr int64_t kUnpack = 1 << 18, kDirect = 1 << 16;
+    hipStream_t s = b->ctx->stream;
+    float* const out[3] = {K, S, V};
+    const int nch[3] = {3, 3, 1};
+    int64_t total = 0;
+    for (int o = 0; o < 3; ++o) total += out[o] ? nch[o] * b->m : 0;
+    const bool direct = total <= kDirect;
+    if (direct && !b->unpack_host)
+      PNT_HIP_CHECK(hipHostMalloc((void**)&b->unpack_host, kDirect * sizeof(float), hipHostMallocMapped));
+    const int64_t need = direct ? 0 : 7 * std::min(b->m, kUnpack);
+    if (need > b->unpack_cap) {
+      dev_free(b->unpack);
+      b->unpack = nullptr;
+      b->unpack_cap = 0;
+      b->unpack = dev_alloc(need);
+      b->unpack_cap = need;
+    }
+    float* stage = b->unpack;
+    if (direct) PNT_HIP_CHECK(hipHostGetDevicePointer((void**)&stage, b->unpack_host, 0));
+    for (int64_t c0 = 0; c0 < b->m; c0 += kUnpack) {
+      const int64_t n = std::min(kUnpack, b->m - c0);
+      float* to[3];
+      int64_t at = 0;
+      for (int o = 0; o < 3; ++o) {
+        to[o] = out[o] ? stage + at : nullptr;
+        at += out[o] ? nch[o] * n : 0;
       }
-      if (V) V[i] = c[6];
+      launch_unpack_cells(n, b->pick + kCell * c0, to[0], to[1], to[2], layout == PNT_PLANAR, s);
+      if (direct) PNT_HIP_CHECK(hipStreamSynchronize(s));
+      const float* src = direct ? b->unpack_host : stage;
+      for (int o = 0; o < 3; ++o) {
+        if (!out[o]) continue;
+        const bool planes = layout == PNT_PLANAR && nch[o] > 1;  // each a piece of its plane
+        for (int c = 0; c < (planes ? nch[o] : 1); ++c) {
+          const int64_t len = planes ? n : nch[o] * n;
+          float* dst = out[o] + (planes ? c * b->m + c0 : nch[o] * c0);
+          if (direct)
+            std::memcpy(dst, src, (size_t)len * sizeof(float));
+          else
+            PNT_HIP_CHECK(hipMemcpyAsync(dst, src, (size_t)len * sizeof(float), hipMemcpyDeviceToHost, s));
+          src += len;
+        }
+      }
+      if (!direct) PNT_HIP_CHECK(hipStreamSynchronize(s));
     }
   });
 }

@@ -117,6 +117,11 @@ struct pnt_brush_s {
   uint64_t geo_gen = 0;        // bumped with every new footprint
   int fbox[4] = {0, 0, 1 << 30, 1 << 30};  // nonzero footprint cells: x0 y0 x1 y1
   float* pick = nullptr;       // pickup map: mstride cells of kCell floats
+  // staging of a pickup map's download: device, a part of the map at a time;
+  // pinned, a small map whole
+  float* unpack = nullptr;
+  int64_t unpack_cap = 0;
+  float* unpack_host = nullptr;
   float* snap = nullptr;       // snapshot: a layer (8 strides of snap_stride)
   int snap_rows = 0, snap_cols = 0;
   int64_t snap_stride = 0, snap_cap = 0;  // floats allocated at snap

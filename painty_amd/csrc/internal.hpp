@@ -163,6 +163,10 @@ void launch_copy_layer(int64_t n, const Layer7& src, const Layer7& dst, hipStrea
 // A layer from seven FP32 planes (V widened exactly), and back (V rounded).
 void launch_layer_from_planes(int64_t n, const Plane7& src, const Layer7& dst, hipStream_t s);
 void launch_planes_from_layer(int64_t n, const Layer7& src, const Plane7& dst, hipStream_t s);
+// n pickup cells into K and S (three values a cell: planes of n, or together)
+// and V; a null destination is left out.
+void launch_unpack_cells(int64_t n, const float* cells, float* K, float* S, float* V, bool planar,
+                         hipStream_t s);
 
 RingBox ring_box(const StampGeom& g, double radius);
 

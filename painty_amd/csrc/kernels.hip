@@ -294,6 +294,23 @@ __global__ __launch_bounds__(kBlock) void k_planes_from_layer(int64_t n, Layer7 
   dst.p[6][i] = (float)src.v[i];
 }
 
+// One cell a thread; bound by the copy to the host that follows.
+__global__ __launch_bounds__(kBlock) void k_unpack_cells(int64_t n, const float* cells, float* K,
+                                                         float* S, float* V, int planar) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const float4* p = reinterpret_cast<const float4*>(cells) + 2 * i;
+  const float4 a = p[0], b = p[1];
+  const float k[3] = {a.x, a.y, a.z}, q[3] = {a.w, b.x, b.y};
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const int64_t at = planar ? c * n + i : 3 * i + c;
+    if (K) K[at] = k[c];
+    if (S) S[at] = q[c];
+  }
+  if (V) V[i] = b.z;
+}
+
 // Canvas::checkDry of one pixel, called directly (Canvas.hxx:123-155).
 __global__ __launch_bounds__(64) void k_check_dry_pixel(DryClock c, Layer7 canvas, int64_t ic) {
   if (threadIdx.x == 0) check_dry(c, canvas, ic);
@@ -387,6 +404,13 @@ void launch_dry_steps(int64_t n, const Layer7& L, const Rgb3& R0, float portion,
 void launch_fill(float* p, int64_t n, float v, hipStream_t s) {
   if (n <= 0) return;
   k_fill<<<blocks_for(n), kBlock, 0, s>>>(p, n, v);
+  PNT_HIP_CHECK(hipGetLastError());
+}
+
+void launch_unpack_cells(int64_t n, const float* cells, float* K, float* S, float* V, bool planar,
+                         hipStream_t s) {
+  if (n <= 0) return;
+  k_unpack_cells<<<blocks_for(n), kBlock, 0, s>>>(n, cells, K, S, V, planar ? 1 : 0);
   PNT_HIP_CHECK(hipGetLastError());
 }
 

@@ -7,11 +7,13 @@ twice); stamps partly or fully off the canvas; snapshot on and off; pickup on
 and off; re-dips; per-stroke footprint sizes (setRadius); drying between
 stamps; paintStroke placement.  Tolerance 1e-5 relative per channel.
 """
+import ctypes as C
 import math
 
 import numpy as np
 import pytest
 
+from painty_amd import _lib
 from painty_amd import workload as W
 from tests.parity import assert_close, compare_canvas, run_gpu, run_oracle
 
@@ -166,3 +168,24 @@ def test_brush_accessors(hip):
     assert b.sizeMap == 92
     b.setRadius(16.0, W.gaussian_core(33, 8.0))
     assert b.sizeMap == 47
+
+
+@pytest.mark.parametrize("radius", [3, 190])  # one part of the download; two
+def test_pickup_map_layouts(hip, oracle, radius):
+    """The pickup map together and as planes, whole and in part, the oracle's."""
+    wl = _wl(60, 70, radius, 5, pickup=True)
+    st = _stamp_array([(31.3, 30.2, 0.4, PA, 0)])
+    ocv, ob = run_oracle(wl, st)
+    gcv, gb = run_gpu(wl, st)
+    compare_canvas("pickup/r%d" % radius, gcv, ocv, pickup=(gb, ob))
+    K, S, V = gb.getPickupMap()
+    m = V.shape[0]
+    planes = np.empty((3, m, m), np.float32)
+    only = np.empty((m, m), np.float32)
+    ptr = lambda a: a.ctypes.data_as(C.POINTER(C.c_float))
+    _lib.call("pnt_brush_get_pickup_map", gb.h, None, ptr(planes), None, _lib.PLANAR)
+    np.testing.assert_array_equal(planes.transpose(1, 2, 0), S)
+    _lib.call("pnt_brush_get_pickup_map", gb.h, ptr(planes), None, ptr(only), _lib.PLANAR)
+    np.testing.assert_array_equal(planes.transpose(1, 2, 0), K)
+    np.testing.assert_array_equal(only, V)
+    assert (V > 0).any()
