@@ -1881,6 +1881,27 @@ int pnt_batch_graph_destroy(pnt_batch_graph g) {
   });
 }
 
+// A mouse stroke's imprints one by one (one launch each, the ring copied
+// whole) or as a planned list (one launch each, the ring by dirty bytes, behind
+// the plan's upload and the setting of every dirty byte: 16 us or so)?
+//   - An edge stamp on its own uploads its shared-pixel lists and waits, 25 us;
+//     a stroke with one goes as a list.
+//   - The ring copied whole costs nothing that shows up to about 65,000 pixels
+//     of ring (radius 64: 5.7 us an imprint either way) and 9 us per million
+//     pixels past that (radius 200: 13.2 against 8.9 us; radius 300: 27.8
+//     against 16.0), which the list's start outweighs for few imprints.
+// Strokes of 1, 2 and 4 imprints at radius 16 took 25, 31 and 43 us as lists, 10,
+// 19 and 38 with two launches an imprint.
+static bool stroke_one_by_one(pnt_brush b, pnt_canvas cv, const std::vector<pnt_stamp>& path) {
+  const int hr = (b->size_map - 1) / 2;
+  for (const pnt_stamp& st : path)
+    if (stamp_dup_axis(st.cx, hr) || stamp_dup_axis(st.cy, hr)) return false;
+  if (!b->use_snap) return true;
+  const double inner = b->size_map, outer = inner + 2.0 * b->radius;
+  const double ring = std::min(outer * outer - inner * inner, (double)cv->n);
+  return (double)path.size() * std::max(ring - 65536.0, 0.0) <= 2e6;
+}
+
 int pnt_paint_stroke(pnt_brush b, pnt_canvas cv, const double* p, int64_t n) {
   return guard([&] {
     check_same_ctx(b, cv);
@@ -1888,15 +1909,18 @@ int pnt_paint_stroke(pnt_brush b, pnt_canvas cv, const double* p, int64_t n) {
     b->ctx->use();
     canvas_tick(cv);
     if (cv->ctx->stream != b->ctx->stream) PNT_HIP_CHECK(hipStreamSynchronize(cv->ctx->stream));
-    // FootprintBrush.hxx:251-267: the imprints as planned lists of at most
-    // kStrokePart (a stroke may be of any length, and the plan is pinned memory
-    // that the brush keeps); the dirty bytes are begun anew (all set) and not
-    // kept past the stroke, as after single imprints
+    // FootprintBrush.hxx:251-267: the imprints one by one, or as planned lists,
+    // of at most kStrokePart (a stroke may be of any length, and the plan is
+    // pinned memory that the brush keeps); a list's dirty bytes are begun anew
+    // (all set) and not kept past the stroke, as after single imprints
     constexpr size_t kStrokePart = 4096;
     std::vector<pnt_stamp> path;
     const auto run = [&] {
       if (path.empty()) return;
-      run_fused(b, cv, path.data(), (int64_t)path.size(), 1);
+      if (stroke_one_by_one(b, cv, path))
+        for (const pnt_stamp& st : path) imprint_plain(b, cv, st.cx, st.cy, st.theta);
+      else
+        run_fused(b, cv, path.data(), (int64_t)path.size(), 1);
       path.clear();
     };
     const struct Forget {

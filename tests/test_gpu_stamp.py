@@ -125,17 +125,31 @@ def test_paint_stroke_placement(hip, oracle):
     compare_canvas("paintStroke", gcv, ocv, pickup=(gb, ob))
 
 
-def test_long_paint_stroke_equals_its_imprints(hip, oracle):
-    """A stroke of more imprints than one planned part holds (4096), doubling
-    back and along column 0, against the imprints one by one, to the bit."""
-    wl = _wl(40, 90, 5, 12)
-    path = [(0.4 + 80.0 * (k % 2) * (k // 8 % 2), 3.3 + (k * 7) % 30) for k in range(1, 130)]
+def _zigzag(n):
+    """Doubling back and along column 0, more imprints than one planned part
+    holds (4096)."""
+    return [(0.4 + 80.0 * (k % 2) * (k // 8 % 2), 3.3 + (k * 7) % 30) for k in range(1, n)]
+
+
+@pytest.mark.parametrize("rows,cols,radius,snap,path", [
+    (40, 90, 5, True, _zigzag(130)),                                    # planned, in two parts
+    (60, 90, 5, True, [(30.2, 20.1), (41.0, 30.7), (50.3, 22.2)]),      # one by one
+    (60, 90, 5, True, [(30.2, 20.1), (30.9, 20.9)]),                    # a single imprint
+    (60, 90, 5, False, [(-3.2, 20.1), (2.4, 30.7), (50.3, 22.2)]),      # over the edge, no snapshot
+    (700, 720, 150, True, [(330.2, 320.1), (350.3, 341.3)]),            # a wide ring: planned
+    (700, 720, 150, True, [(330.2, 320.1), (332.3, 321.3)]),            # few imprints: one by one
+])
+def test_paint_stroke_equals_its_imprints(hip, oracle, rows, cols, radius, snap, path):
+    """Both ways a stroke goes -- imprints one by one, planned parts -- against
+    the imprints by themselves, to the bit."""
+    wl = _wl(rows, cols, radius, 12)
     st = oracle.stroke_stamps(path)
-    assert len(st) > 4200
+    assert len(st) > (4200 if len(path) > 100 else 0)
     out = []
     for whole in (True, False):
         gcv, _ = run_gpu(wl, _stamp_array([]))
         gb = hip.FootprintBrush(wl.radii[0], wl.cores[0])
+        gb.setUseSnapshotBuffer(snap)
         gb.dip(PA)
         if whole:
             gb.paintStroke(path, gcv)
