@@ -25,7 +25,7 @@
 // visit of a shared cell on its own thread, no tiles outside the rotated
 // footprint.  Per wave on 200 stamps of radius 32 on 1024^2: 13,500 cycles
 // before, 8,900 after; 2000 stamps of radius 64 to 96 on 4096^2, 743 launches:
-// 14.7 to 11.3 ms, the pickup map's cells (kCell) and the plan included.  A
+// 13.8 to 10.6 ms, the pickup map's cells (kCell) and the plan included.  A
 // launch there moves 20 MB through the infinity cache, the least that separate
 // launches can; more waves per SIMD change nothing.
 #include <algorithm>

@@ -36,7 +36,7 @@ def _planes(*tensors):
 
 
 class GradRunner(_lib.Owned):
-    """One differentiable stamp list (pnt_grad).  Holds the checkpoints of its
+    """One differentiable stamp list (pnt_grad).  Holds the tape or checkpoints of its
     last forward; backward applies to that forward."""
 
     _kind, _destroy = "grad", "pnt_grad_destroy"
