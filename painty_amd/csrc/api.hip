@@ -1915,20 +1915,28 @@ int pnt_paint_stroke(pnt_brush b, pnt_canvas cv, const double* p, int64_t n) {
     // (all set) and not kept past the stroke, as after single imprints
     constexpr size_t kStrokePart = 4096;
     std::vector<pnt_stamp> path;
+    struct Listed {  // lists ran, and their dirty bytes hold
+      pnt_brush b;
+      bool on = false;
+      ~Listed() {
+        if (on) b->dirty_canvas = nullptr;
+      }
+    } listed{b};
     const auto run = [&] {
       if (path.empty()) return;
-      if (stroke_one_by_one(b, cv, path))
+      if (stroke_one_by_one(b, cv, path)) {
+        listed.on = false;  // a single imprint forgets the dirty bytes
         for (const pnt_stamp& st : path) imprint_plain(b, cv, st.cx, st.cy, st.theta);
-      else
+      } else {
+        if (!listed.on) {
+          cv->epoch++;
+          b->dirty_canvas = nullptr;
+        }
+        listed.on = true;
         run_fused(b, cv, path.data(), (int64_t)path.size(), 1);
+      }
       path.clear();
     };
-    const struct Forget {
-      pnt_brush b;
-      ~Forget() { b->dirty_canvas = nullptr; }
-    } forget{b};
-    cv->epoch++;
-    b->dirty_canvas = nullptr;
     for (int64_t i = 0; i + 1 < n; ++i) {
       const int64_t ipre = i > 0 ? i - 1 : 0;
       const int64_t inext = (i + 2 < n) ? i + 2 : n - 1;

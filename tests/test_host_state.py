@@ -1,7 +1,8 @@
 """Host code of the library on a stand-in for the HIP runtime
 (tests/cpp/host_hip.hpp): what the gradient runner keeps from one call to the
 next, when an allocation fails, and on which stream it copies
-(grad_state.cpp); what a brush holds for a long stroke (stroke_state.cpp).  No
+(grad_state.cpp); what a brush holds for a long stroke and keeps past
+an empty one (stroke_state.cpp).  No
 device is used."""
 import os
 import shutil
@@ -38,7 +39,7 @@ def test_runner_state(program, check):
 
 
 @pytest.mark.skipif(not shutil.which("g++"), reason="needs a C++ compiler")
-def test_a_long_stroke_holds_no_more_memory(tmp_path):
+def test_what_a_stroke_leaves_with_the_brush(tmp_path):
     r = subprocess.run([build(tmp_path, "stroke_state")], capture_output=True, text=True,
                        timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
